@@ -3,16 +3,17 @@
 //
 // Work unit: a tile of 32 output rows per wavefront.  For each filter offset k the wavefront
 // looks up the 32 input rows (neighbour map), skips the offset when none exists, otherwise
-// gathers the rows straight from HBM/L2 into registers (two lanes per row, 64 contiguous
-// bytes each) and multiplies them with W[k] on the matrix cores (v_mfma_f32_32x32x2_f32,
-// fp32 in, fp32 accumulate).  Accumulators stay in registers for all offsets, so every
-// output row is written exactly once and no atomics are needed: the result of a row does
-// not depend on which other rows share its tile, nor on the launch shape.
+// gathers the rows straight from HBM/L2 into registers (two lanes per row) and multiplies them with W[k]
+// on the matrix cores: fp32 operands in three bf16 parts each, fp32 accumulate (see "fp32 products on the
+// bf16 matrix cores").  Accumulators stay in registers for all offsets, so every output row is written
+// exactly once and no atomics are needed: the result of a row does not depend on which other rows share
+// its tile, nor on the launch shape.
 #include <algorithm>
 
 #include "common.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace insc {
 
@@ -143,13 +144,97 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
 }
 
 // ---------------------------------------------------------------------------------------
-// Weight packing.  For filter offset k, input-channel chunk ch (32 channels) and
-// output-channel block nb (32 channels), lane = h*32 + j of the MFMA kernel needs the 16
-// B-operand values W[k][ch*32 + h*16 + s][nb*32 + j], s = 0..15.  The 4 KB tile is stored as
-// four 1 KB quarters; quarter q holds, for lane 0..63 in turn, the values s = 4q..4q+3.  One
-// 16-byte load per lane then reads a quarter fully coalesced.  Channels beyond Cin / Cout
-// are zero.
+// fp32 products on the bf16 matrix cores.  A float is the exact sum of three bf16 numbers of eight
+// significant bits each (x = x0 + x1 + x2, |x1| < 2^-7 |x0|, |x2| < 2^-7 |x1|), so a product of two floats is
+// nine products of bf16 numbers, each exact in fp32; the three smallest (x1 y2, x2 y1, x2 y2, together at most
+// 2^-21 of the product, 2^-25 of it on average) are left out, the other six are summed in fp32.
+// Why: v_mfma_f32_32x32x16_bf16 does 16 times the operations per cycle of v_mfma_f32_32x32x2_f32, six
+// of them still 2.7 times.  Measured for 32x32x32 blocks in a loop, three wavefronts per SIMD: 436 ns a
+// block in fp32 (154 TFLOP/s), 213 ns as six bf16 products, 274 ns with the split of the gathered operand in
+// the loop (241 ns where two output blocks share it).  The rounding that counts is that of the running sum of the
+// leading products x0 y0; the others go into a sum of their own (struct Sum), so it is rounded once per 16 channels,
+// where the fp32 instruction rounds its sum eight times.  2-norm error against 64-bit sums, fp32 instruction -> here:
+// four layers of 32 channels on 500k sites 1.63e-7 -> 0.72e-7, of 64 channels 1.33e-7 -> 0.74e-7, of 128 channels on
+// 5k 1.35e-7 -> 0.77e-7; the seven-scale U-Net on 150k voxels 4.2e-7 -> 2.0e-7.  (All six into one sum: 1.85e-7,
+// 1.48e-7, 1.54e-7 and 4.4e-7 - more than the fp32 instruction's - because each of the six roundings is to the sum.)
+// The gathered operand is split by truncation (and, subtract, byte permute: 5.5 instructions a float; rounding
+// to nearest - convert, unpack, subtract - takes as many and measured 303 ns), the weights, once, by rounding
+// to nearest.  What has no such sum - infinities, NaN, sums that overflow in between - comes out as NaN or
+// infinity; those elements are summed again in plain fp32 (repair_sums), so an infinity stays one.
 // ---------------------------------------------------------------------------------------
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
+
+// 16 channels of one row (8 per half-wave) in three parts: the operand of one 32x32x16 instruction each
+struct Parts {
+  u32x4 p[3];
+};
+
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &p0, unsigned &p1, unsigned &p2) {
+  const unsigned ua = __float_as_uint(a), ub = __float_as_uint(b);
+  p0 = __builtin_amdgcn_perm(ub, ua, 0x07060302);  // the upper halves of both
+  const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
+  const unsigned va = __float_as_uint(ra), vb = __float_as_uint(rb);
+  p1 = __builtin_amdgcn_perm(vb, va, 0x07060302);
+  const float qa = ra - __uint_as_float(va & 0xFFFF0000u), qb = rb - __uint_as_float(vb & 0xFFFF0000u);
+  p2 = __builtin_amdgcn_perm(__float_as_uint(qb), __float_as_uint(qa), 0x07060302);
+}
+
+__device__ __forceinline__ Parts split8(const float4 &lo, const float4 &hi) {
+  const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  Parts s;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    unsigned a, b, c;
+    split_pair(x[2 * j], x[2 * j + 1], a, b, c);
+    s.p[0][j] = a;
+    s.p[1][j] = b;
+    s.p[2][j] = c;
+  }
+  return s;
+}
+
+__device__ __forceinline__ f16v mfma_bf16(const u32x4 &a, const u32x4 &b, f16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8v, a), __builtin_bit_cast(bf8v, b), c, 0, 0, 0);
+}
+
+// A running sum: the products of the leading parts, and apart from them all others, which are 2^-7 of these at most -
+// so the sum that carries the rounding error is rounded once per 16 channels.
+struct Sum {
+  f16v lead, rest;
+};
+__device__ __forceinline__ void sum_start(Sum &a, float bias) {
+#pragma unroll
+  for (int v = 0; v < 16; v++) {
+    a.lead[v] = bias;
+    a.rest[v] = 0.0f;
+  }
+}
+__device__ __forceinline__ f16v sum_of(const Sum &a) {
+  f16v t;
+#pragma unroll
+  for (int v = 0; v < 16; v++) t[v] = a.lead[v] + a.rest[v];
+  return t;
+}
+
+// acc += 16 channels
+__device__ __forceinline__ void mac16(const Parts &a, const Parts &b, Sum &acc) {
+  acc.rest = mfma_bf16(a.p[2], b.p[0], acc.rest);
+  acc.rest = mfma_bf16(a.p[1], b.p[1], acc.rest);
+  acc.rest = mfma_bf16(a.p[0], b.p[2], acc.rest);
+  acc.rest = mfma_bf16(a.p[1], b.p[0], acc.rest);
+  acc.rest = mfma_bf16(a.p[0], b.p[1], acc.rest);
+  acc.lead = mfma_bf16(a.p[0], b.p[0], acc.lead);
+}
+
+// ---------------------------------------------------------------------------------------
+// Weight packing.  For filter offset k, input-channel chunk ch (32 channels) and output-channel block nb (32
+// channels) the weight tile is six 1 KB pieces, one per half s of the chunk and bf16 part i (piece s * 3 + i):
+// lane = h*32 + j reads from it, with one 16-byte load, the eight values W[k][ch*32 + s*16 + h*8 + 0..7][nb*32 + j].
+// A chunk whose second half lies beyond Cin (Cin = 16, 48, ..) is read as its first three pieces only.  Channels
+// beyond Cin / Cout are zero.
+// ---------------------------------------------------------------------------------------
+constexpr int WT_BYTES = 6144;  // a weight tile
 __host__ __device__ static inline int conv_nch(int Cin) { return (Cin + 31) / 32; }
 static inline int conv_nb_per_group(int Cout) {
   const int nbt = (Cout + 31) / 32;
@@ -160,39 +245,109 @@ static inline int conv_nbt_padded(int Cout) {
   return (int)cdiv(nbt, nb) * nb;
 }
 
+// the upper half of a float, rounded to nearest even unless that overflows (an infinity or NaN: as it is)
+__device__ __forceinline__ unsigned bf16_part(float x) {
+  const unsigned u = __float_as_uint(x);
+  if ((u & 0x7F800000u) == 0x7F800000u) return (u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u);
+  const unsigned up = (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+  return (up & 0x7F80u) == 0x7F80u ? u >> 16 : up;
+}
+
 __global__ void pack_weights_kernel(const float *__restrict__ W, int K, int Cin, int Cout, int nch, int nbtp,
-                                    float *__restrict__ Wp) {
-  const int64_t total = (int64_t)K * nch * nbtp * 1024;
+                                    uint16_t *__restrict__ Wp) {
+  const int64_t total = (int64_t)K * nch * nbtp * 1024;  // one (lane, value) of all three parts per thread
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-    const int s = (int)(((e >> 8) & 3) * 4 + (e & 3)), lane = (int)((e >> 2) & 63);
-    int64_t q = e >> 10;
+    const int j8 = (int)(e & 7), lane = (int)((e >> 3) & 63), s = (int)((e >> 9) & 1);
+    const int64_t tile = e >> 10;
+    int64_t q = tile;
     const int nb = (int)(q % nbtp);
     q /= nbtp;
     const int ch = (int)(q % nch), k = (int)(q / nch);
-    const int cin = ch * 32 + (lane >> 5) * 16 + s, col = nb * 32 + (lane & 31);
-    Wp[e] = (cin < Cin && col < Cout) ? W[((int64_t)k * Cin + cin) * Cout + col] : 0.0f;
+    const int cin = ch * 32 + s * 16 + (lane >> 5) * 8 + j8, col = nb * 32 + (lane & 31);
+    float x = (cin < Cin && col < Cout) ? W[((int64_t)k * Cin + cin) * Cout + col] : 0.0f;
+    uint16_t *to = Wp + tile * (WT_BYTES / 2) + s * 1536 + lane * 8 + j8;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const unsigned u = bf16_part(x);
+      to[i * 512] = (uint16_t)u;
+      const float part = __uint_as_float(u << 16);
+      x = (u & 0x7F80u) == 0x7F80u ? 0.0f : x - part;  // (exact)
+    }
+  }
+}
+
+// A weight from its three parts, exactly.
+__device__ __forceinline__ float packed_weight_at(const float *Wp, int64_t tile, int cin32, int col) {
+  const uint16_t *p = reinterpret_cast<const uint16_t *>(Wp) + tile * (WT_BYTES / 2) + (cin32 >> 4) * 1536 +
+                      (((cin32 >> 3) & 1) * 32 + col) * 8 + (cin32 & 7);
+  return (__uint_as_float((unsigned)p[0] << 16) + __uint_as_float((unsigned)p[512] << 16)) +
+         __uint_as_float((unsigned)p[1024] << 16);
+}
+
+// sum + the products of one output element in plain fp32, offsets and channels ascending (cold: repair_sums).
+// map0 / map1 as in the generic kernel.
+__device__ __forceinline__ float plain_sum(float sum, const float *__restrict__ in, int64_t ld_in,
+                                           const float *__restrict__ Wp, const int32_t *__restrict__ map0,
+                                           const int32_t *__restrict__ map1, int mode, int K, int row, int Cin, int nch,
+                                           int nbtp, int c) {
+#pragma unroll 1
+  for (int k = 0; k < K; k++) {
+    const int src = mode == MAP_NBR ? map0[(int64_t)row * K + k]
+                    : mode == MAP_IDENTITY ? row
+                                           : (map1[row] == k ? map0[row] : -1);
+    if (src < 0) continue;
+#pragma unroll 1
+    for (int ci = 0; ci < Cin; ci++)
+      sum = fmaf(in[(int64_t)src * ld_in + ci],
+                 packed_weight_at(Wp, ((int64_t)k * nch + (ci >> 5)) * nbtp + (c >> 5), ci & 31, c & 31), sum);
+  }
+  return sum;
+}
+
+// Elements whose sum of bf16 products is not finite (an infinity or NaN among the inputs or weights, or an
+// overflow on the way) are summed again by plain(j).  Which elements these are depends on the element's own sum
+// alone.  One multiply-add per element finds out that there are none.
+template <int N, class A, class F>
+__device__ __forceinline__ void repair_sums(A &a, const F &plain) {
+  float t = 0.0f;
+#pragma unroll
+  for (int j = 0; j < N; j++) t = fmaf(a[j], 0.0f, t);  // NaN as soon as one is infinite or NaN
+  if (!__any(t != t)) return;
+  unsigned bad = 0;
+#pragma unroll
+  for (int j = 0; j < N; j++) bad |= ((__float_as_uint(a[j]) & 0x7F800000u) == 0x7F800000u ? 1u : 0u) << j;
+#pragma unroll 1
+  for (int j = 0; j < N; j++) {
+    if (!__any((bad >> j) & 1u)) continue;
+    const float x = plain(j);
+#pragma unroll
+    for (int i = 0; i < N; i++) a[i] = (i == j && ((bad >> j) & 1u)) ? x : a[i];
   }
 }
 
 // ---------------------------------------------------------------------------------------
 // MFMA kernel.  Cin % 16 == 0, rows of `in` 16-byte aligned, packed weights.
-// Software pipeline: while the 16*NB MFMAs of one (offset, channel chunk) run, the gather of
+// Software pipeline: while the 12*NB MFMAs of one (offset, channel chunk) run, the gather of
 // the next chunk's input rows and the next weight tile are already in flight.
 // ---------------------------------------------------------------------------------------
+// Gathered row chunk: lane (r, h) holds channels h*8 .. h*8+7 of the chunk's first half (q[0], q[1]) and of its
+// second half (q[2], q[3]).
 struct Frag {
   float4 q[4];
 };
+struct WFrag {
+  Parts s[2];
+};
 
-__device__ __forceinline__ float frag_at(const Frag &f, int s) {
-  const float4 v = f.q[s >> 2];
-  return (s & 3) == 0 ? v.x : (s & 3) == 1 ? v.y : (s & 3) == 2 ? v.z : v.w;
+// acc += chunk a times weight tile b; full: the chunk's second half exists
+__device__ __forceinline__ void mac_chunk(Sum &acc, const Parts (&a)[2], const WFrag &b, bool full) {
+  mac16(a[0], b.s[0], acc);
+  if (full) mac16(a[1], b.s[1], acc);
 }
 
 // Gather: every lane reads the 64 bytes of its own input row that the MFMA A operand needs, with
 // buffer loads: one 32-bit offset per item, rows without a neighbour get an out-of-range offset
-// and the hardware returns zeros, and the weight tile is addressed by a scalar offset - a
-// handful of non-MFMA instructions per 16 MFMAs (ordinary VALU work does not overlap with MFMAs
-// on this part, so it is paid in matrix-core time).
+// and the hardware returns zeros, and the weight tile is addressed by a scalar offset.
 // Items in flight per wavefront (ring depth): whole-tile wavefronts, and wavefronts that share a
 // tile.  (For the latter a ring of four measured 4-10 % slower than one of two at every scale of the
 // U-Net: with 91 instead of 140 registers more wavefronts fit a SIMD, and a turn of the unrolled loop
@@ -204,7 +359,6 @@ __device__ __forceinline__ float frag_at(const Frag &f, int s) {
 #define INSC_CONV_DEPTH_SPLIT 2
 #endif
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // offsets at or beyond this bound make a buffer load return zeros
 constexpr uint32_t BUF_OOB = 0xFFFFF000u;  // room for the per-load immediate on top
 
@@ -213,6 +367,33 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint3
 }
 __device__ __forceinline__ float4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
+
+// the chunk at byte offset voff (BUF_OOB: zeros) of a row; h: half-wave
+__device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on, uint32_t base, int h, bool full) {
+  const uint32_t v0 = on ? base + (uint32_t)(h * 32) : BUF_OOB, v1 = on && full ? base + (uint32_t)(64 + h * 32) : BUF_OOB;
+  Frag f;
+  f.q[0] = buf_load16(rin, v0, 0);
+  f.q[1] = buf_load16(rin, v0 + 16u, 0);
+  f.q[2] = buf_load16(rin, v1, 0);
+  f.q[3] = buf_load16(rin, v1 + 16u, 0);
+  return f;
+}
+// weight tile `tile` of the packed filter (on false: zeros)
+__device__ __forceinline__ WFrag load_wtile(__amdgpu_buffer_rsrc_t rw, int tile, bool on, uint32_t lane16) {
+  const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * WT_BYTES);
+  const uint32_t voff = on ? lane16 : BUF_OOB;
+  WFrag f;
+#pragma unroll
+  for (int i = 0; i < 6; i++)
+    f.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, voff + 1024u * (i & 3), soff + (i >= 4 ? 4096u : 0u)));
+  return f;
+}
+
+// The order in which a wavefront that owns a tile takes the offsets of a 3^3 filter: the centre first, then
+// ascending.  (The filter-in-LDS kernel below has no room in LDS for the centre's weights.)
+__device__ __forceinline__ int first_offset(unsigned mask) {
+  return (mask >> 13) & 1u ? 13 : __builtin_ctz(mask);
 }
 
 // S == 1: every wavefront of the block owns a tile and walks all of its filter offsets.
@@ -273,6 +454,9 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
   // per source (two sources: the blocks from G on gather from the second one, through its own map)
   const int GZ = S == 1 ? 1 : (int)gridDim.z;
   const bool second = S > 1 && ep.src2_in != nullptr && (int)bz >= GZ / 2;
+  const float *const in0 = in, *const bias0 = bias;  // (the first source, whichever this block reads)
+  const int64_t ld_in0 = ld_in;
+  const int32_t *const map00 = map0;
   const int G = (S > 1 && ep.src2_in != nullptr) ? GZ / 2 : GZ, ST = S * G;
   const int ws = wave * G + (S == 1 ? 0 : (int)bz - (second ? G : 0));
   if (second) {
@@ -389,13 +573,11 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
     nitems = __builtin_amdgcn_readfirstlane(cnt);
   }
 
-  f16v acc[NB];
+  Sum sums[NB];
 #pragma unroll
   for (int b = 0; b < NB; b++) {
     const int c = (cb0 + b) * 32 + r;
-    const float bv = (bias && c < Cout && (S == 1 || ws == 0)) ? bias[c] : 0.0f;
-#pragma unroll
-    for (int v = 0; v < 16; v++) acc[b][v] = bv;
+    sum_start(sums[b], (bias && c < Cout && (S == 1 || ws == 0)) ? bias[c] : 0.0f);
   }
 
   // per-channel scale / shift of the fused batch norm for this lane's columns (loaded here so
@@ -433,32 +615,20 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
       return n;
     };
     Cursor first;
-    first.k = __builtin_ctz(rest);
+    first.k = S == 1 && K == 27 ? first_offset(rest) : __builtin_ctz(rest);
     first.ch = ch0(first.k);
-    first.rest = rest & (rest - 1);
+    first.rest = rest & ~(1u << first.k);
 
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
     const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u;
-    // lane (r, h) reads channels ch*32 + h*16 .. +15 of its own row; the second half-wave of a
-    // 16-channel tail chunk has no channels
     auto gather = [&](const Cursor &c) -> Frag {
       const int kk = c.k < 0 ? 0 : c.k;
       const int src = nl[planned ? kk * TILE_M + r : r * K + kk];
-      const bool on = c.k >= 0 && src >= 0 && (h == 0 || Cin - c.ch * 32 >= 32);
-      const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(c.ch * 128 + h * 64) : BUF_OOB;
-      Frag f;
-#pragma unroll
-      for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rin, voff + 16u * q, 0);
-      return f;
+      return gather_chunk(rin, c.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h,
+                          Cin - c.ch * 32 >= 32);
     };
-    auto wload = [&](const Cursor &c, int b) -> Frag {
-      const int tile = ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b;
-      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * 4096);
-      const uint32_t voff = c.k >= 0 ? lane16 : BUF_OOB;
-      Frag f;
-#pragma unroll
-      for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rw, voff + 1024u * q, soff);
-      return f;
+    auto wload = [&](const Cursor &c, int b) -> WFrag {
+      return load_wtile(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
     };
 
     // Pipeline: while item t runs on the matrix cores, the gathers of items t+1 .. t+D-1 are in
@@ -472,7 +642,8 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
     constexpr int D = (S == 1 || S >= 16) ? INSC_CONV_DEPTH : INSC_CONV_DEPTH_SPLIT;
     constexpr bool WRING = NB == 1;                         // weight tiles ride in the same ring
     constexpr int TURN = (WRING || NB % 2 == 0) ? D : (D % 2 == 0 ? D : 2 * D);
-    Frag g[D], bw[WRING ? D : 2];
+    Frag g[D];
+    WFrag bw[WRING ? D : 2];
     Cursor ci = first;  // next item to issue
 #pragma unroll
     for (int d = 0; d < D - 1; d++) {
@@ -490,18 +661,21 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
         g[(u + D - 1) % D] = gather(ci);
         if constexpr (WRING) bw[(u + D - 1) % D] = wload(ci, 0);
         ci = step(ci);
-        const bool real = t0i + u < nitems;
+        const bool real = t0i + u < nitems, full = Cin - c0.ch * 32 >= 32;
+        Parts as[2];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
           const int nn = u * NB + b;
           if constexpr (!WRING) bw[(nn + 1) % 2] = (b + 1 < NB) ? wload(c0, b + 1) : wload(c1, 0);
           asm volatile("" ::: "memory");
           __builtin_amdgcn_sched_barrier(0);
-          const Frag &bf = bw[WRING ? u % D : nn % 2];
+          const WFrag &bf = bw[WRING ? u % D : nn % 2];
           if (real) {
-#pragma unroll
-            for (int s = 0; s < 16; s++)
-              acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[u % D], s), frag_at(bf, s), acc[b], 0, 0, 0);
+            if (b == 0) {
+              as[0] = split8(g[u % D].q[0], g[u % D].q[1]);
+              as[1] = split8(g[u % D].q[2], g[u % D].q[3]);
+            }
+            mac_chunk(sums[b], as, bf, full);
           }
         }
         asm volatile("" ::: "memory");
@@ -511,6 +685,10 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
       }
     }
   }
+
+  f16v acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) acc[b] = sum_of(sums[b]);
 
   if (S > 1) {
     // Every wavefront leaves its partial sum in LDS; each then adds up - in wavefront order - and
@@ -586,6 +764,13 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
       if (lane == 0) pcount[unit * S + wave] = 0;
     }
     const int c = cb0 * 32 + r;
+    repair_sums<NV>(a, [&](int j) -> float {
+      const int v = wave * NV + j, row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+      if (row < 0 || c >= Cout) return 0.0f;
+      float x = plain_sum(bias0 ? bias0[c] : 0.0f, in0, ld_in0, Wp, map00, map1, MODE, K, row, Cin, nch, nbtp, c);
+      if (ep.src2_in) x = plain_sum(x, ep.src2_in, ep.src2_ld, Wp, ep.src2_map, map1, MODE, K, row, Cin, nch, nbtp, c);
+      return x;
+    });
     if (c >= Cout) return;
     if (ep.res) {
 #pragma unroll
@@ -631,6 +816,15 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
   int rid[16];
 #pragma unroll
   for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int c = (cb0 + b) * 32 + r;
+    repair_sums<16>(acc[b], [&](int v) -> float {
+      const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+      if (row < 0 || c >= Cout) return 0.0f;
+      return plain_sum(bias ? bias[c] : 0.0f, in, ld_in, Wp, map0, map1, MODE, K, row, Cin, nch, nbtp, c);
+    });
+  }
   // (the values of the residual input are all fetched before the first store: a store may alias them
   // as far as the compiler knows, and loads issued between the stores would wait one by one)
   if (ep.res) {
@@ -688,45 +882,46 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
 }
 
 // ---------------------------------------------------------------------------------------
-// Narrow 3^3 layers (Cin <= 32, Cout <= 32): the whole packed filter (27 tiles of 4 KB) stays in
-// LDS for the life of the block, so the only traffic between L2 and the CU is the gather itself
-// - with the weight tiles re-read per item that path carries twice the bytes and bounds the
-// kernel.  Blocks are persistent: block b owns every gridDim.x-th tile and its wavefronts draw
-// them one by one.
-// The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (offsets ascending,
-// same MFMA sequence), so both kernels give the same bits.
+// Narrow 3^3 layers (Cin <= 32, Cout <= 32): the packed filter stays in LDS for the life of the block - 26
+// tiles of 6 KB; the centre's, which every tile of a submanifold layer starts with, is read through L1 (all
+// 27 would be 2 KB more than a compute unit has) - so the only traffic between L2 and the CU is the gather and
+// the map.  Blocks are persistent: block b owns every gridDim.x-th tile and its wavefronts draw them one by one.
+// The neighbour ids go from the tile plan straight into registers, a ring of them ahead of the gathers (LDS has no
+// room for a copy, and none is needed: lane r only ever wants the ids of row r).
+// The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (centre, then offsets ascending, same
+// MFMA sequence), so both kernels give the same bits.
 // ---------------------------------------------------------------------------------------
-#ifndef INSC_WL_WAVES
-#define INSC_WL_WAVES 12
-#endif
-constexpr int WL_WAVES = INSC_WL_WAVES;
-#ifndef INSC_WL_DEPTH
-#define INSC_WL_DEPTH 4
-#endif
-constexpr int WL_DEPTH = INSC_WL_DEPTH;
+// (32 -> 32 in four layers with their batch norms, 500k / 150k sites: eight wavefronts 542 / 228 us, twelve 538 / 201;
+// rings of three and four items, which spill at twelve wavefronts, 589 / 232 and 667 / 253)
+constexpr int WL_WAVES = 12;
+constexpr int WL_DEPTH = 2;
 constexpr int WL_MIN_TILES = 4096;  // smaller launches go to conv_mfma_kernel (default of the knob below)
 constexpr int WL_SCHED = 256;  // a block orders up to this many tiles of its own by cost
 
+// KS: halves of the 32-channel chunk that exist (1: 16 input channels, 2: 32)
+template <int KS>
 __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
     const int32_t *__restrict__ rows, const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout,
-    const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t map_bytes, BnEpilogue ep, TilePlan plan) {
-  constexpr int K = 27;
-  constexpr int NSTAGE = (TILE_M * K + 63) / 64;
-  __shared__ __attribute__((aligned(16))) float wl[K * 1024];
-  __shared__ int nbl[WL_WAVES][TILE_M * K];
+    const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t map_bytes, uint32_t wp_bytes, BnEpilogue ep,
+    TilePlan plan) {
+  constexpr int K = 27, D = WL_DEPTH, AHEAD = 2 * D - 2;  // gathers D - 1 items ahead, neighbour ids D - 1 before those
+  constexpr int PIECES = KS * 3, TILE16 = PIECES * 64;    // of a weight tile: 1 KB pieces, 16-byte units
+  __shared__ u32x4 wl[(K - 1) * TILE16];
   __shared__ int next_turn;
   __shared__ int cost_l[WL_SCHED], sched_l[WL_SCHED];
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 31, h = lane >> 5;
 
-  // the filter: 27 KB-quarters x 4, copied as is (already in per-lane order)
+  // the filter but for the centre, already in per-lane order
   {
-    const float4 *src = reinterpret_cast<const float4 *>(Wp);
-    float4 *dst = reinterpret_cast<float4 *>(wl);
-    for (int i = threadIdx.x; i < K * 256; i += WL_WAVES * 64) dst[i] = src[i];
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(Wp);
+    for (int i = threadIdx.x; i < (K - 1) * TILE16; i += WL_WAVES * 64) {
+      const int slot = i / TILE16, e = i - slot * TILE16;
+      wl[i] = src[(slot < 13 ? slot : slot + 1) * (WT_BYTES / 16) + e];
+    }
   }
   if (threadIdx.x == 0) next_turn = 0;
   const int64_t ntiles = (n + TILE_M - 1) / TILE_M;
@@ -760,13 +955,11 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     __syncthreads();
   }
 
-  int *nl = nbl[wave];
-  const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rmap = make_rsrc(map0, map_bytes);
+  const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
   // the outputs are addressed with 32-bit byte offsets as well; rows that do not exist get an
   // out-of-range offset and the hardware drops the store
   const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u);
   const uint32_t ld4 = (uint32_t)ld_in * 4u, ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u;
-  const bool half_on = h == 0 || Cin >= 32;  // a 16-channel layer has nothing for the upper half-wave
   const int col = r;
   const float bv = (bias && col < Cout) ? bias[col] : 0.0f;
   const float ew = (ep.out2 && col < Cout) ? ep.w[col] : 0.0f;
@@ -783,7 +976,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   // gets the first of the second round.)
   const bool dealt = my_tiles < 3 * WL_WAVES;
   int my_turn = wave, my_round = 0;
-  auto draw = [&]() -> int64_t {
+  auto draw = [&]() -> int {
     for (;;) {
       int turn;
       if (dealt) {
@@ -793,184 +986,180 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       } else {
         int v = 0;
         if (lane == 0) v = atomicAdd(&next_turn, 1);
-        turn = __builtin_amdgcn_readfirstlane(v);
+        turn = v;
       }
-      if (turn >= my_tiles) return ntiles;
-      const int64_t t = (int64_t)(lpt ? sched_l[turn] : turn) * gridDim.x + brank;
+      turn = __builtin_amdgcn_readfirstlane(turn);
+      if (turn >= my_tiles) return (int)ntiles;
+      const int t = (lpt ? __builtin_amdgcn_readfirstlane(sched_l[turn]) : turn) * (int)gridDim.x + brank;
       if (!tile_flags || tile_flags[t]) return t;
     }
   };
-  auto load_row = [&](int64_t t) -> int {
-    const int64_t p = t * TILE_M + r;
+  auto load_row = [&](int t) -> int {
+    const int64_t p = (int64_t)t * TILE_M + r;
     return (t < ntiles && p < n) ? (rows ? rows[p] : (int)p) : -1;
   };
-  // issue the loads of a tile's slice of the neighbour map; bit i of the result: element i of
-  // this lane exists (a load sent out of range returns 0, which would pass for a site).  With a
-  // tile plan the slice is 27 coalesced runs that need no row id; the LDS copy is offset-major.
+  // Where a lane finds the neighbour id of offset k: at base + k * pitch of the tile plan (the map transposed into
+  // processing order: one 128-byte run per (offset, tile)), or without a plan of its own row of the map.
   const bool planned = plan.map != nullptr;
-  const __amdgpu_buffer_rsrc_t rplan = make_rsrc(plan.map, planned ? (uint32_t)(plan.ld * K * 4) : 0u);
-  auto stage_issue = [&](int64_t tt, int my_row, int (&st)[NSTAGE]) -> unsigned {
-    unsigned valid = 0;
+  const __amdgpu_buffer_rsrc_t rids = planned ? make_rsrc(plan.map, (uint32_t)(plan.ld * K * 4)) : make_rsrc(map0, map_bytes);
+  const uint32_t pitch = planned ? (uint32_t)plan.ld * 4u : 4u;
+  auto id_base = [&](int t, int row) -> uint32_t {
+    return planned ? (uint32_t)(t * TILE_M + r) * 4u : row >= 0 ? (uint32_t)row * (K * 4u) : BUF_OOB;
+  };
+  // the offsets a tile uses, the centre as bit 0 and the others in their order from bit 1 on: bit q > 0 has its
+  // weights in LDS slot q - 1
+  auto offsets_of = [&](int t, uint32_t base, int v) -> unsigned {
+    unsigned m = 0;
+    if (t >= ntiles) return 0u;
     if (planned) {
-#pragma unroll
-      for (int i = 0; i < NSTAGE; i++) {
-        const int e = i * 64 + lane;  // e = k * 32 + row
-        const bool ok = e < TILE_M * K && tt < ntiles;
-        if (ok) valid |= 1u << i;
-        const uint32_t voff = ok ? (uint32_t)((e >> 5) * (int)plan.ld + (int)(tt * TILE_M) + (e & 31)) * 4u : BUF_OOB;
-        st[i] = __builtin_amdgcn_raw_buffer_load_b32(rplan, (int)voff, 0, 0);
+      m = (unsigned)__builtin_amdgcn_readfirstlane(v) & 0x7FFFFFFu;
+    } else {
+      for (int k = 0; k < K; k++) {
+        const int id = base == BUF_OOB ? -1 : (int)__builtin_amdgcn_raw_buffer_load_b32(rids, (int)(base + k * pitch), 0, 0);
+        m |= __any(id >= 0) ? 1u << k : 0u;
       }
-      return valid;
     }
-    int srow[NSTAGE];
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) srow[i] = __shfl(my_row, ((i * 64 + lane) / K) & (TILE_M - 1), 64);
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = i * 64 + lane;
-      const int kk = e - (e / K) * K;
-      const bool ok = e < TILE_M * K && srow[i] >= 0;
-      if (ok) valid |= 1u << i;
-      st[i] = __builtin_amdgcn_raw_buffer_load_b32(rmap, (int)(ok ? (uint32_t)(srow[i] * K + kk) * 4u : BUF_OOB), 0, 0);
+    return ((m >> 13) & 1u) | ((m & 0x1FFFu) << 1) | (m & 0x7FFC000u);
+  };
+  auto next_q = [](unsigned &rest) -> int {  // past the end: -1
+    const int q = rest ? __builtin_ctz(rest) : -1;
+    rest &= rest - 1;
+    return q;
+  };
+  auto id_load = [&](int q, uint32_t base) -> int {
+    const uint32_t k = q == 0 ? 13u : q <= 13 ? (uint32_t)(q - 1) : (uint32_t)q;
+    return (int)__builtin_amdgcn_raw_buffer_load_b32(rids, (int)(q >= 0 && base != BUF_OOB ? base : BUF_OOB),
+                                                     (int)(q >= 0 ? k * pitch : 0u), 0);
+  };
+  auto gather = [&](int q, int src, uint32_t base) -> Frag {
+    const bool on = q >= 0 && src >= 0 && base != BUF_OOB;  // (a load sent out of range returns 0, which would pass for a site)
+    const uint32_t v0 = on ? (uint32_t)src * ld4 + (uint32_t)(h * 32) : BUF_OOB;
+    Frag f;
+    f.q[0] = buf_load16(rin, v0, 0);
+    f.q[1] = buf_load16(rin, v0 + 16u, 0);
+    if constexpr (KS == 2) {
+      f.q[2] = buf_load16(rin, v0 + 64u, 0);
+      f.q[3] = buf_load16(rin, v0 + 80u, 0);
     }
-    return valid;
+    return f;
   };
 
-  // Software pipeline over tiles: while tile t is computed, the neighbour-map slice of the next
-  // tile and the row ids of the one after it are in flight.
-  int64_t t = draw();
+  // Software pipeline over tiles: while tile t is computed, the neighbour ids of the first items of the next
+  // tile and the row ids and offset mask of the one after it are in flight; the gathers of the next tile's first
+  // items go out before this tile's rows are stored.
+  int t = draw();
+  if (t >= ntiles) return;  // (no workgroup barrier below)
   int my_row = load_row(t);
-  int st[NSTAGE];
-  unsigned valid = stage_issue(t, my_row, st);
-  int64_t tn = t < ntiles ? draw() : ntiles;
+  uint32_t base = id_base(t, my_row);
+  unsigned rest = offsets_of(t, base, planned ? (int)plan.tmask[t] : 0);
+  int ids[AHEAD];  // ids of the items 0 .. AHEAD - 1 of tile t
+  {
+    unsigned rr = rest;
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) ids[i] = id_load(next_q(rr), base);
+  }
+  int tn = draw();
   int my_row_n = load_row(tn);
+  int mask_n_v = planned && tn < ntiles ? (int)plan.tmask[tn] : 0;
+  Frag g[D];
+  WFrag bw;
+  auto prime = [&](unsigned rr, uint32_t b) {  // the gathers of the first items, and the centre's weights
+#pragma unroll
+    for (int i = 0; i < D - 1; i++) g[i] = gather(next_q(rr), ids[i], b);
+#pragma unroll
+    for (int i = 0; i < PIECES; i++)
+      bw.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u, 13u * WT_BYTES + 1024u * i));
+  };
+  prime(rest, base);
 
   while (t < ntiles) {
-    // neighbour-map slice -> LDS (private to the wavefront), and the offsets the tile uses
-    unsigned mymask = 0;
-    if (planned) {
-      mymask = plan.tmask[t];
+    const uint32_t base_n = id_base(tn, my_row_n);
+    const unsigned rest_n = offsets_of(tn, base_n, mask_n_v);
+    // ring of neighbour ids: the item i's is in slot i % D from the step it is loaded in to its gather
+    int ix[D];
 #pragma unroll
-      for (int i = 0; i < NSTAGE; i++) {
-        const int e = i * 64 + lane;
-        if (e < TILE_M * K) nl[e] = st[i];
-      }
-    } else {
+    for (int i = D - 1; i < AHEAD; i++) ix[i % D] = ids[i];
+    {
+      unsigned rr = rest_n;
 #pragma unroll
-      for (int i = 0; i < NSTAGE; i++) {
-        const int e = i * 64 + lane;
-        if (e < TILE_M * K) {
-          const bool have = ((valid >> i) & 1u) && st[i] >= 0;
-          nl[e] = have ? st[i] : -1;
-          if (have) mymask |= 1u << (e % K);
-        }
-      }
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) mymask |= (unsigned)__shfl_xor((int)mymask, d, 64);
+      for (int i = 0; i < AHEAD; i++) ids[i] = id_load(next_q(rr), base_n);
     }
-    unsigned rest = (unsigned)__builtin_amdgcn_readfirstlane((int)mymask);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-    // next tile's loads
-    int stn[NSTAGE];
-    const unsigned valid_n = stage_issue(tn, my_row_n, stn);
-    const int64_t tnn = tn < ntiles ? draw() : ntiles;
+    const int tnn = tn < ntiles ? draw() : (int)ntiles;
     const int my_row_nn = load_row(tnn);
+    const int mask_nn_v = planned && tnn < ntiles ? (int)plan.tmask[tnn] : 0;
 
-    f16v acc;
-#pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = bv;
+    Sum sum;
+    sum_start(sum, bv);
 
     if (rest) {
-      const int nitems = __builtin_popcount(rest);
-      // cursor over the active offsets, branch-free; -1 past the end (loads go out of range)
-      auto next_k = [&]() -> int {
-        const int k = rest ? __builtin_ctz(rest) : -1;
-        rest &= rest - 1;
-        return k;
-      };
-      auto gather = [&](int k) -> Frag {
-        const int kk = k < 0 ? 0 : k;
-        const int src = nl[planned ? kk * TILE_M + r : r * K + kk];
-        const bool on = k >= 0 && src >= 0 && half_on;
-        const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(h * 64) : BUF_OOB;
-        Frag f;
+      // three cursors over the tile's items: the one computed, the one gathered, the one whose id is loaded
+      unsigned rc = rest, rg = rest, ri = rest;
 #pragma unroll
-        for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rin, voff + 16u * q, 0);
-        return f;
-      };
-      auto wread = [&](int k) -> Frag {
-        const float4 *p = reinterpret_cast<const float4 *>(wl + (k < 0 ? 0 : k) * 1024) + lane;
-        Frag f;
+      for (int i = 0; i < D - 1; i++) (void)next_q(rg);
 #pragma unroll
-        for (int q = 0; q < 4; q++) f.q[q] = p[q * 64];
-        return f;
+      for (int i = 0; i < AHEAD; i++) (void)next_q(ri);
+      // step of the item in slot U of the rings
+      auto issue = [&](auto U) {
+        constexpr int u = decltype(U)::value;
+        const int qg = next_q(rg), qi = next_q(ri);
+        g[(u + D - 1) % D] = gather(qg, ix[(u + D - 1) % D], base);
+        ix[(u + AHEAD) % D] = id_load(qi, base);
       };
-      constexpr int D = WL_DEPTH;
-      Frag g[D];
-      int kq[D];  // offsets of the items in the ring
+      auto compute = [&](auto U) {
+        constexpr int u = decltype(U)::value;
+        Parts as[2];
+        as[0] = split8(g[u].q[0], g[u].q[1]);
+        if constexpr (KS == 2) as[1] = split8(g[u].q[2], g[u].q[3]);
+        mac_chunk(sum, as, bw, KS == 2);
+      };
+      auto wread = [&](int q) {
+        const u32x4 *p = wl + (q - 1) * TILE16 + lane;
 #pragma unroll
-      for (int d = 0; d < D - 1; d++) {
-        kq[d] = next_k();
-        g[d] = gather(kq[d]);
+        for (int i = 0; i < PIECES; i++) bw.s[i / 3].p[i % 3] = p[i * 64];
+      };
+      {
+        const int q = next_q(rc);
+        if (q != 0) wread(q);  // (a tile without the centre; bw holds the centre's weights otherwise)
+        __builtin_amdgcn_sched_barrier(0);
+        issue(std::integral_constant<int, 0>());
+        __builtin_amdgcn_sched_barrier(0);
+        compute(std::integral_constant<int, 0>());
       }
-      // The loads of the item D - 1 ahead and the weight tile of the next item are issued in the
-      // shadow of this item's MFMAs (a dependent MFMA issues every 64 cycles; whatever sits between
-      // two of them is free), in four slices pinned by scheduling barriers.
-      // (one turn of the loop covers both rings: D register slots for the gathered rows, two for the weights)
-      constexpr int TURN = D % 2 == 0 ? D : 2 * D;
-      Frag bw[2];
-      bw[0] = wread(kq[0]);
-      for (int i0 = 0; i0 < nitems; i0 += TURN) {
-#pragma unroll
-        for (int u = 0; u < TURN; u++) {
-          const bool real = i0 + u < nitems;
-          const Frag &bf = bw[u % 2];
-          __builtin_amdgcn_sched_barrier(0);
-          if (real) {
-#pragma unroll
-            for (int s = 0; s < 4; s++)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[u % D], s), frag_at(bf, s), acc, 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          const int kn = next_k();
-          kq[(u + D - 1) % D] = kn;
-          const int src = nl[planned ? (kn < 0 ? 0 : kn) * TILE_M + r : r * K + (kn < 0 ? 0 : kn)];
-          __builtin_amdgcn_sched_barrier(0);
-          if (real) {
-#pragma unroll
-            for (int s = 4; s < 8; s++)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[u % D], s), frag_at(bf, s), acc, 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          {
-            const bool on = kn >= 0 && src >= 0 && half_on;
-            const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(h * 64) : BUF_OOB;
-#pragma unroll
-            for (int q = 0; q < 4; q++) g[(u + D - 1) % D].q[q] = buf_load16(rin, voff + 16u * q, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          if (real) {
-#pragma unroll
-            for (int s = 8; s < 12; s++)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[u % D], s), frag_at(bf, s), acc, 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          bw[(u + 1) % 2] = wread(kq[(u + 1) % D]);
-          __builtin_amdgcn_sched_barrier(0);
-          if (real) {
-#pragma unroll
-            for (int s = 12; s < 16; s++)
-              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[u % D], s), frag_at(bf, s), acc, 0, 0, 0);
-          }
-          __builtin_amdgcn_sched_barrier(0);
+      // one turn: the slots 1 .. D - 1, 0
+      auto one = [&](auto U) -> bool {
+        if (!rc) return false;
+        const int q = next_q(rc);
+        wread(q);
+        __builtin_amdgcn_sched_barrier(0);
+        issue(U);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(U);
+        return true;
+      };
+      if constexpr (D == 2) {
+        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 0>())) {
+        }
+      } else if constexpr (D == 3) {
+        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 2>()) &&
+               one(std::integral_constant<int, 0>())) {
+        }
+      } else {
+        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 2>()) &&
+               one(std::integral_constant<int, 3>()) && one(std::integral_constant<int, 0>())) {
         }
       }
     }
+    // the next tile's first gathers and the centre's weights, in flight over this tile's stores
+    prime(rest_n, base_n);
+    __builtin_amdgcn_sched_barrier(0);
+    f16v acc = sum_of(sum);
 
     // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3)
+    repair_sums<16>(acc, [&](int v) -> float {
+      const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+      if (row < 0 || col >= Cout) return 0.0f;
+      return plain_sum(bv, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, 1, 1, col);
+    });
     int rid[16];
 #pragma unroll
     for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
@@ -996,295 +1185,13 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
                                               (int)(ok ? __umul24((unsigned)rid[v], ldo24) + col4 : BUF_OOB), 0, 0);
       }
     }
-    // the next tile overwrites this wavefront's LDS slice: all lanes must be done reading it
-    __builtin_amdgcn_wave_barrier();
-
     t = tn;
     my_row = my_row_n;
-    valid = valid_n;
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) st[i] = stn[i];
+    base = base_n;
+    rest = rest_n;
     tn = tnn;
     my_row_n = my_row_nn;
-  }
-}
-
-// ---------------------------------------------------------------------------------------
-// Wide 3^3 layers with many tiles: persistent blocks of S wavefronts.  A block works through
-// units (tile, output block) of a cost-ordered list (plan.sched: tiles by falling number of active
-// offsets); block b takes the units b, 2B-1-b, 2B+b, ... (every other round reversed, so a block
-// that starts with an expensive unit continues with a cheap one).  While a unit is computed the
-// neighbour-map slice, row ids and tile id of the next ones are in flight, so that no wavefront
-// ever waits for a launch, a map or a row id between two units - with one block per unit the
-// matrix cores idle through 5-10 us of such latencies per wavefront, and the units a compute unit
-// happens to receive differ by 2x in cost.
-// The S wavefronts deal the (offset, chunk) items of the unit exactly as conv_mfma_kernel<1, 27,
-// MAP_NBR, S> with one block per tile does, and the partial sums are added in the same order: both
-// kernels give the same bits.  All wavefronts share the final sum and the stores (8 * 4 / S rows each).
-// ---------------------------------------------------------------------------------------
-template <int S>
-__global__ __launch_bounds__(S * 64) __attribute__((amdgpu_waves_per_eu(3, 3))) void conv_pers_kernel(
-    const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
-    const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
-    const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
-  constexpr int K = 27;
-  constexpr int NSTAGE = (TILE_M * K + 64 * S - 1) / (64 * S);
-  constexpr int VPW = 16 / S;  // accumulator registers (groups of 4 rows x 2 half-waves) a wavefront finishes
-  __shared__ int nl[2][TILE_M * K];
-  __shared__ float red[2][S][16 * 64];
-  const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
-  const int64_t ntiles = (n + TILE_M - 1) / TILE_M, units = ntiles * nbt;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int r = lane & 31, h = lane >> 5;
-  const int nch = conv_nch(Cin);
-  const int64_t B = gridDim.x, b = blockIdx.x;
-  const __amdgpu_buffer_rsrc_t rplan = make_rsrc(plan.map, (uint32_t)(plan.ld * K * 4));
-  // unit j of this block: b, 2B - 1 - b, 2B + b, ...
-  auto unit_at = [&](int64_t j) -> int64_t { return j * B + ((j & 1) ? B - 1 - b : b); };
-  // Tile id, tile flag and offset mask of a unit are the same for every lane, but they are fetched
-  // with vector loads: scalar loads share their counter with the LDS reads of the item loop, which
-  // would then wait for them.
-  const __amdgpu_buffer_rsrc_t rsched = make_rsrc(plan.sched, (uint32_t)(ntiles * 4));
-  const __amdgpu_buffer_rsrc_t rtmask = make_rsrc(plan.tmask, (uint32_t)(ntiles * 4));
-  const __amdgpu_buffer_rsrc_t rflag = make_rsrc(tile_flags, tile_flags ? (uint32_t)ntiles : 0u);
-  auto tile_issue = [&](int64_t u) -> int {  // out of range: 0, never used
-    return __builtin_amdgcn_raw_buffer_load_b32(rsched, (int)(u < units ? (uint32_t)(u / nbt) * 4u : BUF_OOB), 0, 0);
-  };
-  auto stage_issue = [&](int tile, int (&st)[NSTAGE]) {
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (i * S + wave) * 64 + lane;  // e = k * 32 + row
-      const bool ok = tile >= 0 && e < TILE_M * K;  // (the value of a load sent out of range is never used)
-      const uint32_t voff = ok ? (uint32_t)((e >> 5) * (int)plan.ld + tile * TILE_M + (e & 31)) * 4u : BUF_OOB;
-      st[i] = __builtin_amdgcn_raw_buffer_load_b32(rplan, (int)voff, 0, 0);
-    }
-  };
-  auto row_of = [&](int tile) -> int {
-    const int64_t p = (int64_t)tile * TILE_M + r;
-    return (tile >= 0 && p < n) ? (rows ? rows[p] : (int)p) : -1;
-  };
-  auto flag_issue = [&](int tile) -> int {
-    return (int)__builtin_amdgcn_raw_buffer_load_b8(rflag, (int)(tile >= 0 ? (uint32_t)tile : BUF_OOB), 0, 0);
-  };
-  auto mask_issue = [&](int tile) -> int {
-    return __builtin_amdgcn_raw_buffer_load_b32(rtmask, (int)(tile >= 0 ? (uint32_t)tile * 4u : BUF_OOB), 0, 0);
-  };
-
-  const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
-  const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u;
-  // outputs and the residual input are addressed with 32-bit byte offsets as well (the host checks
-  // the sizes); rows that do not exist get an out-of-range offset and the hardware drops the access
-  const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u);
-  const __amdgpu_buffer_rsrc_t rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
-  const __amdgpu_buffer_rsrc_t rbias = make_rsrc(bias, bias ? (uint32_t)Cout * 4u : 0u);
-  const __amdgpu_buffer_rsrc_t rew = make_rsrc(ep.w, ep.out2 ? (uint32_t)Cout * 4u : 0u);
-  const __amdgpu_buffer_rsrc_t reb = make_rsrc(ep.b, ep.out2 ? (uint32_t)Cout * 4u : 0u);
-  const uint32_t ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u, ldr4 = (uint32_t)ep.ldr * 4u;
-  // Offsets of which this wavefront holds at least 1, 2, .. items (it takes, of offset k, the chunks
-  // ch0(k), ch0(k) + S, ... with ch0(k) = (wave - k * nch) mod S): the items of a tile with offset
-  // mask m are then counted with a few population counts.
-  constexpr int MAXQ = 4;  // nch <= MAXQ * S
-  unsigned kmask[MAXQ];
-#pragma unroll
-  for (int q = 0; q < MAXQ; q++) kmask[q] = 0;
-  for (int k = 0; k < K; k++) {
-    const int c0 = (wave - k * nch) & (S - 1);
-    const int cnt = c0 < nch ? (nch - c0 + S - 1) / S : 0;
-#pragma unroll
-    for (int q = 0; q < MAXQ; q++)
-      if (cnt > q) kmask[q] |= 1u << k;
-  }
-  // bias and the fused batch norm's scale / shift for this lane's column of output block ob (sent
-  // out of range, they read as zero)
-  auto col_issue = [&](int ob, float &bv, float &ew, float &eb) {
-    const uint32_t off = (uint32_t)(ob * 32 + r) * 4u;
-    bv = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rbias, (int)(wave == 0 ? off : BUF_OOB), 0, 0));
-    ew = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rew, (int)off, 0, 0));
-    eb = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(reb, (int)off, 0, 0));
-  };
-
-  // LDS copies of the map slice and of the partial sums are double buffered (parity par): one
-  // barrier per unit publishes the partial sums of this unit and the map slice of the next
-  // Pipeline over the units of this block: while unit j is computed, the map slice, row ids, flag
-  // and mask of unit j + 1 and the tile id of unit j + 2 are in flight.
-  int64_t j = 0, u = unit_at(0);
-  int tile_c = u < units ? __builtin_amdgcn_readfirstlane(tile_issue(u)) : -1;
-  int tile_n = unit_at(1) < units ? __builtin_amdgcn_readfirstlane(tile_issue(unit_at(1))) : -1;
-  int par = 0;
-  {
-    int st[NSTAGE];
-    stage_issue(tile_c, st);
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (i * S + wave) * 64 + lane;
-      if (e < TILE_M * K) nl[0][e] = st[i];
-    }
-  }
-  int my_row = row_of(tile_c);
-  bool live = tile_c >= 0 && (!tile_flags || __builtin_amdgcn_readfirstlane(flag_issue(tile_c)) != 0);
-  unsigned tmask_c = (unsigned)__builtin_amdgcn_readfirstlane(mask_issue(tile_c));
-  float bv, ew, eb;
-  col_issue((int)(u % nbt), bv, ew, eb);
-  __syncthreads();
-
-  while (u < units) {
-    const int ob = (int)(u % nbt);
-    const int64_t un = unit_at(j + 1), unn = unit_at(j + 2);
-    const int tile_nn_v = tile_issue(unn);
-    int stn[NSTAGE];
-    stage_issue(tile_n, stn);
-    const int my_row_n = row_of(tile_n);
-    const int flag_n_v = flag_issue(tile_n);
-    const int tmask_n_v = mask_issue(tile_n);
-    float bv_n, ew_n, eb_n;
-    col_issue((int)(un % nbt), bv_n, ew_n, eb_n);
-    const int *nlc = nl[par];
-    const int c = ob * 32 + r;
-    f16v acc;
-    int rid[VPW];
-    float rv[VPW];
-
-    if (live) {
-      // Items (active offset k, 32-channel chunk ch), dealt by (k * nch + ch) % S: wavefront w takes,
-      // of offset k, the chunks ch0(k), ch0(k) + S, ... with ch0(k) = (w - k * nch) mod S.
-      const unsigned rest = tmask_c & kmask[0];
-      int nitems = 0;
-#pragma unroll
-      for (int q = 0; q < MAXQ; q++) nitems += __builtin_popcount(tmask_c & kmask[q]);
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[v] = bv;
-
-      if (rest) {
-        struct Cursor {
-          int k, ch;
-          unsigned rest;
-        };
-        auto ch0 = [&](int k) -> int { return (wave - k * nch) & (S - 1); };
-        auto step = [&](const Cursor &cu) -> Cursor {
-          const bool wrap = cu.ch + S >= nch;
-          const int nk = cu.rest ? __builtin_ctz(cu.rest) : -1;
-          Cursor nx;
-          nx.ch = wrap ? ch0(nk) : cu.ch + S;
-          nx.k = wrap ? nk : cu.k;
-          nx.rest = wrap ? (cu.rest & (cu.rest - 1)) : cu.rest;
-          return nx;
-        };
-        Cursor first;
-        first.k = __builtin_ctz(rest);
-        first.ch = ch0(first.k);
-        first.rest = rest & (rest - 1);
-        auto gather = [&](const Cursor &cu) -> Frag {
-          const int kk = cu.k < 0 ? 0 : cu.k;
-          const int src = nlc[kk * TILE_M + r];
-          const bool on = cu.k >= 0 && src >= 0 && (h == 0 || Cin - cu.ch * 32 >= 32);
-          const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128 + h * 64) : BUF_OOB;
-          Frag f;
-#pragma unroll
-          for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rin, voff + 16u * q, 0);
-          return f;
-        };
-        auto wload = [&](const Cursor &cu) -> Frag {
-          const int tile = ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob;
-          const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * 4096);
-          const uint32_t voff = cu.k >= 0 ? lane16 : BUF_OOB;
-          Frag f;
-#pragma unroll
-          for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rw, voff + 1024u * q, soff);
-          return f;
-        };
-        // the same ring of D items in flight as in conv_mfma_kernel
-        constexpr int D = INSC_CONV_DEPTH_SPLIT;
-        Frag g[D], bw[D];
-        Cursor ci = first;
-#pragma unroll
-        for (int d = 0; d < D - 1; d++) {
-          g[d] = gather(ci);
-          bw[d] = wload(ci);
-          ci = step(ci);
-        }
-        for (int t0i = 0; t0i < nitems; t0i += D) {
-#pragma unroll
-          for (int uu = 0; uu < D; uu++) {
-            g[(uu + D - 1) % D] = gather(ci);
-            bw[(uu + D - 1) % D] = wload(ci);
-            ci = step(ci);
-            const bool real = t0i + uu < nitems;
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-            if (real) {
-#pragma unroll
-              for (int s2 = 0; s2 < 16; s2++)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[uu], s2), frag_at(bw[uu], s2), acc, 0, 0, 0);
-            }
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
-      }
-
-    }
-    // the next unit's slice of the map and its scalars (taken before the loads and stores of this
-    // unit's output are issued: a wait for them placed later would wait for those as well)
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (i * S + wave) * 64 + lane;
-      if (e < TILE_M * K) nl[par ^ 1][e] = stn[i];
-    }
-    const int tile_nn = unn < units ? __builtin_amdgcn_readfirstlane(tile_nn_v) : -1;
-    const bool live_n = tile_n >= 0 && (!tile_flags || __builtin_amdgcn_readfirstlane(flag_n_v) != 0);
-    const unsigned tmask_n = tile_n >= 0 ? (unsigned)__builtin_amdgcn_readfirstlane(tmask_n_v) : 0u;
-    if (live) {
-      // partial sums of all wavefronts through LDS
-#pragma unroll
-      for (int v = 0; v < 16; v++) red[par][wave][v * 64 + lane] = acc[v];
-      // rows this wavefront will store, and their residual input (in flight across the barrier)
-#pragma unroll
-      for (int q = 0; q < VPW; q++) {
-        const int v = wave * VPW + q;
-        rid[q] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-        if (c >= Cout) rid[q] = -1;
-        rv[q] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(
-            rres, (int)(rid[q] >= 0 ? __umul24((unsigned)rid[q], ldr4) + (uint32_t)c * 4u : BUF_OOB), 0, 0));
-      }
-    }
-    __syncthreads();
-    if (live) {
-      // wavefront w adds the partial sums, in wavefront order, for the accumulator registers
-      // w * VPW .. and stores those rows
-      float a[VPW];
-#pragma unroll
-      for (int q = 0; q < VPW; q++) {
-        const int v = wave * VPW + q;
-        a[q] = red[par][0][v * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < S; w++) a[q] += red[par][w][v * 64 + lane];
-        if (ep.res) a[q] += rv[q];
-      }
-#pragma unroll
-      for (int q = 0; q < VPW; q++) {
-        const uint32_t c4 = (uint32_t)c * 4u;
-        if (out)
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a[q]), rout,
-                                                (int)(rid[q] >= 0 ? __umul24((unsigned)rid[q], ldo4) + c4 : BUF_OOB), 0, 0);
-        if (ep.out2) {
-          const float y = fmaf(a[q], ew, eb);  // fused batch norm + leaky ReLU
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : ep.leak)), rout2,
-                                                (int)(rid[q] >= 0 ? __umul24((unsigned)rid[q], ldo24) + c4 : BUF_OOB), 0, 0);
-        }
-      }
-    }
-    j++;
-    u = un;
-    tile_c = tile_n;
-    tile_n = tile_nn;
-    my_row = my_row_n;
-    live = live_n;
-    tmask_c = tmask_n;
-    bv = bv_n;
-    ew = ew_n;
-    eb = eb_n;
-    par ^= 1;
+    mask_n_v = mask_nn_v;
   }
 }
 
@@ -1299,7 +1206,7 @@ __global__ __launch_bounds__(S * 64) __attribute__((amdgpu_waves_per_eu(3, 3))) 
 // kernel's ST partial sums - the items (k, ch) with (k * nch + ch) % ST == p, in ascending order,
 // bias in sum 0 - in ST accumulators per output block and adds them in order at the end.
 // Blocks are persistent over units (group of four tiles, NB output blocks) taken from the cost-
-// ordered group schedule as in conv_pers_kernel.
+// ordered group schedule: block b takes the units b, 2B - 1 - b, 2B + b, ..
 // The two weight buffers and the two A slots alternate with the parity of the step, and the step
 // loop is unrolled by two so that each is a compile-time choice: the compiler then knows that a
 // read of one weight buffer cannot touch the load into the other that is still in flight (for a
@@ -1307,16 +1214,18 @@ __global__ __launch_bounds__(S * 64) __attribute__((amdgpu_waves_per_eu(3, 3))) 
 // ---------------------------------------------------------------------------------------
 #define INSC_LDS_PTR(x) ((__attribute__((address_space(3))) void *)(x))
 template <int NB, int ST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4 ? 2 : 3, NB * ST > 4 ? 2 : 3))) void conv_wshare_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 : 3, NB > 1 ? 2 : 3))) void conv_wshare_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
+    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
+    const int32_t *__restrict__ rows,
     const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
   constexpr int K = 27, WV = 4;
   constexpr int NSTAGE = (TILE_M * K + 63) / 64;  // 14 loads of 64 entries; the last one half empty
   __shared__ int nl[WV][NSTAGE * 64];
-  __shared__ float4 wl0[NB][256];
-  __shared__ float4 wl1[NB][256];
+  __shared__ u32x4 wl0[NB][6 * 64];
+  __shared__ u32x4 wl1[NB][6 * 64];
+  __shared__ u32x4 wl2[NB][6 * 64];
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int ntiles = (int)((n + TILE_M - 1) / TILE_M), ngroups = (ntiles + WV - 1) / WV;
   const int nug = (nbt + NB - 1) / NB;  // units per group
@@ -1324,6 +1233,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const int r = lane & 31, h = lane >> 5;
   const int nch = conv_nch(Cin);
+  // offsets that hold items of partial sum p
+  unsigned hm[ST];
+#pragma unroll
+  for (int p = 0; p < ST; p++) hm[p] = (unsigned)__ballot(lane < K && ((p - lane * nch) & (ST - 1)) < nch);
   const int64_t B = gridDim.x, b = blockIdx.x;
   const __amdgpu_buffer_rsrc_t rplan = make_rsrc(plan.map, (uint32_t)(plan.ld * K * 4));
   const __amdgpu_buffer_rsrc_t rsched = make_rsrc(plan.sched + (plan.ld + 31) / 32, (uint32_t)ngroups * 4u);  // group schedule
@@ -1369,17 +1282,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
     return (tile >= 0 && p < n) ? (rows ? rows[p] : (int)p) : -1;
   };
   struct Step {
-    int k, ch;
+    int k, ch, p;
     unsigned rest;
-  };
-  auto step_next = [&](const Step &c) -> Step {  // past the end: k = -1
-    Step nx;
-    const bool wrap = c.ch + 1 >= nch;
-    const int nk = c.rest ? __builtin_ctz(c.rest) : -1;
-    nx.ch = wrap ? 0 : c.ch + 1;
-    nx.k = wrap ? nk : c.k;
-    nx.rest = wrap ? (c.rest & (c.rest - 1)) : c.rest;
-    return nx;
   };
 
   int64_t j = 0, u = unit_at(0);
@@ -1422,99 +1326,112 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
         ew[o] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rew, (int)off, 0, 0));
         eb[o] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(reb, (int)off, 0, 0));
       }
-      f16v acc[ST][NB];  // partial sum p holds the items with (k * nch + ch) % ST == p; bias in sum 0
+      // the running partial sum and the sum of the finished ones; bias in partial sum 0
+      Sum acc[NB];
+      f16v total[NB];
 #pragma unroll
-      for (int pp = 0; pp < ST; pp++) {
+      for (int o = 0; o < NB; o++) sum_start(acc[o], bv[o]);
+      int cur = 0;  // the partial sum in acc
+      auto step_next = [&](const Step &c) -> Step {  // past the end: k = -1
+        Step nx = c;
+        nx.ch = c.ch + ST;
+        if (nx.ch >= nch || c.k < 0) {
 #pragma unroll
-        for (int o = 0; o < NB; o++) {
-#pragma unroll
-          for (int v = 0; v < 16; v++) acc[pp][o][v] = pp == 0 ? bv[o] : 0.0f;
+          for (int p = 1; p < ST; p++) {
+            if (nx.rest == 0 && nx.p < p) {
+              nx.p = p;
+              nx.rest = uni & hm[p];
+            }
+          }
+          nx.k = nx.rest ? __builtin_ctz(nx.rest) : -1;
+          nx.ch = (nx.p - nx.k * nch) & (ST - 1);
+          nx.rest &= nx.rest - 1;
         }
-      }
-      const int nsteps = __builtin_popcount(uni) * nch;
-      // weight tiles of a step -> LDS, a quarter (1 KB) per wavefront and output block
-      auto w_issue0 = [&](const Step &c) {
-#pragma unroll
-        for (int o = 0; o < NB; o++) {
-          const uint32_t soff = (uint32_t)(((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + ob0 + o) * 4096u;
-          const bool ok = c.k >= 0 && ob0 + o < nbt;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, INSC_LDS_PTR(&wl0[o][wave * 64]), 16,
-                                                   (int)(ok ? (uint32_t)(wave * 1024 + lane * 16) : BUF_OOB), (int)soff, 0, 0);
-        }
+        return nx;
       };
-      auto w_issue1 = [&](const Step &c) {
+      // weight tiles of a step -> LDS, their 1 KB pieces dealt to the four wavefronts
+      auto w_issue = [&](const Step &c, u32x4 (*wl)[6 * 64]) {
 #pragma unroll
-        for (int o = 0; o < NB; o++) {
-          const uint32_t soff = (uint32_t)(((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + ob0 + o) * 4096u;
+        for (int i = 0; i < (6 * NB + WV - 1) / WV; i++) {
+          const int piece = i * WV + wave, o = piece / 6;
+          if (piece >= 6 * NB) break;
+          const uint32_t soff = (uint32_t)(((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + ob0 + o) * (uint32_t)WT_BYTES;
           const bool ok = c.k >= 0 && ob0 + o < nbt;
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, INSC_LDS_PTR(&wl1[o][wave * 64]), 16,
-                                                   (int)(ok ? (uint32_t)(wave * 1024 + lane * 16) : BUF_OOB), (int)soff, 0, 0);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              rw, INSC_LDS_PTR(&wl[0][piece * 64]), 16,
+              (int)(ok ? (uint32_t)((piece - o * 6) * 1024 + lane * 16) : BUF_OOB), (int)soff, 0, 0);
         }
       };
       auto gather = [&](const Step &c) -> Frag {
         const int kk = c.k < 0 ? 0 : c.k;
         const int src = nlw[kk * TILE_M + r];
-        const bool on = c.k >= 0 && ((mine >> kk) & 1u) && src >= 0 && (h == 0 || Cin - c.ch * 32 >= 32);
-        const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(c.ch * 128 + h * 64) : BUF_OOB;
-        Frag f;
-#pragma unroll
-        for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rin, voff + 16u * q, 0);
-        return f;
+        const bool on = c.k >= 0 && ((mine >> kk) & 1u) && src >= 0;
+        return gather_chunk(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h, Cin - c.ch * 32 >= 32);
       };
-      auto compute = [&](const Step &c, const Frag &a, const float4 (*wl)[256]) {
+      auto compute = [&](const Step &c, const Frag &a, const u32x4 (*wl)[6 * 64]) {
         if (c.k < 0 || !((mine >> c.k) & 1u)) return;  // (the same for every lane of the wavefront)
-        const int part = (c.k * nch + c.ch) & (ST - 1);
+        const bool full = Cin - c.ch * 32 >= 32;
+        if (c.p != cur) {
+#pragma unroll
+          for (int o = 0; o < NB; o++) {
+            const f16v part = sum_of(acc[o]);
+#pragma unroll
+            for (int v = 0; v < 16; v++) total[o][v] = cur == 0 ? part[v] : total[o][v] + part[v];
+            sum_start(acc[o], 0.0f);
+          }
+          cur = c.p;
+        }
+        const Parts as[2] = {split8(a.q[0], a.q[1]), split8(a.q[2], a.q[3])};
 #pragma unroll
         for (int o = 0; o < NB; o++) {
           if (ob0 + o >= nbt) break;
-          Frag bf;
+          WFrag bf;
 #pragma unroll
-          for (int q = 0; q < 4; q++) bf.q[q] = wl[o][q * 64 + lane];
-#pragma unroll
-          for (int pp = 0; pp < ST; pp++) {
-            if (part != pp) continue;  // (one copy of the MFMA block per partial sum: the accumulator is a compile-time choice)
-#pragma unroll
-            for (int s2 = 0; s2 < 16; s2++)
-              acc[pp][o] = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(a, s2), frag_at(bf, s2), acc[pp][o], 0, 0, 0);
-          }
+          for (int i = 0; i < 6; i++) bf.s[i / 3].p[i % 3] = wl[o][i * 64 + lane];
+          mac_chunk(acc[o], as, bf, full);
         }
       };
-      Step c0;  // step on the matrix cores
-      c0.k = __builtin_ctz(uni);
-      c0.ch = 0;
-      c0.rest = uni & (uni - 1);
-      Step c1 = step_next(c0);
+      // Two steps' weights and gathers are in flight over the step on the matrix cores; weight buffers and gather
+      // slots go round in three turns, each a compile-time choice.
+      Step c0, c1, c2;
+      c0.k = -1;
+      c0.ch = nch;
+      c0.p = 0;
+      c0.rest = uni & hm[0];
+      c0 = step_next(c0);
+      c1 = step_next(c0);
       __builtin_amdgcn_sched_barrier(0);
-      w_issue0(c0);
+      w_issue(c0, wl0);
       __builtin_amdgcn_sched_barrier(0);
-      Frag a0 = gather(c0), a1;
+      Frag a0 = gather(c0), a1, a2;
       __builtin_amdgcn_sched_barrier(0);
-      // Before a barrier every wavefront waits until its own quarter of the step's weight tiles has
-      // landed in LDS: everything but the four gather loads issued after it (vmcnt(4); the order of
-      // the loads is pinned).
-      for (int s0 = 0; s0 < nsteps; s0 += 2) {
-        // even step: weights in wl0, chunk in a0
-        __builtin_amdgcn_s_waitcnt(0x0F74);
-        __syncthreads();  // W(s0) is complete for every wavefront, and nobody reads wl1 any more
+      w_issue(c1, wl1);
+      __builtin_amdgcn_sched_barrier(0);
+      a1 = gather(c1);
+      __builtin_amdgcn_sched_barrier(0);
+      // Before a barrier every wavefront waits until its own pieces of the step's weight tiles have
+      // landed in LDS: everything but what was issued after them - the step's four gather loads and the next
+      // step's (at least 6 NB / 4) pieces and four gather loads; the order of the loads is pinned.
+      auto turn = [&](Step &c, Step &cp2, const Frag &a, Frag &ap2, const Step &cp1, u32x4 (*wl)[6 * 64],
+                      u32x4 (*wlp2)[6 * 64]) {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (8 + 6 * NB / WV));
+        __syncthreads();  // the step's weights are complete for every wavefront, and nobody reads the oldest buffer any more
         __builtin_amdgcn_sched_barrier(0);
-        w_issue1(c1);
+        cp2 = step_next(cp1);
+        w_issue(cp2, wlp2);
         __builtin_amdgcn_sched_barrier(0);
-        a1 = gather(c1);
+        ap2 = gather(cp2);
         __builtin_amdgcn_sched_barrier(0);
-        compute(c0, a0, wl0);
-        c0 = step_next(c1);
-        // odd step: weights in wl1, chunk in a1
+        compute(c, a, wl);
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(0x0F74);
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        w_issue0(c0);
-        __builtin_amdgcn_sched_barrier(0);
-        a0 = gather(c0);
-        __builtin_amdgcn_sched_barrier(0);
-        compute(c1, a1, wl1);
-        c1 = step_next(c0);
-        __builtin_amdgcn_sched_barrier(0);
+      };
+      for (;;) {
+        turn(c0, c2, a0, a2, c1, wl0, wl2);
+        if (c1.k < 0) break;
+        turn(c1, c0, a1, a0, c2, wl1, wl0);
+        if (c2.k < 0) break;
+        turn(c2, c1, a2, a1, c0, wl2, wl1);
+        if (c0.k < 0) break;
       }
       __syncthreads();  // the weight buffers are free for the next unit
 
@@ -1528,6 +1445,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
         for (int o = 0; o < NB; o++) {
           const int cc = (ob0 + o) * 32 + r;
           if (ob0 + o >= nbt) break;
+          f16v sum = sum_of(acc[o]);
+          if (cur != 0) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) sum[v] = total[o][v] + sum[v];
+          }
+          repair_sums<16>(sum, [&](int v) -> float {
+            const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+            if (row < 0 || cc >= Cout) return 0.0f;
+            return plain_sum(bias ? bias[cc] : 0.0f, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, nch, nbtp, cc);
+          });
           float rv[16];
 #pragma unroll
           for (int v = 0; v < 16; v++)
@@ -1536,9 +1463,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
 #pragma unroll
           for (int v = 0; v < 16; v++) {
             const bool ok = rid[v] >= 0 && cc < Cout;
-            float a = acc[0][o][v];
-#pragma unroll
-            for (int pp = 1; pp < ST; pp++) a += acc[pp][o][v];
+            float a = sum[v];
             if (ep.res) a += rv[v];
             if (out)
               __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), rout,
@@ -1577,11 +1502,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB * ST > 4
 // D = items in flight per wavefront (2 with three wavefronts per SIMD; deeper rings at two wavefronts per
 // SIMD measured the same, and so did fewer wavefronts that draw their units from a counter: what the
 // launch lasts is the SIMD with the largest sum of items, hence the fixed assignment below).
-constexpr int OWN_WAVES = 12;  // one block per compute unit, three wavefronts per SIMD
+// (two wavefronts per SIMD: at three the sums, parts and weights do not fit the registers - 64 -> 64 at 39k sites
+// 55 us with 30 of them spilled against 47)
+constexpr int OWN_WAVES = 8;  // one block per compute unit
 template <int ST, int D>
-__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(3, 3))) void conv_own_kernel(
+__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_own_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
+    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
+    const int32_t *__restrict__ rows,
     const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
   constexpr int K = 27;
@@ -1594,6 +1522,10 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   const int nch = conv_nch(Cin);
   int *nl = nlb[wave];
   // (wavefronts are on their own: no workgroup barrier anywhere below)
+  // offsets that hold items of partial sum p
+  unsigned hm[ST];
+#pragma unroll
+  for (int p = 0; p < ST; p++) hm[p] = (unsigned)__ballot(lane < K && ((p - lane * nch) & (ST - 1)) < nch);
   // One block per compute unit; wavefront w sits on SIMD w % 4, so bin = (block, w % 4) names a SIMD and
   // turn = w / 4 one of its three wavefronts.  Units come by falling cost: the first turn hands them to the
   // bins in order, every later turn in reverse order, so the SIMDs that drew the expensive units of the
@@ -1633,24 +1565,31 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-  f16v acc[ST];
-#pragma unroll
-  for (int pp = 0; pp < ST; pp++) {
-#pragma unroll
-    for (int v = 0; v < 16; v++) acc[pp][v] = pp == 0 ? bv : 0.0f;
-  }
+  // the running partial sum and the sum of the finished ones; bias in partial sum 0
+  Sum acc;
+  sum_start(acc, bv);
+  f16v total;
+  int cur = 0;  // the partial sum in acc
   if (tmask) {
     struct Cursor {
-      int k, ch;
+      int k, ch, p;
       unsigned rest;
     };
     auto step = [&](const Cursor &cu) -> Cursor {  // past the end: k = -1
-      const bool wrap = cu.ch + 1 >= nch;
-      const int nk = cu.rest ? __builtin_ctz(cu.rest) : -1;
-      Cursor nx;
-      nx.ch = wrap ? 0 : cu.ch + 1;
-      nx.k = wrap ? nk : cu.k;
-      nx.rest = wrap ? (cu.rest & (cu.rest - 1)) : cu.rest;
+      Cursor nx = cu;
+      nx.ch = cu.ch + ST;
+      if (nx.ch >= nch || cu.k < 0) {
+#pragma unroll
+        for (int p = 1; p < ST; p++) {
+          if (nx.rest == 0 && nx.p < p) {
+            nx.p = p;
+            nx.rest = tmask & hm[p];
+          }
+        }
+        nx.k = nx.rest ? __builtin_ctz(nx.rest) : -1;
+        nx.ch = (nx.p - nx.k * nch) & (ST - 1);
+        nx.rest &= nx.rest - 1;
+      }
       return nx;
     };
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
@@ -1658,28 +1597,21 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
     auto gather = [&](const Cursor &cu) -> Frag {
       const int kk = cu.k < 0 ? 0 : cu.k;
       const int src = nl[kk * TILE_M + r];
-      const bool on = cu.k >= 0 && src >= 0 && (h == 0 || Cin - cu.ch * 32 >= 32);
-      const uint32_t voff = on ? (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128 + h * 64) : BUF_OOB;
-      Frag f;
-#pragma unroll
-      for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rin, voff + 16u * q, 0);
-      return f;
+      return gather_chunk(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), h,
+                          Cin - cu.ch * 32 >= 32);
     };
-    auto wload = [&](const Cursor &cu) -> Frag {
-      const int wt = ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob;
-      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(wt * 4096);
-      const uint32_t voff = cu.k >= 0 ? lane16 : BUF_OOB;
-      Frag f;
-#pragma unroll
-      for (int q = 0; q < 4; q++) f.q[q] = buf_load16(rw, voff + 1024u * q, soff);
-      return f;
+    auto wload = [&](const Cursor &cu) -> WFrag {
+      return load_wtile(rw, ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob, cu.k >= 0, lane16);
     };
     const int nitems = __builtin_popcount(tmask) * nch;
     Cursor first;
-    first.k = __builtin_ctz(tmask);
-    first.ch = 0;
-    first.rest = tmask & (tmask - 1);
-    Frag g[D], bw[D];
+    first.k = -1;
+    first.ch = nch;
+    first.p = 0;
+    first.rest = tmask & hm[0];
+    first = step(first);
+    Frag g[D];
+    WFrag bw[D];
     Cursor ci = first, c0 = first;
 #pragma unroll
     for (int d = 0; d < D - 1; d++) {
@@ -1693,16 +1625,19 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
         g[(uu + D - 1) % D] = gather(ci);
         bw[(uu + D - 1) % D] = wload(ci);
         ci = step(ci);
-        // which partial sum the item on the matrix cores belongs to (-1 past the last item)
-        const int part = t0i + uu < nitems ? ((c0.k * nch + c0.ch) & (ST - 1)) : -1;
+        const bool full = Cin - c0.ch * 32 >= 32;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        if (t0i + uu < nitems) {
+          if (c0.p != cur) {
+            const f16v part = sum_of(acc);
 #pragma unroll
-        for (int pp = 0; pp < ST; pp++) {
-          if (part != pp) continue;  // (one copy of the MFMA block per partial sum: the accumulator is a compile-time choice)
-#pragma unroll
-          for (int s2 = 0; s2 < 16; s2++)
-            acc[pp] = __builtin_amdgcn_mfma_f32_32x32x2f32(frag_at(g[uu], s2), frag_at(bw[uu], s2), acc[pp], 0, 0, 0);
+            for (int v = 0; v < 16; v++) total[v] = cur == 0 ? part[v] : total[v] + part[v];
+            sum_start(acc, 0.0f);
+            cur = c0.p;
+          }
+          const Parts as[2] = {split8(g[uu].q[0], g[uu].q[1]), split8(g[uu].q[2], g[uu].q[3])};
+          mac_chunk(acc, as, bw[uu], full);
         }
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -1717,6 +1652,16 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   int rid[16];
 #pragma unroll
   for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+  f16v sum = sum_of(acc);
+  if (cur != 0) {
+#pragma unroll
+    for (int v = 0; v < 16; v++) sum[v] = total[v] + sum[v];
+  }
+  repair_sums<16>(sum, [&](int v) -> float {
+    const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+    if (row < 0 || c >= Cout) return 0.0f;
+    return plain_sum(bv, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, nch, nbtp, c);
+  });
   float rv[16];
 #pragma unroll
   for (int v = 0; v < 16; v++)
@@ -1725,9 +1670,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int v = 0; v < 16; v++) {
     const bool ok = rid[v] >= 0 && c < Cout;
-    float a = acc[0][v];
-#pragma unroll
-    for (int pp = 1; pp < ST; pp++) a += acc[pp][v];
+    float a = sum[v];
     if (ep.res) a += rv[v];
     if (out)
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), rout,
@@ -1935,23 +1878,19 @@ static bool conv_uses_mfma(const float *in, int64_t ld_in, int Cin, int K) {
 }
 
 int64_t packed_floats(int K, int Cin, int Cout) {
-  return (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * 1024;
+  return (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * (WT_BYTES / 4);
 }
 
 int pack_weights(const float *W, int K, int Cin, int Cout, float *Wp, hipStream_t s) {
-  const int64_t total = packed_floats(K, Cin, Cout);
+  const int64_t total = (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * 1024;
   hipLaunchKernelGGL(pack_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, K, Cin, Cout,
-                     conv_nch(Cin), conv_nbt_padded(Cout), Wp);
+                     conv_nch(Cin), conv_nbt_padded(Cout), reinterpret_cast<uint16_t *>(Wp));
   INSC_LAUNCH_CHECK();
   return INSC_OK;
 }
 
 // Launch policy of wide 3^3 layers (64..159 input channels, a tile schedule).  All kernels give the same
 // bits; the bounds only move time.
-// The persistent kernel is off by default: since the one-block-per-unit kernel keeps two items in flight
-// and numbers its blocks for balance across the compute units it is the faster one at every size measured
-// (96 -> 96 at 10k sites: 37 us against 43 us; 64 -> 64 at 21k sites: 36 against 46).
-static std::atomic<int64_t> g_pers_min_units{INT64_MAX};
 // With at least this many (group of four tiles, output block) units: the kernel whose blocks share the
 // weight tiles through LDS (faster from about 60k sites at 64 channels).
 static std::atomic<int64_t> g_shared_min_units{896};
@@ -2038,8 +1977,12 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       // persistent blocks, a multiple of the XCD count, at most one per compute unit
       const int64_t want = cdiv(tiles, WL_WAVES);
       const unsigned nblk = (unsigned)std::min<int64_t>(device_cus(), want);
-      hipLaunchKernelGGL(conv_wlds_kernel, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias,
-                         map0, rows, d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, ep, plan);
+      if (Cin == 16)
+        hipLaunchKernelGGL(conv_wlds_kernel<1>, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias,
+                           map0, rows, d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, wp_bytes, ep, plan);
+      else
+        hipLaunchKernelGGL(conv_wlds_kernel<2>, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias,
+                           map0, rows, d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, wp_bytes, ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
     }
@@ -2088,7 +2031,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
         }
         const int64_t wunits = cdiv(tiles, 4) * cdiv(nbt, 2);
         const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu4, wunits);
-        hipLaunchKernelGGL((conv_wshare_kernel<2, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
+        hipLaunchKernelGGL((conv_wshare_kernel<2, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, map0, rows,
                            d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
         INSC_LAUNCH_CHECK();
         return INSC_OK;
@@ -2100,7 +2043,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       }
       const int64_t wunits = cdiv(tiles, 4) * nbt;
       const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu2, wunits);
-      hipLaunchKernelGGL((conv_wshare_kernel<1, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
+      hipLaunchKernelGGL((conv_wshare_kernel<1, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, map0, rows,
                          d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
@@ -2109,21 +2052,8 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     if (wide_planned && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
       // one wavefront per (tile, output block): enough units that every SIMD gets one to three
       hipLaunchKernelGGL((conv_own_kernel<4, 2>), dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
-                         ld_out, Wp, bias, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep,
-                         plan);
-      INSC_LAUNCH_CHECK();
-      return INSC_OK;
-    }
-    if (wide_planned && tiles * nbt >= g_pers_min_units.load(std::memory_order_relaxed)) {
-      // persistent blocks, as many as fit on the device at once
-      static int per_cu = 0;
-      if (!per_cu) {
-        INSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, conv_pers_kernel<4>, 256, 0));
-        if (per_cu < 1) per_cu = 1;
-      }
-      const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu, tiles * nbt);
-      hipLaunchKernelGGL(conv_pers_kernel<4>, dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
-                         d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
+                         ld_out, Wp, bias, map0, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes,
+                         ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
     }
@@ -2231,9 +2161,9 @@ using namespace insc;
 
 extern "C" {
 
+// (kept for callers: the kernel that this bound chose was the slower one at every size and is gone)
 int insc_conv_set_persistent_min_units(int64_t units) {
   INSC_REQUIRE(units >= 1, INSC_ERR_ARG, "insc_conv_set_persistent_min_units: units must be >= 1");
-  g_pers_min_units.store(units, std::memory_order_relaxed);
   return INSC_OK;
 }
 

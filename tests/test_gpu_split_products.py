@@ -1,0 +1,120 @@
+"""fp32 products as sums of bf16 products (csrc/conv.hip): what such a sum can get wrong - infinities and NaN,
+magnitudes far from one, the error against 64-bit sums - on every matrix-core kernel."""
+import numpy as np
+import pytest
+import torch
+
+from workloads import scenes
+
+pytestmark = pytest.mark.gpu
+SZ = torch.LongTensor([4096, 4096, 4096])
+NEVER = 1 << 40
+# (Cin, Cout, filter-in-LDS from, wavefront per unit from, shared weights from): one kernel each
+KERNELS = [(16, 16, 1, NEVER, NEVER), (32, 32, 1, NEVER, NEVER), (32, 20, NEVER, NEVER, NEVER), (48, 64, NEVER, NEVER, NEVER),
+           (64, 64, NEVER, 1, NEVER), (64, 96, NEVER, NEVER, 1), (80, 32, NEVER, NEVER, 1), (96, 64, NEVER, NEVER, NEVER),
+           (128, 128, NEVER, NEVER, NEVER), (160, 100, NEVER, NEVER, NEVER)]
+
+
+@pytest.fixture(scope="module")
+def scene():
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import ensure_init
+
+    ensure_init(0)
+    pts = scenes.boxes_scene(seed=7, n=2300)
+    m = S.Metadata_3()
+    out = torch.empty(0, device="cuda")
+    S.InputLayer_updateOutput(m, SZ, torch.from_numpy(pts.astype(np.int64)), torch.ones((len(pts), 1), device="cuda"), out, 0, 4)
+    sc = m.ssc_rulebook(SZ)
+    return S, m, sc, sc.nbr.t[:sc.n].cpu().numpy()
+
+
+def layer(scene, x, W, b, case):
+    from sparseconvnet._lib import lib
+
+    S, m, sc, _ = scene
+    out = torch.full((sc.n, W.shape[2]), 7.0, device="cuda")
+    try:
+        lib.insc_conv_set_filter_lds_min_tiles(case[2])
+        lib.insc_conv_set_wavefront_per_unit_min_units(case[3])
+        lib.insc_conv_set_shared_weights_min_units(case[4])
+        S.ssc_rows_planned(torch.from_numpy(x).cuda(), out, torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda(), sc, m.ssc_plan(sc))
+    finally:
+        lib.insc_conv_set_filter_lds_min_tiles(4096)
+        lib.insc_conv_set_wavefront_per_unit_min_units(1750)
+        lib.insc_conv_set_shared_weights_min_units(896)
+    return out.cpu().numpy()
+
+
+def sums64(nbr, x, W, b):
+    ref = np.tile(b.astype(np.float64), (len(nbr), 1))
+    for k in range(27):
+        i = np.flatnonzero(nbr[:, k] >= 0)
+        with np.errstate(invalid="ignore"):
+            ref[i] += x[nbr[i, k]].astype(np.float64) @ W[k].astype(np.float64)
+    return ref
+
+
+def data(scene, case):
+    rng = np.random.default_rng(case[0] + case[1])
+    n = scene[2].n
+    x = rng.normal(size=(n, case[0])).astype(np.float32)
+    W = (rng.normal(size=(27,) + case[:2]) * (2.0 / case[0] / 27) ** 0.5).astype(np.float32)
+    return rng, x, W, rng.normal(size=case[1]).astype(np.float32)
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_error_against_64_bit_sums(scene, case):
+    """Per element: each fp32 rounding of the running sum is half a unit in the last place of a partial sum, which
+    |b| + sum |x||w| bounds; there are at most 27 * Cin / 8 of them in a fp32 chain of this length."""
+    _, x, W, b = data(scene, case)
+    got, nbr = layer(scene, x, W, b, case), scene[3]
+    ref, mag = sums64(nbr, x, W, b), sums64(nbr, np.abs(x), np.abs(W), np.abs(b))
+    err = np.abs(got - ref)
+    assert (err <= 2.0 ** -24 * 27 * case[0] / 8 * mag).all()
+    # and over all of them: no more than a chain of fp32 multiply-adds, which rounds its sum once per product, shows on
+    # a sample of the same rows (here it is rounded once per 16 channels: a quarter of that is expected)
+    some = np.random.default_rng(1).integers(0, len(x), 200)
+    acc = np.tile(b, (len(some), 1))
+    for k in range(27):
+        src = nbr[some, k]
+        for ci in range(case[0]):
+            step = (x[src, ci].astype(np.float64)[:, None] * W[k, ci].astype(np.float64) + acc).astype(np.float32)
+            acc = np.where(src[:, None] >= 0, step, acc)
+    assert np.linalg.norm(err[some]) <= np.linalg.norm(acc - ref[some])
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_magnitudes_far_from_one(scene, case):
+    """Powers of two move through exactly: three parts of eight bits each keep the whole exponent range."""
+    _, x, W, b = data(scene, case)
+    base = layer(scene, x, W, b, case)
+    for e in (-60, 60):
+        s = np.float32(2.0 ** e)
+        assert (layer(scene, x * s, W, b * s, case) == base * s).all()
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_infinities_and_nan(scene, case):
+    """An infinity stays one (three parts of it would be infinity minus infinity), NaN stays NaN, and no
+    other row changes."""
+    rng, x, W, b = data(scene, case)
+    base = layer(scene, x, W, b, case)
+    n = len(x)
+    x[rng.integers(0, n, 5), rng.integers(0, case[0], 5)] = np.inf
+    x[rng.integers(0, n, 5), rng.integers(0, case[0], 5)] = -np.inf
+    x[rng.integers(0, n, 3), rng.integers(0, case[0], 3)] = np.nan
+    got, ref = layer(scene, x, W, b, case), sums64(scene[3], x, W, b)
+    assert np.isinf(ref).any() and np.isnan(ref).any()
+    fin = np.isfinite(ref)
+    assert (got[fin] == base[fin]).all()
+    assert (np.isnan(got) == np.isnan(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
+    # the largest floats: their upper halves would round to infinity
+    _, x, W, b = data(scene, case)
+    x[7, 0] = np.float32(3.4e38)
+    W[:, 0, :] = np.clip(W[:, 0, :], -0.01, 0.01)
+    W[13, 1, 0] = np.float32(-3.4e38)
+    x[:, 1] = 0
+    got, ref = layer(scene, x, W, b, case), sums64(scene[3], x, W, b)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - ref) <= 1e-5 * np.abs(ref) + 1e-4 * np.abs(sums64(scene[3], np.minimum(np.abs(x), 9), np.minimum(np.abs(W), 9), b))).all()
