@@ -197,6 +197,13 @@ int insc_conv_nbr(const float *d_in, int64_t ld_in, int64_t n_in_rows, float *d_
  * insc_conv_packed_floats gives the size of d_Wp in floats. */
 int64_t insc_conv_packed_floats(int K, int Cin, int Cout);
 int insc_conv_pack_weights(const float *d_W, int K, int Cin, int Cout, float *d_Wp, void *stream);
+/* The layout the kernels themselves read: every weight as three bf16 parts whose sum is exactly the weight
+ * (insc_conv_split_floats floats, 16-byte aligned).  Every d_Wp argument takes such weights as well: pass their address
+ * with its lowest bit set, INSC_SPLIT_WEIGHTS(d_Ws).  Packed fp32 weights are split on every call instead, into
+ * scratch memory. */
+int64_t insc_conv_split_floats(int K, int Cin, int Cout);
+int insc_conv_split_weights(const float *d_W, int K, int Cin, int Cout, float *d_Ws, void *stream);
+#define INSC_SPLIT_WEIGHTS(d_Ws) ((const float *)((uintptr_t)(d_Ws) | 1))
 /* Tile plan of a 3^3 neighbour map for one processing order (no counterpart in the reference;
  * its chunk rulebook, SubmanifoldRules_cuda.cpp:572-1112, plays this role for its kernel):
  * d_plan[k*plan_ld + p] = d_nbr[d_order[p]*27 + k] for p < n_rows and -1 up to the next multiple of
@@ -216,13 +223,13 @@ int insc_conv_ssc_plan(const float *d_in, int64_t ld_in, int64_t n_in_rows, floa
                        const int32_t *d_order, const int32_t *d_n_rows, int64_t n_rows, int Cin, int Cout,
                        void *stream);
 /* Launch policy of a 3^3 layer of 64..159 input channels with a tile schedule: by default one block per
- * (tile, 32-column output block) pair; persistent blocks once it has at least `units` pairs (off by
- * default: the one-block-per-pair kernel measures faster at every size); with at least `units` (four
- * consecutive tiles, output block) pairs (default 896) the kernel whose blocks share the weight tiles
- * through LDS.  Same bits in all cases: tuning and test knobs with no counterpart in the reference. */
+ * (tile, 32-column output block) pair; with at least `units` (four consecutive tiles, output block) pairs
+ * (default 896) the kernel whose blocks share the weight tiles through LDS.  Same bits in all cases: tuning and
+ * test knobs with no counterpart in the reference.  (The persistent-block kernel that the first one chose was slower
+ * at every size and is gone; the call is accepted and changes nothing.) */
 int insc_conv_set_persistent_min_units(int64_t units);
 int insc_conv_set_shared_weights_min_units(int64_t units);
-/* ... and between the two, from `units` (tile, output block) pairs up (default 2400; half as many again
+/* ... and between the two, from `units` (tile, output block) pairs up (default 1750; half as many again
  * for more than 64 input channels), on the kernel that gives every pair a wavefront of its own.  Same
  * bits again. */
 int insc_conv_set_wavefront_per_unit_min_units(int64_t units);

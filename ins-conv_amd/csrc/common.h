@@ -148,7 +148,14 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
 bool conv_two_sources_ok(int mode, int K, const float *in, int64_t ld_in, const float *in2, int64_t ld_in2,
                          int64_t in2_rows, int Cin, int latency);
 int64_t packed_floats(int K, int Cin, int Cout);
-int pack_weights(const float *W, int K, int Cin, int Cout, float *Wp, hipStream_t s);
+int64_t split_floats(int K, int Cin, int Cout);
+// Ws = the three-part layout of raw weights W, or of packed ones Wp
+int split_weights(const float *W, const float *Wp, int K, int Cin, int Cout, float *Ws, hipStream_t s);
+// A pointer to weights in the three-part layout, where packed weights are asked for: the address (16-byte aligned)
+// with its lowest bit set.
+static inline const float *split_ref(const float *Ws) { return Ws ? (const float *)((uintptr_t)Ws | 1) : nullptr; }
+static inline bool is_split(const float *p) { return ((uintptr_t)p & 1) != 0; }
+static inline const float *split_address(const float *p) { return (const float *)((uintptr_t)p & ~(uintptr_t)1); }
 int launch_bn(const float *in, int64_t ld_in, float *out, int64_t ld_out, const float *mean, const float *var,
               const float *gamma, const float *beta, float eps, float leak, const int32_t *rows,
               const int32_t *d_n_rows, int64_t n_rows, int C, const uint8_t *row_mask, hipStream_t s);

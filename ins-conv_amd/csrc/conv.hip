@@ -253,8 +253,25 @@ __device__ __forceinline__ unsigned bf16_part(float x) {
   return (up & 0x7F80u) == 0x7F80u ? u >> 16 : up;
 }
 
+// The fp32 layout of insc_conv_pack_weights: a tile is 4 KB, four 1 KB quarters; quarter q holds, for lane 0..63 in
+// turn, the values W[k][ch*32 + h*16 + s][nb*32 + j], s = 4q..4q+3.
 __global__ void pack_weights_kernel(const float *__restrict__ W, int K, int Cin, int Cout, int nch, int nbtp,
-                                    uint16_t *__restrict__ Wp) {
+                                    float *__restrict__ Wp) {
+  const int64_t total = (int64_t)K * nch * nbtp * 1024;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
+    const int s = (int)(((e >> 8) & 3) * 4 + (e & 3)), lane = (int)((e >> 2) & 63);
+    int64_t q = e >> 10;
+    const int nb = (int)(q % nbtp);
+    q /= nbtp;
+    const int ch = (int)(q % nch), k = (int)(q / nch);
+    const int cin = ch * 32 + (lane >> 5) * 16 + s, col = nb * 32 + (lane & 31);
+    Wp[e] = (cin < Cin && col < Cout) ? W[((int64_t)k * Cin + cin) * Cout + col] : 0.0f;
+  }
+}
+
+// The three-part layout that the kernels read, from raw weights (W) or from the fp32 layout (Wp).
+__global__ void split_weights_kernel(const float *__restrict__ W, const float *__restrict__ Wp, int K, int Cin, int Cout,
+                                     int nch, int nbtp, uint16_t *__restrict__ Ws) {
   const int64_t total = (int64_t)K * nch * nbtp * 1024;  // one (lane, value) of all three parts per thread
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
     const int j8 = (int)(e & 7), lane = (int)((e >> 3) & 63), s = (int)((e >> 9) & 1);
@@ -263,9 +280,12 @@ __global__ void pack_weights_kernel(const float *__restrict__ W, int K, int Cin,
     const int nb = (int)(q % nbtp);
     q /= nbtp;
     const int ch = (int)(q % nch), k = (int)(q / nch);
-    const int cin = ch * 32 + s * 16 + (lane >> 5) * 8 + j8, col = nb * 32 + (lane & 31);
-    float x = (cin < Cin && col < Cout) ? W[((int64_t)k * Cin + cin) * Cout + col] : 0.0f;
-    uint16_t *to = Wp + tile * (WT_BYTES / 2) + s * 1536 + lane * 8 + j8;
+    const int cin32 = s * 16 + (lane >> 5) * 8 + j8, cin = ch * 32 + cin32, col = nb * 32 + (lane & 31);
+    float x = 0.0f;
+    if (cin < Cin && col < Cout)
+      x = Wp ? Wp[tile * 1024 + ((cin32 >> 2) & 3) * 256 + ((cin32 >> 4) * 32 + (lane & 31)) * 4 + (cin32 & 3)]
+             : W[((int64_t)k * Cin + cin) * Cout + col];
+    uint16_t *to = Ws + tile * (WT_BYTES / 2) + s * 1536 + lane * 8 + j8;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
       const unsigned u = bf16_part(x);
@@ -890,6 +910,9 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
 // room for a copy, and none is needed: lane r only ever wants the ids of row r).
 // The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (centre, then offsets ascending, same
 // MFMA sequence), so both kernels give the same bits.
+// What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in about 105 us a layer (6 TB/s; a pure
+// gather reaches 8.7), against 25 us of matrix-core time; 115 us with fp32 instructions, whose 65 us it also waited for.
+// (A contiguous eighth of the tiles per XCD instead of interleaved ones: 531 against 511 us for four layers.)
 // ---------------------------------------------------------------------------------------
 // (32 -> 32 in four layers with their batch norms, 500k / 150k sites: eight wavefronts 542 / 228 us, twelve 538 / 201;
 // rings of three and four items, which spill at twelve wavefronts, 589 / 232 and 667 / 253)
@@ -1196,21 +1219,23 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Wide 3^3 layers with many tiles, second design: the bytes a compute unit pulls through its L1
-// bound these layers (8 KB per 16 MFMAs: a gathered chunk and a weight tile), so here the four
-// wavefronts of a block work on four consecutive tiles and walk the union of their offsets in
-// step: the weight tile of a step goes from L2 into LDS once per block (buffer loads that write
-// LDS directly, a quarter per wavefront) and is read from there by all four, and a wavefront
-// computes NB output blocks from one gathered chunk.  A wavefront owns its tile: no partial sums
-// cross wavefronts.  To give the bits of conv_mfma_kernel<1, 27, MAP_NBR, ST> it keeps that
-// kernel's ST partial sums - the items (k, ch) with (k * nch + ch) % ST == p, in ascending order,
-// bias in sum 0 - in ST accumulators per output block and adds them in order at the end.
+// Wide 3^3 layers with many tiles: the four wavefronts of a block work on four consecutive tiles and walk the union
+// of their offsets in step: the weight tile of a step goes from L2 into LDS once per block (buffer loads that write
+// LDS directly, 1 KB pieces dealt to the wavefronts) and is read from there by all four, and a wavefront
+// computes NB output blocks from one gathered chunk, split into parts once.  A wavefront owns its tile: no partial
+// sums cross wavefronts.  To give the bits of conv_mfma_kernel<1, 27, MAP_NBR, ST> it forms that kernel's ST partial
+// sums - the items (k, ch) with (k * nch + ch) % ST == p, in ascending order, bias in sum 0 - one after the other and
+// adds each to the total when it is done: two accumulators per output block, whatever ST.
 // Blocks are persistent over units (group of four tiles, NB output blocks) taken from the cost-
 // ordered group schedule: block b takes the units b, 2B - 1 - b, 2B + b, ..
-// The two weight buffers and the two A slots alternate with the parity of the step, and the step
-// loop is unrolled by two so that each is a compile-time choice: the compiler then knows that a
-// read of one weight buffer cannot touch the load into the other that is still in flight (for a
-// single array it would wait for every outstanding load before each LDS read).
+// Weights and gathers of two steps are in flight over the step on the matrix cores; the three weight buffers and A
+// slots are compile-time choices (the step loop is unrolled by three): the compiler then knows that a read of one
+// weight buffer cannot touch a load into another that is still in flight (for a single array it would wait for every
+// outstanding load before each LDS read).
+// What bounds it (64 -> 64 at 500k sites, four layers with batch norms 1920 us in fp32, 1435-1500 now): 2.5 GB through
+// L1 per launch at 7.5 TB/s, 45 % of the requests beyond L2; matrix cores busy 34 %, VALU 36 %.  Eight tiles per block,
+// which halves the weight bytes: 1542 us (the wavefronts wait for one another); units in site order per XCD, which
+// would hit L2: 1741 us (unbalanced).
 // ---------------------------------------------------------------------------------------
 #define INSC_LDS_PTR(x) ((__attribute__((address_space(3))) void *)(x))
 template <int NB, int ST>
@@ -1494,10 +1519,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 // Wide 3^3 layers of middling size (a few hundred to a few thousand tiles): one wavefront per unit
 // (tile, output block), nothing shared between wavefronts - no barrier, no partial sums through LDS,
 // no wait for the slowest of four.  To give the bits of conv_mfma_kernel<1, 27, MAP_NBR, ST> the
-// wavefront keeps that kernel's ST partial sums - the items (k, ch) with (k * nch + ch) % ST == p, in
-// ascending order, bias in sum 0 - in ST accumulators and adds them in order at the end.  Units
+// wavefront forms that kernel's ST partial sums one after the other (as the kernel above).  Units
 // follow the cost-ordered tile schedule, output blocks of a tile side by side on neighbouring SIMDs of
 // one compute unit, so they meet the tile's map slice and gathered rows in L1.
+// What bounds it: 10 KB through L1 per item (4 KB of rows, 6 KB of weights): 64 -> 64 at 39k sites 53 -> 48 us.
 // ---------------------------------------------------------------------------------------
 // D = items in flight per wavefront (2 with three wavefronts per SIMD; deeper rings at two wavefronts per
 // SIMD measured the same, and so did fewer wavefronts that draw their units from a counter: what the
@@ -1527,7 +1552,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int p = 0; p < ST; p++) hm[p] = (unsigned)__ballot(lane < K && ((p - lane * nch) & (ST - 1)) < nch);
   // One block per compute unit; wavefront w sits on SIMD w % 4, so bin = (block, w % 4) names a SIMD and
-  // turn = w / 4 one of its three wavefronts.  Units come by falling cost: the first turn hands them to the
+  // turn = w / 4 one of its two wavefronts.  Units come by falling cost: the first turn hands them to the
   // bins in order, every later turn in reverse order, so the SIMDs that drew the expensive units of the
   // first turn get the cheap ones afterwards (largest sum of a SIMD at 39k sites and 64 channels: 72 items against
   // 90 when every SIMD takes three units in a row; 66 is the best any assignment reaches).
@@ -1878,13 +1903,22 @@ static bool conv_uses_mfma(const float *in, int64_t ld_in, int Cin, int K) {
 }
 
 int64_t packed_floats(int K, int Cin, int Cout) {
-  return (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * (WT_BYTES / 4);
+  return (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * 1024;
+}
+int64_t split_floats(int K, int Cin, int Cout) { return packed_floats(K, Cin, Cout) / 1024 * (WT_BYTES / 4); }
+
+static int pack_weights(const float *W, int K, int Cin, int Cout, float *Wp, hipStream_t s) {
+  const int64_t total = packed_floats(K, Cin, Cout);
+  hipLaunchKernelGGL(pack_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, K, Cin, Cout,
+                     conv_nch(Cin), conv_nbt_padded(Cout), Wp);
+  INSC_LAUNCH_CHECK();
+  return INSC_OK;
 }
 
-int pack_weights(const float *W, int K, int Cin, int Cout, float *Wp, hipStream_t s) {
-  const int64_t total = (int64_t)K * conv_nch(Cin) * conv_nbt_padded(Cout) * 1024;
-  hipLaunchKernelGGL(pack_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, K, Cin, Cout,
-                     conv_nch(Cin), conv_nbt_padded(Cout), reinterpret_cast<uint16_t *>(Wp));
+int split_weights(const float *W, const float *Wp, int K, int Cin, int Cout, float *Ws, hipStream_t s) {
+  const int64_t total = packed_floats(K, Cin, Cout);
+  hipLaunchKernelGGL(split_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, Wp, K, Cin, Cout,
+                     conv_nch(Cin), conv_nbt_padded(Cout), reinterpret_cast<uint16_t *>(Ws));
   INSC_LAUNCH_CHECK();
   return INSC_OK;
 }
@@ -1905,8 +1939,8 @@ static std::atomic<int64_t> g_own_min_units{1750};
 // Same bits either way.
 static std::atomic<int64_t> g_wl_min_tiles{WL_MIN_TILES};
 
-// W: raw [K,Cin,Cout] weights (always needed by the generic kernel); Wp: packed weights or
-// null, in which case they are packed into scratch memory first.
+// W: raw [K,Cin,Cout] weights (always needed by the generic kernel); Wp: split weights (split_ref), or packed
+// fp32 ones or null, in which case their parts are made in scratch memory first.
 // Whether one launch can gather from two sources (BnEpilogue::src2_*): the shapes that the split
 // kernel serves - 3^3 layers of a residual frame (latency != 0) and stride-2 deconvolutions, from 32
 // input channels on.
@@ -1943,18 +1977,21 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
   plan.cus = (unsigned)device_cus();
   if (conv_uses_mfma(in, ld_in, Cin, K)) {
     // the gather addresses rows with 32-bit byte offsets (buffer loads)
-    const int64_t in_bytes64 = in_rows * ld_in * 4, wp_bytes64 = packed_floats(K, Cin, Cout) * 4;
+    const int64_t in_bytes64 = in_rows * ld_in * 4, wp_bytes64 = split_floats(K, Cin, Cout) * 4;
     if (in_rows < 0 || in_bytes64 >= (int64_t)BUF_OOB || wp_bytes64 >= (int64_t)BUF_OOB) {
       set_error("conv: input matrix (%lld rows x %lld floats) or weights exceed the 4 GB the kernel addresses",
                 (long long)in_rows, (long long)ld_in);
       return INSC_ERR_ARG;
     }
     const uint32_t in_bytes = (uint32_t)in_bytes64, wp_bytes = (uint32_t)wp_bytes64;
-    if (!Wp) {
+    if (is_split(Wp)) {
+      Wp = split_address(Wp);
+    } else {
+      // raw weights, or packed ones in fp32: their parts are made for this call
       void *ws;
-      int rc = workspace(WS_API, s, sizeof(float) * (size_t)packed_floats(K, Cin, Cout), &ws);
+      int rc = workspace(WS_API, s, sizeof(float) * (size_t)split_floats(K, Cin, Cout), &ws);
       if (rc) return rc;
-      rc = pack_weights(W, K, Cin, Cout, (float *)ws, s);
+      rc = split_weights(W, Wp, K, Cin, Cout, (float *)ws, s);
       if (rc) return rc;
       Wp = (const float *)ws;
     }
@@ -2194,6 +2231,17 @@ int insc_conv_pack_weights(const float *d_W, int K, int Cin, int Cout, float *d_
   INSC_REQUIRE(d_W && d_Wp && K > 0 && K <= MAXK && Cin > 0 && Cout > 0, INSC_ERR_ARG,
                "insc_conv_pack_weights: bad arguments");
   return pack_weights(d_W, K, Cin, Cout, d_Wp, (hipStream_t)stream);
+}
+
+int64_t insc_conv_split_floats(int K, int Cin, int Cout) {
+  if (K <= 0 || Cin <= 0 || Cout <= 0) return 0;
+  return split_floats(K, Cin, Cout);
+}
+
+int insc_conv_split_weights(const float *d_W, int K, int Cin, int Cout, float *d_Ws, void *stream) {
+  INSC_REQUIRE(d_W && d_Ws && K > 0 && K <= MAXK && Cin > 0 && Cout > 0 && ((uintptr_t)d_Ws & 15) == 0, INSC_ERR_ARG,
+               "insc_conv_split_weights: bad arguments");
+  return split_weights(d_W, nullptr, K, Cin, Cout, d_Ws, (hipStream_t)stream);
 }
 
 int insc_conv_nbr(const float *d_in, int64_t ld_in, int64_t n_in_rows, float *d_out, int64_t ld_out,

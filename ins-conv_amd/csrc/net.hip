@@ -67,7 +67,7 @@ struct Tensor {
 struct Op {
   int kind = 0, in0 = -1, in1 = -1, out = -1;
   const float *W = nullptr, *bias = nullptr, *mean = nullptr, *var = nullptr, *gamma = nullptr, *beta = nullptr;
-  float *Wp = nullptr;  // packed weights, owned
+  float *Wp = nullptr;  // weights in the three-part layout, owned
   float eps = 0, leak = 0;
   int Cin = 0, Cout = 0;
   // batch norm folded into the kernel that produces its input
@@ -577,26 +577,26 @@ static int run_op(insc_net *net, const Op &op, bool incremental, hipStream_t s) 
   switch (op.kind) {
     case OP_SSC: {
       if (d && d->compact)  // tiles made of the set's rows only (no tile plan: its positions are the full order's)
-        return launch_conv(in0, ld0, rows0, out, ld_out, op.W, op.Wp, op.bias, Lo.nbr, nullptr, MAP_NBR, 27, d->crows,
+        return launch_conv(in0, ld0, rows0, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lo.nbr, nullptr, MAP_NBR, 27, d->crows,
                            d->ccount, n_up, op.Cin, op.Cout, nullptr, d->mask, s, ep, TilePlan(), 0, d->expect_rows);
       TilePlan plan;
       plan.map = Lo.plan;
       plan.ld = Lo.cap;
       plan.tmask = Lo.tmask;
       plan.sched = Lo.sched;
-      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, op.Wp, op.bias, Lo.nbr, nullptr, MAP_NBR, 27, Lo.order, d_n,
+      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lo.nbr, nullptr, MAP_NBR, 27, Lo.order, d_n,
                          n_up, op.Cin, op.Cout, d ? d->tflag : nullptr, d ? d->mask : nullptr, s, ep, plan);
     }
     case OP_NIN:
-      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, op.Wp, op.bias, nullptr, nullptr, MAP_IDENTITY, 1, Lo.order,
+      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, split_ref(op.Wp), op.bias, nullptr, nullptr, MAP_IDENTITY, 1, Lo.order,
                          d_n, n_up, op.Cin, op.Cout, d ? d->tflag : nullptr, d ? d->mask : nullptr, s, ep);
     case OP_CONV: {
       const Level &Lf = net->levels[To.level - 1];
-      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, op.Wp, op.bias, Lf.child, nullptr, MAP_NBR, 8, Lo.order, d_n,
+      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lf.child, nullptr, MAP_NBR, 8, Lo.order, d_n,
                          n_up, op.Cin, op.Cout, d ? d->tflag : nullptr, d ? d->mask : nullptr, s, ep);
     }
     case OP_DECONV:
-      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, op.Wp, op.bias, Lo.parent, Lo.offset, MAP_PARENT, 8,
+      return launch_conv(in0, ld0, rows0, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lo.parent, Lo.offset, MAP_PARENT, 8,
                          Lo.bo_order, d_n, n_up, op.Cin, op.Cout, d ? d->tflag_bo : nullptr, d ? d->mask : nullptr,
                          s, ep);
     case OP_BN:
@@ -943,10 +943,10 @@ int insc_net_finalize(insc_net *net, int out_tensor, int64_t capacity_sites, voi
     if (op.kind == OP_SSC || op.kind == OP_CONV || op.kind == OP_DECONV || op.kind == OP_NIN) {
       const int K = op.kind == OP_SSC ? 27 : op.kind == OP_NIN ? 1 : 8;
       if (op.Cin % 16 == 0) {
-        const int64_t nf = packed_floats(K, op.Cin, op.Cout);
+        const int64_t nf = split_floats(K, op.Cin, op.Cout);
         int rc = dev_alloc(&op.Wp, (size_t)nf);
         if (rc) return rc;
-        rc = pack_weights(op.W, K, op.Cin, op.Cout, op.Wp, s);
+        rc = split_weights(op.W, nullptr, K, op.Cin, op.Cout, op.Wp, s);
         if (rc) return rc;
       }
     }
@@ -1076,7 +1076,7 @@ int insc_net_refresh_weights(insc_net *net, void *stream) {
   for (Op &op : net->ops)
     if (op.Wp) {
       const int K = op.kind == OP_SSC ? 27 : op.kind == OP_NIN ? 1 : 8;
-      int rc = pack_weights(op.W, K, op.Cin, op.Cout, op.Wp, (hipStream_t)stream);
+      int rc = split_weights(op.W, nullptr, K, op.Cin, op.Cout, op.Wp, (hipStream_t)stream);
       if (rc) return rc;
     }
   for (Op &op : net->ops)
@@ -1577,17 +1577,17 @@ static int run_op_residual(insc_net *net, int index, hipStream_t s) {
           R.bn_done[(size_t)tail.fused_bn] = 1;
         }
       }
-      return incre_conv_ssc(in0, ld0, pre0, ldp0, n_pre_in, out, ld_out, op.W, op.Wp, op.bias, Lo.nbr,
+      return incre_conv_ssc(in0, ld0, pre0, ldp0, n_pre_in, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lo.nbr,
                             R.nbr_pre[To.level], n, op.Cin, op.Cout, ep, s);
     case OP_NIN:
-      return launch_conv(in0, ld0, n_in, out, ld_out, op.W, op.Wp, op.bias, nullptr, nullptr, MAP_IDENTITY, 1, nullptr,
+      return launch_conv(in0, ld0, n_in, out, ld_out, op.W, split_ref(op.Wp), op.bias, nullptr, nullptr, MAP_IDENTITY, 1, nullptr,
                          nullptr, n, op.Cin, op.Cout, nullptr, nullptr, s, ep);
     case OP_CONV:
-      return launch_conv(in0, ld0, n_in, out, ld_out, op.W, op.Wp, op.bias, R.levels[li].child, nullptr, MAP_NBR, 8,
+      return launch_conv(in0, ld0, n_in, out, ld_out, op.W, split_ref(op.Wp), op.bias, R.levels[li].child, nullptr, MAP_NBR, 8,
                          nullptr, nullptr, n, op.Cin, op.Cout, nullptr, nullptr, s, ep);
     case OP_DECONV:
       INSC_REQUIRE(pre0, INSC_ERR_STATE, "residual frame: the input of a deconvolution was not kept");
-      return incre_deconv_down2(in0, ld0, n_in, pre0, ldp0, n_pre_in, out, ld_out, op.W, op.Wp, op.bias, Lo.parent,
+      return incre_deconv_down2(in0, ld0, n_in, pre0, ldp0, n_pre_in, out, ld_out, op.W, split_ref(op.Wp), op.bias, Lo.parent,
                                 Lo.offset, R.pre_exist[li], R.pre_exist[To.level], n, op.Cin, op.Cout, ep.res, ep.ldr, s,
                                 R.parent2[To.level]);
     case OP_BN:

@@ -338,8 +338,8 @@ def _rows_args(rows, count, n_upper):
 
 
 def packed_weight(weight, K):
-    """Weights in the matrix-core operand layout.  The packed copy is kept on the tensor
-    object itself and reused until the tensor is modified in place or re-assigned."""
+    """Weights in the matrix-core operand layout (three bf16 parts a value).  The packed copy is kept on the
+    tensor object itself and reused until the tensor is modified in place or re-assigned."""
     Cin, Cout = weight.size(-2), weight.size(-1)
     if Cin % 16:
         return None
@@ -350,9 +350,9 @@ def packed_weight(weight, K):
     w = weight.detach()
     if not w.is_contiguous():
         w = w.contiguous()
-    n = int(lib.insc_conv_packed_floats(int(K), int(Cin), int(Cout)))
+    n = int(lib.insc_conv_split_floats(int(K), int(Cin), int(Cout)))
     wp = torch.empty(n, dtype=torch.float32, device=weight.device)
-    lib.insc_conv_pack_weights(ptr(w), int(K), int(Cin), int(Cout), ptr(wp), stream_ptr())
+    lib.insc_conv_split_weights(ptr(w), int(K), int(Cin), int(Cout), ptr(wp), stream_ptr())
     try:
         weight._insc_packed = (tag, wp)
     except AttributeError:
@@ -360,11 +360,16 @@ def packed_weight(weight, K):
     return wp
 
 
+def _split_ptr(wp):
+    """How the C ABI takes such weights in the place of packed ones: their address with its lowest bit set."""
+    return None if wp is None else wp.data_ptr() | 1
+
+
 def conv_rows(in_f, out_f, weight, bias, nbr, K, rows, count, n_rows):
     """insc_conv_nbr on a row subset; in_f/out_f may be column slices of wider buffers."""
     Cin, Cout = weight.size(-2), weight.size(-1)
     lib.insc_conv_nbr(ptr(in_f), I64(_ld(in_f)), I64(in_f.size(0)), ptr(out_f), I64(_ld(out_f)), ptr(weight),
-                      ptr(packed_weight(weight, K)), ptr(bias), ptr(nbr), int(K), ptr(rows), ptr(count),
+                      _split_ptr(packed_weight(weight, K)), ptr(bias), ptr(nbr), int(K), ptr(rows), ptr(count),
                       I64(int(n_rows)), int(Cin), int(Cout), None, stream_ptr())
 
 
@@ -372,7 +377,7 @@ def ssc_rows_planned(in_f, out_f, weight, bias, sc, plan):
     """insc_conv_ssc_plan over all sites of a scale in its processing order."""
     Cin, Cout = weight.size(-2), weight.size(-1)
     lib.insc_conv_ssc_plan(ptr(in_f), I64(_ld(in_f)), I64(in_f.size(0)), ptr(out_f), I64(_ld(out_f)), ptr(weight),
-                           ptr(packed_weight(weight, 27)), ptr(bias), ptr(sc.nbr.t), ptr(plan[0]), I64(plan[2]),
+                           _split_ptr(packed_weight(weight, 27)), ptr(bias), ptr(sc.nbr.t), ptr(plan[0]), I64(plan[2]),
                            ptr(plan[1]), ptr(plan[3]), ptr(sc.order.t), None, I64(int(sc.n)), int(Cin), int(Cout),
                            stream_ptr())
 
@@ -380,7 +385,7 @@ def ssc_rows_planned(in_f, out_f, weight, bias, sc, plan):
 def deconv_rows(in_f, out_f, weight, bias, parent, offset, rows, count, n_rows):
     Cin, Cout = weight.size(-2), weight.size(-1)
     lib.insc_deconv_down2(ptr(in_f), I64(_ld(in_f)), I64(in_f.size(0)), ptr(out_f), I64(_ld(out_f)), ptr(weight),
-                          ptr(packed_weight(weight, 8)), ptr(bias), ptr(parent), ptr(offset), ptr(rows), ptr(count),
+                          _split_ptr(packed_weight(weight, 8)), ptr(bias), ptr(parent), ptr(offset), ptr(rows), ptr(count),
                           I64(int(n_rows)), int(Cin), int(Cout), stream_ptr())
 
 
@@ -625,7 +630,7 @@ def Incre_SubmanifoldConvolution_updateOutput(inputSize, filterSize, m, input_fe
     nbr_pre = m.incre_ssc_map(inputSize, pre_m)
     Cin, Cout = w.size(1), w.size(2)
     lib.insc_incre_conv_ssc(ptr(input_features), I64(_ld(input_features)), ptr(pre), I64(_ld(pre)), I64(n_pre),
-                            ptr(output_features), I64(_ld(output_features)), ptr(w), ptr(packed_weight(w, 27)),
+                            ptr(output_features), I64(_ld(output_features)), ptr(w), _split_ptr(packed_weight(w, 27)),
                             ptr(b), ptr(sc.nbr.t), ptr(nbr_pre), I64(sc.n), int(Cin), int(Cout), stream_ptr())
     if not count_muladds:
         return 0.0
@@ -660,7 +665,7 @@ def Incre_Deconvolution_updateOutput(inputSize, outputSize, filterSize, filterSt
     pe_out = m.pre_exist_map(outputSize, pre_m)
     lib.insc_incre_deconv_down2(ptr(input_features), I64(_ld(input_features)), I64(coarse.n), ptr(pre), I64(_ld(pre)),
                                 I64(n_pre), ptr(output_features), I64(_ld(output_features)), ptr(w),
-                                ptr(packed_weight(w, 8)), ptr(b), ptr(d.parent.t), ptr(d.offset.t), ptr(pe_in),
+                                _split_ptr(packed_weight(w, 8)), ptr(b), ptr(d.parent.t), ptr(d.offset.t), ptr(pe_in),
                                 ptr(pe_out), I64(fine.n), int(w.size(1)), int(w.size(2)), stream_ptr())
     return float(fine.n) * w.size(1) * w.size(2)
 

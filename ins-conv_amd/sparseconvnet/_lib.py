@@ -36,6 +36,7 @@ _SIGS = {
     "insc_conv_nbr": [vp, c_i64, c_i64, vp, c_i64, vp, vp, vp, vp, c_int, vp, vp, c_i64, c_int, c_int,
                       ctypes.POINTER(ctypes.c_double), vp],
     "insc_conv_pack_weights": [vp, c_int, c_int, c_int, vp, vp],
+    "insc_conv_split_weights": [vp, c_int, c_int, c_int, vp, vp],
     "insc_plan_build": [vp, vp, vp, c_i64, c_i64, vp, vp, vp, vp],
     "insc_conv_ssc_plan": [vp, c_i64, c_i64, vp, c_i64, vp, vp, vp, vp, vp, c_i64, vp, vp, vp, vp, c_i64, c_int, c_int,
                            vp],
@@ -111,6 +112,7 @@ _OTHER = {
     "insc_grid_count_ptr": (vp, [vp]),
     "insc_grid_capacity": (c_i64, [vp]),
     "insc_conv_packed_floats": (c_i64, [c_int, c_int, c_int]),
+    "insc_conv_split_floats": (c_i64, [c_int, c_int, c_int]),
     "insc_net_op_count": (c_int, [vp]),
 }
 

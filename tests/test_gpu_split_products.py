@@ -118,3 +118,23 @@ def test_infinities_and_nan(scene, case):
     got, ref = layer(scene, x, W, b, case), sums64(scene[3], x, W, b)
     assert np.isfinite(got).all()
     assert (np.abs(got - ref) <= 1e-5 * np.abs(ref) + 1e-4 * np.abs(sums64(scene[3], np.minimum(np.abs(x), 9), np.minimum(np.abs(W), 9), b))).all()
+
+
+@pytest.mark.parametrize("Cin,Cout", [(16, 16), (48, 224), (96, 33)])
+def test_raw_packed_and_split_weights_give_the_same_bits(scene, Cin, Cout):
+    from sparseconvnet._lib import lib, ptr, stream_ptr
+
+    S, m, sc, _ = scene
+    _, x, W, b = data(scene, (Cin, Cout))
+    xd, Wd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda()
+    packed = torch.empty(lib.insc_conv_packed_floats(27, Cin, Cout), device="cuda")
+    split = torch.empty(lib.insc_conv_split_floats(27, Cin, Cout), device="cuda")
+    lib.insc_conv_pack_weights(ptr(Wd), 27, Cin, Cout, ptr(packed), stream_ptr())
+    lib.insc_conv_split_weights(ptr(Wd), 27, Cin, Cout, ptr(split), stream_ptr())
+    got = []
+    for raw, wp in ((ptr(Wd), None), (None, ptr(packed)), (None, ptr(split) | 1)):
+        out = torch.full((sc.n, Cout), 7.0, device="cuda")
+        lib.insc_conv_nbr(ptr(xd), Cin, sc.n, ptr(out), Cout, raw, wp, ptr(bd), ptr(sc.nbr.t), 27, None, None, sc.n, Cin, Cout,
+                          None, stream_ptr())
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
