@@ -56,7 +56,7 @@ struct SortJob {
   int64_t n;
 };
 constexpr int SORT_BATCH_MAX_JOBS = 8;
-constexpr int64_t SORT_BATCH_MAX_N = 262144;
+constexpr int64_t SORT_BATCH_MAX_N = 524288;
 int sort_pairs_u64_into_batch(const SortJob *jobs, int n_jobs, int key_bits, hipStream_t s);
 int sort_pairs_u64(uint64_t *keys, int32_t *vals, int64_t n, int key_bits, hipStream_t s);
 

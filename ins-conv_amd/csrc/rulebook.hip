@@ -268,6 +268,9 @@ int insc_order_build(const insc_grid *g, const int32_t *d_nbr, int64_t first, in
   return sort_pairs_u64_into(keys, ids, d_order + first, n, ORDER_KEY_BITS, s);
 }
 
+// (what the header promises; the shared launches themselves take twice as many)
+static constexpr int64_t ORDER_SCALES_MAX_N = 262144;
+
 int insc_order_build_scales(const insc_grid *const *grids, const int32_t *const *d_nbr, const int32_t *const *d_offset,
                             const int64_t *n, int n_scales, int32_t *const *d_order, int32_t *const *d_pos,
                             int32_t *const *d_bo_order, int32_t *const *d_bo_pos, void *stream) {
@@ -275,9 +278,9 @@ int insc_order_build_scales(const insc_grid *const *grids, const int32_t *const 
                "insc_order_build_scales: 1..%d scales, no null array", SORT_BATCH_MAX_JOBS);
   OrderBuildJob jobs[SORT_BATCH_MAX_JOBS];
   for (int i = 0; i < n_scales; i++) {
-    INSC_REQUIRE(grids[i] && n[i] >= 1 && n[i] <= SORT_BATCH_MAX_N && n[i] <= insc_grid_capacity(grids[i]), INSC_ERR_ARG,
+    INSC_REQUIRE(grids[i] && n[i] >= 1 && n[i] <= ORDER_SCALES_MAX_N && n[i] <= insc_grid_capacity(grids[i]), INSC_ERR_ARG,
                  "insc_order_build_scales: scale %d has %lld sites (1..%lld, within the grid's capacity)", i,
-                 (long long)n[i], (long long)SORT_BATCH_MAX_N);
+                 (long long)n[i], (long long)ORDER_SCALES_MAX_N);
     const int32_t *off = d_offset ? d_offset[i] : nullptr;
     INSC_REQUIRE(d_nbr[i] && d_order[i] && d_pos[i] && (!off || (d_bo_order && d_bo_pos && d_bo_order[i] && d_bo_pos[i])),
                  INSC_ERR_ARG, "insc_order_build_scales: null pointer at scale %d", i);
