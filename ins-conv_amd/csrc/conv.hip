@@ -1933,6 +1933,9 @@ static std::atomic<int64_t> g_shared_min_units{896};
 // (64 -> 64 at 39k sites = 2452 units: 50 us against 56 us; 2084 units: 48 against 50; 1840: 41 against 44;
 // 1716: 41.1 against 41.5; 1472: 41 against 39 - the split kernel's launch is whole rounds of 1024 blocks, four to
 // a compute unit, this kernel's is the SIMD with the most units).
+// Those figures are from the fp32 instruction; with bf16 parts the order is the same.  Four layers with their batch norms,
+// wavefront per unit / one block per unit / shared weights: 64 -> 64 at 39k sites 229 / 238-250 / 248-273 us, at 150k
+// 647 / 710 / 552, 96 -> 96 at 10k 251 / 195 / 194-390.
 static std::atomic<int64_t> g_own_min_units{1750};
 // Narrow 3^3 layers (Cin, Cout <= 32) with at least this many 32-row tiles run on the persistent
 // kernel that keeps the whole filter in LDS; smaller ones on the one-wavefront-per-tile kernel.
