@@ -234,7 +234,7 @@ int insc_conv_set_shared_weights_min_units(int64_t units);
  * bits again. */
 int insc_conv_set_wavefront_per_unit_min_units(int64_t units);
 /* A 3^3 layer with at most 32 input and 32 output channels runs, from `tiles` 32-row tiles up
- * (default 4096, i.e. 131k sites), on persistent blocks that keep the whole filter in LDS; below,
+ * (default 2048, i.e. 65k sites; four times as many without a tile plan), on persistent blocks that keep the whole filter in LDS; below,
  * one wavefront per tile.  Same bits in both cases: a tuning and test knob like the two above. */
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles);
 /* Size-2 stride-2 deconvolution: out[i,:] = bias + in[parent[i],:] . W[offset[i]]

@@ -918,7 +918,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
 // rings of three and four items, which spill at twelve wavefronts, 589 / 232 and 667 / 253)
 constexpr int WL_WAVES = 12;
 constexpr int WL_DEPTH = 2;
-constexpr int WL_MIN_TILES = 4096;  // smaller launches go to conv_mfma_kernel (default of the knob below)
+constexpr int WL_MIN_TILES = 2048;  // smaller launches go to conv_mfma_kernel (default of the knob below)
 constexpr int WL_SCHED = 256;  // a block orders up to this many tiles of its own by cost
 
 // KS: halves of the 32-channel chunk that exist (1: 16 input channels, 2: 32)
@@ -2008,11 +2008,11 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const bool small_ids = in_rows < (1 << 24) && out_rows < (1 << 24) && ld_out * 4 < (1 << 24) &&
                            ep.ld2 * 4 < (1 << 24) && out_rows * ld_out * 4 < (int64_t)BUF_OOB &&
                            out_rows * ep.ld2 * 4 < (int64_t)BUF_OOB;
-    // (below some four thousand tiles the persistent kernel's start-up - every block copies the
-    // whole filter into LDS - costs more than it saves: 34 us against 21 us at 32k sites, even at
-    // 150k; both kernels give the same bits)
+    // (below some two thousand tiles the persistent kernel's start-up - every block copies the whole filter into LDS -
+    // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1476 / 1440 us, 100k 1641 / 1669.
+    // Without a plan every tile looks its offsets up first: four times as many.  Both kernels give the same bits.)
     if (mode == MAP_NBR && K == 27 && Cin <= 32 && Cout <= 32 && map_bytes64 < (int64_t)BUF_OOB && small_ids &&
-        cdiv(expect_rows, TILE_M) >= g_wl_min_tiles.load(std::memory_order_relaxed) && !latency) {
+        cdiv(expect_rows, TILE_M) >= g_wl_min_tiles.load(std::memory_order_relaxed) * (plan.map ? 1 : 4) && !latency) {
       const uint32_t map_bytes = (uint32_t)map_bytes64;
       // persistent blocks, a multiple of the XCD count, at most one per compute unit
       const int64_t want = cdiv(tiles, WL_WAVES);
