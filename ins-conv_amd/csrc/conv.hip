@@ -2012,7 +2012,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1476 / 1440 us, 100k 1641 / 1669.
     // Without a plan every tile looks its offsets up first: four times as many.  Both kernels give the same bits.)
     if (mode == MAP_NBR && K == 27 && Cin <= 32 && Cout <= 32 && map_bytes64 < (int64_t)BUF_OOB && small_ids &&
-        cdiv(expect_rows, TILE_M) >= g_wl_min_tiles.load(std::memory_order_relaxed) * (plan.map ? 1 : 4) && !latency) {
+        cdiv(expect_rows, TILE_M) / (plan.map ? 1 : 4) >= g_wl_min_tiles.load(std::memory_order_relaxed) && !latency) {
       const uint32_t map_bytes = (uint32_t)map_bytes64;
       // persistent blocks, a multiple of the XCD count, at most one per compute unit
       const int64_t want = cdiv(tiles, WL_WAVES);
