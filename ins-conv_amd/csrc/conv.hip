@@ -296,52 +296,48 @@ __global__ void split_weights_kernel(const float *__restrict__ W, const float *_
   }
 }
 
-// A weight from its three parts, exactly.
-__device__ __forceinline__ float packed_weight_at(const float *Wp, int64_t tile, int cin32, int col) {
-  const uint16_t *p = reinterpret_cast<const uint16_t *>(Wp) + tile * (WT_BYTES / 2) + (cin32 >> 4) * 1536 +
-                      (((cin32 >> 3) & 1) * 32 + col) * 8 + (cin32 & 7);
-  return (__uint_as_float((unsigned)p[0] << 16) + __uint_as_float((unsigned)p[512] << 16)) +
-         __uint_as_float((unsigned)p[1024] << 16);
+// The lane's number, formed where it is asked for: what rarely runs or runs once per tile would otherwise have its
+// addresses formed ahead of the kernel's loop and kept, or spilled, across it (the sums formed again below took
+// conv_wshare_kernel from 1455 to 1736 us, 64 -> 64 at 500k sites).
+__device__ __forceinline__ int lane_again() {
+  int all = -1;
+  asm volatile("" : "+s"(all));
+  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)all, __builtin_amdgcn_mbcnt_lo((unsigned)all, 0));
 }
 
-// sum + the products of one output element in plain fp32, offsets and channels ascending (cold: repair_sums).
-// map0 / map1 as in the generic kernel.
-__device__ __forceinline__ float plain_sum(float sum, const float *__restrict__ in, int64_t ld_in,
-                                           const float *__restrict__ Wp, const int32_t *__restrict__ map0,
-                                           const int32_t *__restrict__ map1, int mode, int K, int row, int Cin, int nch,
-                                           int nbtp, int c) {
-#pragma unroll 1
-  for (int k = 0; k < K; k++) {
-    const int src = mode == MAP_NBR ? map0[(int64_t)row * K + k]
-                    : mode == MAP_IDENTITY ? row
-                                           : (map1[row] == k ? map0[row] : -1);
-    if (src < 0) continue;
-#pragma unroll 1
-    for (int ci = 0; ci < Cin; ci++)
-      sum = fmaf(in[(int64_t)src * ld_in + ci],
-                 packed_weight_at(Wp, ((int64_t)k * nch + (ci >> 5)) * nbtp + (c >> 5), ci & 31, c & 31), sum);
-  }
-  return sum;
+// Rows of a tile that the elements of this lane's 32x32 sums belong to (element v: row 8 * (v / 4) + 4 * h + v % 4), from
+// the lanes that hold them.
+__device__ __forceinline__ void rows_of_elements(int my_row, int (&rid)[16]) {
+  const int base = (lane_again() >> 5) * 16;
+#pragma unroll
+  for (int v = 0; v < 16; v++) rid[v] = __builtin_amdgcn_ds_bpermute(base + 4 * (8 * (v >> 2) + (v & 3)), my_row);
 }
 
-// Elements whose sum of bf16 products is not finite (an infinity or NaN among the inputs or weights, or an
-// overflow on the way) are summed again by plain(j).  Which elements these are depends on the element's own sum
-// alone.  One multiply-add per element finds out that there are none.
+// Elements whose sum of bf16 products is not finite (an infinity or NaN among the inputs or weights, or an overflow on
+// the way) are formed again in plain fp32: tile_sums() gives them for the wavefront's tile (add_plain_products below), v0
+// is the first of this lane's N elements among its sixteen.  Which elements these are depends on the element's own sum
+// alone - but for an infinite weight, which makes NaN of the zeros of rows without its offset as well: these come out right,
+// with the rounding of this sum.  One multiply-add per element finds out that there are none.
+__device__ __forceinline__ bool is_bad(float x) { return (__float_as_uint(x) & 0x7F800000u) == 0x7F800000u; }
+template <int N, class A>
+__device__ __forceinline__ float not_finite(const A &a, float t) {  // NaN as soon as one is infinite or NaN
+#pragma unroll
+  for (int j = 0; j < N; j++) t = fmaf(a[j], 0.0f, t);
+  return t;
+}
 template <int N, class A, class F>
-__device__ __forceinline__ void repair_sums(A &a, const F &plain) {
-  float t = 0.0f;
+__device__ __forceinline__ void repair_sums(A &a, int v0, const F &tile_sums) {
+  const float t = not_finite<N>(a, 0.0f);
+  if (__builtin_expect(!__any(t != t), 1)) return;
+  const f16v x = tile_sums();
 #pragma unroll
-  for (int j = 0; j < N; j++) t = fmaf(a[j], 0.0f, t);  // NaN as soon as one is infinite or NaN
-  if (!__any(t != t)) return;
-  unsigned bad = 0;
-#pragma unroll
-  for (int j = 0; j < N; j++) bad |= ((__float_as_uint(a[j]) & 0x7F800000u) == 0x7F800000u ? 1u : 0u) << j;
-#pragma unroll 1
   for (int j = 0; j < N; j++) {
-    if (!__any((bad >> j) & 1u)) continue;
-    const float x = plain(j);
+    float y = x[j];
+    if (N < 16) {
 #pragma unroll
-    for (int i = 0; i < N; i++) a[i] = (i == j && ((bad >> j) & 1u)) ? x : a[i];
+      for (int v = 0; v < 16; v++) y = v == v0 + j ? x[v] : y;
+    }
+    a[j] = is_bad(a[j]) ? y : a[j];
   }
 }
 
@@ -410,6 +406,47 @@ __device__ __forceinline__ WFrag load_wtile(__amdgpu_buffer_rsrc_t rw, int tile,
   return f;
 }
 
+// sums += the products of a tile's rows with output block nb in plain fp32 (v_mfma_f32_32x32x2_f32), offsets and channels
+// ascending: what repair_sums falls back to.  id_of(k): input row of offset k of tile row lane & 31, -1: none.  A row
+// takes no part in an offset that it does not have (its zeros would turn an infinite weight into NaN).
+// Cold, so it waits for every load; but one NaN of a scan reaches whole scales, which then pass through it: 32 -> 32 at
+// 500k sites 0.15 ms finite, 0.34 all NaN (element by element in scalar code: 12.9), 64 -> 64 at 500k 0.42 and 1.25 (54.5),
+// 96 -> 96 at 10k 0.07 and 0.21 (3.7).
+template <class Ids>
+__device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of, int K, __amdgpu_buffer_rsrc_t rin,
+                                                   uint32_t ld4, __amdgpu_buffer_rsrc_t rw, int Cin, int nch, int nbtp,
+                                                   int nb) {
+  const int lane = lane_again(), h = lane >> 5;
+#pragma unroll 1
+  for (int k = 0; k < K; k++) {
+    const int src = id_of(k);
+    const unsigned have = (unsigned)__ballot(src >= 0) >> (4 * h);  // (the two half-waves agree; bit of this lane's rows)
+    if (!__any(have != 0)) continue;
+    const f16v before = sums;
+#pragma unroll 1
+    for (int c16 = 0; c16 * 16 < Cin; c16++) {
+      const uint32_t voff = src >= 0 ? (uint32_t)src * ld4 + (uint32_t)(c16 * 64 + h * 32) : BUF_OOB;
+      const float4 lo = buf_load16(rin, voff, 0), hi = buf_load16(rin, voff + 16u, 0);
+      const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(((k * nch + (c16 >> 1)) * nbtp + nb) * WT_BYTES +
+                                                                     (c16 & 1) * 3072);
+      u32x4 p[3];
+#pragma unroll
+      for (int i = 0; i < 3; i++) p[i] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u + 1024u * i, soff));
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        float w = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 3; i++)  // (exact)
+          w += __uint_as_float(j & 1 ? p[i][j >> 1] & 0xFFFF0000u : p[i][j >> 1] << 16);
+        sums = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], w, sums, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) sums[v] = have & (1u << (8 * (v >> 2) + (v & 3))) ? sums[v] : before[v];
+  }
+}
+
 // The order in which a wavefront that owns a tile takes the offsets of a 3^3 filter: the centre first, then
 // ascending.  (The filter-in-LDS kernel below has no room in LDS for the centre's weights.)
 __device__ __forceinline__ int first_offset(unsigned mask) {
@@ -427,7 +464,7 @@ __device__ __forceinline__ int first_offset(unsigned mask) {
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
 template <int NB, int K, int MODE, int S>
-__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kernel(
+__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) void conv_mfma_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
     const int32_t *__restrict__ map1, const int32_t *__restrict__ rows,
@@ -476,6 +513,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
   const bool second = S > 1 && ep.src2_in != nullptr && (int)bz >= GZ / 2;
   const float *const in0 = in, *const bias0 = bias;  // (the first source, whichever this block reads)
   const int64_t ld_in0 = ld_in;
+  const uint32_t in_bytes0 = in_bytes;
   const int32_t *const map00 = map0;
   const int G = (S > 1 && ep.src2_in != nullptr) ? GZ / 2 : GZ, ST = S * G;
   const int ws = wave * G + (S == 1 ? 0 : (int)bz - (second ? G : 0));
@@ -706,6 +744,40 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
     }
   }
 
+  // input row of this lane's output row at offset k (cold: from memory, through a source's own map)
+  auto id_at = [&](const int32_t *map, int k) -> int {
+    if (planned) return plan.map[(int64_t)k * plan.ld + t0 + (lane_again() & 31)];
+    if (my_row < 0) return -1;
+    return MODE == MAP_NBR ? map[(int64_t)my_row * K + k] : MODE == MAP_IDENTITY ? my_row : map1[my_row] == k ? map[my_row] : -1;
+  };
+  if (S == 1) {
+    // (put back into the running sums, one block at a time: copies of all blocks' totals would cost NB = 3 its second
+    // wavefront per SIMD, 32 -> 96 at 200k sites 99 -> 124 us)
+    float t = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NB; b++) t = not_finite<16>(sum_of(sums[b]), t);
+    if (__builtin_expect(__any(t != t), 0)) {
+#pragma unroll 1
+      for (int bb = 0; bb < NB; bb++) {
+        const int c = (cb0 + bb) * 32 + r;
+        f16v x;
+#pragma unroll
+        for (int v = 0; v < 16; v++) x[v] = (bias && c < Cout) ? bias[c] : 0.0f;
+        add_plain_products(x, [&](int k) { return id_at(map0, k); }, K, make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u,
+                           make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, cb0 + bb);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          if (b != bb) continue;
+#pragma unroll
+          for (int v = 0; v < 16; v++)
+            if (is_bad(sums[b].lead[v] + sums[b].rest[v])) {
+              sums[b].lead[v] = x[v];
+              sums[b].rest[v] = 0.0f;
+            }
+        }
+      }
+    }
+  }
   f16v acc[NB];
 #pragma unroll
   for (int b = 0; b < NB; b++) acc[b] = sum_of(sums[b]);
@@ -784,12 +856,18 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
       if (lane == 0) pcount[unit * S + wave] = 0;
     }
     const int c = cb0 * 32 + r;
-    repair_sums<NV>(a, [&](int j) -> float {
-      const int v = wave * NV + j, row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-      if (row < 0 || c >= Cout) return 0.0f;
-      float x = plain_sum(bias0 ? bias0[c] : 0.0f, in0, ld_in0, Wp, map00, map1, MODE, K, row, Cin, nch, nbtp, c);
-      if (ep.src2_in) x = plain_sum(x, ep.src2_in, ep.src2_ld, Wp, ep.src2_map, map1, MODE, K, row, Cin, nch, nbtp, c);
-      return x;
+    repair_sums<NV>(a, wave * NV, [&]() -> f16v {
+      f16v t;
+#pragma unroll
+      for (int v = 0; v < 16; v++) t[v] = (bias0 && c < Cout) ? bias0[c] : 0.0f;
+      const __amdgpu_buffer_rsrc_t rw = make_rsrc(Wp, wp_bytes);
+      add_plain_products(t, [&](int k) { return id_at(map00, k); }, K, make_rsrc(in0, in_bytes0), (uint32_t)ld_in0 * 4u, rw, Cin,
+                         nch, nbtp, cb0);
+      if (ep.src2_in)
+        add_plain_products(t, [&](int k) { return id_at(ep.src2_map, k); }, K,
+                           make_rsrc(ep.src2_in, (uint32_t)(ep.src2_rows * ep.src2_ld * 4)), (uint32_t)ep.src2_ld * 4u, rw, Cin, nch,
+                           nbtp, cb0);
+      return t;
     });
     if (c >= Cout) return;
     if (ep.res) {
@@ -834,17 +912,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64) void conv_mfma_kern
   // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3).
   // All row ids are fetched from their lanes first, then the stores go out back to back.
   int rid[16];
-#pragma unroll
-  for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const int c = (cb0 + b) * 32 + r;
-    repair_sums<16>(acc[b], [&](int v) -> float {
-      const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-      if (row < 0 || c >= Cout) return 0.0f;
-      return plain_sum(bias ? bias[c] : 0.0f, in, ld_in, Wp, map0, map1, MODE, K, row, Cin, nch, nbtp, c);
-    });
-  }
+  rows_of_elements(my_row, rid);
   // (the values of the residual input are all fetched before the first store: a store may alias them
   // as far as the compiler knows, and loads issued between the stores would wait one by one)
   if (ep.res) {
@@ -1178,14 +1246,17 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     f16v acc = sum_of(sum);
 
     // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3)
-    repair_sums<16>(acc, [&](int v) -> float {
-      const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-      if (row < 0 || col >= Cout) return 0.0f;
-      return plain_sum(bv, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, 1, 1, col);
+    repair_sums<16>(acc, 0, [&]() -> f16v {
+      f16v x;
+#pragma unroll
+      for (int v = 0; v < 16; v++) x[v] = bv;
+      add_plain_products(
+          x, [&](int k) { return base == BUF_OOB ? -1 : (int)__builtin_amdgcn_raw_buffer_load_b32(rids, (int)(base + k * pitch), 0, 0); },
+          K, rin, ld4, rw, Cin, 1, 1, 0);
+      return x;
     });
     int rid[16];
-#pragma unroll
-    for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+    rows_of_elements(my_row, rid);
     const uint32_t col4 = (uint32_t)col * 4u;
     // (the residual input is fetched before the first store, which may alias it as far as the
     // compiler knows: loads issued between the stores would wait one by one)
@@ -1241,8 +1312,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
 template <int NB, int ST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 : 3, NB > 1 ? 2 : 3))) void conv_wshare_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
-    const int32_t *__restrict__ rows,
+    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
     const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
   constexpr int K = 27, WV = 4;
@@ -1294,11 +1364,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
   // same for every i, the rest is a scalar)
   auto stage_issue = [&](int tile) {
     if (tile < 0) return;  // no such tile: its wavefront never reads the slice
-    const uint32_t base = (uint32_t)(h * (int)plan.ld + tile * TILE_M + r) * 4u;
+    const int l = lane_again();
+    const uint32_t base = (uint32_t)((l >> 5) * (int)plan.ld + tile * TILE_M + (l & 31)) * 4u;
     const uint32_t pair = (uint32_t)plan.ld * 8u;
 #pragma unroll
     for (int i = 0; i < NSTAGE; i++) {
-      const uint32_t voff = (2 * i + 1 < K || h == 0) ? base : BUF_OOB;
+      const uint32_t voff = (2 * i + 1 < K || l < 32) ? base : BUF_OOB;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rplan, INSC_LDS_PTR(nlw + i * 64), 4, (int)voff, (int)(i * pair), 0, 0);
     }
   };
@@ -1462,9 +1533,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 
       // this unit's rows; the next unit's map slice goes out first (nobody reads nl any more)
       stage_issue(tile_n);
-      int rid[16];
-#pragma unroll
-      for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
       if (mine) {
 #pragma unroll
         for (int o = 0; o < NB; o++) {
@@ -1475,11 +1543,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 #pragma unroll
             for (int v = 0; v < 16; v++) sum[v] = total[o][v] + sum[v];
           }
-          repair_sums<16>(sum, [&](int v) -> float {
-            const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-            if (row < 0 || cc >= Cout) return 0.0f;
-            return plain_sum(bias ? bias[cc] : 0.0f, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, nch, nbtp, cc);
+          repair_sums<16>(sum, 0, [&]() -> f16v {
+            f16v x;
+#pragma unroll
+            for (int v = 0; v < 16; v++) x[v] = bv[o];
+            add_plain_products(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K, rin, ld4,
+                               rw, Cin, nch, nbtp, ob0 + o);
+            return x;
           });
+          int rid[16];
+          rows_of_elements(my_row, rid);
           float rv[16];
 #pragma unroll
           for (int v = 0; v < 16; v++)
@@ -1533,8 +1606,7 @@ constexpr int OWN_WAVES = 8;  // one block per compute unit
 template <int ST, int D>
 __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_own_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
-    const int32_t *__restrict__ rows,
+    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
     const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
   constexpr int K = 27;
@@ -1675,17 +1747,19 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   const __amdgpu_buffer_rsrc_t rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
   const uint32_t ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u, ldr4 = (uint32_t)ep.ldr * 4u;
   int rid[16];
-#pragma unroll
-  for (int v = 0; v < 16; v++) rid[v] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+  rows_of_elements(my_row, rid);
   f16v sum = sum_of(acc);
   if (cur != 0) {
 #pragma unroll
     for (int v = 0; v < 16; v++) sum[v] = total[v] + sum[v];
   }
-  repair_sums<16>(sum, [&](int v) -> float {
-    const int row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
-    if (row < 0 || c >= Cout) return 0.0f;
-    return plain_sum(bv, in, ld_in, Wp, map0, nullptr, MAP_NBR, K, row, Cin, nch, nbtp, c);
+  repair_sums<16>(sum, 0, [&]() -> f16v {
+    f16v x;
+#pragma unroll
+    for (int v = 0; v < 16; v++) x[v] = bv;
+    add_plain_products(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K,
+                       make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u, make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, ob);
+    return x;
   });
   float rv[16];
 #pragma unroll
@@ -2071,7 +2145,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
         }
         const int64_t wunits = cdiv(tiles, 4) * cdiv(nbt, 2);
         const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu4, wunits);
-        hipLaunchKernelGGL((conv_wshare_kernel<2, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, map0, rows,
+        hipLaunchKernelGGL((conv_wshare_kernel<2, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
                            d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
         INSC_LAUNCH_CHECK();
         return INSC_OK;
@@ -2083,7 +2157,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       }
       const int64_t wunits = cdiv(tiles, 4) * nbt;
       const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu2, wunits);
-      hipLaunchKernelGGL((conv_wshare_kernel<1, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, map0, rows,
+      hipLaunchKernelGGL((conv_wshare_kernel<1, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
                          d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
@@ -2092,8 +2166,8 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     if (wide_planned && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
       // one wavefront per (tile, output block): enough units that every SIMD gets one to three
       hipLaunchKernelGGL((conv_own_kernel<4, 2>), dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
-                         ld_out, Wp, bias, map0, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes,
-                         ep, plan);
+                         ld_out, Wp, bias, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep,
+                         plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
     }

@@ -29,16 +29,25 @@ def scene():
     return S, m, sc, sc.nbr.t[:sc.n].cpu().numpy()
 
 
-def layer(scene, x, W, b, case):
+def layer(scene, x, W, b, case, n_in=None, events=None):
     from sparseconvnet._lib import lib
 
     S, m, sc, _ = scene
     out = torch.full((sc.n, W.shape[2]), 7.0, device="cuda")
+    xd, Wd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda()
+    plan = m.ssc_plan(sc)
     try:
         lib.insc_conv_set_filter_lds_min_tiles(case[2])
         lib.insc_conv_set_wavefront_per_unit_min_units(case[3])
         lib.insc_conv_set_shared_weights_min_units(case[4])
-        S.ssc_rows_planned(torch.from_numpy(x).cuda(), out, torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda(), sc, m.ssc_plan(sc))
+        S.packed_weight(Wd, 27)
+        if events is not None:
+            events += [torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)]
+            torch.cuda.synchronize()
+            events[0].record()
+        S.ssc_rows_planned(xd[:n_in], out, Wd, bd, sc, plan)
+        if events is not None:
+            events[1].record()
     finally:
         lib.insc_conv_set_filter_lds_min_tiles(4096)
         lib.insc_conv_set_wavefront_per_unit_min_units(1750)
@@ -138,3 +147,142 @@ def test_raw_packed_and_split_weights_give_the_same_bits(scene, Cin, Cout):
                           None, stream_ptr())
         got.append(out)
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_repeated_sums_read_inside_the_input_matrix(scene, case):
+    """Map entries beyond n_in_rows count as rows of zeros (the gather is bounds-checked against it), also in the sums
+    that are formed a second time because they are not finite."""
+    S, m, sc, nbr = scene
+    rng, x, W, b = data(scene, case)
+    half = sc.n // 2
+    x[rng.integers(0, half, 40), 0] = np.nan
+    x[rng.integers(0, half, 40), 0] = np.inf
+    x[half:] = 1e30  # (allocated, but not part of the matrix that is handed over)
+    got = layer(scene, x, W, b, case, n_in=half)
+    x[half:] = 0
+    ref = sums64(nbr, x, W, b)
+    assert np.isnan(ref).any() and np.isinf(ref).any()
+    assert (np.isnan(got) == np.isnan(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
+    fin = np.isfinite(ref)
+    assert (np.abs(got[fin] - ref[fin]) <= 1e-4).all()
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_a_layer_of_nan_costs_a_few_times_a_finite_one(scene, case):
+    """One NaN of a scan reaches every site of the coarse scales: a layer whose sums are all repeated may take a few times
+    as long (some ten at these sizes, where a finite layer is one short launch), not hundreds of times."""
+    _, x, W, b = data(scene, case)
+
+    def best(x):
+        ts = []
+        for _ in range(5):
+            e = []
+            layer(scene, x, W, b, case, events=e)
+            ts.append(e[0].elapsed_time(e[1]))
+        return min(ts)
+
+    assert best(np.full_like(x, np.nan)) < 25 * best(x)
+
+
+@pytest.mark.parametrize("case", KERNELS)
+def test_an_infinite_weight_reaches_only_rows_that_have_its_offset(scene, case):
+    """A row without a neighbour takes no part in that offset, whatever its tile mates do: zero times infinity does not
+    come in.  (Its sum may be formed the other way, so it is compared within the error of a fp32 sum, not bit for bit.)"""
+    _, x, W, b = data(scene, case)
+    mag = sums64(scene[3], np.abs(x), np.abs(W), np.abs(b))
+    W[3, 5, 1], W[26, 7, 0] = np.inf, -np.inf
+    got, ref = layer(scene, x, W, b, case), sums64(scene[3], x, W, b)
+    fin = np.isfinite(ref)
+    assert np.isinf(ref).any() and (got[~fin] == ref[~fin]).all()
+    assert (np.abs(got[fin] - ref[fin]) <= 2.0 ** -24 * 27 * case[0] * mag[fin]).all()
+
+
+def sums64_through(maps, x, W, b):
+    """Like sums64, for any map [rows, K] and several sources."""
+    ref = np.tile(b.astype(np.float64), (len(maps[0]), 1))
+    for nbr, src in zip(maps, x):
+        for k in range(W.shape[0]):
+            i = np.flatnonzero(nbr[:, k] >= 0)
+            with np.errstate(invalid="ignore"):
+                ref[i] += src[nbr[i, k]].astype(np.float64) @ W[k].astype(np.float64)
+    return ref
+
+
+@pytest.mark.parametrize("kind,Cin,Cout", [("nin", 48, 96), ("nin", 192, 64), ("down", 16, 32), ("down", 48, 70), ("down", 64, 96),
+                                           ("up", 32, 16), ("up", 64, 40), ("up", 128, 64), ("incre", 32, 32),
+                                           ("incre", 64, 40), ("incre", 128, 128), ("incre_up", 32, 16), ("incre_up", 96, 64)])
+def test_the_other_maps(kind, Cin, Cout):
+    """1x1, 2^3 stride-2, deconvolutions and the two sources of a residual frame, with infinities and NaN in some rows: every
+    kernel has a form of its own for each map."""
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import ensure_init
+
+    ensure_init(0)
+    rng = np.random.default_rng(Cin + Cout)
+    vox = scenes.boxes_scene(seed=11, n=2600)
+    old, new = vox[:1700], np.concatenate([vox[rng.choice(1700, 500, replace=False)], vox[1700:]])
+    half = SZ // 2
+
+    def sites(pts):
+        m, e = S.Metadata_3(), torch.empty(0, device="cuda")
+        S.InputLayer_updateOutput(m, SZ, torch.from_numpy(pts.astype(np.int64)), torch.ones((len(pts), 1), device="cuda"), e, 0, 4)
+        return m
+
+    m = sites(new)
+    fine, coarse, d = m.down_rulebook(SZ, half)
+    cpu = lambda t, n: t[:n].cpu().numpy()
+    parent, off = cpu(d.parent.t, fine.n), cpu(d.offset.t, fine.n)
+    K = {"nin": 1, "incre": 27}.get(kind, 8)
+    W = (rng.normal(size=(K, Cin, Cout)) * (2.0 / Cin / K) ** 0.5).astype(np.float32)
+    b = rng.normal(size=Cout).astype(np.float32)
+    n_in = coarse.n if kind.endswith("up") else fine.n
+
+    def spoil(x):
+        x[rng.integers(0, len(x), 6), rng.integers(0, Cin, 6)] = np.inf
+        x[rng.integers(0, len(x), 6), rng.integers(0, Cin, 6)] = -np.inf
+        x[rng.integers(0, len(x), 4), rng.integers(0, Cin, 4)] = np.nan
+        return x
+
+    up = np.where(np.arange(8) == off[:, None], parent[:, None], -1)
+    x = rng.normal(size=(n_in, Cin)).astype(np.float32)
+    sets, maps = [x], {"nin": np.arange(fine.n)[:, None], "down": cpu(d.child.t, coarse.n), "up": up, "incre_up": up}
+    if kind.startswith("incre"):
+        ma = sites(old)
+        _, coarse_a, _ = ma.down_rulebook(SZ, half)
+        sets.append(rng.normal(size=(coarse_a.n if kind == "incre_up" else 1700, Cin)).astype(np.float32))
+    if kind == "incre":
+        maps = [cpu(m.ssc_rulebook(SZ).nbr.t, fine.n), cpu(m.incre_ssc_map(SZ, ma), fine.n)]
+    elif kind == "incre_up":
+        pe_c, pe_f = m.pre_exist_map(half, ma).cpu().numpy(), m.pre_exist_map(SZ, ma).cpu().numpy()
+        maps = [up, np.where((up >= 0) & (pe_f < 0)[:, None], pe_c[up], -1)]
+    else:
+        maps = [maps[kind]]
+
+    def run(sets):
+        xs, Wd, bd = [torch.from_numpy(v).cuda() for v in sets], torch.from_numpy(W).cuda(), torch.from_numpy(b).cuda()
+        out = torch.full((len(maps[0]), Cout), 7.0, device="cuda")
+        two, e = torch.LongTensor([2, 2, 2]), torch.empty(0, device="cuda")
+        if kind == "nin":
+            S.NetworkInNetwork_updateOutput(xs[0], e, Wd[0], bd)
+            return e.cpu().numpy()
+        if kind == "down":
+            S.conv_rows(xs[0], out, Wd, bd, d.child.t, 8, None, None, coarse.n)
+        elif kind == "up":
+            S.deconv_rows(xs[0], out, Wd, bd, d.parent.t, d.offset.t, None, None, fine.n)
+        elif kind == "incre":
+            S.Incre_SubmanifoldConvolution_updateOutput(SZ, torch.LongTensor([3, 3, 3]), m, xs[0], e, Wd, bd, ma, xs[1])
+            return e.cpu().numpy()
+        else:
+            S.Incre_Deconvolution_updateOutput(half, SZ, two, two, m, xs[0], e, Wd, bd, ma, xs[1])
+            return e.cpu().numpy()
+        return out.cpu().numpy()
+
+    base, ref = run(sets), sums64_through(maps, sets, W, b)
+    mag = sums64_through(maps, [np.abs(v) for v in sets], np.abs(W), np.abs(b))
+    assert (np.abs(base - ref) <= 2.0 ** -24 * (K * Cin / 8 + 2) * mag).all()
+    bad = [spoil(v.copy()) for v in sets]
+    got, ref = run(bad), sums64_through(maps, bad, W, b)
+    fin = np.isfinite(ref)
+    assert np.isnan(ref).any() and np.isinf(ref).any() and (got[fin] == base[fin]).all()
+    assert (np.isnan(got) == np.isnan(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
