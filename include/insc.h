@@ -197,7 +197,7 @@ int insc_conv_nbr(const float *d_in, int64_t ld_in, int64_t n_in_rows, float *d_
  * insc_conv_packed_floats gives the size of d_Wp in floats. */
 int64_t insc_conv_packed_floats(int K, int Cin, int Cout);
 int insc_conv_pack_weights(const float *d_W, int K, int Cin, int Cout, float *d_Wp, void *stream);
-/* The layout the kernels themselves read: every weight as three bf16 parts whose sum is exactly the weight
+/* The layout the kernels themselves read: every weight as three bf16 parts that hold it exactly
  * (insc_conv_split_floats floats, 16-byte aligned).  Every d_Wp argument takes such weights as well: pass their address
  * with its lowest bit set, INSC_SPLIT_WEIGHTS(d_Ws).  Packed fp32 weights are split on every call instead, into
  * scratch memory. */

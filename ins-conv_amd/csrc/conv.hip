@@ -146,21 +146,25 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
 // ---------------------------------------------------------------------------------------
 // fp32 products on the bf16 matrix cores.  A float is the exact sum of three bf16 numbers of eight
 // significant bits each (x = x0 + x1 + x2, |x1| < 2^-7 |x0|, |x2| < 2^-7 |x1|), so a product of two floats is
-// nine products of bf16 numbers, each exact in fp32; the three smallest (x1 y2, x2 y1, x2 y2, together at most
-// 2^-21 of the product, 2^-25 of it on average) are left out, the other six are summed in fp32.
-// Why: v_mfma_f32_32x32x16_bf16 does 16 times the operations per cycle of v_mfma_f32_32x32x2_f32, six
-// of them still 2.7 times.  Measured for 32x32x32 blocks in a loop, three wavefronts per SIMD: 436 ns a
-// block in fp32 (154 TFLOP/s), 213 ns as six bf16 products, 274 ns with the split of the gathered operand in
-// the loop (241 ns where two output blocks share it).  The rounding that counts is that of the running sum of the
+// nine products of bf16 numbers, each exact in fp32; the smallest (x2 y2, at most 2^-30 of the product) is left out, the
+// other eight are summed in fp32, so that a single product comes out as the fp32 instruction rounds it (worst error 6.0e-8,
+// 2-norm 2.5e-8 either way; without x1 y2 and x2 y1 as well it would be 1.9e-7 and 3.1e-8, at 6 % less time for the
+// U-Net on 6k voxels, 2 % on 150k).
+// Exact needs the third part to be a bf16 number too: both operands are split 2^23 times their size, which takes the
+// last bit of the smallest float to 2^-126, the smallest normal bf16 number.  (Unscaled, bits drop out of operands below
+// 2^-110: 2-norm error 4.4e-6 at 2^-116, 4.5e-3 at 2^-126.)  The sums are 2^46 times the true ones until they are final.
+// Why: v_mfma_f32_32x32x16_bf16 does 16 times the operations per cycle of v_mfma_f32_32x32x2_f32, eight
+// of them still twice.  Measured for 32x32x32 blocks in a loop, three wavefronts per SIMD: 441 ns a
+// block in fp32 (152 TFLOP/s), 291 ns as eight bf16 products, 365 ns with the split of the gathered operand in
+// the loop (324 ns where two output blocks share it).  The rounding that counts is that of the running sum of the
 // leading products x0 y0; the others go into a sum of their own (struct Sum), so it is rounded once per 16 channels,
 // where the fp32 instruction rounds its sum eight times.  2-norm error against 64-bit sums, fp32 instruction -> here:
-// four layers of 32 channels on 500k sites 1.63e-7 -> 0.72e-7, of 64 channels 1.33e-7 -> 0.74e-7, of 128 channels on
-// 5k 1.35e-7 -> 0.77e-7; the seven-scale U-Net on 150k voxels 4.2e-7 -> 2.0e-7.  (All six into one sum: 1.85e-7,
-// 1.48e-7, 1.54e-7 and 4.4e-7 - more than the fp32 instruction's - because each of the six roundings is to the sum.)
-// The gathered operand is split by truncation (and, subtract, byte permute: 5.5 instructions a float; rounding
-// to nearest - convert, unpack, subtract - takes as many and measured 303 ns), the weights, once, by rounding
-// to nearest.  What has no such sum - infinities, NaN, sums that overflow in between - comes out as NaN or
-// infinity; those elements are summed again in plain fp32 (repair_sums), so an infinity stays one.
+// four layers of 32 channels on 500k sites 1.63e-7 -> 0.69e-7, of 64 channels 1.33e-7 -> 0.73e-7, of 128 channels on
+// 5k 1.35e-7 -> 0.77e-7; the seven-scale U-Net on 150k voxels 4.2e-7 -> 2.0e-7.
+// The gathered operand is split by truncation (multiply, and, subtract, byte permute: 6.5 instructions a float; rounding
+// to nearest - convert, unpack, subtract - takes as many and is slower), the weights, once, by rounding to nearest.
+// What has no such sum - infinities, NaN, weights from 2^104, sums from 2^82 - comes out as NaN or infinity;
+// those elements are summed again in plain fp32 (repair_sums), so an infinity stays one.
 // ---------------------------------------------------------------------------------------
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
@@ -170,7 +174,12 @@ struct Parts {
   u32x4 p[3];
 };
 
+constexpr float SPLIT_SCALE = 0x1p23f;                            // of either operand
+constexpr float SUM_SCALE = 0x1p46f, SUM_UNSCALE = 0x1p-46f;      // of their products
+
 __device__ __forceinline__ void split_pair(float a, float b, unsigned &p0, unsigned &p1, unsigned &p2) {
+  a *= SPLIT_SCALE;
+  b *= SPLIT_SCALE;
   const unsigned ua = __float_as_uint(a), ub = __float_as_uint(b);
   p0 = __builtin_amdgcn_perm(ub, ua, 0x07060302);  // the upper halves of both
   const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
@@ -199,14 +208,14 @@ __device__ __forceinline__ f16v mfma_bf16(const u32x4 &a, const u32x4 &b, f16v c
 }
 
 // A running sum: the products of the leading parts, and apart from them all others, which are 2^-7 of these at most -
-// so the sum that carries the rounding error is rounded once per 16 channels.
+// so the sum that carries the rounding error is rounded once per 16 channels.  (Both times SUM_SCALE.)
 struct Sum {
   f16v lead, rest;
 };
 __device__ __forceinline__ void sum_start(Sum &a, float bias) {
 #pragma unroll
   for (int v = 0; v < 16; v++) {
-    a.lead[v] = bias;
+    a.lead[v] = bias * SUM_SCALE;
     a.rest[v] = 0.0f;
   }
 }
@@ -217,8 +226,17 @@ __device__ __forceinline__ f16v sum_of(const Sum &a) {
   return t;
 }
 
+// the sums of products themselves, of a total of such sums
+template <int N, class A>
+__device__ __forceinline__ void unscale(A &a) {
+#pragma unroll
+  for (int j = 0; j < N; j++) a[j] *= SUM_UNSCALE;
+}
+
 // acc += 16 channels
 __device__ __forceinline__ void mac16(const Parts &a, const Parts &b, Sum &acc) {
+  acc.rest = mfma_bf16(a.p[1], b.p[2], acc.rest);
+  acc.rest = mfma_bf16(a.p[2], b.p[1], acc.rest);
   acc.rest = mfma_bf16(a.p[2], b.p[0], acc.rest);
   acc.rest = mfma_bf16(a.p[1], b.p[1], acc.rest);
   acc.rest = mfma_bf16(a.p[0], b.p[2], acc.rest);
@@ -245,12 +263,16 @@ static inline int conv_nbt_padded(int Cout) {
   return (int)cdiv(nbt, nb) * nb;
 }
 
-// the upper half of a float, rounded to nearest even unless that overflows (an infinity or NaN: as it is)
+// the upper half of a float that is not large, rounded to nearest even
 __device__ __forceinline__ unsigned bf16_part(float x) {
   const unsigned u = __float_as_uint(x);
-  if ((u & 0x7F800000u) == 0x7F800000u) return (u >> 16) | ((u & 0xFFFFu) ? 0x40u : 0u);
-  const unsigned up = (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
-  return (up & 0x7F80u) == 0x7F80u ? u >> 16 : up;
+  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+}
+
+// A weight from its three parts, exactly (cold).
+__device__ __forceinline__ float weight_of(unsigned p0, unsigned p1, unsigned p2) {
+  if ((p0 & 0x7F80u) == 0x7F80u) return __uint_as_float((p1 << 16) | p2);
+  return (__uint_as_float(p0 << 16) + __uint_as_float(p1 << 16) + __uint_as_float(p2 << 16)) * (1.0f / SPLIT_SCALE);
 }
 
 // The fp32 layout of insc_conv_pack_weights: a tile is 4 KB, four 1 KB quarters; quarter q holds, for lane 0..63 in
@@ -286,13 +308,20 @@ __global__ void split_weights_kernel(const float *__restrict__ W, const float *_
       x = Wp ? Wp[tile * 1024 + ((cin32 >> 2) & 3) * 256 + ((cin32 >> 4) * 32 + (lane & 31)) * 4 + (cin32 & 3)]
              : W[((int64_t)k * Cin + cin) * Cout + col];
     uint16_t *to = Ws + tile * (WT_BYTES / 2) + s * 1536 + lane * 8 + j8;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      const unsigned u = bf16_part(x);
-      to[i * 512] = (uint16_t)u;
-      const float part = __uint_as_float(u << 16);
-      x = (u & 0x7F80u) == 0x7F80u ? 0.0f : x - part;  // (exact)
+    // (weights that the scale would take to the end of the range, infinities and NaN: NaN in the first part, so that their
+    // sums are formed again, and the weight itself in the other two)
+    const unsigned u = __float_as_uint(x);
+    unsigned p0 = 0x7FC0u, p1 = u >> 16, p2 = u & 0xFFFFu;
+    if (fabsf(x) < 0x1p104f) {
+      x *= SPLIT_SCALE;
+      p0 = bf16_part(x);
+      x -= __uint_as_float(p0 << 16);  // (exact)
+      p1 = bf16_part(x);
+      p2 = bf16_part(x - __uint_as_float(p1 << 16));
     }
+    to[0] = (uint16_t)p0;
+    to[512] = (uint16_t)p1;
+    to[1024] = (uint16_t)p2;
   }
 }
 
@@ -343,7 +372,7 @@ __device__ __forceinline__ void repair_sums(A &a, int v0, const F &tile_sums) {
 
 // ---------------------------------------------------------------------------------------
 // MFMA kernel.  Cin % 16 == 0, rows of `in` 16-byte aligned, packed weights.
-// Software pipeline: while the 12*NB MFMAs of one (offset, channel chunk) run, the gather of
+// Software pipeline: while the 16*NB MFMAs of one (offset, channel chunk) run, the gather of
 // the next chunk's input rows and the next weight tile are already in flight.
 // ---------------------------------------------------------------------------------------
 // Gathered row chunk: lane (r, h) holds channels h*8 .. h*8+7 of the chunk's first half (q[0], q[1]) and of its
@@ -435,10 +464,10 @@ __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of,
       for (int i = 0; i < 3; i++) p[i] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u + 1024u * i, soff));
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        float w = 0.0f;
+        unsigned q[3];
 #pragma unroll
-        for (int i = 0; i < 3; i++)  // (exact)
-          w += __uint_as_float(j & 1 ? p[i][j >> 1] & 0xFFFF0000u : p[i][j >> 1] << 16);
+        for (int i = 0; i < 3; i++) q[i] = j & 1 ? p[i][j >> 1] >> 16 : p[i][j >> 1] & 0xFFFFu;
+        const float w = weight_of(q[0], q[1], q[2]);
         sums = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], w, sums, 0, 0, 0);
       }
     }
@@ -750,12 +779,18 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     if (my_row < 0) return -1;
     return MODE == MAP_NBR ? map[(int64_t)my_row * K + k] : MODE == MAP_IDENTITY ? my_row : map1[my_row] == k ? map[my_row] : -1;
   };
+  f16v acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) acc[b] = sum_of(sums[b]);
   if (S == 1) {
-    // (put back into the running sums, one block at a time: copies of all blocks' totals would cost NB = 3 its second
-    // wavefront per SIMD, 32 -> 96 at 200k sites 99 -> 124 us)
+    // (one block at a time: copies of all blocks' repeated sums would cost NB = 3 its second wavefront per SIMD, 32 -> 96 at
+    // 200k sites 99 -> 124 us)
     float t = 0.0f;
 #pragma unroll
-    for (int b = 0; b < NB; b++) t = not_finite<16>(sum_of(sums[b]), t);
+    for (int b = 0; b < NB; b++) {
+      unscale<16>(acc[b]);
+      t = not_finite<16>(acc[b], t);
+    }
     if (__builtin_expect(__any(t != t), 0)) {
 #pragma unroll 1
       for (int bb = 0; bb < NB; bb++) {
@@ -769,18 +804,11 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
         for (int b = 0; b < NB; b++) {
           if (b != bb) continue;
 #pragma unroll
-          for (int v = 0; v < 16; v++)
-            if (is_bad(sums[b].lead[v] + sums[b].rest[v])) {
-              sums[b].lead[v] = x[v];
-              sums[b].rest[v] = 0.0f;
-            }
+          for (int v = 0; v < 16; v++) acc[b][v] = is_bad(acc[b][v]) ? x[v] : acc[b][v];
         }
       }
     }
   }
-  f16v acc[NB];
-#pragma unroll
-  for (int b = 0; b < NB; b++) acc[b] = sum_of(sums[b]);
 
   if (S > 1) {
     // Every wavefront leaves its partial sum in LDS; each then adds up - in wavefront order - and
@@ -856,6 +884,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       if (lane == 0) pcount[unit * S + wave] = 0;
     }
     const int c = cb0 * 32 + r;
+    unscale<NV>(a);
     repair_sums<NV>(a, wave * NV, [&]() -> f16v {
       f16v t;
 #pragma unroll
@@ -1155,11 +1184,12 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   Frag g[D];
   WFrag bw;
   auto prime = [&](unsigned rr, uint32_t b) {  // the gathers of the first items, and the centre's weights
+    const uint32_t lane16 = (uint32_t)lane_again() * 16u;  // (not a constant of the loop: the weights would be, and spilled)
 #pragma unroll
     for (int i = 0; i < D - 1; i++) g[i] = gather(next_q(rr), ids[i], b);
 #pragma unroll
     for (int i = 0; i < PIECES; i++)
-      bw.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u, 13u * WT_BYTES + 1024u * i));
+      bw.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, lane16, 13u * WT_BYTES + 1024u * i));
   };
   prime(rest, base);
 
@@ -1244,6 +1274,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     prime(rest_n, base_n);
     __builtin_amdgcn_sched_barrier(0);
     f16v acc = sum_of(sum);
+    unscale<16>(acc);
 
     // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3)
     repair_sums<16>(acc, 0, [&]() -> f16v {
@@ -1543,6 +1574,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 #pragma unroll
             for (int v = 0; v < 16; v++) sum[v] = total[o][v] + sum[v];
           }
+          unscale<16>(sum);
           repair_sums<16>(sum, 0, [&]() -> f16v {
             f16v x;
 #pragma unroll
@@ -1753,6 +1785,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int v = 0; v < 16; v++) sum[v] = total[v] + sum[v];
   }
+  unscale<16>(sum);
   repair_sums<16>(sum, 0, [&]() -> f16v {
     f16v x;
 #pragma unroll

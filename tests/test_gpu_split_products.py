@@ -95,7 +95,7 @@ def test_error_against_64_bit_sums(scene, case):
 
 @pytest.mark.parametrize("case", KERNELS)
 def test_magnitudes_far_from_one(scene, case):
-    """Powers of two move through exactly: three parts of eight bits each keep the whole exponent range."""
+    """Powers of two move through exactly."""
     _, x, W, b = data(scene, case)
     base = layer(scene, x, W, b, case)
     for e in (-60, 60):
@@ -286,3 +286,35 @@ def test_the_other_maps(kind, Cin, Cout):
     fin = np.isfinite(ref)
     assert np.isnan(ref).any() and np.isinf(ref).any() and (got[fin] == base[fin]).all()
     assert (np.isnan(got) == np.isnan(ref)).all() and (got[np.isinf(ref)] == ref[np.isinf(ref)]).all()
+
+
+@pytest.mark.parametrize("case", KERNELS)
+@pytest.mark.parametrize("ex,ew", [(0, 0), (-104, 60), (-112, 60), (-126, 100), (-140, 100), (90, -112), (90, -126), (90, -140)])
+def test_a_single_product_is_rounded_as_in_fp32(scene, case, ex, ew):
+    """One input channel and the centre's offset alone: the result is one product, whatever the size of its factors
+    (subnormal ones among them).  Its error is that of a fp32 product, half a unit in the last place, and at most 2^-27 of the
+    product on top: 2^-30 from the part product that is left out and seven roundings of a sum of 2^-6 of it."""
+    rng, x, W, b = data(scene, case)
+    n = len(x)
+    one, j = np.zeros_like(x), rng.integers(0, case[0], n)
+    one[np.arange(n), j] = (x[np.arange(n), j].astype(np.float64) * 2.0 ** ex).astype(np.float32)
+    Wc = np.zeros_like(W)
+    Wc[13] = (W[13].astype(np.float64) * 2.0 ** ew).astype(np.float32)
+    got, ref = layer(scene, one, Wc, np.zeros_like(b), case), one.astype(np.float64) @ Wc[13].astype(np.float64)
+    err, fp32 = np.abs(got - ref), np.abs(ref.astype(np.float32) - ref)
+    assert (err <= np.abs(ref) * (2.0 ** -24 + 2.0 ** -27)).all()
+    assert np.linalg.norm(err) <= 1.02 * np.linalg.norm(fp32)
+
+
+@pytest.mark.parametrize("case", KERNELS)
+@pytest.mark.parametrize("ex,ew", [(-112, 60), (-126, 100), (-140, 100), (90, -126), (-60, -60), (100, 10), (10, 110), (60, 60)])
+def test_error_against_64_bit_sums_far_from_one(scene, case, ex, ew):
+    """The bound of test_error_against_64_bit_sums at both ends of the range, where parts of eight bits would run out of
+    exponents (and, from sums of 2^82 and weights of 2^104 up, where the sums are formed in plain fp32: a rounding per
+    product pair)."""
+    rng, x, W, b = data(scene, case)
+    x, W = ((v.astype(np.float64) * 2.0 ** e).astype(np.float32) for v, e in ((x, ex), (W, ew)))
+    b = (b.astype(np.float64) * 2.0 ** (ex + ew)).astype(np.float32)
+    got, nbr = layer(scene, x, W, b, case), scene[3]
+    ref, mag = sums64(nbr, x, W, b), sums64(nbr, np.abs(x), np.abs(W), np.abs(b))
+    assert (np.abs(got - ref) <= 2.0 ** -24 * 27 * case[0] / (8 if ex + ew < 70 and ew < 100 else 2) * mag).all()
