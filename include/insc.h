@@ -183,8 +183,9 @@ int insc_order_append(const insc_grid *g, const int32_t *d_nbr, const int32_t *d
  * (CUDA/Convolution.cpp:152-218); K = 8 with a child map is Convolution_updateOutput for
  * size 2 / stride 2 (CUDA/Convolution.cpp:52-81); K = 1 with d_nbr = NULL (identity map) is
  * NetworkInNetwork_updateOutput (CUDA/NetworkInNetwork.cpp:9-25).  d_W is [K,Cin,Cout]; d_Wp
- * (nullable) is the same weights packed by insc_conv_pack_weights - give it to skip the
- * per-call packing (then d_W may be NULL when Cin is a multiple of 16).
+ * (nullable) is the same weights packed by insc_conv_pack_weights or, faster, split by insc_conv_split_weights - give it
+ * to skip the per-call work, which is a launch more and scratch memory of the stream, allocated when it has to grow:
+ * do not capture calls with raw weights alone (with d_Wp, d_W may be NULL when Cin is a multiple of 16).
  * n_in_rows = rows of d_in (the gather is bounds-checked against it; n_in_rows*ld_in*4 must stay
  * below 4 GB).  h_muladds (nullable) receives the multiply-add count the reference returns
  * (synchronises). */
@@ -199,8 +200,9 @@ int64_t insc_conv_packed_floats(int K, int Cin, int Cout);
 int insc_conv_pack_weights(const float *d_W, int K, int Cin, int Cout, float *d_Wp, void *stream);
 /* The layout the kernels themselves read: every weight as three bf16 parts that hold it exactly
  * (insc_conv_split_floats floats, 16-byte aligned).  Every d_Wp argument takes such weights as well: pass their address
- * with its lowest bit set, INSC_SPLIT_WEIGHTS(d_Ws).  Packed fp32 weights are split on every call instead, into
- * scratch memory. */
+ * with its lowest bit set, INSC_SPLIT_WEIGHTS(d_Ws).  Packed fp32 weights give the same bits; the kernels split each
+ * tile of them as they read it, which takes longer (64 -> 64 at 39k sites 54 us against 48, at 500k 411 against 337).
+ * Either layout must stay below 4 GB. */
 int64_t insc_conv_split_floats(int K, int Cin, int Cout);
 int insc_conv_split_weights(const float *d_W, int K, int Cin, int Cout, float *d_Ws, void *stream);
 #define INSC_SPLIT_WEIGHTS(d_Ws) ((const float *)((uintptr_t)(d_Ws) | 1))

@@ -149,8 +149,8 @@ bool conv_two_sources_ok(int mode, int K, const float *in, int64_t ld_in, const 
                          int64_t in2_rows, int Cin, int latency);
 int64_t packed_floats(int K, int Cin, int Cout);
 int64_t split_floats(int K, int Cin, int Cout);
-// Ws = the three-part layout of raw weights W, or of packed ones Wp
-int split_weights(const float *W, const float *Wp, int K, int Cin, int Cout, float *Ws, hipStream_t s);
+// Ws = the three-part layout of raw weights W
+int split_weights(const float *W, int K, int Cin, int Cout, float *Ws, hipStream_t s);
 // A pointer to weights in the three-part layout, where packed weights are asked for: the address (16-byte aligned)
 // with its lowest bit set.
 static inline const float *split_ref(const float *Ws) { return Ws ? (const float *)((uintptr_t)Ws | 1) : nullptr; }

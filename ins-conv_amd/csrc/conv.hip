@@ -263,10 +263,9 @@ static inline int conv_nbt_padded(int Cout) {
   return (int)cdiv(nbt, nb) * nb;
 }
 
-// the upper half of a float that is not large, rounded to nearest even
+// a float rounded to bf16, to nearest even
 __device__ __forceinline__ unsigned bf16_part(float x) {
-  const unsigned u = __float_as_uint(x);
-  return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+  return __builtin_bit_cast(uint16_t, (__bf16)x);
 }
 
 // A weight from its three parts, exactly (cold).
@@ -291,9 +290,9 @@ __global__ void pack_weights_kernel(const float *__restrict__ W, int K, int Cin,
   }
 }
 
-// The three-part layout that the kernels read, from raw weights (W) or from the fp32 layout (Wp).
-__global__ void split_weights_kernel(const float *__restrict__ W, const float *__restrict__ Wp, int K, int Cin, int Cout,
-                                     int nch, int nbtp, uint16_t *__restrict__ Ws) {
+// The three-part layout.
+__global__ void split_weights_kernel(const float *__restrict__ W, int K, int Cin, int Cout, int nch, int nbtp,
+                                     uint16_t *__restrict__ Ws) {
   const int64_t total = (int64_t)K * nch * nbtp * 1024;  // one (lane, value) of all three parts per thread
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
     const int j8 = (int)(e & 7), lane = (int)((e >> 3) & 63), s = (int)((e >> 9) & 1);
@@ -303,19 +302,16 @@ __global__ void split_weights_kernel(const float *__restrict__ W, const float *_
     q /= nbtp;
     const int ch = (int)(q % nch), k = (int)(q / nch);
     const int cin32 = s * 16 + (lane >> 5) * 8 + j8, cin = ch * 32 + cin32, col = nb * 32 + (lane & 31);
-    float x = 0.0f;
-    if (cin < Cin && col < Cout)
-      x = Wp ? Wp[tile * 1024 + ((cin32 >> 2) & 3) * 256 + ((cin32 >> 4) * 32 + (lane & 31)) * 4 + (cin32 & 3)]
-             : W[((int64_t)k * Cin + cin) * Cout + col];
+    float x = (cin < Cin && col < Cout) ? W[((int64_t)k * Cin + cin) * Cout + col] : 0.0f;
     uint16_t *to = Ws + tile * (WT_BYTES / 2) + s * 1536 + lane * 8 + j8;
     // (weights that the scale would take to the end of the range, infinities and NaN: NaN in the first part, so that their
     // sums are formed again, and the weight itself in the other two)
     const unsigned u = __float_as_uint(x);
-    unsigned p0 = 0x7FC0u, p1 = u >> 16, p2 = u & 0xFFFFu;
-    if (fabsf(x) < 0x1p104f) {
-      x *= SPLIT_SCALE;
-      p0 = bf16_part(x);
-      x -= __uint_as_float(p0 << 16);  // (exact)
+    unsigned p0 = bf16_part(x * SPLIT_SCALE), p1 = u >> 16, p2 = u & 0xFFFFu;
+    if ((p0 & 0x7F80u) == 0x7F80u) {
+      p0 = 0x7FC0u;
+    } else {
+      x = x * SPLIT_SCALE - __uint_as_float(p0 << 16);  // (exact)
       p1 = bf16_part(x);
       p2 = bf16_part(x - __uint_as_float(p1 << 16));
     }
@@ -380,14 +376,55 @@ __device__ __forceinline__ void repair_sums(A &a, int v0, const F &tile_sums) {
 struct Frag {
   float4 q[4];
 };
+// A weight tile as it is loaded.  PW: from the packed fp32 layout (what insc_conv_pack_weights makes and callers of the C
+// ABI may hold): sixteen weights a lane, which are split as split_weights_kernel does it, so either layout gives the same
+// bits.  Costs about as many instructions per tile as the gathered chunk's parts: 64 -> 64 at 500k sites 411 us against 337,
+// 39k sites 54 against 48; in scratch memory, once per call, it would cost a launch, an allocation now and then, and
+// so capture into a graph.
+template <bool PW>
 struct WFrag {
   Parts s[2];
 };
+template <>
+struct WFrag<true> {
+  float4 q[4];
+};
+constexpr int pw_pieces(bool pw, int halves) { return pw ? 4 : 3 * halves; }  // of a tile: 1 KB each
+constexpr int wt_bytes(bool pw) { return pw ? 4096 : WT_BYTES; }
+
+typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+typedef float fl2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {  // (one instruction)
+  const fl2v v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf2v));
+}
+// eight weights, as split_weights_kernel
+__device__ __forceinline__ Parts split8_nearest(const float4 &lo, const float4 &hi) {
+  const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+  Parts s;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    float a = x[2 * j] * SPLIT_SCALE, b = x[2 * j + 1] * SPLIT_SCALE;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const unsigned p = bf16_pair(a, b);
+      s.p[i][j] = p;
+      a -= __uint_as_float(p << 16);
+      b -= __uint_as_float(p & 0xFFFF0000u);
+    }
+  }
+  return s;
+}
+__device__ __forceinline__ const Parts &parts_of(const WFrag<false> &w, int half) { return w.s[half]; }
+__device__ __forceinline__ Parts parts_of(const WFrag<true> &w, int half) {
+  return split8_nearest(w.q[2 * half], w.q[2 * half + 1]);
+}
 
 // acc += chunk a times weight tile b; full: the chunk's second half exists
-__device__ __forceinline__ void mac_chunk(Sum &acc, const Parts (&a)[2], const WFrag &b, bool full) {
-  mac16(a[0], b.s[0], acc);
-  if (full) mac16(a[1], b.s[1], acc);
+template <bool PW>
+__device__ __forceinline__ void mac_chunk(Sum &acc, const Parts (&a)[2], const WFrag<PW> &b, bool full) {
+  mac16(a[0], parts_of(b, 0), acc);
+  if (full) mac16(a[1], parts_of(b, 1), acc);
 }
 
 // Gather: every lane reads the 64 bytes of its own input row that the MFMA A operand needs, with
@@ -424,14 +461,22 @@ __device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on
   f.q[3] = buf_load16(rin, v1 + 16u, 0);
   return f;
 }
-// weight tile `tile` of the packed filter (on false: zeros)
-__device__ __forceinline__ WFrag load_wtile(__amdgpu_buffer_rsrc_t rw, int tile, bool on, uint32_t lane16) {
-  const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * WT_BYTES);
-  const uint32_t voff = on ? lane16 : BUF_OOB;
-  WFrag f;
+// weight tile `tile` of the filter (on false: zeros)
+template <bool PW>
+__device__ __forceinline__ WFrag<PW> load_wtile(__amdgpu_buffer_rsrc_t rw, int tile, bool on, uint32_t lane16) {
+  const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * wt_bytes(PW));
+  WFrag<PW> f;
+  if constexpr (PW) {
+    // (half s, channels h * 8 ..: quarters 2h and 2h + 1, there at lane s * 32 + column)
+    const uint32_t voff = on ? (lane16 & 512u) * 4u + (lane16 & 511u) : BUF_OOB;
 #pragma unroll
-  for (int i = 0; i < 6; i++)
-    f.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, voff + 1024u * (i & 3), soff + (i >= 4 ? 4096u : 0u)));
+    for (int i = 0; i < 4; i++) f.q[i] = buf_load16(rw, voff + (i >> 1) * 512u + (i & 1) * 1024u, soff);
+  } else {
+    const uint32_t voff = on ? lane16 : BUF_OOB;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+      f.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, voff + 1024u * (i & 3), soff + (i >= 4 ? 4096u : 0u)));
+  }
   return f;
 }
 
@@ -441,7 +486,7 @@ __device__ __forceinline__ WFrag load_wtile(__amdgpu_buffer_rsrc_t rw, int tile,
 // Cold, so it waits for every load; but one NaN of a scan reaches whole scales, which then pass through it: 32 -> 32 at
 // 500k sites 0.15 ms finite, 0.34 all NaN (element by element in scalar code: 12.9), 64 -> 64 at 500k 0.42 and 1.25 (54.5),
 // 96 -> 96 at 10k 0.07 and 0.21 (3.7).
-template <class Ids>
+template <bool PW, class Ids>
 __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of, int K, __amdgpu_buffer_rsrc_t rin,
                                                    uint32_t ld4, __amdgpu_buffer_rsrc_t rw, int Cin, int nch, int nbtp,
                                                    int nb) {
@@ -457,19 +502,30 @@ __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of,
       const uint32_t voff = src >= 0 ? (uint32_t)src * ld4 + (uint32_t)(c16 * 64 + h * 32) : BUF_OOB;
       const float4 lo = buf_load16(rin, voff, 0), hi = buf_load16(rin, voff + 16u, 0);
       const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(((k * nch + (c16 >> 1)) * nbtp + nb) * WT_BYTES +
-                                                                     (c16 & 1) * 3072);
-      u32x4 p[3];
+      const int tile = (k * nch + (c16 >> 1)) * nbtp + nb;
+      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * wt_bytes(PW) + (c16 & 1) * (PW ? 512 : 3072));
+      float wv[8];
+      if constexpr (PW) {
+        const uint32_t wo = (uint32_t)(h * 2048 + (lane & 31) * 16);
+        const float4 wlo = buf_load16(rw, wo, soff), whi = buf_load16(rw, wo + 1024u, soff);
+        const float t[8] = {wlo.x, wlo.y, wlo.z, wlo.w, whi.x, whi.y, whi.z, whi.w};
 #pragma unroll
-      for (int i = 0; i < 3; i++) p[i] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u + 1024u * i, soff));
+        for (int j = 0; j < 8; j++) wv[j] = t[j];
+      } else {
+        u32x4 p[3];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        unsigned q[3];
+        for (int i = 0; i < 3; i++) p[i] = __builtin_bit_cast(u32x4, buf_load16(rw, (uint32_t)lane * 16u + 1024u * i, soff));
 #pragma unroll
-        for (int i = 0; i < 3; i++) q[i] = j & 1 ? p[i][j >> 1] >> 16 : p[i][j >> 1] & 0xFFFFu;
-        const float w = weight_of(q[0], q[1], q[2]);
-        sums = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], w, sums, 0, 0, 0);
+        for (int j = 0; j < 8; j++) {
+          unsigned q[3];
+#pragma unroll
+          for (int i = 0; i < 3; i++) q[i] = j & 1 ? p[i][j >> 1] >> 16 : p[i][j >> 1] & 0xFFFFu;
+          wv[j] = weight_of(q[0], q[1], q[2]);
+        }
       }
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        sums = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], wv[j], sums, 0, 0, 0);
     }
 #pragma unroll
     for (int v = 0; v < 16; v++) sums[v] = have & (1u << (8 * (v >> 2) + (v & 3))) ? sums[v] : before[v];
@@ -492,7 +548,7 @@ __device__ __forceinline__ int first_offset(unsigned mask) {
 //         With gridDim.z = G > 1 the deal goes over S * G wavefronts in G blocks (different
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
-template <int NB, int K, int MODE, int S>
+template <int NB, int K, int MODE, int S, bool PW>
 __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) void conv_mfma_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
@@ -714,8 +770,8 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       return gather_chunk(rin, c.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h,
                           Cin - c.ch * 32 >= 32);
     };
-    auto wload = [&](const Cursor &c, int b) -> WFrag {
-      return load_wtile(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
+    auto wload = [&](const Cursor &c, int b) -> WFrag<PW> {
+      return load_wtile<PW>(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
     };
 
     // Pipeline: while item t runs on the matrix cores, the gathers of items t+1 .. t+D-1 are in
@@ -730,7 +786,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     constexpr bool WRING = NB == 1;                         // weight tiles ride in the same ring
     constexpr int TURN = (WRING || NB % 2 == 0) ? D : (D % 2 == 0 ? D : 2 * D);
     Frag g[D];
-    WFrag bw[WRING ? D : 2];
+    WFrag<PW> bw[WRING ? D : 2];
     Cursor ci = first;  // next item to issue
 #pragma unroll
     for (int d = 0; d < D - 1; d++) {
@@ -756,7 +812,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
           if constexpr (!WRING) bw[(nn + 1) % 2] = (b + 1 < NB) ? wload(c0, b + 1) : wload(c1, 0);
           asm volatile("" ::: "memory");
           __builtin_amdgcn_sched_barrier(0);
-          const WFrag &bf = bw[WRING ? u % D : nn % 2];
+          const WFrag<PW> &bf = bw[WRING ? u % D : nn % 2];
           if (real) {
             if (b == 0) {
               as[0] = split8(g[u % D].q[0], g[u % D].q[1]);
@@ -798,7 +854,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
         f16v x;
 #pragma unroll
         for (int v = 0; v < 16; v++) x[v] = (bias && c < Cout) ? bias[c] : 0.0f;
-        add_plain_products(x, [&](int k) { return id_at(map0, k); }, K, make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u,
+        add_plain_products<PW>(x, [&](int k) { return id_at(map0, k); }, K, make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u,
                            make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, cb0 + bb);
 #pragma unroll
         for (int b = 0; b < NB; b++) {
@@ -890,10 +946,10 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
 #pragma unroll
       for (int v = 0; v < 16; v++) t[v] = (bias0 && c < Cout) ? bias0[c] : 0.0f;
       const __amdgpu_buffer_rsrc_t rw = make_rsrc(Wp, wp_bytes);
-      add_plain_products(t, [&](int k) { return id_at(map00, k); }, K, make_rsrc(in0, in_bytes0), (uint32_t)ld_in0 * 4u, rw, Cin,
+      add_plain_products<PW>(t, [&](int k) { return id_at(map00, k); }, K, make_rsrc(in0, in_bytes0), (uint32_t)ld_in0 * 4u, rw, Cin,
                          nch, nbtp, cb0);
       if (ep.src2_in)
-        add_plain_products(t, [&](int k) { return id_at(ep.src2_map, k); }, K,
+        add_plain_products<PW>(t, [&](int k) { return id_at(ep.src2_map, k); }, K,
                            make_rsrc(ep.src2_in, (uint32_t)(ep.src2_rows * ep.src2_ld * 4)), (uint32_t)ep.src2_ld * 4u, rw, Cin, nch,
                            nbtp, cb0);
       return t;
@@ -1019,7 +1075,7 @@ constexpr int WL_MIN_TILES = 2048;  // smaller launches go to conv_mfma_kernel (
 constexpr int WL_SCHED = 256;  // a block orders up to this many tiles of its own by cost
 
 // KS: halves of the 32-channel chunk that exist (1: 16 input channels, 2: 32)
-template <int KS>
+template <int KS, bool PW>
 __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
@@ -1035,8 +1091,17 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 31, h = lane >> 5;
 
-  // the filter but for the centre, already in per-lane order
-  {
+  // the filter but for the centre, in per-lane order
+  if constexpr (PW) {
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(Wp, wp_bytes);
+    for (int i = threadIdx.x; i < (K - 1) * KS * 64; i += WL_WAVES * 64) {
+      const int slot = i / (KS * 64), e = i - slot * (KS * 64), half = e >> 6, l = e & 63;
+      const uint32_t from = (uint32_t)((slot < 13 ? slot : slot + 1) * 4096 + (l >> 5) * 2048 + half * 512 + (l & 31) * 16);
+      const Parts p = split8_nearest(buf_load16(rw, from, 0), buf_load16(rw, from + 1024u, 0));
+#pragma unroll
+      for (int q = 0; q < 3; q++) wl[slot * TILE16 + (half * 3 + q) * 64 + l] = p.p[q];
+    }
+  } else {
     const u32x4 *src = reinterpret_cast<const u32x4 *>(Wp);
     for (int i = threadIdx.x; i < (K - 1) * TILE16; i += WL_WAVES * 64) {
       const int slot = i / TILE16, e = i - slot * TILE16;
@@ -1182,14 +1247,19 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   int my_row_n = load_row(tn);
   int mask_n_v = planned && tn < ntiles ? (int)plan.tmask[tn] : 0;
   Frag g[D];
-  WFrag bw;
+  WFrag<false> bw;  // of the item on the matrix cores
+  WFrag<PW> cw;     // the centre's
   auto prime = [&](unsigned rr, uint32_t b) {  // the gathers of the first items, and the centre's weights
     const uint32_t lane16 = (uint32_t)lane_again() * 16u;  // (not a constant of the loop: the weights would be, and spilled)
 #pragma unroll
     for (int i = 0; i < D - 1; i++) g[i] = gather(next_q(rr), ids[i], b);
+    if constexpr (PW) {
+      cw = load_wtile<PW>(rw, 13, true, lane16);
+    } else {
 #pragma unroll
-    for (int i = 0; i < PIECES; i++)
-      bw.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, lane16, 13u * WT_BYTES + 1024u * i));
+      for (int i = 0; i < PIECES; i++)
+        bw.s[i / 3].p[i % 3] = __builtin_bit_cast(u32x4, buf_load16(rw, lane16, 13u * WT_BYTES + 1024u * i));
+    }
   };
   prime(rest, base);
 
@@ -1240,7 +1310,12 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       };
       {
         const int q = next_q(rc);
-        if (q != 0) wread(q);  // (a tile without the centre; bw holds the centre's weights otherwise)
+        if (q != 0) {  // (a tile without the centre; bw or cw holds the centre's weights otherwise)
+          wread(q);
+        } else if constexpr (PW) {
+#pragma unroll
+          for (int i = 0; i < KS; i++) bw.s[i] = parts_of(cw, i);
+        }
         __builtin_amdgcn_sched_barrier(0);
         issue(std::integral_constant<int, 0>());
         __builtin_amdgcn_sched_barrier(0);
@@ -1281,7 +1356,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       f16v x;
 #pragma unroll
       for (int v = 0; v < 16; v++) x[v] = bv;
-      add_plain_products(
+      add_plain_products<PW>(
           x, [&](int k) { return base == BUF_OOB ? -1 : (int)__builtin_amdgcn_raw_buffer_load_b32(rids, (int)(base + k * pitch), 0, 0); },
           K, rin, ld4, rw, Cin, 1, 1, 0);
       return x;
@@ -1340,7 +1415,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
 // would hit L2: 1741 us (unbalanced).
 // ---------------------------------------------------------------------------------------
 #define INSC_LDS_PTR(x) ((__attribute__((address_space(3))) void *)(x))
-template <int NB, int ST>
+template <int NB, int ST, bool PW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 : 3, NB > 1 ? 2 : 3))) void conv_wshare_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
@@ -1348,10 +1423,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
   constexpr int K = 27, WV = 4;
   constexpr int NSTAGE = (TILE_M * K + 63) / 64;  // 14 loads of 64 entries; the last one half empty
+  constexpr int PC = pw_pieces(PW, 2);            // pieces of a weight tile
   __shared__ int nl[WV][NSTAGE * 64];
-  __shared__ u32x4 wl0[NB][6 * 64];
-  __shared__ u32x4 wl1[NB][6 * 64];
-  __shared__ u32x4 wl2[NB][6 * 64];
+  __shared__ u32x4 wl0[NB][PC * 64];
+  __shared__ u32x4 wl1[NB][PC * 64];
+  __shared__ u32x4 wl2[NB][PC * 64];
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int ntiles = (int)((n + TILE_M - 1) / TILE_M), ngroups = (ntiles + WV - 1) / WV;
   const int nug = (nbt + NB - 1) / NB;  // units per group
@@ -1477,16 +1553,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
         return nx;
       };
       // weight tiles of a step -> LDS, their 1 KB pieces dealt to the four wavefronts
-      auto w_issue = [&](const Step &c, u32x4 (*wl)[6 * 64]) {
+      auto w_issue = [&](const Step &c, u32x4 (*wl)[PC * 64]) {
 #pragma unroll
-        for (int i = 0; i < (6 * NB + WV - 1) / WV; i++) {
-          const int piece = i * WV + wave, o = piece / 6;
-          if (piece >= 6 * NB) break;
-          const uint32_t soff = (uint32_t)(((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + ob0 + o) * (uint32_t)WT_BYTES;
+        for (int i = 0; i < (PC * NB + WV - 1) / WV; i++) {
+          const int piece = i * WV + wave, o = piece / PC;
+          if (piece >= PC * NB) break;
+          const uint32_t soff = (uint32_t)(((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + ob0 + o) * (uint32_t)wt_bytes(PW);
           const bool ok = c.k >= 0 && ob0 + o < nbt;
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               rw, INSC_LDS_PTR(&wl[0][piece * 64]), 16,
-              (int)(ok ? (uint32_t)((piece - o * 6) * 1024 + lane * 16) : BUF_OOB), (int)soff, 0, 0);
+              (int)(ok ? (uint32_t)((piece - o * PC) * 1024 + lane * 16) : BUF_OOB), (int)soff, 0, 0);
         }
       };
       auto gather = [&](const Step &c) -> Frag {
@@ -1495,7 +1571,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
         const bool on = c.k >= 0 && ((mine >> kk) & 1u) && src >= 0;
         return gather_chunk(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h, Cin - c.ch * 32 >= 32);
       };
-      auto compute = [&](const Step &c, const Frag &a, const u32x4 (*wl)[6 * 64]) {
+      auto compute = [&](const Step &c, const Frag &a, const u32x4 (*wl)[PC * 64]) {
         if (c.k < 0 || !((mine >> c.k) & 1u)) return;  // (the same for every lane of the wavefront)
         const bool full = Cin - c.ch * 32 >= 32;
         if (c.p != cur) {
@@ -1512,9 +1588,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 #pragma unroll
         for (int o = 0; o < NB; o++) {
           if (ob0 + o >= nbt) break;
-          WFrag bf;
+          WFrag<PW> bf;
+          if constexpr (PW) {
 #pragma unroll
-          for (int i = 0; i < 6; i++) bf.s[i / 3].p[i % 3] = wl[o][i * 64 + lane];
+            for (int i = 0; i < 4; i++)
+              bf.q[i] = __builtin_bit_cast(float4, wl[o][(2 * h + (i & 1)) * 64 + (i >> 1) * 32 + r]);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 6; i++) bf.s[i / 3].p[i % 3] = wl[o][i * 64 + lane];
+          }
           mac_chunk(acc[o], as, bf, full);
         }
       };
@@ -1538,10 +1620,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
       __builtin_amdgcn_sched_barrier(0);
       // Before a barrier every wavefront waits until its own pieces of the step's weight tiles have
       // landed in LDS: everything but what was issued after them - the step's four gather loads and the next
-      // step's (at least 6 NB / 4) pieces and four gather loads; the order of the loads is pinned.
-      auto turn = [&](Step &c, Step &cp2, const Frag &a, Frag &ap2, const Step &cp1, u32x4 (*wl)[6 * 64],
-                      u32x4 (*wlp2)[6 * 64]) {
-        __builtin_amdgcn_s_waitcnt(0x0F70 | (8 + 6 * NB / WV));
+      // step's (at least PC * NB / 4) pieces and four gather loads; the order of the loads is pinned.
+      auto turn = [&](Step &c, Step &cp2, const Frag &a, Frag &ap2, const Step &cp1, u32x4 (*wl)[PC * 64],
+                      u32x4 (*wlp2)[PC * 64]) {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (8 + PC * NB / WV));
         __syncthreads();  // the step's weights are complete for every wavefront, and nobody reads the oldest buffer any more
         __builtin_amdgcn_sched_barrier(0);
         cp2 = step_next(cp1);
@@ -1579,7 +1661,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
             f16v x;
 #pragma unroll
             for (int v = 0; v < 16; v++) x[v] = bv[o];
-            add_plain_products(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K, rin, ld4,
+            add_plain_products<PW>(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K, rin, ld4,
                                rw, Cin, nch, nbtp, ob0 + o);
             return x;
           });
@@ -1635,7 +1717,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 // (two wavefronts per SIMD: at three the sums, parts and weights do not fit the registers - 64 -> 64 at 39k sites
 // 55 us with 30 of them spilled against 47)
 constexpr int OWN_WAVES = 8;  // one block per compute unit
-template <int ST, int D>
+template <int ST, int D, bool PW>
 __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_own_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
@@ -1729,8 +1811,8 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
       return gather_chunk(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), h,
                           Cin - cu.ch * 32 >= 32);
     };
-    auto wload = [&](const Cursor &cu) -> WFrag {
-      return load_wtile(rw, ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob, cu.k >= 0, lane16);
+    auto wload = [&](const Cursor &cu) -> WFrag<PW> {
+      return load_wtile<PW>(rw, ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob, cu.k >= 0, lane16);
     };
     const int nitems = __builtin_popcount(tmask) * nch;
     Cursor first;
@@ -1740,7 +1822,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
     first.rest = tmask & hm[0];
     first = step(first);
     Frag g[D];
-    WFrag bw[D];
+    WFrag<PW> bw[D];
     Cursor ci = first, c0 = first;
 #pragma unroll
     for (int d = 0; d < D - 1; d++) {
@@ -1790,7 +1872,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
     f16v x;
 #pragma unroll
     for (int v = 0; v < 16; v++) x[v] = bv;
-    add_plain_products(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K,
+    add_plain_products<PW>(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K,
                        make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u, make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, ob);
     return x;
   });
@@ -2022,9 +2104,9 @@ static int pack_weights(const float *W, int K, int Cin, int Cout, float *Wp, hip
   return INSC_OK;
 }
 
-int split_weights(const float *W, const float *Wp, int K, int Cin, int Cout, float *Ws, hipStream_t s) {
+int split_weights(const float *W, int K, int Cin, int Cout, float *Ws, hipStream_t s) {
   const int64_t total = packed_floats(K, Cin, Cout);
-  hipLaunchKernelGGL(split_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, Wp, K, Cin, Cout,
+  hipLaunchKernelGGL(split_weights_kernel, dim3(grid_for(total, 256, 4096)), dim3(256), 0, s, W, K, Cin, Cout,
                      conv_nch(Cin), conv_nbt_padded(Cout), reinterpret_cast<uint16_t *>(Ws));
   INSC_LAUNCH_CHECK();
   return INSC_OK;
@@ -2049,8 +2131,9 @@ static std::atomic<int64_t> g_own_min_units{1750};
 // Same bits either way.
 static std::atomic<int64_t> g_wl_min_tiles{WL_MIN_TILES};
 
-// W: raw [K,Cin,Cout] weights (always needed by the generic kernel); Wp: split weights (split_ref), or packed
-// fp32 ones or null, in which case their parts are made in scratch memory first.
+// W: raw [K,Cin,Cout] weights (always needed by the generic kernel); Wp: split weights (split_ref), packed
+// fp32 ones, or null, in which case the raw ones are split (or, where that layout would pass 4 GB, packed) into scratch
+// memory first.
 // Whether one launch can gather from two sources (BnEpilogue::src2_*): the shapes that the split
 // kernel serves - 3^3 layers of a residual frame (latency != 0) and stride-2 deconvolutions, from 32
 // input channels on.
@@ -2087,7 +2170,9 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
   plan.cus = (unsigned)device_cus();
   if (conv_uses_mfma(in, ld_in, Cin, K)) {
     // the gather addresses rows with 32-bit byte offsets (buffer loads)
-    const int64_t in_bytes64 = in_rows * ld_in * 4, wp_bytes64 = split_floats(K, Cin, Cout) * 4;
+    const int64_t split_bytes = split_floats(K, Cin, Cout) * 4, packed_bytes = packed_floats(K, Cin, Cout) * 4;
+    const bool pw = is_split(Wp) ? false : Wp ? true : split_bytes >= (int64_t)BUF_OOB;
+    const int64_t in_bytes64 = in_rows * ld_in * 4, wp_bytes64 = pw ? packed_bytes : split_bytes;
     if (in_rows < 0 || in_bytes64 >= (int64_t)BUF_OOB || wp_bytes64 >= (int64_t)BUF_OOB) {
       set_error("conv: input matrix (%lld rows x %lld floats) or weights exceed the 4 GB the kernel addresses",
                 (long long)in_rows, (long long)ld_in);
@@ -2096,12 +2181,11 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const uint32_t in_bytes = (uint32_t)in_bytes64, wp_bytes = (uint32_t)wp_bytes64;
     if (is_split(Wp)) {
       Wp = split_address(Wp);
-    } else {
-      // raw weights, or packed ones in fp32: their parts are made for this call
+    } else if (!Wp) {
       void *ws;
-      int rc = workspace(WS_API, s, sizeof(float) * (size_t)split_floats(K, Cin, Cout), &ws);
+      int rc = workspace(WS_API, s, (size_t)wp_bytes64, &ws);
       if (rc) return rc;
-      rc = split_weights(W, Wp, K, Cin, Cout, (float *)ws, s);
+      rc = pw ? pack_weights(W, K, Cin, Cout, (float *)ws, s) : split_weights(W, K, Cin, Cout, (float *)ws, s);
       if (rc) return rc;
       Wp = (const float *)ws;
     }
@@ -2124,12 +2208,10 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       // persistent blocks, a multiple of the XCD count, at most one per compute unit
       const int64_t want = cdiv(tiles, WL_WAVES);
       const unsigned nblk = (unsigned)std::min<int64_t>(device_cus(), want);
-      if (Cin == 16)
-        hipLaunchKernelGGL(conv_wlds_kernel<1>, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias,
-                           map0, rows, d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, wp_bytes, ep, plan);
-      else
-        hipLaunchKernelGGL(conv_wlds_kernel<2>, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias,
-                           map0, rows, d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, wp_bytes, ep, plan);
+      auto kernel = Cin == 16 ? (pw ? conv_wlds_kernel<1, true> : conv_wlds_kernel<1, false>)
+                              : (pw ? conv_wlds_kernel<2, true> : conv_wlds_kernel<2, false>);
+      hipLaunchKernelGGL(kernel, dim3(nblk), dim3(WL_WAVES * 64), 0, s, in, ld_in, out, ld_out, Wp, bias, map0, rows,
+                         d_n_rows, n_rows, Cin, Cout, tile_flags, in_bytes, map_bytes, wp_bytes, ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
     }
@@ -2171,26 +2253,30 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       // with enough units left, two output blocks per gathered chunk (eight accumulators: two
       // wavefronts per SIMD instead of three, but a third fewer bytes per MFMA)
       if (nbt >= 2 && cdiv(tiles, 4) * cdiv(nbt, 2) * 3 >= g_shared_min_units.load(std::memory_order_relaxed) * 2) {
-        static int per_cu4 = 0;
+        static int per_cu4_of[2] = {0, 0};
+        int &per_cu4 = per_cu4_of[pw];
+        auto kernel = pw ? conv_wshare_kernel<2, 4, true> : conv_wshare_kernel<2, 4, false>;
         if (!per_cu4) {
-          INSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu4, conv_wshare_kernel<2, 4>, 256, 0));
+          INSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu4, kernel, 256, 0));
           if (per_cu4 < 1) per_cu4 = 1;
         }
         const int64_t wunits = cdiv(tiles, 4) * cdiv(nbt, 2);
         const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu4, wunits);
-        hipLaunchKernelGGL((conv_wshare_kernel<2, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
+        hipLaunchKernelGGL(kernel, dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
                            d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
         INSC_LAUNCH_CHECK();
         return INSC_OK;
       }
-      static int per_cu2 = 0;
+      static int per_cu2_of[2] = {0, 0};
+      int &per_cu2 = per_cu2_of[pw];
+      auto kernel = pw ? conv_wshare_kernel<1, 4, true> : conv_wshare_kernel<1, 4, false>;
       if (!per_cu2) {
-        INSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, conv_wshare_kernel<1, 4>, 256, 0));
+        INSC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, kernel, 256, 0));
         if (per_cu2 < 1) per_cu2 = 1;
       }
       const int64_t wunits = cdiv(tiles, 4) * nbt;
       const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu2, wunits);
-      hipLaunchKernelGGL((conv_wshare_kernel<1, 4>), dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
+      hipLaunchKernelGGL(kernel, dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
                          d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
@@ -2198,7 +2284,8 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const int64_t own_min = g_own_min_units.load(std::memory_order_relaxed);
     if (wide_planned && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
       // one wavefront per (tile, output block): enough units that every SIMD gets one to three
-      hipLaunchKernelGGL((conv_own_kernel<4, 2>), dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
+      auto kernel = pw ? conv_own_kernel<4, 2, true> : conv_own_kernel<4, 2, false>;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
                          ld_out, Wp, bias, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep,
                          plan);
       INSC_LAUNCH_CHECK();
@@ -2219,7 +2306,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     }
     bool shape_ok = true;
 #define INSC_CONV_LAUNCH(NBV, KV, MV, SV)                                                                       \
-  hipLaunchKernelGGL((conv_mfma_kernel<NBV, KV, MV, SV>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
+  hipLaunchKernelGGL((pw ? conv_mfma_kernel<NBV, KV, MV, SV, true> : conv_mfma_kernel<NBV, KV, MV, SV, false>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
                      map0, map1, rows, d_n_rows, n_rows, Cin, Cout, nbtp, tile_flags, in_bytes, wp_bytes, ep, part,  \
                      pcount, plan)
 #define INSC_CONV_CASE(NBV)                                      \
@@ -2351,7 +2438,7 @@ int64_t insc_conv_split_floats(int K, int Cin, int Cout) {
 int insc_conv_split_weights(const float *d_W, int K, int Cin, int Cout, float *d_Ws, void *stream) {
   INSC_REQUIRE(d_W && d_Ws && K > 0 && K <= MAXK && Cin > 0 && Cout > 0 && ((uintptr_t)d_Ws & 15) == 0, INSC_ERR_ARG,
                "insc_conv_split_weights: bad arguments");
-  return split_weights(d_W, nullptr, K, Cin, Cout, d_Ws, (hipStream_t)stream);
+  return split_weights(d_W, K, Cin, Cout, d_Ws, (hipStream_t)stream);
 }
 
 int insc_conv_nbr(const float *d_in, int64_t ld_in, int64_t n_in_rows, float *d_out, int64_t ld_out,

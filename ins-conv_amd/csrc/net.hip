@@ -946,7 +946,7 @@ int insc_net_finalize(insc_net *net, int out_tensor, int64_t capacity_sites, voi
         const int64_t nf = split_floats(K, op.Cin, op.Cout);
         int rc = dev_alloc(&op.Wp, (size_t)nf);
         if (rc) return rc;
-        rc = split_weights(op.W, nullptr, K, op.Cin, op.Cout, op.Wp, s);
+        rc = split_weights(op.W, K, op.Cin, op.Cout, op.Wp, s);
         if (rc) return rc;
       }
     }
@@ -1076,7 +1076,7 @@ int insc_net_refresh_weights(insc_net *net, void *stream) {
   for (Op &op : net->ops)
     if (op.Wp) {
       const int K = op.kind == OP_SSC ? 27 : op.kind == OP_NIN ? 1 : 8;
-      int rc = split_weights(op.W, nullptr, K, op.Cin, op.Cout, op.Wp, (hipStream_t)stream);
+      int rc = split_weights(op.W, K, op.Cin, op.Cout, op.Wp, (hipStream_t)stream);
       if (rc) return rc;
     }
   for (Op &op : net->ops)
