@@ -1,5 +1,7 @@
 // Internal view of the hash grid, shared by grid.hip and the network executor.
 #pragma once
+#include <atomic>
+
 #include "common.h"
 
 namespace insc {
@@ -35,9 +37,17 @@ struct insc_grid {
   int64_t scratch_rows = 0;
   int32_t *part = nullptr;  // partition counters and offsets of the large insert (PART_INTS words, zero between calls)
   int device = 0;
+  // The clearing of a new grid is queued on the null stream; `made` is recorded behind it, and a call on another stream
+  // waits for it there (grid_wait_made) until a call has waited for such a stream on the host.
+  hipEvent_t made = nullptr;
+  mutable std::atomic<bool> made_pending{false};
 };
 
 namespace insc {
+
+// Work queued on s from here on finds the grid cleared.  Every call that reads or writes a grid that may never have been
+// inserted into starts with it.
+int grid_wait_made(const insc_grid *g, hipStream_t s);
 
 // Point coordinate that the insert skips silently (site -1, no error): used to pad a fixed-size
 // launch whose real length is only known on the device.

@@ -854,8 +854,19 @@ static int grid_alloc_table(insc_grid *g, int64_t capacity_sites) {
   return INSC_OK;
 }
 
+int grid_wait_made(const insc_grid *g, hipStream_t s) {
+  if (s == nullptr || !g->made_pending.load(std::memory_order_acquire)) return INSC_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  INSC_HIP(hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone) return INSC_OK;  // (a capture cannot wait for what was queued before it)
+  INSC_HIP(hipStreamWaitEvent(s, g->made, 0));
+  return INSC_OK;
+}
+
 static int grid_sync_errors(insc_grid *g, hipStream_t s, const char *who) {
   int32_t h[2];
+  int rc = grid_wait_made(g, s);
+  if (rc) return rc;
   if (g->h_fresh && g->h_stream == (void *)s) {
     // the last insert left both words in pinned host memory: waiting for its stream is all it takes
     // (two small device-to-host copies and their waits cost ~50 us per call, most of a 220 000-point insert)
@@ -869,6 +880,7 @@ static int grid_sync_errors(insc_grid *g, hipStream_t s, const char *who) {
     h[0] = both[0];
     h[1] = both[16];
   }
+  g->made_pending.store(false, std::memory_order_release);  // (s has been waited for, and it had waited)
   g->n_exact = h[0];
   g->n_upper = h[0];
   if (h[1]) {
@@ -913,8 +925,9 @@ static int grid_ensure_scratch(insc_grid *g, int64_t P, hipStream_t s) {
 // the insert proper: the caller has made sure that P more sites fit
 static int grid_insert_launch(insc_grid *g, const int32_t *d_coords4, int64_t P, int32_t *d_site_of_point,
                               hipStream_t s) {
-  int rc = grid_ensure_scratch(g, P, s);
+  int rc = grid_wait_made(g, s);
   if (rc) return rc;
+  if ((rc = grid_ensure_scratch(g, P, s))) return rc;
   const int64_t mask = g->n_slots - 1;
   const unsigned nb = grid_for(P, 256);
   int32_t *total = g->flags + g->scratch_rows;  // spare int after the flags
@@ -1232,6 +1245,8 @@ int grid_clear_batch(insc_grid *const *grids, int32_t *const *minus1, const int6
   int64_t most = zero_bytes / 4;
   for (int i = 0; i < n; i++) {
     insc_grid *g = grids[i];
+    const int rc = grid_wait_made(g, s);
+    if (rc) return rc;
     b.job[i] = ClearJob{g->table, g->n_slots, g->d_n, g->d_err, minus1 ? minus1[i] : nullptr,
                         (minus1 && minus1[i]) ? n_minus1[i] : 0};
     most = std::max(most, std::max(g->n_slots, b.job[i].n_minus1));
@@ -1643,6 +1658,8 @@ int frame_insert_levels(const FrameInsertLevel *lv, int n_levels, const int32_t 
       set_error("frame_insert_levels: the table of scale %d has more than 2^30 slots", l);
       return INSC_ERR_ARG;
     }
+    const int rc = grid_wait_made(g, s);
+    if (rc) return rc;
     a.lv[l] = FrameLevelDev{g->table, g->n_slots - 1, g->capacity_sites, g->coords, g->d_n, g->d_err,
                             lv[l].parent, lv[l].offset, lv[l].child};
   }
@@ -1804,6 +1821,10 @@ int incre_links_batch(const insc_grid *const *grids, const insc_grid *const *pre
     return INSC_ERR_ARG;
   }
   IncreLinkBatch b;
+  for (int i = 0; i < n; i++) {
+    const int rc = grid_wait_made(pre[i], s);
+    if (rc) return rc;
+  }
   for (int i = 0; i < n; i++)
     b.job[i] = IncreLinkJob{pre[i]->table, pre[i]->n_slots - 1, grids[i]->coords, grids[i]->d_n,
                             i + 1 < n ? d_parent[i] : nullptr, d_pre_exist[i], d_nbr_pre[i],
@@ -1869,7 +1890,11 @@ int insc_grid_create(int64_t capacity_sites, insc_grid **out) {
     INSC_HIP(hipMemsetAsync(g->part, 0, sizeof(int32_t) * PART_INTS, nullptr));
     const int e = insc_grid_clear(g, nullptr);
     if (e) return e;
-    INSC_HIP(hipStreamSynchronize(nullptr));  // (the caller's stream need not wait for the null stream by itself)
+    // (the host does not wait: with work queued on the null stream that would be for all of it.  A stream that the null
+    // stream does not order by itself waits for the event.)
+    INSC_HIP(hipEventCreateWithFlags(&g->made, hipEventDisableTiming));
+    INSC_HIP(hipEventRecord(g->made, nullptr));
+    g->made_pending.store(true, std::memory_order_release);
     return INSC_OK;
   };
   if (!rc) rc = rest();
@@ -1909,6 +1934,7 @@ int insc_grid_destroy(insc_grid *g) {
     }
     if (!kept) (void)hipHostFree(g->h_n);
   }
+  if (g->made) (void)hipEventDestroy(g->made);
   if (dev != g->device) (void)hipSetDevice(dev);
   delete g;
   return INSC_OK;
@@ -1916,6 +1942,8 @@ int insc_grid_destroy(insc_grid *g) {
 
 int insc_grid_clear(insc_grid *g, void *stream) {
   INSC_REQUIRE(g, INSC_ERR_ARG, "insc_grid_clear: grid is null");
+  int rc = grid_wait_made(g, (hipStream_t)stream);
+  if (rc) return rc;
   hipLaunchKernelGGL(grid_clear_kernel, dim3(grid_for(g->n_slots, 256, 8192)), dim3(256), 0, (hipStream_t)stream,
                      g->table, g->n_slots, g->d_n, g->d_err);
   INSC_LAUNCH_CHECK();
@@ -1930,11 +1958,12 @@ int insc_grid_reserve(insc_grid *g, int64_t capacity_sites, void *stream) {
   INSC_REQUIRE(capacity_sites < (1ll << 30), INSC_ERR_ARG, "insc_grid_reserve: capacity out of range");
   if (capacity_sites <= g->capacity_sites) return INSC_OK;
   hipStream_t s = (hipStream_t)stream;
+  int rc = grid_wait_made(g, s);
+  if (rc) return rc;
   INSC_HIP(hipStreamSynchronize(s));
   g->h_fresh = false;
   int32_t *coords = nullptr;
-  int rc_coords = pool_alloc(g->device, grid_coord_bytes(capacity_sites), (void **)&coords);
-  if (rc_coords) return rc_coords;
+  if ((rc = pool_alloc(g->device, grid_coord_bytes(capacity_sites), (void **)&coords))) return rc;
   INSC_HIP(hipMemcpyAsync(coords, g->coords, sizeof(int32_t) * 4 * (size_t)g->capacity_sites,
                           hipMemcpyDeviceToDevice, s));
   INSC_HIP(hipStreamSynchronize(s));
@@ -1944,8 +1973,7 @@ int insc_grid_reserve(insc_grid *g, int64_t capacity_sites, void *stream) {
   if (g->n_slots < 2 * capacity_sites) {
     INSC_HIP(hipFree(g->table));
     g->table = nullptr;
-    int rc = grid_alloc_table(g, capacity_sites);
-    if (rc) return rc;
+    if ((rc = grid_alloc_table(g, capacity_sites))) return rc;
     // clear the new table but keep the counter
     int32_t n_keep = 0;
     INSC_HIP(hipMemcpy(&n_keep, g->d_n, sizeof(int32_t), hipMemcpyDeviceToHost));
@@ -2010,6 +2038,7 @@ int insc_grid_insert_noalloc(insc_grid *g, const int32_t *d_coords4, int64_t P, 
     int32_t *slot_of_point = nullptr;
     int rc = scratch_on_current_device(&slot_of_point);
     if (rc) return rc;
+    if ((rc = grid_wait_made(g, s))) return rc;
     // this entry point never grows the grid: the host-side bound (every row a new site) must fit
     INSC_REQUIRE(g->n_upper + P <= g->capacity_sites, INSC_ERR_CAPACITY,
                  "insc_grid_insert_noalloc: up to %lld sites + %lld points may exceed the capacity of %lld; call "
@@ -2048,6 +2077,8 @@ int insc_grid_query(const insc_grid *g, const int32_t *d_coords4, int64_t Q, int
   INSC_REQUIRE(g, INSC_ERR_ARG, "insc_grid_query: grid is null");
   INSC_REQUIRE(Q >= 0 && (Q == 0 || (d_coords4 && d_site)), INSC_ERR_ARG, "insc_grid_query: bad arguments");
   if (Q == 0) return INSC_OK;
+  int rc = grid_wait_made(g, (hipStream_t)stream);
+  if (rc) return rc;
   hipLaunchKernelGGL(grid_query_kernel, dim3(grid_for(Q, 256)), dim3(256), 0, (hipStream_t)stream, g->table,
                      g->n_slots - 1, d_coords4, Q, d_site);
   INSC_LAUNCH_CHECK();
@@ -2097,6 +2128,8 @@ int insc_incre_rulebook_ssc3(const insc_grid *g, const insc_grid *pre, const int
   INSC_REQUIRE(n >= 0 && n <= g->capacity_sites, INSC_ERR_ARG, "insc_incre_rulebook_ssc3: n outside capacity");
   INSC_REQUIRE(n == 0 || (d_pre_exist && d_nbr_pre), INSC_ERR_ARG, "insc_incre_rulebook_ssc3: null pointer");
   if (n == 0) return INSC_OK;
+  int rc = grid_wait_made(pre, (hipStream_t)stream);
+  if (rc) return rc;
   hipLaunchKernelGGL(incre_ssc3_nbr_kernel, dim3(grid_for(n * 27, 256, 1ll << 30)), dim3(256), 0, (hipStream_t)stream,
                      pre->table, pre->n_slots - 1, g->coords, d_pre_exist, n, d_nbr_pre);
   INSC_LAUNCH_CHECK();

@@ -308,6 +308,8 @@ int insc_labels_count(insc_labels *l, int64_t *h_n, void *stream) {
 int insc_labels_export(insc_labels *l, int32_t *d_out4, float *d_conf, int64_t rows, void *stream) {
   INSC_REQUIRE(l && rows >= 0 && (rows == 0 || d_out4), INSC_ERR_ARG, "insc_labels_export: bad arguments");
   if (rows == 0) return INSC_OK;
+  int rc = grid_wait_made(l->grid, (hipStream_t)stream);
+  if (rc) return rc;
   hipLaunchKernelGGL(labels_export_kernel, dim3(grid_for(rows, 256)), dim3(256), 0, (hipStream_t)stream,
                      insc_grid_coords(l->grid), l->grid->d_n, rows, l->kind, l->C, l->label, l->conf, l->scores, d_out4,
                      d_conf);

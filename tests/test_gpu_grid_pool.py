@@ -69,3 +69,73 @@ def test_threads_and_streams_share_the_pool(orc):
     for t in threads:
         t.join()
     assert not bad
+
+
+def _busy(ms=40):
+    """Work of about that many milliseconds queued on the current stream."""
+    a = torch.randn(4096, 4096, device="cuda")
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    a @ a
+    torch.cuda.synchronize()
+    e[0].record()
+    a @ a
+    e[1].record()
+    torch.cuda.synchronize()
+    n = int(ms / e[0].elapsed_time(e[1])) + 1
+    for _ in range(n):
+        a @ a
+
+
+def test_creation_does_not_wait_for_queued_work():
+    import ctypes
+    import time
+
+    from sparseconvnet._lib import ensure_init, lib
+
+    ensure_init(0)
+    for _ in range(2):  # (the first grid of a size may have to allocate)
+        g = ctypes.c_void_p()
+        _busy()
+        t0 = time.perf_counter()
+        lib.insc_grid_create(ctypes.c_int64(200000), ctypes.byref(g))
+        t1 = time.perf_counter()
+        torch.cuda.synchronize()
+        t2 = time.perf_counter()
+        lib.insc_grid_destroy(g)
+    assert t1 - t0 < 0.25 * (t2 - t0), "creation took %.1f of %.1f ms" % ((t1 - t0) * 1e3, (t2 - t0) * 1e3)
+
+
+@pytest.mark.parametrize("n", [3000, 60000])
+def test_a_new_grid_is_cleared_before_any_stream_uses_it(orc, n):
+    """Work is queued on the null stream, where a new grid's clearing waits behind it; another stream inserts into the grid
+    and queries it meanwhile."""
+    import ctypes
+
+    from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
+
+    ensure_init(0)
+    I64 = ctypes.c_int64
+    side = torch.cuda.Stream()
+    for seed in range(3):  # (the second and third grid take the first one's memory)
+        pts = scenes.boxes_scene(seed=70 + seed, n=n)
+        sop, sc, _ = orc.grid_build(pts)
+        c4 = np.zeros((n, 4), np.int32)
+        c4[:, :pts.shape[1]] = pts
+        d = torch.from_numpy(c4).cuda()
+        site = torch.empty(n, dtype=torch.int32, device="cuda")
+        found = torch.empty(n, dtype=torch.int32, device="cuda")
+        empty = torch.empty(n, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        _busy(20)
+        a, b, count = ctypes.c_void_p(), ctypes.c_void_p(), I64(0)
+        lib.insc_grid_create(I64(n), ctypes.byref(a))
+        lib.insc_grid_create(I64(n), ctypes.byref(b))
+        with torch.cuda.stream(side):
+            lib.insc_grid_query(b, ptr(d), I64(n), ptr(empty), stream_ptr())
+            lib.insc_grid_insert(a, ptr(d), I64(n), ptr(site), ctypes.byref(count), stream_ptr())
+            lib.insc_grid_query(a, ptr(d), I64(n), ptr(found), stream_ptr())
+        torch.cuda.synchronize()
+        assert count.value == len(sc) and (site.cpu().numpy() == sop).all() and (found.cpu().numpy() == sop).all()
+        assert (empty.cpu().numpy() == -1).all()
+        lib.insc_grid_destroy(a)
+        lib.insc_grid_destroy(b)
