@@ -57,6 +57,9 @@ const char *insc_version(void);
  * ------------------------------------------------------------------------------------- */
 int insc_grid_create(int64_t capacity_sites, insc_grid **out);
 int insc_grid_destroy(insc_grid *g);
+/* Up to 256 MB of the memory of destroyed grids is kept for the grids to come.  This call gives back what is kept on
+ * the current device; the library does so itself when an allocation of its own fails there. */
+int insc_grid_pool_trim(void);
 /* Forget all sites, keep the allocation (reference: Metadata<D>::clear, Metadata.cpp:68-75). */
 int insc_grid_clear(insc_grid *g, void *stream);
 /* Grow so that capacity_sites fit; rehashes the existing sites, ids unchanged. */

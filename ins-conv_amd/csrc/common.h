@@ -39,6 +39,8 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 // insc_grid_insert_scales (whose helpers use arenas 0-2).
 enum { WS_SCAN = 0, WS_SORT = 1, WS_API = 2, WS_CONV = 3, WS_LABELS = 4, WS_INCRE = 5, WS_INSERT = 6 };
 int workspace(int which, hipStream_t stream, size_t bytes, void **out);
+// hipMalloc on the current device; the memory that destroyed grids left for the next ones is given up for it
+int device_malloc(void **p, size_t bytes);
 int device_cus();
 // `count` int32 counters per (device, stream), zero at kernel start; users leave them at zero
 int zero_counters(hipStream_t stream, size_t count, int32_t **out);

@@ -19,12 +19,11 @@
 //
 // Numbering: a site's id is its rank among first occurrences in the inserted list, offset by
 // the count before the call - deterministic and append-only.
-#include <list>
 #include <mutex>
-#include <vector>
 
 #include "common.h"
 #include "grid.h"
+#include "grid_pool.h"
 
 namespace insc {
 
@@ -760,84 +759,31 @@ __global__ void ssc3_nbr_fill_batch_kernel(NewSitesBatch b) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += stride) j.nbr[i] = -1;
 }
 
-// Memory of grids that are gone, for the grids to come.  A scan makes a grid per scale and drops them with its
-// Metadata: five grids of 220 000 points took 0.54 ms to allocate and 1.9 ms to free, of the 4.1 ms that the whole
-// structure took.  Blocks come in size classes an eighth apart, so that scans of about the same size find one
-// another's.  A block enters when its grid is destroyed, after the device has been waited for (nothing of any stream
-// uses it any more), and belongs to its device.  The pool holds at most GRID_POOL_BYTES over all devices: the blocks
-// that have been in it longest are freed first, and all of the device's when an allocation fails.
-constexpr size_t GRID_POOL_BYTES = (size_t)256 << 20;
-constexpr size_t GRID_POOL_HOST = 64;  // pinned words of destroyed grids that are kept
-struct PoolBlock {
-  int device;
-  size_t bytes;
-  void *p;
+struct HipMem {
+  static constexpr int OUT_OF_MEMORY = (int)hipErrorOutOfMemory;
+  static int device(void **p, size_t bytes) { return done(hipMalloc(p, bytes)); }
+  static void free_device(void *p) { (void)hipFree(p); }
+  static int host(void **p, size_t bytes) { return done(hipHostMalloc(p, bytes, hipHostMallocDefault)); }
+  static void free_host(void *p) { (void)hipHostFree(p); }
+  static int done(hipError_t e) {
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+    return (int)e;
+  }
 };
-static std::mutex g_pool_mu;
+constexpr size_t GRID_HOST_BYTES = 64;
 // (never destroyed: a grid may be given up after the destructors of this file's statics have run)
-static std::list<PoolBlock> &g_pool = *new std::list<PoolBlock>();  // oldest first
-static size_t g_pool_bytes = 0;
-static std::vector<int32_t *> &g_pool_host = *new std::vector<int32_t *>();
+static GridPool<HipMem> &g_pool = *new GridPool<HipMem>((size_t)256 << 20, 64);
 
-static size_t pool_class(size_t bytes) {
-  size_t step = 256;
-  while (step * 16 <= bytes) step <<= 1;  // 8 to 16 steps: at most an eighth on top
-  return (bytes + step - 1) / step * step;
-}
-
-static int pool_alloc(int device, size_t bytes, void **out) {
-  bytes = pool_class(bytes);
-  {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    for (auto it = g_pool.begin(); it != g_pool.end(); ++it)
-      if (it->device == device && it->bytes == bytes) {
-        *out = it->p;
-        g_pool_bytes -= bytes;
-        g_pool.erase(it);
-        return INSC_OK;
-      }
-  }
-  hipError_t e = hipMalloc(out, bytes);
-  if (e == hipErrorOutOfMemory) {
-    (void)hipGetLastError();
-    {
-      std::lock_guard<std::mutex> lk(g_pool_mu);
-      for (auto it = g_pool.begin(); it != g_pool.end();) {
-        if (it->device != device) {
-          ++it;
-          continue;
-        }
-        (void)hipFree(it->p);
-        g_pool_bytes -= it->bytes;
-        it = g_pool.erase(it);
-      }
-    }
-    e = hipMalloc(out, bytes);
-  }
-  INSC_HIP(e);
+int device_malloc(void **p, size_t bytes) {
+  int dev = 0;
+  INSC_HIP(hipGetDevice(&dev));
+  INSC_HIP((hipError_t)g_pool.outside(dev, bytes, p));
   return INSC_OK;
 }
 
-// p: a block of pool_alloc(device, bytes) that no work in flight uses
-static void pool_give(int device, size_t bytes, void *p) {
-  if (!p) return;
-  bytes = pool_class(bytes);
-  if (bytes > GRID_POOL_BYTES / 2) {
-    (void)hipFree(p);
-    return;
-  }
-  std::lock_guard<std::mutex> lk(g_pool_mu);
-  while (g_pool_bytes + bytes > GRID_POOL_BYTES) {
-    (void)hipFree(g_pool.front().p);
-    g_pool_bytes -= g_pool.front().bytes;
-    g_pool.pop_front();
-  }
-  try {
-    g_pool.push_back(PoolBlock{device, bytes, p});
-    g_pool_bytes += bytes;
-  } catch (...) {
-    (void)hipFree(p);
-  }
+static int pool_alloc(int device, size_t bytes, void **out) {
+  INSC_HIP((hipError_t)g_pool.alloc(device, bytes, out));
+  return INSC_OK;
 }
 
 static size_t grid_table_bytes(int64_t slots) { return sizeof(Slot) * (size_t)slots; }
@@ -1876,15 +1822,8 @@ int insc_grid_create(int64_t capacity_sites, insc_grid **out) {
   rc = pool_alloc(g->device, grid_coord_bytes(capacity_sites), (void **)&g->coords);
   if (!rc) rc = pool_alloc(g->device, 256, (void **)&g->d_n);
   if (!rc) rc = pool_alloc(g->device, sizeof(int32_t) * PART_INTS, (void **)&g->part);
-  if (!rc) {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    if (!g_pool_host.empty()) {
-      g->h_n = g_pool_host.back();
-      g_pool_host.pop_back();
-    }
-  }
   auto rest = [&]() -> int {
-    if (!g->h_n) INSC_HIP(hipHostMalloc((void **)&g->h_n, 64, hipHostMallocDefault));
+    INSC_HIP((hipError_t)g_pool.alloc_host(g->device, GRID_HOST_BYTES, (void **)&g->h_n));
     g->d_err = g->d_n + 16;
     g->h_n[0] = g->h_n[1] = 0;
     INSC_HIP(hipMemsetAsync(g->part, 0, sizeof(int32_t) * PART_INTS, nullptr));
@@ -1914,7 +1853,7 @@ int insc_grid_destroy(insc_grid *g) {
   const bool idle = hipDeviceSynchronize() == hipSuccess;  // (a block in the pool must be free on every stream)
   auto give = [&](size_t bytes, void *p) {
     if (idle)
-      pool_give(g->device, bytes, p);
+      g_pool.give(g->device, bytes, p);
     else if (p)
       (void)hipFree(p);
   };
@@ -1924,19 +1863,20 @@ int insc_grid_destroy(insc_grid *g) {
   give(grid_slot_bytes(g->scratch_rows), g->slot_of_point);
   give(grid_flag_bytes(g->scratch_rows), g->flags);
   give(sizeof(int32_t) * PART_INTS, g->part);
-  if (g->h_n) {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    bool kept = idle && g_pool_host.size() < GRID_POOL_HOST;
-    try {
-      if (kept) g_pool_host.push_back(g->h_n);
-    } catch (...) {
-      kept = false;
-    }
-    if (!kept) (void)hipHostFree(g->h_n);
-  }
+  if (idle)
+    g_pool.give_host(g->device, GRID_HOST_BYTES, g->h_n);
+  else if (g->h_n)
+    (void)hipHostFree(g->h_n);
   if (g->made) (void)hipEventDestroy(g->made);
   if (dev != g->device) (void)hipSetDevice(dev);
   delete g;
+  return INSC_OK;
+}
+
+int insc_grid_pool_trim(void) {
+  int dev = 0;
+  INSC_HIP(hipGetDevice(&dev));
+  g_pool.trim(dev);
   return INSC_OK;
 }
 

@@ -168,7 +168,8 @@ __global__ void labels_compact_kernel(const int32_t *__restrict__ coords, const 
 template <typename T>
 static int regrow(T **p, size_t old_count, size_t new_count, hipStream_t s) {
   T *q = nullptr;
-  INSC_HIP(hipMalloc((void **)&q, sizeof(T) * (new_count ? new_count : 1)));
+  int rc = device_malloc((void **)&q, sizeof(T) * (new_count ? new_count : 1));
+  if (rc) return rc;
   if (*p && old_count) INSC_HIP(hipMemcpyAsync(q, *p, sizeof(T) * old_count, hipMemcpyDeviceToDevice, s));
   INSC_HIP(hipStreamSynchronize(s));
   if (*p) INSC_HIP(hipFree(*p));

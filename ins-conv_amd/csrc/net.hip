@@ -357,14 +357,14 @@ template <typename T>
 static int dev_alloc(T **p, size_t count) {
   *p = nullptr;
   if (count == 0) count = 1;
-  INSC_HIP(hipMalloc((void **)p, sizeof(T) * count));
-  return INSC_OK;
+  return device_malloc((void **)p, sizeof(T) * count);
 }
 
 template <typename T>
 static int dev_grow(T **p, size_t old_count, size_t new_count, hipStream_t s) {
   T *q = nullptr;
-  INSC_HIP(hipMalloc((void **)&q, sizeof(T) * (new_count ? new_count : 1)));
+  int rc = device_malloc((void **)&q, sizeof(T) * (new_count ? new_count : 1));
+  if (rc) return rc;
   if (*p && old_count) INSC_HIP(hipMemcpyAsync(q, *p, sizeof(T) * old_count, hipMemcpyDeviceToDevice, s));
   INSC_HIP(hipStreamSynchronize(s));
   if (*p) INSC_HIP(hipFree(*p));
@@ -463,7 +463,10 @@ static int level_reserve(insc_net *net, int l, int64_t cap, hipStream_t s) {
   if (bytes > net->mask_arena_bytes) {
     INSC_HIP(hipStreamSynchronize(s));
     if (net->mask_arena) INSC_HIP(hipFree(net->mask_arena));
-    INSC_HIP(hipMalloc((void **)&net->mask_arena, bytes));
+    net->mask_arena = nullptr;
+    net->mask_arena_bytes = 0;
+    int rc = device_malloc((void **)&net->mask_arena, bytes);
+    if (rc) return rc;
     net->mask_arena_bytes = bytes;
   }
   size_t off = 0;
@@ -479,7 +482,8 @@ static int level_reserve(insc_net *net, int l, int64_t cap, hipStream_t s) {
       INSC_HIP(hipStreamSynchronize(s));
       if (d.crows) INSC_HIP(hipFree(d.crows));
       d.crows = nullptr;
-      INSC_HIP(hipMalloc((void **)&d.crows, sizeof(int32_t) * c));
+      int rc = device_malloc((void **)&d.crows, sizeof(int32_t) * c);
+      if (rc) return rc;
       d.crows_cap = (int64_t)c;
     }
   }

@@ -49,7 +49,8 @@ static int arena_get(int which, hipStream_t stream, size_t bytes, void **out) {
     }
     size_t want = bytes + bytes / 2;
     if (want < (1u << 20)) want = 1u << 20;
-    INSC_HIP(hipMalloc(&a.p, want));
+    int rc = device_malloc(&a.p, want);
+    if (rc) return rc;
     a.bytes = want;
   }
   *out = a.p;
@@ -77,7 +78,8 @@ int zero_counters(hipStream_t stream, size_t count, int32_t **out) {
       c.count = 0;
     }
     size_t want = count < 16384 ? 16384 : count + count / 2;
-    INSC_HIP(hipMalloc((void **)&c.p, want * sizeof(int32_t)));
+    int rc = device_malloc((void **)&c.p, want * sizeof(int32_t));
+    if (rc) return rc;
     INSC_HIP(hipMemsetAsync(c.p, 0, want * sizeof(int32_t), stream));
     c.count = want;
   }

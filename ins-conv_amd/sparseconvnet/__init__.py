@@ -20,6 +20,6 @@ from .networkInNetwork import NetworkInNetwork  # noqa: E402
 from .pooling import MaxPooling, AveragePooling, UnPooling, SparseToDense  # noqa: E402
 from .networkArchitectures import UNet  # noqa: E402
 from .utils import (toLongTensor, optionalTensor, checkpoint_save, checkpoint_restore,  # noqa: E402
-                    ssc_offset_permutation, convert_zmajor_state_dict)
+                    ssc_offset_permutation, convert_zmajor_state_dict, empty_cache)
 from .compiled import compile, CompiledNet  # noqa: E402
 from .incremental import set_mode as set_incremental_mode, get_mode as get_incremental_mode  # noqa: E402

@@ -5,6 +5,14 @@ import os
 import torch
 
 
+def empty_cache():
+    """Gives the memory that destroyed Metadata objects left for the next ones (256 MB at most) back to the current
+    device, for other allocators."""
+    from ._lib import lib
+
+    lib.insc_grid_pool_trim()
+
+
 def toLongTensor(dimension, x):
     if isinstance(x, torch.Tensor) and x.dtype == torch.long:
         return x

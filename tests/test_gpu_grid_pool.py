@@ -139,3 +139,20 @@ def test_a_new_grid_is_cleared_before_any_stream_uses_it(orc, n):
         assert (empty.cpu().numpy() == -1).all()
         lib.insc_grid_destroy(a)
         lib.insc_grid_destroy(b)
+
+
+def test_the_kept_memory_is_given_back():
+    import sparseconvnet as scn
+    from sparseconvnet._lib import ensure_init
+
+    ensure_init(0)
+    scn.empty_cache()
+    torch.cuda.synchronize()
+    structure(scenes.boxes_scene(seed=3, n=60000))
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    structure(scenes.boxes_scene(seed=3, n=60000))
+    torch.cuda.empty_cache()
+    assert torch.cuda.mem_get_info()[0] >= free  # (the second scene's grids took the first one's memory)
+    scn.empty_cache()
+    assert torch.cuda.mem_get_info()[0] > free
