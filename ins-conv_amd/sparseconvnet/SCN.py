@@ -81,12 +81,24 @@ class _Down(object):
         self.by_offset_n = 0
 
 
+class _Grid(ctypes.c_void_p):
+    """A hash grid of the library, destroyed with the last reference to it."""
+
+    def __del__(self):
+        try:
+            if self.value:
+                lib.insc_grid_destroy(self)
+                self.value = None
+        except Exception:  # (at interpreter exit the library may be gone)
+            pass
+
+
 class _Scale(object):
     """Active sites of one spatial size and everything derived from them."""
 
     def __init__(self, device):
         self.device = device
-        self.grid = ctypes.c_void_p()
+        self.grid = _Grid()
         self.n = 0
         self.nbr = _Buf(27, torch.int32, device)
         self.nbr_n = 0
@@ -105,24 +117,24 @@ class _Scale(object):
         return int(lib.insc_grid_capacity(self.grid)) if self.grid else 0
 
     def destroy(self):
-        if self.grid:
-            lib.insc_grid_destroy(self.grid)
-            self.grid = ctypes.c_void_p()
+        self.grid = _Grid()  # (the old one goes with its last view)
 
     def coords_view(self):
-        """int32 [n,4] view (x,y,z,batch) of the grid's own coordinate table."""
+        """int32 [n,4] view (x,y,z,batch) of the grid's own coordinate table.  It keeps the grid's memory, also when its
+        Metadata goes; sites that are added later may move the table, so take a new view then."""
         if self.n == 0:
             return torch.empty((0, 4), dtype=torch.int32, device=self.device)
         addr = lib.insc_grid_coords(self.grid)
-        return _from_ptr(addr, (self.n, 4), torch.int32, self.device)
+        return _from_ptr(addr, (self.n, 4), torch.int32, self.device, self.grid)
 
 
-def _from_ptr(addr, shape, dtype, device):
-    """Wrap library-owned device memory as a torch tensor (no copy, no ownership)."""
+def _from_ptr(addr, shape, dtype, device, owner=None):
+    """Wrap library-owned device memory as a torch tensor (no copy); the tensor keeps a reference to `owner`."""
     class _Holder(object):
         pass
 
     h = _Holder()
+    h.owner = owner
     h.__cuda_array_interface__ = {
         "shape": tuple(shape),
         "typestr": {torch.int32: "<i4", torch.float32: "<f4", torch.uint8: "|u1"}[dtype],

@@ -156,3 +156,32 @@ def test_the_kept_memory_is_given_back():
     assert torch.cuda.mem_get_info()[0] >= free  # (the second scene's grids took the first one's memory)
     scn.empty_cache()
     assert torch.cuda.mem_get_info()[0] > free
+
+
+def test_a_view_of_the_coordinates_keeps_its_scene():
+    """The memory of a scene whose coordinates are still looked at does not go to the next scene."""
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import ensure_init
+
+    ensure_init(0)
+
+    def scene(seed):
+        pts = scenes.boxes_scene(seed=seed, n=5000)
+        m = S.Metadata_3()
+        out = torch.empty(0, device="cuda")
+        S.InputLayer_updateOutput(m, SZ, torch.from_numpy(pts.astype(np.int64)), torch.ones((len(pts), 1), device="cuda"), out, 0, 4)
+        return m
+
+    m = scene(90)
+    view = m.scale(SZ).coords_view()
+    want = view.cpu().numpy().copy()
+    del m
+    others = [scene(91 + i) for i in range(3)]
+    assert (view.cpu().numpy() == want).all()
+    assert not (others[0].scale(SZ).coords_view()[:100].cpu().numpy() == want[:100]).all()
+    m = scene(95)
+    part = m.scale(SZ).coords_view()[7:9]  # (a slice of a view is one as well)
+    want = part.cpu().numpy().copy()
+    m.clear()
+    others += [scene(96), scene(97)]
+    assert (part.cpu().numpy() == want).all()
