@@ -786,6 +786,14 @@ static int pool_alloc(int device, size_t bytes, void **out) {
   return INSC_OK;
 }
 
+// p: a block of the grid that it has outgrown.  (hipFree would wait for the device as well.)
+static int grid_outgrow(const insc_grid *g, size_t bytes, void *p) {
+  if (!p) return INSC_OK;
+  INSC_HIP(hipDeviceSynchronize());
+  g_pool.give(g->device, bytes, p);
+  return INSC_OK;
+}
+
 static size_t grid_table_bytes(int64_t slots) { return sizeof(Slot) * (size_t)slots; }
 static size_t grid_coord_bytes(int64_t capacity) { return sizeof(int32_t) * 4 * (size_t)capacity; }
 static size_t grid_slot_bytes(int64_t rows) { return sizeof(int32_t) * 5 * (size_t)rows; }
@@ -850,16 +858,17 @@ static int grid_sync_errors(insc_grid *g, hipStream_t s, const char *who) {
 static int grid_ensure_scratch(insc_grid *g, int64_t P, hipStream_t s) {
   if (g->scratch_rows < P) {
     INSC_HIP(hipStreamSynchronize(s));
-    if (g->slot_of_point) INSC_HIP(hipFree(g->slot_of_point));
-    if (g->flags) INSC_HIP(hipFree(g->flags));
+    const int64_t old = g->scratch_rows;
+    int32_t *const old_slots = g->slot_of_point, *const old_flags = g->flags;
     g->slot_of_point = g->flags = nullptr;
+    g->scratch_rows = 0;
+    int rc = grid_outgrow(g, grid_slot_bytes(old), old_slots), rc2 = grid_outgrow(g, grid_flag_bytes(old), old_flags);
+    if (rc || rc2) return rc ? rc : rc2;
     int64_t rows = (P + P / 2 + 1) & ~1ll;
     // (with the large insert's row states, slots and keys: five arrays of `rows` words)
-    g->scratch_rows = 0;
-    int rc = pool_alloc(g->device, grid_slot_bytes(rows), (void **)&g->slot_of_point);
-    if (rc) return rc;
+    if ((rc = pool_alloc(g->device, grid_slot_bytes(rows), (void **)&g->slot_of_point))) return rc;
     if ((rc = pool_alloc(g->device, grid_flag_bytes(rows), (void **)&g->flags))) {
-      (void)hipFree(g->slot_of_point);
+      g_pool.give(g->device, grid_slot_bytes(rows), g->slot_of_point);
       g->slot_of_point = nullptr;
       return rc;
     }
@@ -1907,12 +1916,15 @@ int insc_grid_reserve(insc_grid *g, int64_t capacity_sites, void *stream) {
   INSC_HIP(hipMemcpyAsync(coords, g->coords, sizeof(int32_t) * 4 * (size_t)g->capacity_sites,
                           hipMemcpyDeviceToDevice, s));
   INSC_HIP(hipStreamSynchronize(s));
-  INSC_HIP(hipFree(g->coords));
+  int32_t *const old_coords = g->coords;
+  const int64_t old_capacity = g->capacity_sites;
   g->coords = coords;
   g->capacity_sites = capacity_sites;
+  if ((rc = grid_outgrow(g, grid_coord_bytes(old_capacity), old_coords))) return rc;
   if (g->n_slots < 2 * capacity_sites) {
-    INSC_HIP(hipFree(g->table));
+    void *const old_table = g->table;
     g->table = nullptr;
+    if ((rc = grid_outgrow(g, grid_table_bytes(g->n_slots), old_table))) return rc;
     if ((rc = grid_alloc_table(g, capacity_sites))) return rc;
     // clear the new table but keep the counter
     int32_t n_keep = 0;

@@ -185,3 +185,38 @@ def test_a_view_of_the_coordinates_keeps_its_scene():
     m.clear()
     others += [scene(96), scene(97)]
     assert (part.cpu().numpy() == want).all()
+
+
+def test_growing_grids_take_and_leave_kept_memory(orc):
+    """A grid that is inserted into piece by piece outgrows its table, coordinates and scratch memory several times; a second
+    one takes over what the first outgrew and needs no more of the device."""
+    import ctypes
+
+    import sparseconvnet as scn
+    from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
+
+    ensure_init(0)
+    scn.empty_cache()
+    I64 = ctypes.c_int64
+    pts = scenes.boxes_scene(seed=33, n=60000)
+    sop, sc, _ = orc.grid_build(pts)
+    c4 = np.zeros((len(pts), 4), np.int32)
+    c4[:, :pts.shape[1]] = pts
+    d = torch.from_numpy(c4).cuda()
+    site = torch.empty(len(pts), dtype=torch.int32, device="cuda")
+    free = []
+    for _ in range(3):
+        g, n = ctypes.c_void_p(), I64(0)
+        lib.insc_grid_create(I64(1024), ctypes.byref(g))
+        a = 0
+        for step in (500, 3000, 9000, 20000, len(pts)):
+            b = min(a + step, len(pts))
+            lib.insc_grid_insert(g, ptr(d[a:b]), I64(b - a), ptr(site[a:b]), ctypes.byref(n), stream_ptr())
+            a = b
+        assert n.value == len(sc) and (site.cpu().numpy() == sop).all()
+        lib.insc_grid_query(g, ptr(d), I64(len(pts)), ptr(site), stream_ptr())
+        assert (site.cpu().numpy() == sop).all()
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+        lib.insc_grid_destroy(g)
+    assert free[1] == free[2]
