@@ -144,7 +144,7 @@ def conv_roofline(device, reps=200, warm=300):
     lib.insc_conv_set_filter_lds_min_tiles(1 << 40)
     for _ in range(warm):
         SCN.ssc_rows_planned(x.features, out, w, None, sc, plan)
-    lib.insc_conv_set_filter_lds_min_tiles(4096)
+    lib.insc_conv_reset_launch_policy()
     for _ in range(10):
         SCN.ssc_rows_planned(x.features, out, w, None, sc, plan)
     torch.cuda.synchronize()

@@ -242,6 +242,8 @@ int insc_conv_set_wavefront_per_unit_min_units(int64_t units);
  * (default 2048, i.e. 65k sites; four times as many without a tile plan), on persistent blocks that keep the whole filter in LDS; below,
  * one wavefront per tile.  Same bits in both cases: a tuning and test knob like the two above. */
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles);
+/* All of these back to their defaults. */
+int insc_conv_reset_launch_policy(void);
 /* Size-2 stride-2 deconvolution: out[i,:] = bias + in[parent[i],:] . W[offset[i]]
  * (Deconvolution_updateOutput, CUDA/Deconvolution.cpp:28-58: the convolution's rules with
  * the roles of input and output swapped). */

@@ -2116,7 +2116,8 @@ int split_weights(const float *W, int K, int Cin, int Cout, float *Ws, hipStream
 // bits; the bounds only move time.
 // With at least this many (group of four tiles, output block) units: the kernel whose blocks share the
 // weight tiles through LDS (faster from about 60k sites at 64 channels).
-static std::atomic<int64_t> g_shared_min_units{896};
+constexpr int64_t SHARED_MIN_UNITS = 896;
+static std::atomic<int64_t> g_shared_min_units{SHARED_MIN_UNITS};
 // Below that, with at least this many (tile, output block) units - half as many again for layers of more
 // than 64 input channels, whose units are longer - the kernel that gives every unit a wavefront of its own
 // (64 -> 64 at 39k sites = 2452 units: 50 us against 56 us; 2084 units: 48 against 50; 1840: 41 against 44;
@@ -2125,7 +2126,8 @@ static std::atomic<int64_t> g_shared_min_units{896};
 // Those figures are from the fp32 instruction; with bf16 parts the order is the same.  Four layers with their batch norms,
 // wavefront per unit / one block per unit / shared weights: 64 -> 64 at 39k sites 229 / 238-250 / 248-273 us, at 150k
 // 647 / 710 / 552, 96 -> 96 at 10k 251 / 195 / 194-390.
-static std::atomic<int64_t> g_own_min_units{1750};
+constexpr int64_t OWN_MIN_UNITS = 1750;
+static std::atomic<int64_t> g_own_min_units{OWN_MIN_UNITS};
 // Narrow 3^3 layers (Cin, Cout <= 32) with at least this many 32-row tiles run on the persistent
 // kernel that keeps the whole filter in LDS; smaller ones on the one-wavefront-per-tile kernel.
 // Same bits either way.
@@ -2416,6 +2418,13 @@ int insc_conv_set_wavefront_per_unit_min_units(int64_t units) {
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles) {
   INSC_REQUIRE(tiles >= 1, INSC_ERR_ARG, "insc_conv_set_filter_lds_min_tiles: tiles must be >= 1");
   g_wl_min_tiles.store(tiles, std::memory_order_relaxed);
+  return INSC_OK;
+}
+
+int insc_conv_reset_launch_policy(void) {
+  g_shared_min_units.store(SHARED_MIN_UNITS, std::memory_order_relaxed);
+  g_own_min_units.store(OWN_MIN_UNITS, std::memory_order_relaxed);
+  g_wl_min_tiles.store(WL_MIN_TILES, std::memory_order_relaxed);
   return INSC_OK;
 }
 

@@ -19,6 +19,7 @@ _SIGS = {
     "insc_grid_create": [c_i64, ctypes.POINTER(vp)],
     "insc_grid_destroy": [vp],
     "insc_grid_pool_trim": [],
+    "insc_conv_reset_launch_policy": [],
     "insc_grid_clear": [vp, vp],
     "insc_grid_reserve": [vp, c_i64, vp],
     "insc_grid_insert": [vp, vp, c_i64, vp, ctypes.POINTER(c_i64), vp],

@@ -11,30 +11,26 @@ from test_gpu_incremental import _frames, _inp
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(params=[(512, 896, 4096, 2000), (1, 1 << 40, 4096, 1 << 40), (512, 1, 4096, 2000), (512, 896, 1, 2000),
-                        (512, 1 << 40, 4096, 1)],
-                ids=["default-launch-policy", "persistent-kernel-forced", "shared-weights-kernel-forced",
-                     "filter-in-lds-kernel-forced", "wavefront-per-unit-kernel-forced"])
-def persistent_min_units(request):
-    """The 3^3 layers of these small scenes stay below the thresholds of the three persistent
-    kernels; the second, third and fifth run force the wide layers onto one of them, the fourth the
-    narrow layers (at most 32 channels) onto the kernel that keeps its filter in LDS - each with the
-    fused batch norm / residual epilogues and the dirty-tile flags of the executor."""
+@pytest.fixture(params=[None, (1, 4096, 1 << 40), (1 << 40, 1, 1 << 40), (1 << 40, 4096, 1)],
+                ids=["default-launch-policy", "shared-weights-kernel-forced", "filter-in-lds-kernel-forced",
+                     "wavefront-per-unit-kernel-forced"])
+def launch_policy(request):
+    """The 3^3 layers of these small scenes stay below the thresholds of the kernels for larger ones; the second and fourth
+    run force the wide layers onto one of them, the third the narrow layers (at most 32 channels) onto the kernel that
+    keeps its filter in LDS - each with the fused batch norm / residual epilogues and the dirty-tile flags of the
+    executor."""
     from sparseconvnet._lib import lib
 
-    lib.insc_conv_set_persistent_min_units(request.param[0])
-    lib.insc_conv_set_shared_weights_min_units(request.param[1])
-    lib.insc_conv_set_filter_lds_min_tiles(request.param[2])
-    lib.insc_conv_set_wavefront_per_unit_min_units(request.param[3])
+    if request.param:
+        lib.insc_conv_set_shared_weights_min_units(request.param[0])
+        lib.insc_conv_set_filter_lds_min_tiles(request.param[1])
+        lib.insc_conv_set_wavefront_per_unit_min_units(request.param[2])
     yield request.param
-    lib.insc_conv_set_persistent_min_units((1 << 63) - 1)
-    lib.insc_conv_set_shared_weights_min_units(896)
-    lib.insc_conv_set_filter_lds_min_tiles(4096)
-    lib.insc_conv_set_wavefront_per_unit_min_units(2400)
+    lib.insc_conv_reset_launch_policy()
 
 
 @pytest.mark.parametrize("levels,m", [(3, 16), (7, 32)])
-def test_compiled_full_and_incremental(levels, m, persistent_min_units):
+def test_compiled_full_and_incremental(levels, m, launch_policy):
     import sparseconvnet as scn
     from workloads.netdefs import NaiveUNet
 

@@ -81,11 +81,11 @@ def test_submanifold_convolution(S, orc, Cin, Cout, bias):
 
 @pytest.mark.parametrize("Cin,Cout,bias", [(64, 64, False), (64, 32, True), (96, 96, False), (80, 48, True),
                                             (112, 100, False)])
-def test_persistent_kernels_give_the_bits_of_the_per_tile_kernel(S, orc, Cin, Cout, bias):
+def test_the_kernels_of_wide_layers_give_the_same_bits(S, orc, Cin, Cout, bias):
     """Wide 3^3 layers (64..127 input channels) have three kernels: one block per (tile, output
-    block), persistent blocks that walk a cost-ordered tile schedule, and persistent blocks of four
-    tiles that share the weight tiles through LDS.  They must agree bit for bit (an incremental frame
-    and a full frame may take different ones), and with the oracle to the float tolerance."""
+    block), one wavefront per (tile, output block), and persistent blocks of four tiles that share the weight tiles through
+    LDS.  They must agree bit for bit (an incremental frame and a full frame may take different ones), and with the
+    oracle to the float tolerance."""
     from sparseconvnet._lib import lib
 
     pts = scenes.boxes_scene(seed=5, n=7000)
@@ -96,7 +96,6 @@ def test_persistent_kernels_give_the_bits_of_the_per_tile_kernel(S, orc, Cin, Co
     b = rng.normal(size=Cout).astype(np.float32) if bias else None
     bt = cu(b) if bias else None
     a = torch.full((sc.n, Cout), 3.0, device="cuda")
-    c = torch.full((sc.n, Cout), -3.0, device="cuda")
     d = torch.full((sc.n, Cout), 5.0, device="cuda")
     e = torch.full((sc.n, Cout), 11.0, device="cuda")
     try:
@@ -104,13 +103,10 @@ def test_persistent_kernels_give_the_bits_of_the_per_tile_kernel(S, orc, Cin, Co
         lib.insc_conv_set_wavefront_per_unit_min_units(1)  # a wavefront of its own per (tile, output block)
         S.ssc_rows_planned(feats, e, W, bt, sc, m.ssc_plan(sc))
         lib.insc_conv_set_wavefront_per_unit_min_units(1 << 40)
-        lib.insc_conv_set_persistent_min_units(1)
         S.ssc_rows_planned(feats, a, W, bt, sc, m.ssc_plan(sc))
-        lib.insc_conv_set_persistent_min_units(1 << 40)
-        S.ssc_rows_planned(feats, c, W, bt, sc, m.ssc_plan(sc))
         lib.insc_conv_set_shared_weights_min_units(1)  # two output blocks per gathered chunk where there are two
         S.ssc_rows_planned(feats, d, W, bt, sc, m.ssc_plan(sc))
-        assert torch.equal(d, c)
+        assert torch.equal(d, a)
         # one output block per unit: enough units for that, too few for pairs of output blocks (with
         # three output blocks the pairs always qualify as well)
         groups, nbt = ((sc.n + 31) // 32 + 3) // 4, (Cout + 31) // 32
@@ -118,12 +114,9 @@ def test_persistent_kernels_give_the_bits_of_the_per_tile_kernel(S, orc, Cin, Co
         d.fill_(9.0)
         S.ssc_rows_planned(feats, d, W, bt, sc, m.ssc_plan(sc))
     finally:
-        lib.insc_conv_set_persistent_min_units((1 << 63) - 1)
-        lib.insc_conv_set_shared_weights_min_units(896)
-        lib.insc_conv_set_wavefront_per_unit_min_units(2400)
-    assert torch.equal(a, c)
-    assert torch.equal(d, c)
-    assert torch.equal(e, c)
+        lib.insc_conv_reset_launch_policy()
+    assert torch.equal(d, a)
+    assert torch.equal(e, a)
     nt = (sc.n + 31) // 32
     plan = m.ssc_plan(sc)
     sched = plan[3][:nt].cpu().numpy()
@@ -146,7 +139,7 @@ def test_persistent_kernels_give_the_bits_of_the_per_tile_kernel(S, orc, Cin, Co
 @pytest.mark.parametrize("Cin,Cout,bias", [(16, 16, False), (16, 16, True), (32, 32, False), (32, 32, True),
                                             (16, 32, True), (32, 20, False)])
 def test_filter_in_lds_kernel_against_oracle_and_per_tile_kernel(S, orc, Cin, Cout, bias):
-    """Narrow 3^3 layers (Cin, Cout <= 32) have two kernels: one wavefront per tile, and - from 4096
+    """Narrow 3^3 layers (Cin, Cout <= 32) have two kernels: one wavefront per tile, and - from 2048
     tiles up by default - persistent blocks that keep the whole filter in LDS (the kernel the
     HBM-roofline figure is quoted on).  Here the threshold is lowered so that the 20k-voxel scene of
     workload 1 runs on the second one, planned and unplanned staging, and the result is compared with
@@ -173,7 +166,7 @@ def test_filter_in_lds_kernel_against_oracle_and_per_tile_kernel(S, orc, Cin, Co
         S.conv_rows(feats, lds_unplanned, W, bt, sc.nbr.t, 27, sc.order.t, None, sc.n)
         S.conv_rows(feats, lds_permuted, W, bt, sc.nbr.t, 27, perm, None, sc.n)
     finally:
-        lib.insc_conv_set_filter_lds_min_tiles(4096)
+        lib.insc_conv_reset_launch_policy()
     assert torch.equal(lds_planned, per_tile)
     assert torch.equal(lds_unplanned, per_tile)
     assert torch.equal(lds_permuted, per_tile)
@@ -184,9 +177,9 @@ def test_filter_in_lds_kernel_against_oracle_and_per_tile_kernel(S, orc, Cin, Co
 
 
 @pytest.mark.parametrize("n", [1, 20, 33, 130, 1025])
-def test_persistent_kernels_on_tiny_and_ragged_scenes(S, n):
+def test_the_kernels_of_wide_layers_on_tiny_and_ragged_scenes(S, n):
     """One site, one tile, two tiles, a group of four tiles with a partial fifth, a partial last tile:
-    all four kernels of a 64->64 layer give the same bits."""
+    all three kernels of a 64->64 layer give the same bits."""
     from sparseconvnet._lib import lib
 
     rng = np.random.default_rng(n)
@@ -199,22 +192,40 @@ def test_persistent_kernels_on_tiny_and_ragged_scenes(S, n):
     W = cu((rng.normal(size=(27, 64, 64)) * 0.05).astype(np.float32))
     outs = []
     try:
-        for pers, shared, own in [(1 << 40, 1 << 40, 1 << 40), (1, 1 << 40, 1 << 40), (1 << 40, 1, 1 << 40),
-                                  (1 << 40, 1 << 40, 1)]:
-            lib.insc_conv_set_persistent_min_units(pers)
+        for shared, own in [(1 << 40, 1 << 40), (1, 1 << 40), (1 << 40, 1)]:
             lib.insc_conv_set_shared_weights_min_units(shared)
             lib.insc_conv_set_wavefront_per_unit_min_units(own)
             o = torch.full((sc.n, 64), float(len(outs)), device="cuda")
             S.ssc_rows_planned(feats, o, W, None, sc, m.ssc_plan(sc))
             outs.append(o)
     finally:
-        lib.insc_conv_set_persistent_min_units((1 << 63) - 1)
-        lib.insc_conv_set_shared_weights_min_units(896)
-        lib.insc_conv_set_wavefront_per_unit_min_units(2400)
+        lib.insc_conv_reset_launch_policy()
     assert torch.equal(outs[0], outs[1])
     assert torch.equal(outs[0], outs[2])
-    assert torch.equal(outs[0], outs[3])
     assert torch.isfinite(outs[0]).all() and outs[0].abs().max().item() > 0
+
+
+@pytest.mark.parametrize("Cin,Cout,n", [(16, 16, 66000), (32, 32, 100000), (32, 20, 131000), (64, 64, 30000), (64, 64, 62000),
+                                        (96, 64, 45000)])
+def test_the_default_launch_policy_gives_the_bits_of_the_per_tile_kernel(S, Cin, Cout, n):
+    """Sizes at which the policy that ships leaves the kernel of small scenes: the filter in LDS from 65k sites, a wavefront
+    per unit from 28k at 64 channels, shared weights from 57k."""
+    from sparseconvnet._lib import lib
+
+    lib.insc_conv_reset_launch_policy()
+    m, x, feats = setup_sites(S, scenes.boxes_scene(seed=2, n=n), Cin, seed=Cin)
+    sc = m.ssc_rulebook(SZ)
+    W = cu((np.random.default_rng(Cout).normal(size=(27, Cin, Cout)) * (2.0 / Cin / 27) ** 0.5).astype(np.float32))
+    shipped, small = (torch.full((sc.n, Cout), v, device="cuda") for v in (3.0, -3.0))
+    S.ssc_rows_planned(feats, shipped, W, None, sc, m.ssc_plan(sc))
+    try:
+        lib.insc_conv_set_filter_lds_min_tiles(1 << 40)
+        lib.insc_conv_set_wavefront_per_unit_min_units(1 << 40)
+        lib.insc_conv_set_shared_weights_min_units(1 << 40)
+        S.ssc_rows_planned(feats, small, W, None, sc, m.ssc_plan(sc))
+    finally:
+        lib.insc_conv_reset_launch_policy()
+    assert sc.n >= 0.9 * n and torch.equal(shipped, small)
 
 
 def test_submanifold_convolution_cfg1_vs_dense_conv3d(S):

@@ -49,9 +49,7 @@ def layer(scene, x, W, b, case, n_in=None, events=None):
         if events is not None:
             events[1].record()
     finally:
-        lib.insc_conv_set_filter_lds_min_tiles(4096)
-        lib.insc_conv_set_wavefront_per_unit_min_units(1750)
-        lib.insc_conv_set_shared_weights_min_units(896)
+        lib.insc_conv_reset_launch_policy()
     return out.cpu().numpy()
 
 
