@@ -1332,17 +1332,8 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
         compute(U);
         return true;
       };
-      if constexpr (D == 2) {
-        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 0>())) {
-        }
-      } else if constexpr (D == 3) {
-        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 2>()) &&
-               one(std::integral_constant<int, 0>())) {
-        }
-      } else {
-        while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 2>()) &&
-               one(std::integral_constant<int, 3>()) && one(std::integral_constant<int, 0>())) {
-        }
+      static_assert(D == 2, "the turns of the rings are written out");
+      while (one(std::integral_constant<int, 1>()) && one(std::integral_constant<int, 0>())) {
       }
     }
     // the next tile's first gathers and the centre's weights, in flight over this tile's stores
@@ -2326,7 +2317,6 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     break;
     if (S > 1 && mode == MAP_NBR && K == 27) {
       switch (S) {
-        case 2: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 2); break;
         case 4: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 4); break;
         case 8: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 8); break;
         default: shape_ok = false;
