@@ -36,7 +36,9 @@ for p in (ROOT, os.path.join(ROOT, "ins-conv_amd")):
         sys.path.insert(0, p)
 
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
-MFMA_FP32_PEAK_TFLOPS = 157.3
+# fp32 products as the convolution kernels form them: eight bf16 products each, at the dense bf16 peak
+BF16_PEAK_TFLOPS = 2500.0
+MFMA_PEAK_TFLOPS = BF16_PEAK_TFLOPS / 8
 
 
 def profile_records(name):
@@ -161,26 +163,28 @@ def conv_roofline(device, reps=200, warm=300):
     bytes_alg = n_rules * (4 * Cin + 8) + sc.n * 4 * Cout + 27 * Cin * Cout * 4
     flops = 2.0 * n_rules * Cin * Cout
     achieved = bytes_alg / t / 1e9
-    traffic, traffic_note = profiled_traffic("conv_wlds_ssc32_500k.txt", "insc::conv_wlds_kernel")
+    traffic, traffic_note = profiled_traffic("conv_wlds_ssc32_500k.txt", "insc::conv_wlds_kernel<2,false>")
     return {
         "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-        "bound_in_practice": "mfma issue: `achieved` counts ALGORITHMIC bytes (every gathered row once per rule); the L2 "
-                             "serves most of that reuse, so the HBM itself moves `traffic` bytes per launch "
-                             "(hbm_GB/s_on_traffic), and what the kernel waits for is matrix-core issue (mfma_frac)",
+        "bound_in_practice": "the gather: `achieved` counts ALGORITHMIC bytes (every gathered row once per rule), which is "
+                             "what passes through the compute units' L1; the L2 serves most of that reuse, so the HBM "
+                             "itself moves `traffic` bytes per launch (hbm_GB/s_on_traffic); mfma_frac is against eight "
+                             "bf16 products per fp32 product at the dense bf16 peak",
         "hbm_GB/s_on_traffic": round(traffic / t / 1e9, 1) if traffic else None,
         "hbm_frac_on_traffic": round(traffic / t / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
         "kernel": "conv_wlds_kernel (SSC 3^3, 32->32, filter in LDS, persistent blocks; 500k sites, %d rules)" % n_rules,
         "avg_us": round(t * 1e6, 1), "algorithmic_bytes": int(bytes_alg),
         "traffic_note": traffic_note,
-        "mfma_tflops": round(flops / t / 1e12, 2), "mfma_frac": round(flops / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+        "mfma_tflops": round(flops / t / 1e12, 2), "mfma_frac": round(flops / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
         "ssc_msites_per_s": round(sc.n / t / 1e6, 1),
     }
 
 
 def wide_conv_row(device, C=64, reps=40, warm=60):
-    """The 64-channel submanifold convolution of workload 3 (500k voxels), which is bound by the
-    matrix cores rather than by HBM: us per launch and the fraction of the fp32 MFMA peak."""
+    """The 64-channel submanifold convolution of workload 3 (500k voxels), which is bound by the bytes its compute units
+    pull through L1 rather than by HBM: us per launch and the fraction of the matrix-core peak for fp32 products
+    as eight bf16 products."""
     import torch
 
     from sparseconvnet import SCN
@@ -197,7 +201,7 @@ def wide_conv_row(device, C=64, reps=40, warm=60):
     lib.insc_conv_set_shared_weights_min_units(1 << 40)
     for _ in range(warm):
         SCN.ssc_rows_planned(x.features, out, conv.weight, None, sc, plan)
-    lib.insc_conv_set_shared_weights_min_units(896)
+    lib.insc_conv_reset_launch_policy()
     for _ in range(5):
         SCN.ssc_rows_planned(x.features, out, conv.weight, None, sc, plan)
     torch.cuda.synchronize()
@@ -211,8 +215,9 @@ def wide_conv_row(device, C=64, reps=40, warm=60):
     flops = 2.0 * info["rules"] * C * C
     bytes_alg = info["rules"] * (4 * C + 8) + sc.n * 4 * C + 27 * C * C * 4
     return {"kernel": "conv_wshare_kernel<2, 4> (SSC 3^3, %d->%d, persistent blocks of four tiles sharing weight tiles through LDS, two output blocks per gathered chunk; 500k sites)" % (C, C),
-            "bound": "mfma", "avg_us": round(t * 1e6, 1), "achieved": round(flops / t / 1e12, 2),
-            "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(flops / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+            "bound": "mfma", "bound_in_practice": "gathered rows and weight tiles through L1",
+            "avg_us": round(t * 1e6, 1), "achieved": round(flops / t / 1e12, 2),
+            "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(flops / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
             "GB/s_on_algorithmic_bytes": round(bytes_alg / t / 1e9, 1)}
 
 
@@ -220,7 +225,7 @@ def split_layer_row(device, C=96, shift=2, reps=200, warm=200):
     """The kernel the incremental frame spends most of its time in - conv_mfma_kernel<1, 27, 0, 4>,
     the items of a 32-row tile dealt to four wavefronts - on the layer it serves most often: 3^3,
     96 -> 96 channels, at the third scale of the 150 000-voxel scene (10 414 sites), alone in a loop.
-    Useful and issued flops against the fp32 MFMA peak."""
+    Useful and issued flops against the matrix-core peak for fp32 products as eight bf16 products."""
     import numpy as np
     import torch
 
@@ -260,10 +265,10 @@ def split_layer_row(device, C=96, shift=2, reps=200, warm=200):
     return {"kernel": "conv_mfma_kernel<1, 27, 0, 4> (SSC 3^3, %d->%d, one 32-row tile and output block per block of four "
                       "wavefronts; %d sites = scale %d of the 150 000-voxel scene, %d rules, %d tiles)"
                       % (C, C, sc.n, shift, rules, tiles),
-            "bound": "mfma", "avg_us": round(t * 1e6, 1), "unit": "TFLOP/s", "peak": MFMA_FP32_PEAK_TFLOPS,
-            "achieved": round(useful / t / 1e12, 2), "frac": round(useful / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+            "bound": "mfma", "avg_us": round(t * 1e6, 1), "unit": "TFLOP/s", "peak": MFMA_PEAK_TFLOPS,
+            "achieved": round(useful / t / 1e12, 2), "frac": round(useful / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
             "issued_tflops": round(issued / t / 1e12, 2),
-            "issued_frac": round(issued / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+            "issued_frac": round(issued / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
             "rule_slot_fill": round(useful / issued, 3),
             "offsets_used_per_tile": round(slots / 32.0 / tiles, 2),
             "note": "alone in a loop, plain epilogue; inside a frame the same layer also adds the residual, applies the "
@@ -545,7 +550,7 @@ def frame_work_summary(net, frame_ms):
     2 * rules * Cin * Cout summed over its convolutions, issued = 2 * 32 * (offsets used per 32-row
     tile) * Cin * Cout (what the matrix cores are handed, empty rule slots included; the 3-channel
     stem runs on the vector units and counts as issued = useful), both over the whole frame's
-    wall time against the fp32 MFMA peak."""
+    wall time against the matrix-core peak for fp32 products as eight bf16 products."""
     useful = issued = 0.0
     by_scale = {}
     for w in net.frame_work():
@@ -561,8 +566,8 @@ def frame_work_summary(net, frame_ms):
     t = frame_ms * 1e-3
     return {"useful_gflop": round(useful / 1e9, 2), "issued_gflop": round(issued / 1e9, 2),
             "useful_tflops": round(useful / t / 1e12, 2), "issued_tflops": round(issued / t / 1e12, 2),
-            "useful_frac_of_fp32_mfma_peak": round(useful / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
-            "issued_frac_of_fp32_mfma_peak": round(issued / t / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+            "useful_frac_of_mfma_peak": round(useful / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
+            "issued_frac_of_mfma_peak": round(issued / t / 1e12 / MFMA_PEAK_TFLOPS, 4),
             "rule_slot_fill": round(useful / issued, 3) if issued else None,
             "by_scale": [{"scale": l, "convolutions": b[2], "useful_gflop": round(b[0] / 1e9, 2),
                           "issued_gflop": round(b[1] / 1e9, 2)} for l, b in sorted(by_scale.items())],
@@ -933,7 +938,7 @@ def main():
         extra["dirty_rows_last_frame"] = [
             {"scale": l, "sites": int(sites[l]), "min": min(r for _, r in sets), "max": max(r for _, r in sets)}
             for l, sets in enumerate(net.dirty_rows()) if sets]
-        # flop accounting of the last timed frame against the fp32 MFMA peak (the frame is bound by
+        # flop accounting of the last timed frame against the matrix-core peak (the frame is bound by
         # matrix-core issue at the coarse scales, not by HBM)
         extra["frame"] = frame_work_summary(net, per_frame[-1])
         extra["frame_phases_ms"] = sweep_phases(lambda x, inc: model.linear(net(x, increment=inc)), net, frames, first)

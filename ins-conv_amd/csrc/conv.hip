@@ -163,8 +163,9 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
 // 5k 1.35e-7 -> 0.77e-7; the seven-scale U-Net on 150k voxels 4.2e-7 -> 2.0e-7.
 // The gathered operand is split by truncation (multiply, and, subtract, byte permute: 6.5 instructions a float; rounding
 // to nearest - convert, unpack, subtract - takes as many and is slower), the weights, once, by rounding to nearest.
-// What has no such sum - infinities, NaN, weights from 2^104, sums from 2^82 - comes out as NaN or infinity;
+// What has no such sum - infinities, NaN, weights from 2^105, sums from 2^82 - comes out as NaN or infinity;
 // those elements are summed again in plain fp32 (repair_sums), so an infinity stays one.
+// (Times of variants that the comments below say were not taken are with six products instead of eight.)
 // ---------------------------------------------------------------------------------------
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
@@ -1063,8 +1064,8 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
 // room for a copy, and none is needed: lane r only ever wants the ids of row r).
 // The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (centre, then offsets ascending, same
 // MFMA sequence), so both kernels give the same bits.
-// What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in about 105 us a layer (6 TB/s; a pure
-// gather reaches 8.7), against 25 us of matrix-core time; 115 us with fp32 instructions, whose 65 us it also waited for.
+// What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in 103 us a layer (6.2 TB/s; a pure
+// gather reaches 8.7), against 35 us of matrix-core time; 115 us with fp32 instructions, whose 65 us it also waited for.
 // (A contiguous eighth of the tiles per XCD instead of interleaved ones: 531 against 511 us for four layers.)
 // ---------------------------------------------------------------------------------------
 // (32 -> 32 in four layers with their batch norms, 500k / 150k sites: eight wavefronts 542 / 228 us, twelve 538 / 201;
@@ -1400,10 +1401,10 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
 // slots are compile-time choices (the step loop is unrolled by three): the compiler then knows that a read of one
 // weight buffer cannot touch a load into another that is still in flight (for a single array it would wait for every
 // outstanding load before each LDS read).
-// What bounds it (64 -> 64 at 500k sites, four layers with batch norms 1920 us in fp32, 1435-1500 now): 2.5 GB through
-// L1 per launch at 7.5 TB/s, 45 % of the requests beyond L2; matrix cores busy 34 %, VALU 36 %.  Eight tiles per block,
-// which halves the weight bytes: 1542 us (the wavefronts wait for one another); units in site order per XCD, which
-// would hit L2: 1741 us (unbalanced).
+// What bounds it (64 -> 64 at 500k sites, a launch 414 us in fp32, 342 now; four layers with batch norms 1920 and
+// 1540-1600): 2.2 GB from L2 into L1 per launch at 6.5 TB/s; matrix cores busy 41 %.  Not taken: eight tiles per block,
+// which halves the weight bytes, 1542 us instead of 1436 (the wavefronts wait for one another); units in site order per
+// XCD, which would hit L2, 1741 instead of 1460 (unbalanced).
 // ---------------------------------------------------------------------------------------
 #define INSC_LDS_PTR(x) ((__attribute__((address_space(3))) void *)(x))
 template <int NB, int ST, bool PW>
@@ -1700,7 +1701,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
 // wavefront forms that kernel's ST partial sums one after the other (as the kernel above).  Units
 // follow the cost-ordered tile schedule, output blocks of a tile side by side on neighbouring SIMDs of
 // one compute unit, so they meet the tile's map slice and gathered rows in L1.
-// What bounds it: 10 KB through L1 per item (4 KB of rows, 6 KB of weights): 64 -> 64 at 39k sites 53 -> 48 us.
+// What bounds it: 10 KB through L1 per item (4 KB of rows, 6 KB of weights): 64 -> 64 at 39k sites 52 us in fp32, 48 now.
 // ---------------------------------------------------------------------------------------
 // D = items in flight per wavefront (2 with three wavefronts per SIMD; deeper rings at two wavefronts per
 // SIMD measured the same, and so did fewer wavefronts that draw their units from a counter: what the
@@ -2115,8 +2116,8 @@ static std::atomic<int64_t> g_shared_min_units{SHARED_MIN_UNITS};
 // 1716: 41.1 against 41.5; 1472: 41 against 39 - the split kernel's launch is whole rounds of 1024 blocks, four to
 // a compute unit, this kernel's is the SIMD with the most units).
 // Those figures are from the fp32 instruction; with bf16 parts the order is the same.  Four layers with their batch norms,
-// wavefront per unit / one block per unit / shared weights: 64 -> 64 at 39k sites 229 / 238-250 / 248-273 us, at 150k
-// 647 / 710 / 552, 96 -> 96 at 10k 251 / 195 / 194-390.
+// wavefront per unit / one block per unit / shared weights: 64 -> 64 at 39k sites 244 / 250 / 319 us, at 150k
+// 655 / 685 / 607, 96 -> 96 at 10k 264 / 185 / 413.
 constexpr int64_t OWN_MIN_UNITS = 1750;
 static std::atomic<int64_t> g_own_min_units{OWN_MIN_UNITS};
 // Narrow 3^3 layers (Cin, Cout <= 32) with at least this many 32-row tiles run on the persistent
@@ -2193,7 +2194,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
                            ep.ld2 * 4 < (1 << 24) && out_rows * ld_out * 4 < (int64_t)BUF_OOB &&
                            out_rows * ep.ld2 * 4 < (int64_t)BUF_OOB;
     // (below some two thousand tiles the persistent kernel's start-up - every block copies the whole filter into LDS -
-    // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1476 / 1440 us, 100k 1641 / 1669.
+    // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1509 / 1462 us, 100k 1654 / 1669.
     // Without a plan every tile looks its offsets up first: four times as many.  Both kernels give the same bits.)
     if (mode == MAP_NBR && K == 27 && Cin <= 32 && Cout <= 32 && map_bytes64 < (int64_t)BUF_OOB && small_ids &&
         cdiv(expect_rows, TILE_M) / (plan.map ? 1 : 4) >= g_wl_min_tiles.load(std::memory_order_relaxed) && !latency) {
