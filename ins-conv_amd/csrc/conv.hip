@@ -465,7 +465,7 @@ __device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on
 // weight tile `tile` of the filter (on false: zeros)
 template <bool PW>
 __device__ __forceinline__ WFrag<PW> load_wtile(__amdgpu_buffer_rsrc_t rw, int tile, bool on, uint32_t lane16) {
-  const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * wt_bytes(PW));
+  const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)tile * (uint32_t)wt_bytes(PW)));
   WFrag<PW> f;
   if constexpr (PW) {
     // (half s, channels h * 8 ..: quarters 2h and 2h + 1, there at lane s * 32 + column)
@@ -504,7 +504,8 @@ __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of,
       const float4 lo = buf_load16(rin, voff, 0), hi = buf_load16(rin, voff + 16u, 0);
       const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
       const int tile = (k * nch + (c16 >> 1)) * nbtp + nb;
-      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(tile * wt_bytes(PW) + (c16 & 1) * (PW ? 512 : 3072));
+      const uint32_t soff = (uint32_t)__builtin_amdgcn_readfirstlane(
+          (int)((uint32_t)tile * (uint32_t)wt_bytes(PW) + (uint32_t)((c16 & 1) * (PW ? 512 : 3072))));
       float wv[8];
       if constexpr (PW) {
         const uint32_t wo = (uint32_t)(h * 2048 + (lane & 31) * 16);

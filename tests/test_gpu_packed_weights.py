@@ -82,3 +82,10 @@ def test_weights_of_3_gb(raw):
     for a in range(0, C, 5504):
         ref = x.double() @ W[:, a:a + 5504].double()
         assert ((out[:, a:a + 5504] - ref).abs().max() <= 1e-5 * ref.abs().max()).item()
+    # (sums that are formed again read the same tiles)
+    rows = out.clone()
+    x[5, C - 7] = float("inf")
+    run()
+    assert torch.equal(out[5], torch.sign(W[C - 7]) * float("inf"))
+    rows[5] = out[5]
+    assert torch.equal(out, rows)
