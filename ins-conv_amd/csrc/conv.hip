@@ -452,7 +452,7 @@ __device__ __forceinline__ float4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t 
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
 
-// the chunk at byte offset voff (BUF_OOB: zeros) of a row; h: half-wave
+// The 32-channel chunk at byte offset `base` (BUF_OOB: zeros) of a lane's own row, every lane its 64 bytes of it.
 __device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on, uint32_t base, int h, bool full) {
   const uint32_t v0 = on ? base + (uint32_t)(h * 32) : BUF_OOB, v1 = on && full ? base + (uint32_t)(64 + h * 32) : BUF_OOB;
   Frag f;
@@ -460,6 +460,57 @@ __device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on
   f.q[1] = buf_load16(rin, v0 + 16u, 0);
   f.q[2] = buf_load16(rin, v1, 0);
   f.q[3] = buf_load16(rin, v1 + 16u, 0);
+  return f;
+}
+
+// The same chunk two lanes at a time: loads 0 and 1 of an even lane and its odd neighbour bring 32 consecutive bytes of the
+// even and of the odd lane's row (loads 2 and 3: 64 bytes further on), and the two lanes exchange what is the other's
+// (own_rows).  Why: the address unit takes a quad of lanes per cycle and line they touch, whatever they read of it, so four
+// rows a quad are four cycles for 64 bytes: rows that all lie in L1 came in at 9.3 TB/s that way and at 13.7 two rows a quad;
+// 500k sites of 32 channels at 8.5 and 11.1.  (A line a quad reaches 17.0 and 12.3, but its exchange over four lanes takes 32
+// instructions and not 16: 32 -> 32 at 500k sites 104, 99 and 102 us a layer with one, two and four lanes a row.)
+// Kernels whose launches are shorter than a few wavefronts per SIMD wait for their own instructions, not for the address
+// unit, and gather row by row (U-Net on 6k voxels 977 us, two lanes a row 1020).
+template <int CTRL>
+__device__ __forceinline__ uint32_t lane_perm(uint32_t x) {  // (an operand modifier of the instruction that uses it)
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t pair_piece(int lane) { return (uint32_t)((lane & 1) * 16 + (lane & 32)); }
+__device__ __forceinline__ Frag gather_pairs(__amdgpu_buffer_rsrc_t rin, bool on, uint32_t base, uint32_t piece, bool full) {
+  const uint32_t b = on ? base : BUF_OOB;
+  const uint32_t v0 = lane_perm<0xA0>(b) + piece, v1 = lane_perm<0xF5>(b) + piece;  // quad_perm [0,0,2,2] and [1,1,3,3]
+  Frag f;
+  f.q[0] = buf_load16(rin, v0, 0);
+  f.q[1] = buf_load16(rin, v1, 0);
+  f.q[2] = buf_load16(rin, full ? v0 + 64u : BUF_OOB, 0);
+  f.q[3] = buf_load16(rin, full ? v1 + 64u : BUF_OOB, 0);
+  return f;
+}
+// x of even lanes stays, x of odd ones goes to their even neighbour's y; y the other way round.  Eight v_cndmask with a lane
+// permutation on one operand, a form that the compiler does not make by itself.  (The wait states in front are those
+// of an operand that the instruction before has written; every lane is active where this is called.)
+__device__ __forceinline__ void exchange(float4 &x, float4 &y) {
+  float4 t, u;
+  asm("s_nop 0\n\ts_mov_b64 vcc, %16\n\t"
+      "v_cndmask_b32_dpp %0, %12, %8, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %1, %13, %9, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %2, %14, %10, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %3, %15, %11, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "s_not_b64 vcc, vcc\n\t"
+      "v_cndmask_b32_dpp %4, %8, %12, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %5, %9, %13, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %6, %10, %14, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_dpp %7, %11, %15, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "=&v"(t.x), "=&v"(t.y), "=&v"(t.z), "=&v"(t.w), "=&v"(u.x), "=&v"(u.y), "=&v"(u.z), "=&v"(u.w)
+      : "v"(x.x), "v"(x.y), "v"(x.z), "v"(x.w), "v"(y.x), "v"(y.y), "v"(y.z), "v"(y.w), "s"(0x5555555555555555ull)
+      : "vcc", "scc");
+  x = t;
+  y = u;
+}
+// what gather_pairs has loaded, sorted out: as gather_chunk gives it
+__device__ __forceinline__ Frag own_rows(Frag f) {
+  exchange(f.q[0], f.q[1]);
+  exchange(f.q[2], f.q[3]);
   return f;
 }
 // weight tile `tile` of the filter (on false: zeros)
@@ -534,6 +585,57 @@ __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of,
   }
 }
 
+// The rows of a tile: residual sum, the raw rows, the batch norm's rows - whole passes over the sixteen rows of a lane, so
+// that nothing branches per row.  Rows that do not exist (my_row < 0) go out of range.
+__device__ __forceinline__ void element_offsets(int my_row, uint32_t ld4, uint32_t (&off)[16]) {
+  int o[16];
+  rows_of_elements((int)(my_row >= 0 ? __umul24((unsigned)my_row, ld4) : BUF_OOB), o);
+  const uint32_t col4 = (uint32_t)(lane_again() & 31) * 4u;
+#pragma unroll
+  for (int v = 0; v < 16; v++) off[v] = (uint32_t)o[v] + col4;
+}
+// block: the first column (a multiple of 32); on: this lane's column exists
+__device__ __forceinline__ void store_tile(f16v &sum, int my_row, int block, bool on, __amdgpu_buffer_rsrc_t rout,
+                                           uint32_t ldo4, __amdgpu_buffer_rsrc_t rout2, uint32_t ld24,
+                                           __amdgpu_buffer_rsrc_t rres, uint32_t ldr4, float ew, float eb, float leak,
+                                           bool has_out, bool has_out2, bool has_res) {
+  uint32_t off[16];
+  if (has_res) {
+    element_offsets(my_row, ldr4, off);
+    if (on) {
+      float rv[16];
+#pragma unroll
+      for (int v = 0; v < 16; v++)
+        rv[v] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(rres, (int)off[v], block * 4, 0));
+      __builtin_amdgcn_sched_barrier(0);  // (all of them requested before the first is waited for)
+#pragma unroll
+      for (int v = 0; v < 16; v++) sum[v] += rv[v];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (the sums stay above the stores)
+  }
+  if (has_out) {
+    element_offsets(my_row, ldo4, off);
+    if (on) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const float x = sum[v];  // (a bit cast applied to the vector element itself reads element 0)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rout, (int)off[v], block * 4, 0);
+      }
+    }
+  }
+  if (has_out2) {
+    // fused batch norm + leaky ReLU
+    element_offsets(my_row, ld24, off);
+    if (on) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const float y = fmaf(sum[v], ew, eb);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : leak)), rout2, (int)off[v], block * 4, 0);
+      }
+    }
+  }
+}
+
 // The order in which a wavefront that owns a tile takes the offsets of a 3^3 filter: the centre first, then
 // ascending.  (The filter-in-LDS kernel below has no room in LDS for the centre's weights.)
 __device__ __forceinline__ int first_offset(unsigned mask) {
@@ -550,7 +652,7 @@ __device__ __forceinline__ int first_offset(unsigned mask) {
 //         With gridDim.z = G > 1 the deal goes over S * G wavefronts in G blocks (different
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
-template <int NB, int K, int MODE, int S, bool PW>
+template <int NB, int K, int MODE, int S, bool PW, bool PAIRS>
 __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) void conv_mfma_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
@@ -765,12 +867,13 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     first.rest = rest & ~(1u << first.k);
 
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
-    const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u;
+    const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u, piece = pair_piece(lane);
     auto gather = [&](const Cursor &c) -> Frag {
       const int kk = c.k < 0 ? 0 : c.k;
       const int src = nl[planned ? kk * TILE_M + r : r * K + kk];
-      return gather_chunk(rin, c.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h,
-                          Cin - c.ch * 32 >= 32);
+      const bool on = c.k >= 0 && src >= 0, full = Cin - c.ch * 32 >= 32;
+      const uint32_t base = (uint32_t)src * ld4 + (uint32_t)(c.ch * 128);
+      return PAIRS ? gather_pairs(rin, on, base, piece, full) : gather_chunk(rin, on, base, h, full);
     };
     auto wload = [&](const Cursor &c, int b) -> WFrag<PW> {
       return load_wtile<PW>(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
@@ -817,8 +920,9 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
           const WFrag<PW> &bf = bw[WRING ? u % D : nn % 2];
           if (real) {
             if (b == 0) {
-              as[0] = split8(g[u % D].q[0], g[u % D].q[1]);
-              as[1] = split8(g[u % D].q[2], g[u % D].q[3]);
+              const Frag a = PAIRS ? own_rows(g[u % D]) : g[u % D];
+              as[0] = split8(a.q[0], a.q[1]);
+              as[1] = split8(a.q[2], a.q[3]);
             }
             mac_chunk(sums[b], as, bf, full);
           }
@@ -1091,7 +1195,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   __shared__ int cost_l[WL_SCHED], sched_l[WL_SCHED];
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = lane & 31, h = lane >> 5;
+  const int r = lane & 31;
 
   // the filter but for the centre, in per-lane order
   if constexpr (PW) {
@@ -1145,8 +1249,9 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
   // the outputs are addressed with 32-bit byte offsets as well; rows that do not exist get an
   // out-of-range offset and the hardware drops the store
-  const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u);
-  const uint32_t ld4 = (uint32_t)ld_in * 4u, ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u;
+  const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u), rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
+  const uint32_t ld4 = (uint32_t)ld_in * 4u, ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u, ldr4 = (uint32_t)ep.ldr * 4u;
+  const uint32_t piece = pair_piece(lane);
   const int col = r;
   const float bv = (bias && col < Cout) ? bias[col] : 0.0f;
   const float ew = (ep.out2 && col < Cout) ? ep.w[col] : 0.0f;
@@ -1220,15 +1325,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   };
   auto gather = [&](int q, int src, uint32_t base) -> Frag {
     const bool on = q >= 0 && src >= 0 && base != BUF_OOB;  // (a load sent out of range returns 0, which would pass for a site)
-    const uint32_t v0 = on ? (uint32_t)src * ld4 + (uint32_t)(h * 32) : BUF_OOB;
-    Frag f;
-    f.q[0] = buf_load16(rin, v0, 0);
-    f.q[1] = buf_load16(rin, v0 + 16u, 0);
-    if constexpr (KS == 2) {
-      f.q[2] = buf_load16(rin, v0 + 64u, 0);
-      f.q[3] = buf_load16(rin, v0 + 80u, 0);
-    }
-    return f;
+    return gather_pairs(rin, on, (uint32_t)src * ld4, piece, KS == 2);
   };
 
   // Software pipeline over tiles: while tile t is computed, the neighbour ids of the first items of the next
@@ -1295,14 +1392,18 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       auto issue = [&](auto U) {
         constexpr int u = decltype(U)::value;
         const int qg = next_q(rg), qi = next_q(ri);
-        g[(u + D - 1) % D] = gather(qg, ix[(u + D - 1) % D], base);
+        // (the id first: its wait, a step on, is then not one for the gathers behind it as well)
+        const int here = ix[(u + D - 1) % D];
         ix[(u + AHEAD) % D] = id_load(qi, base);
+        __builtin_amdgcn_sched_barrier(0);
+        g[(u + D - 1) % D] = gather(qg, here, base);
       };
       auto compute = [&](auto U) {
         constexpr int u = decltype(U)::value;
         Parts as[2];
-        as[0] = split8(g[u].q[0], g[u].q[1]);
-        if constexpr (KS == 2) as[1] = split8(g[u].q[2], g[u].q[3]);
+        const Frag a = own_rows(g[u]);
+        as[0] = split8(a.q[0], a.q[1]);
+        if constexpr (KS == 2) as[1] = split8(a.q[2], a.q[3]);
         mac_chunk(sum, as, bw, KS == 2);
       };
       auto wread = [&](int q) {
@@ -1354,30 +1455,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
           K, rin, ld4, rw, Cin, 1, 1, 0);
       return x;
     });
-    int rid[16];
-    rows_of_elements(my_row, rid);
-    const uint32_t col4 = (uint32_t)col * 4u;
-    // (the residual input is fetched before the first store, which may alias it as far as the
-    // compiler knows: loads issued between the stores would wait one by one)
-    float rv[16];
-#pragma unroll
-    for (int v = 0; v < 16; v++)
-      rv[v] = (ep.res && rid[v] >= 0 && col < Cout) ? ep.res[(int64_t)rid[v] * ep.ldr + col] : 0.0f;
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-      const bool ok = rid[v] >= 0 && col < Cout;
-      float av = acc[v];  // (a bit cast applied to the vector element itself reads element 0)
-      if (ep.res && ok) av += rv[v];
-      if (out)
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(av), rout,
-                                              (int)(ok ? __umul24((unsigned)rid[v], ldo4) + col4 : BUF_OOB), 0, 0);
-      if (ep.out2) {
-        // fused batch norm + leaky ReLU
-        const float y = fmaf(av, ew, eb);
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : ep.leak)), rout2,
-                                              (int)(ok ? __umul24((unsigned)rid[v], ldo24) + col4 : BUF_OOB), 0, 0);
-      }
-    }
+    store_tile(acc, my_row, 0, col < Cout, rout, ldo4, rout2, ldo24, rres, ldr4, ew, eb, ep.leak, out != nullptr, ep.out2 != nullptr, ep.res != nullptr);
     t = tn;
     my_row = my_row_n;
     base = base_n;
@@ -1445,6 +1523,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
   const __amdgpu_buffer_rsrc_t reb = make_rsrc(ep.b, ep.out2 ? (uint32_t)Cout * 4u : 0u);
   const uint32_t ld4 = (uint32_t)ld_in * 4u, ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u,
                  ldr4 = (uint32_t)ep.ldr * 4u;
+  const uint32_t piece = pair_piece(lane);
   int *nlw = nl[wave];
 
   auto unit_at = [&](int64_t j) -> int64_t { return j * B + ((j & 1) ? B - 1 - b : b); };
@@ -1562,7 +1641,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
         const int kk = c.k < 0 ? 0 : c.k;
         const int src = nlw[kk * TILE_M + r];
         const bool on = c.k >= 0 && ((mine >> kk) & 1u) && src >= 0;
-        return gather_chunk(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), h, Cin - c.ch * 32 >= 32);
+        return gather_pairs(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), piece, Cin - c.ch * 32 >= 32);
       };
       auto compute = [&](const Step &c, const Frag &a, const u32x4 (*wl)[PC * 64]) {
         if (c.k < 0 || !((mine >> c.k) & 1u)) return;  // (the same for every lane of the wavefront)
@@ -1577,7 +1656,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
           }
           cur = c.p;
         }
-        const Parts as[2] = {split8(a.q[0], a.q[1]), split8(a.q[2], a.q[3])};
+        const Frag w = own_rows(a);
+        const Parts as[2] = {split8(w.q[0], w.q[1]), split8(w.q[2], w.q[3])};
 #pragma unroll
         for (int o = 0; o < NB; o++) {
           if (ob0 + o >= nbt) break;
@@ -1658,27 +1738,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
                                rw, Cin, nch, nbtp, ob0 + o);
             return x;
           });
-          int rid[16];
-          rows_of_elements(my_row, rid);
-          float rv[16];
-#pragma unroll
-          for (int v = 0; v < 16; v++)
-            rv[v] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(
-                rres, (int)((rid[v] >= 0 && cc < Cout) ? __umul24((unsigned)rid[v], ldr4) + (uint32_t)cc * 4u : BUF_OOB), 0, 0));
-#pragma unroll
-          for (int v = 0; v < 16; v++) {
-            const bool ok = rid[v] >= 0 && cc < Cout;
-            float a = sum[v];
-            if (ep.res) a += rv[v];
-            if (out)
-              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), rout,
-                                                    (int)(ok ? __umul24((unsigned)rid[v], ldo4) + (uint32_t)cc * 4u : BUF_OOB), 0, 0);
-            if (ep.out2) {
-              const float y = fmaf(a, ew[o], eb[o]);
-              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : ep.leak)), rout2,
-                                                    (int)(ok ? __umul24((unsigned)rid[v], ldo24) + (uint32_t)cc * 4u : BUF_OOB), 0, 0);
-            }
-          }
+          store_tile(sum, my_row, (ob0 + o) * 32, cc < Cout, rout, ldo4, rout2, ldo24, rres, ldr4, ew[o], eb[o], ep.leak, out != nullptr,
+                     ep.out2 != nullptr, ep.res != nullptr);
         }
       }
     } else {
@@ -1722,7 +1783,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int64_t ntiles = (n + TILE_M - 1) / TILE_M, units = ntiles * nbt;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int r = lane & 31, h = lane >> 5;
+  const int r = lane & 31;
   const int nch = conv_nch(Cin);
   int *nl = nlb[wave];
   // (wavefronts are on their own: no workgroup barrier anywhere below)
@@ -1797,11 +1858,11 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
       return nx;
     };
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
-    const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u;
+    const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u, piece = pair_piece(lane);
     auto gather = [&](const Cursor &cu) -> Frag {
       const int kk = cu.k < 0 ? 0 : cu.k;
       const int src = nl[kk * TILE_M + r];
-      return gather_chunk(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), h,
+      return gather_pairs(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), piece,
                           Cin - cu.ch * 32 >= 32);
     };
     auto wload = [&](const Cursor &cu) -> WFrag<PW> {
@@ -1840,7 +1901,8 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
             sum_start(acc, 0.0f);
             cur = c0.p;
           }
-          const Parts as[2] = {split8(g[uu].q[0], g[uu].q[1]), split8(g[uu].q[2], g[uu].q[3])};
+          const Frag a = own_rows(g[uu]);
+          const Parts as[2] = {split8(a.q[0], a.q[1]), split8(a.q[2], a.q[3])};
           mac_chunk(acc, as, bw[uu], full);
         }
         asm volatile("" ::: "memory");
@@ -1853,8 +1915,6 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
   const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u);
   const __amdgpu_buffer_rsrc_t rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
   const uint32_t ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u, ldr4 = (uint32_t)ep.ldr * 4u;
-  int rid[16];
-  rows_of_elements(my_row, rid);
   f16v sum = sum_of(acc);
   if (cur != 0) {
 #pragma unroll
@@ -1869,25 +1929,8 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
                        make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u, make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, ob);
     return x;
   });
-  float rv[16];
-#pragma unroll
-  for (int v = 0; v < 16; v++)
-    rv[v] = __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(
-        rres, (int)((rid[v] >= 0 && c < Cout) ? __umul24((unsigned)rid[v], ldr4) + (uint32_t)c * 4u : BUF_OOB), 0, 0));
-#pragma unroll
-  for (int v = 0; v < 16; v++) {
-    const bool ok = rid[v] >= 0 && c < Cout;
-    float a = sum[v];
-    if (ep.res) a += rv[v];
-    if (out)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a), rout,
-                                            (int)(ok ? __umul24((unsigned)rid[v], ldo4) + (uint32_t)c * 4u : BUF_OOB), 0, 0);
-    if (ep.out2) {
-      const float y = fmaf(a, ew, eb);  // fused batch norm + leaky ReLU
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : ep.leak)), rout2,
-                                            (int)(ok ? __umul24((unsigned)rid[v], ldo24) + (uint32_t)c * 4u : BUF_OOB), 0, 0);
-    }
-  }
+  store_tile(sum, my_row, ob * 32, c < Cout, rout, ldo4, rout2, ldo24, rres, ldr4, ew, eb, ep.leak, out != nullptr, ep.out2 != nullptr,
+             ep.res != nullptr);
   }  // units of this wavefront
 }
 
@@ -2193,7 +2236,8 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     // (row ids and row strides go through 24-bit multiplies)
     const bool small_ids = in_rows < (1 << 24) && out_rows < (1 << 24) && ld_out * 4 < (1 << 24) &&
                            ep.ld2 * 4 < (1 << 24) && out_rows * ld_out * 4 < (int64_t)BUF_OOB &&
-                           out_rows * ep.ld2 * 4 < (int64_t)BUF_OOB;
+                           out_rows * ep.ld2 * 4 < (int64_t)BUF_OOB && ep.ldr * 4 < (1 << 24) &&
+                           out_rows * ep.ldr * 4 < (int64_t)BUF_OOB;
     // (below some two thousand tiles the persistent kernel's start-up - every block copies the whole filter into LDS -
     // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1509 / 1462 us, 100k 1654 / 1669.
     // Without a plan every tile looks its offsets up first: four times as many.  Both kernels give the same bits.)
@@ -2240,7 +2284,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     }
     if (G > 1) S = 4;
     const bool wide_planned = mode == MAP_NBR && K == 27 && S == 4 && G == 1 && !lat && plan.map && plan.sched &&
-                              small_ids && ep.ldr * 4 < (1 << 24) && out_rows * ep.ldr * 4 < (int64_t)BUF_OOB;
+                              small_ids;
     // (a layer with one output block has half the weight bytes per gathered row to share: 64 -> 32 at 150k
     // sites takes 95 us there against 88 us with a wavefront per unit, so its bound is twice as high)
     if (wide_planned && cdiv(tiles, 4) * nbt >= g_shared_min_units.load(std::memory_order_relaxed) * (nbt == 1 ? 2 : 1)) {
@@ -2300,8 +2344,10 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       if ((rc = zero_counters(s, units * (size_t)S, &pcount))) return rc;  // one counter per wavefront of a unit
     }
     bool shape_ok = true;
+    // (two lanes a row from one wavefront per SIMD on; layers of a residual frame are short whatever their grids)
+    const bool pairs = !latency && (int64_t)grid.x * grid.y * grid.z * (block.x / 64) >= (int64_t)plan.cus * 4;
 #define INSC_CONV_LAUNCH(NBV, KV, MV, SV)                                                                       \
-  hipLaunchKernelGGL((pw ? conv_mfma_kernel<NBV, KV, MV, SV, true> : conv_mfma_kernel<NBV, KV, MV, SV, false>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
+  hipLaunchKernelGGL((pw ? conv_mfma_kernel<NBV, KV, MV, SV, true, false> : pairs ? conv_mfma_kernel<NBV, KV, MV, SV, false, true> : conv_mfma_kernel<NBV, KV, MV, SV, false, false>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
                      map0, map1, rows, d_n_rows, n_rows, Cin, Cout, nbtp, tile_flags, in_bytes, wp_bytes, ep, part,  \
                      pcount, plan)
 #define INSC_CONV_CASE(NBV)                                      \
