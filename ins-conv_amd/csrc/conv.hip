@@ -431,17 +431,6 @@ __device__ __forceinline__ void mac_chunk(Sum &acc, const Parts (&a)[2], const W
 // Gather: every lane reads the 64 bytes of its own input row that the MFMA A operand needs, with
 // buffer loads: one 32-bit offset per item, rows without a neighbour get an out-of-range offset
 // and the hardware returns zeros, and the weight tile is addressed by a scalar offset.
-// Items in flight per wavefront (ring depth): whole-tile wavefronts, and wavefronts that share a
-// tile.  (For the latter a ring of four measured 4-10 % slower than one of two at every scale of the
-// U-Net: with 91 instead of 140 registers more wavefronts fit a SIMD, and a turn of the unrolled loop
-// wastes fewer steps past a wavefront's last item.)
-#ifndef INSC_CONV_DEPTH
-#define INSC_CONV_DEPTH 2
-#endif
-#ifndef INSC_CONV_DEPTH_SPLIT
-#define INSC_CONV_DEPTH_SPLIT 2
-#endif
-
 // offsets at or beyond this bound make a buffer load return zeros
 constexpr uint32_t BUF_OOB = 0xFFFFF000u;  // room for the per-load immediate on top
 
@@ -636,14 +625,18 @@ __device__ __forceinline__ void store_tile(f16v &sum, int my_row, int block, boo
   }
 }
 
-// The order in which a wavefront that owns a tile takes the offsets of a 3^3 filter: the centre first, then
-// ascending.  (The filter-in-LDS kernel below has no room in LDS for the centre's weights.)
-__device__ __forceinline__ int first_offset(unsigned mask) {
-  return (mask >> 13) & 1u ? 13 : __builtin_ctz(mask);
+// Narrow 3^3 layers (fewer than 64 input channels, so one or two chunks): a row's sum is formed as two partial sums, of the even
+// offsets and of the odd ones - each ascending, with one chunk the odd ones beginning with the centre, whose weights the
+// filter-in-LDS kernel has no room for -, the bias in the former, added at the end.  So a tile can go to one wavefront, which
+// forms them one after the other, or to two: what a launch of few tiles lasts is its longest wavefront.
+constexpr unsigned EVEN_OFFSETS = 0x5555555u, ODD_OFFSETS = 0x2AAAAAAu;  // of 27
+__device__ __forceinline__ int pick_offset(unsigned rest, bool centre_first) {
+  return centre_first && ((rest >> 13) & 1u) ? 13 : __builtin_ctz(rest);
 }
 
-// S == 1: every wavefront of the block owns a tile and walks all of its filter offsets.
-// S  > 1: the S wavefronts of a block share ONE tile; the (offset, channel chunk) items are dealt
+// S == 1: every wavefront of the block owns a tile and walks all of its filter offsets (a narrow 3^3 layer: partial sum by
+//         partial sum).
+// S  > 1: the S wavefronts of a block share ONE tile (and NB output blocks of it); the (offset, channel chunk) items are dealt
 //         out round robin and the partial sums are added in wavefront order at the end.  This is for
 //         the coarse scales of a U-Net, where a layer has a handful of tiles but hundreds of
 //         channels and a single wavefront would run tens of thousands of dependent MFMAs.  Which
@@ -653,17 +646,16 @@ __device__ __forceinline__ int first_offset(unsigned mask) {
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
 template <int NB, int K, int MODE, int S, bool PW, bool PAIRS>
-__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) void conv_mfma_kernel(
+__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2 && K == 27) ? 2 : 1) void conv_mfma_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
     const int32_t *__restrict__ map1, const int32_t *__restrict__ rows,
     const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbtp,
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep,
     float *__restrict__ part, int32_t *__restrict__ pcount, TilePlan plan) {
-  static_assert(S == 1 || NB == 1, "split tiles use one output block per wavefront");
   constexpr int WAVES = S == 1 ? CONV_WAVES : S;
   __shared__ int nbl[S == 1 ? WAVES : 1][TILE_M * K];
-  __shared__ float red[S > 1 ? S : 1][S > 1 ? 16 * 64 : 1];  // (slot S - 1: only when all wavefronts share the tail)
+  __shared__ float red[S > 1 ? S : 1][S > 1 ? NB * 16 * 64 : 1];  // (slot S - 1: only when all wavefronts share the tail)
   __shared__ unsigned wmask[S];
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   // (the wavefront's number as a scalar: the item cursor below then runs on the scalar unit)
@@ -781,7 +773,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
   // folded element-wise sum, the saved rows of a residual frame's batch norm - is asked for here, for
   // the rows the wavefront finishes, so that the main loop hides these loads.
   constexpr int NVP = S > 1 ? 16 / S : 1;
-  float pre_res[NVP], pre_pin[NVP], pre_pout[NVP];
+  float pre_res[NB][NVP], pre_pin[NVP], pre_pout[NVP];
   int pre_pe[NVP];
   if (S > 1) {
     const int c = cb0 * 32 + r;
@@ -790,7 +782,9 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       const int v = wave * NVP + j, src_lane = 8 * (v >> 2) + 4 * h + (v & 3);
       const int row = __shfl(my_row, src_lane, 64);
       pre_pe[j] = __shfl(my_pe, src_lane, 64);
-      pre_res[j] = (ep.res && row >= 0 && c < Cout) ? ep.res[(int64_t)row * ep.ldr + c] : 0.0f;
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        pre_res[b][j] = (ep.res && row >= 0 && c + b * 32 < Cout) ? ep.res[(int64_t)row * ep.ldr + c + b * 32] : 0.0f;
       const bool sv = pre_pe[j] >= 0 && c < Cout;
       pre_pin[j] = sv ? ep.pre_in[(int64_t)pre_pe[j] * ep.ld_pin + c] : 0.0f;
       pre_pout[j] = sv ? ep.pre_out[(int64_t)pre_pe[j] * ep.ld_pout + c] : 0.0f;
@@ -811,16 +805,21 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     for (int w = 0; w < S; w++) act |= wmask[w];
     act = (unsigned)__builtin_amdgcn_readfirstlane((int)act);
     // (lane k looks at offset k: one ballot and a sum over the lanes instead of a scalar loop over the offsets)
-    const int c0 = (ws - lane * nch) & (ST - 1);
+    // (two wavefronts: a narrow layer's two partial sums)
+    const int c0 = S == 2 ? ((ws ^ lane) & 1) * nch : (ws - lane * nch) & (ST - 1);
     const bool has = lane < K && ((act >> (lane & 31)) & 1u) && c0 < nch;
     rest = (unsigned)__ballot(has);
-    int cnt = has ? (nch - c0 + ST - 1) >> __builtin_ctz(ST) : 0;
+    int cnt = !has ? 0 : S == 2 ? nch : (nch - c0 + ST - 1) >> __builtin_ctz(ST);
 #pragma unroll
     for (int d = 16; d > 0; d >>= 1) cnt += __shfl_xor(cnt, d, 64);
     nitems = __builtin_amdgcn_readfirstlane(cnt);
   }
 
+  // (one wavefront, several partial sums: the running one and the sum of the finished ones)
+  constexpr bool SEQ = S == 1 && K == 27 && MODE == MAP_NBR;
   Sum sums[NB];
+  f16v total[SEQ ? NB : 1];
+  int cur = 0;  // the partial sum in sums
 #pragma unroll
   for (int b = 0; b < NB; b++) {
     const int c = (cb0 + b) * 32 + r;
@@ -848,23 +847,43 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     // last item it yields k = -1, and loads for such an item are sent out of range: they
     // return zeros and move no data.
     struct Cursor {
-      int k, ch;
+      int k, ch, p;
       unsigned rest;
     };
-    auto ch0 = [&](int k) -> int { return S == 1 ? 0 : ((ws - k * nch) & (ST - 1)); };
+    const bool centre_first = K == 27 && nch == 1;
+    auto ch0 = [&](int k) -> int { return S <= 2 ? 0 : ((ws - k * nch) & (ST - 1)); };
     auto step = [&](const Cursor &c) -> Cursor {
-      const bool wrap = c.ch + ST >= nch;
+      Cursor n = c;
+      if (SEQ) {
+        const bool next = c.ch + 1 >= nch, over = next && c.rest == 0 && c.p == 0;
+        const unsigned left = over ? rest & ODD_OFFSETS : c.rest;
+        const int nk = left ? pick_offset(left, centre_first) : -1;
+        n.ch = next ? 0 : c.ch + 1;
+        n.p = over ? 1 : c.p;
+        n.k = next ? nk : c.k;
+        n.rest = next ? left & ~(1u << (nk & 31)) : c.rest;
+        return n;
+      }
+      const int stride = S == 2 ? 1 : ST;
+      const bool wrap = c.ch + stride >= nch;
       const int nk = c.rest ? __builtin_ctz(c.rest) : -1;
-      Cursor n;
-      n.ch = wrap ? ch0(nk) : c.ch + ST;
+      n.ch = wrap ? ch0(nk) : c.ch + stride;
       n.k = wrap ? nk : c.k;
       n.rest = wrap ? (c.rest & (c.rest - 1)) : c.rest;
       return n;
     };
     Cursor first;
-    first.k = S == 1 && K == 27 ? first_offset(rest) : __builtin_ctz(rest);
-    first.ch = ch0(first.k);
-    first.rest = rest & ~(1u << first.k);
+    if (SEQ) {
+      first.k = first.p = 0;
+      first.ch = nch;
+      first.rest = rest & EVEN_OFFSETS;
+      first = step(first);
+    } else {
+      first.k = pick_offset(rest, centre_first);
+      first.ch = ch0(first.k);
+      first.p = 0;
+      first.rest = rest & ~(1u << first.k);
+    }
 
     const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
     const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u, piece = pair_piece(lane);
@@ -879,59 +898,56 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       return load_wtile<PW>(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
     };
 
-    // Pipeline: while item t runs on the matrix cores, the gathers of items t+1 .. t+D-1 are in
-    // flight; so are their weight tiles when a wavefront owns a single output block (otherwise
-    // the weight tiles of the (item, block) sequence are fetched one step ahead).  Register
-    // slots are compile-time (the body is unrolled over a full turn of the rings) because
+    // Pipeline: while item t runs on the matrix cores, the gathers of item t+1 are in flight; so are its weights when a
+    // wavefront owns a single output block (otherwise the weight tiles of the (item, block) sequence are fetched one step
+    // ahead).  Register slots are compile-time (the body is unrolled over the two turns of the rings) because
     // copying a fragment would wait for the load that fills it.  Every load is issued
     // unconditionally: a load under a branch would force the wait before the MFMAs to drain
     // all outstanding loads.  The sched_barrier / memory-clobber pairs keep the loads above the
     // MFMAs they overlap and their consumers below.
-    constexpr int D = (S == 1 || S >= 16) ? INSC_CONV_DEPTH : INSC_CONV_DEPTH_SPLIT;
-    constexpr bool WRING = NB == 1;                         // weight tiles ride in the same ring
-    constexpr int TURN = (WRING || NB % 2 == 0) ? D : (D % 2 == 0 ? D : 2 * D);
-    Frag g[D];
-    WFrag<PW> bw[WRING ? D : 2];
-    Cursor ci = first;  // next item to issue
-#pragma unroll
-    for (int d = 0; d < D - 1; d++) {
-      g[d] = gather(ci);
-      if constexpr (WRING) bw[d] = wload(ci, 0);
-      ci = step(ci);
-    }
+    // (Rings of three and four items spill or leave room for fewer wavefronts; a list of the items in LDS instead of the
+    // cursor, and the next item split between the MFMAs of this one, measured the same at 32 channels and slower above.)
+    Frag g[2];
+    WFrag<PW> bw[2];
+    g[0] = gather(first);
+    bw[0] = wload(first, 0);
     Cursor c0 = first, c1 = step(first);  // item on the matrix cores and its successor
-    if constexpr (!WRING) bw[0] = wload(c0, 0);
-    // One loop turn = TURN items; the last turn may run past the last item: those steps issue
-    // out-of-range loads and skip their MFMAs (a uniform branch around the MFMAs only).
-    for (int t0i = 0; t0i < nitems; t0i += TURN) {
-#pragma unroll
-      for (int u = 0; u < TURN; u++) {
-        g[(u + D - 1) % D] = gather(ci);
-        if constexpr (WRING) bw[(u + D - 1) % D] = wload(ci, 0);
-        ci = step(ci);
-        const bool real = t0i + u < nitems, full = Cin - c0.ch * 32 >= 32;
-        Parts as[2];
+    auto turn = [&](auto U) -> bool {
+      constexpr int u = decltype(U)::value;
+      g[u ^ 1] = gather(c1);
+      if constexpr (NB == 1) bw[u ^ 1] = wload(c1, 0);
+      const bool full = Cin - c0.ch * 32 >= 32;
+      if (SEQ && c0.p != cur) {
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-          const int nn = u * NB + b;
-          if constexpr (!WRING) bw[(nn + 1) % 2] = (b + 1 < NB) ? wload(c0, b + 1) : wload(c1, 0);
-          asm volatile("" ::: "memory");
-          __builtin_amdgcn_sched_barrier(0);
-          const WFrag<PW> &bf = bw[WRING ? u % D : nn % 2];
-          if (real) {
-            if (b == 0) {
-              const Frag a = PAIRS ? own_rows(g[u % D]) : g[u % D];
-              as[0] = split8(a.q[0], a.q[1]);
-              as[1] = split8(a.q[2], a.q[3]);
-            }
-            mac_chunk(sums[b], as, bf, full);
-          }
+          const f16v part = sum_of(sums[b]);
+#pragma unroll
+          for (int v = 0; v < 16; v++) total[b][v] = cur == 0 ? part[v] : total[b][v] + part[v];
+          sum_start(sums[b], 0.0f);
         }
+        cur = c0.p;
+      }
+      Parts as[2];
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const int nn = u * NB + b;
+        if constexpr (NB > 1) bw[(nn + 1) & 1] = (b + 1 < NB) ? wload(c0, b + 1) : wload(c1, 0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-        c0 = c1;
-        c1 = step(c1);
+        if (b == 0) {
+          const Frag a = PAIRS ? own_rows(g[u]) : g[u];
+          as[0] = split8(a.q[0], a.q[1]);
+          as[1] = split8(a.q[2], a.q[3]);
+        }
+        mac_chunk(sums[b], as, bw[NB == 1 ? u : nn & 1], full);
       }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      c0 = c1;
+      c1 = step(c1);
+      return --nitems > 0;
+    };
+    while (turn(std::integral_constant<int, 0>()) && turn(std::integral_constant<int, 1>())) {
     }
   }
 
@@ -943,7 +959,13 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
   };
   f16v acc[NB];
 #pragma unroll
-  for (int b = 0; b < NB; b++) acc[b] = sum_of(sums[b]);
+  for (int b = 0; b < NB; b++) {
+    acc[b] = sum_of(sums[b]);
+    if (SEQ && cur != 0) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[b][v] = total[b][v] + acc[b][v];
+    }
+  }
   if (S == 1) {
     // (one block at a time: copies of all blocks' repeated sums would cost NB = 3 its second wavefront per SIMD, 32 -> 96 at
     // 200k sites 99 -> 124 us)
@@ -979,16 +1001,22 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
     // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3).
     constexpr int NV = 16 / (S > 1 ? S : 16);
 #pragma unroll
-    for (int v = 0; v < 16; v++) red[wave][v * 64 + lane] = acc[0][v];
+    for (int b = 0; b < NB; b++) {
+#pragma unroll
+      for (int v = 0; v < 16; v++) red[wave][(b * 16 + v) * 64 + lane] = acc[b][v];
+    }
     __syncthreads();
-    float a[NV];
+    float a[NB][NV];
     int rid[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) {
       const int v = wave * NV + j;
-      a[j] = red[0][v * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < S; w++) a[j] += red[w][v * 64 + lane];
+      for (int b = 0; b < NB; b++) {
+        a[b][j] = red[0][(b * 16 + v) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < S; w++) a[b][j] += red[w][(b * 16 + v) * 64 + lane];
+      }
       rid[j] = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
     }
     if (GZ > 1) {
@@ -1011,9 +1039,13 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       // (they emit no instructions).  An acquire/release pair at agent scope would say the same in the
       // language's terms but writes back and invalidates the whole L2.
       const int unit = (int)(bx * gridDim.y + by);
-      float *mine = part + ((int64_t)unit * GZ + bz) * 1024 + (wave * NV) * 64 + lane;
+      float *mine = part + ((int64_t)unit * GZ + bz) * (NB * 1024) + (wave * NV) * 64 + lane;
 #pragma unroll
-      for (int j = 0; j < NV; j++) __hip_atomic_store(mine + j * 64, a[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int b = 0; b < NB; b++) {
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+          __hip_atomic_store(mine + b * 1024 + j * 64, a[b][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the stores have been acknowledged
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -1021,49 +1053,57 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
       if (lane == 0) old = atomicAdd(pcount + unit * S + wave, 1);
       if (__builtin_amdgcn_readfirstlane(old) != GZ - 1) return;
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      const float *all = part + (int64_t)unit * GZ * 1024 + (wave * NV) * 64 + lane;
+      const float *all = part + (int64_t)unit * GZ * (NB * 1024) + (wave * NV) * 64 + lane;
       // (the sums of eight blocks at a time are requested together and added in block order: one trip
       // to memory per eight blocks instead of one per block)
-      constexpr int GP = 8;
+      constexpr int GP = NB == 1 ? 8 : 4;
       for (int g0 = 0; g0 < GZ; g0 += GP) {
-        float pv[GP][NV];
+        float pv[GP][NB][NV];
 #pragma unroll
         for (int gg = 0; gg < GP; gg++) {
           if (g0 + gg < GZ) {
 #pragma unroll
-            for (int j = 0; j < NV; j++)
-              pv[gg][j] = __hip_atomic_load(all + (g0 + gg) * 1024 + j * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int b = 0; b < NB; b++) {
+#pragma unroll
+              for (int j = 0; j < NV; j++)
+                pv[gg][b][j] = __hip_atomic_load(all + ((g0 + gg) * NB + b) * 1024 + j * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
           }
         }
 #pragma unroll
         for (int gg = 0; gg < GP; gg++) {
           if (g0 + gg < GZ) {
 #pragma unroll
-            for (int j = 0; j < NV; j++) a[j] = (g0 + gg == 0) ? pv[0][j] : a[j] + pv[gg][j];
+            for (int b = 0; b < NB; b++) {
+#pragma unroll
+              for (int j = 0; j < NV; j++) a[b][j] = (g0 + gg == 0) ? pv[0][b][j] : a[b][j] + pv[gg][b][j];
+            }
           }
         }
       }
       if (lane == 0) pcount[unit * S + wave] = 0;
     }
-    const int c = cb0 * 32 + r;
-    unscale<NV>(a);
-    repair_sums<NV>(a, wave * NV, [&]() -> f16v {
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+    const int c = (cb0 + b) * 32 + r;
+    unscale<NV>(a[b]);
+    repair_sums<NV>(a[b], wave * NV, [&]() -> f16v {
       f16v t;
 #pragma unroll
       for (int v = 0; v < 16; v++) t[v] = (bias0 && c < Cout) ? bias0[c] : 0.0f;
       const __amdgpu_buffer_rsrc_t rw = make_rsrc(Wp, wp_bytes);
       add_plain_products<PW>(t, [&](int k) { return id_at(map00, k); }, K, make_rsrc(in0, in_bytes0), (uint32_t)ld_in0 * 4u, rw, Cin,
-                         nch, nbtp, cb0);
+                         nch, nbtp, cb0 + b);
       if (ep.src2_in)
         add_plain_products<PW>(t, [&](int k) { return id_at(ep.src2_map, k); }, K,
                            make_rsrc(ep.src2_in, (uint32_t)(ep.src2_rows * ep.src2_ld * 4)), (uint32_t)ep.src2_ld * 4u, rw, Cin, nch,
-                           nbtp, cb0);
+                           nbtp, cb0 + b);
       return t;
     });
-    if (c >= Cout) return;
+    if (c >= Cout) continue;
     if (ep.res) {
 #pragma unroll
-      for (int j = 0; j < NV; j++) a[j] += pre_res[j];
+      for (int j = 0; j < NV; j++) a[b][j] += pre_res[b][j];
     }
     float sv[NV];
     if (MODE == MAP_PARENT && ep.side_in) {
@@ -1076,26 +1116,27 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
 #pragma unroll
       for (int j = 0; j < NV; j++) {
         if (rid[j] < 0) continue;
-        if (out) out[(int64_t)rid[j] * ld_out + c] = a[j];
-        const float o = fmaf(a[j], ew[0], eb[0]);
+        if (out) out[(int64_t)rid[j] * ld_out + c] = a[b][j];
+        const float o = fmaf(a[b][j], ew[b], eb[b]);
         const float y =
-            pre_pe[j] >= 0 ? sub_exact(leaky(fmaf(pre_pin[j], ew[0], o), ep.leak), pre_pout[j]) : leaky(o, ep.leak);
+            pre_pe[j] >= 0 ? sub_exact(leaky(fmaf(pre_pin[j], ew[b], o), ep.leak), pre_pout[j]) : leaky(o, ep.leak);
         ep.out2[(int64_t)rid[j] * ep.ld2 + c] = y;
       }
-      return;
+      continue;
     }
 #pragma unroll
     for (int j = 0; j < NV; j++) {
       if (rid[j] < 0) continue;
-      if (out) out[(int64_t)rid[j] * ld_out + c] = a[j];
+      if (out) out[(int64_t)rid[j] * ld_out + c] = a[b][j];
       if (ep.out2) {
-        const float y = fmaf(a[j], ew[0], eb[0]);  // fused batch norm + leaky ReLU
+        const float y = fmaf(a[b][j], ew[b], eb[b]);  // fused batch norm + leaky ReLU
         ep.out2[(int64_t)rid[j] * ep.ld2 + c] = y * ((y > 0.0f) ? 1.0f : ep.leak);
       }
       if (MODE == MAP_PARENT && ep.side_in) {
-        const float y = fmaf(sv[j], sw[0], sb[0]);  // batch norm of the other half of a joined matrix
+        const float y = fmaf(sv[j], sw[b], sb[b]);  // batch norm of the other half of a joined matrix
         ep.side_out[(int64_t)rid[j] * ep.ld2 + c] = y * ((y > 0.0f) ? 1.0f : ep.leak);
       }
+    }
     }
     return;
   }
@@ -1168,7 +1209,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 ? 2 : 1) vo
 // The neighbour ids go from the tile plan straight into registers, a ring of them ahead of the gathers (LDS has no
 // room for a copy, and none is needed: lane r only ever wants the ids of row r).
 // The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (centre, then offsets ascending, same
-// MFMA sequence), so both kernels give the same bits.
+// MFMA sequence; the odd offsets' partial sum, with the centre, before the even ones'), so both kernels give the same bits.
 // What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in 103 us a layer (6.2 TB/s; a pure
 // gather reaches 8.7), against 35 us of matrix-core time; 115 us with fp32 instructions, whose 65 us it also waited for.
 // (A contiguous eighth of the tiles per XCD instead of interleaved ones: 531 against 511 us for four layers.)
@@ -1197,12 +1238,16 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 31;
 
+  // The order of a tile's offsets: q = 0 the centre, 1 .. 12 the other odd ones, 13 .. 26 the even ones; offset q > 0 has its
+  // weights in LDS slot q - 1.
+  auto k_of = [](int q) -> int { return 2 * q + (q == 0 ? 13 : q <= 6 ? -1 : q <= 12 ? 1 : -26); };
+
   // the filter but for the centre, in per-lane order
   if constexpr (PW) {
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(Wp, wp_bytes);
     for (int i = threadIdx.x; i < (K - 1) * KS * 64; i += WL_WAVES * 64) {
       const int slot = i / (KS * 64), e = i - slot * (KS * 64), half = e >> 6, l = e & 63;
-      const uint32_t from = (uint32_t)((slot < 13 ? slot : slot + 1) * 4096 + (l >> 5) * 2048 + half * 512 + (l & 31) * 16);
+      const uint32_t from = (uint32_t)(k_of(slot + 1) * 4096 + (l >> 5) * 2048 + half * 512 + (l & 31) * 16);
       const Parts p = split8_nearest(buf_load16(rw, from, 0), buf_load16(rw, from + 1024u, 0));
 #pragma unroll
       for (int q = 0; q < 3; q++) wl[slot * TILE16 + (half * 3 + q) * 64 + l] = p.p[q];
@@ -1211,7 +1256,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     const u32x4 *src = reinterpret_cast<const u32x4 *>(Wp);
     for (int i = threadIdx.x; i < (K - 1) * TILE16; i += WL_WAVES * 64) {
       const int slot = i / TILE16, e = i - slot * TILE16;
-      wl[i] = src[(slot < 13 ? slot : slot + 1) * (WT_BYTES / 16) + e];
+      wl[i] = src[k_of(slot + 1) * (WT_BYTES / 16) + e];
     }
   }
   if (threadIdx.x == 0) next_turn = 0;
@@ -1298,8 +1343,14 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   auto id_base = [&](int t, int row) -> uint32_t {
     return planned ? (uint32_t)(t * TILE_M + r) * 4u : row >= 0 ? (uint32_t)row * (K * 4u) : BUF_OOB;
   };
-  // the offsets a tile uses, the centre as bit 0 and the others in their order from bit 1 on: bit q > 0 has its
-  // weights in LDS slot q - 1
+  // the offsets a tile uses, bit q
+  auto every_other = [](unsigned x) -> unsigned {  // bits 0, 2, .. 30 of x
+    x &= 0x55555555u;
+    x = (x | x >> 1) & 0x33333333u;
+    x = (x | x >> 2) & 0x0F0F0F0Fu;
+    x = (x | x >> 4) & 0x00FF00FFu;
+    return (x | x >> 8) & 0xFFFFu;
+  };
   auto offsets_of = [&](int t, uint32_t base, int v) -> unsigned {
     unsigned m = 0;
     if (t >= ntiles) return 0u;
@@ -1311,7 +1362,8 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
         m |= __any(id >= 0) ? 1u << k : 0u;
       }
     }
-    return ((m >> 13) & 1u) | ((m & 0x1FFFu) << 1) | (m & 0x7FFC000u);
+    const unsigned odd = every_other(m >> 1), even = every_other(m);
+    return ((odd >> 6) & 1u) | ((odd & 0x3Fu) << 1) | ((odd >> 7) << 7) | (even << 13);
   };
   auto next_q = [](unsigned &rest) -> int {  // past the end: -1
     const int q = rest ? __builtin_ctz(rest) : -1;
@@ -1319,7 +1371,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     return q;
   };
   auto id_load = [&](int q, uint32_t base) -> int {
-    const uint32_t k = q == 0 ? 13u : q <= 13 ? (uint32_t)(q - 1) : (uint32_t)q;
+    const uint32_t k = (uint32_t)k_of(q);
     return (int)__builtin_amdgcn_raw_buffer_load_b32(rids, (int)(q >= 0 && base != BUF_OOB ? base : BUF_OOB),
                                                      (int)(q >= 0 ? k * pitch : 0u), 0);
   };
@@ -1378,8 +1430,16 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     const int my_row_nn = load_row(tnn);
     const int mask_nn_v = planned && tnn < ntiles ? (int)plan.tmask[tnn] : 0;
 
+    // the odd offsets' partial sum, then - with the bias - the even ones'
     Sum sum;
-    sum_start(sum, bv);
+    f16v total;
+    bool second = false;
+    sum_start(sum, 0.0f);
+    auto fold = [&]() {
+      total = sum_of(sum);
+      sum_start(sum, bv);
+      second = true;
+    };
 
     if (rest) {
       // three cursors over the tile's items: the one computed, the one gathered, the one whose id is loaded
@@ -1413,6 +1473,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       };
       {
         const int q = next_q(rc);
+        if (q >= 13) fold();
         if (q != 0) {  // (a tile without the centre; bw or cw holds the centre's weights otherwise)
           wread(q);
         } else if constexpr (PW) {
@@ -1428,6 +1489,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       auto one = [&](auto U) -> bool {
         if (!rc) return false;
         const int q = next_q(rc);
+        if (q >= 13 && !second) fold();
         wread(q);
         __builtin_amdgcn_sched_barrier(0);
         issue(U);
@@ -1442,7 +1504,10 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
     // the next tile's first gathers and the centre's weights, in flight over this tile's stores
     prime(rest_n, base_n);
     __builtin_amdgcn_sched_barrier(0);
+    if (!second) fold();
     f16v acc = sum_of(sum);
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] += total[v];
     unscale<16>(acc);
 
     // D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3)
@@ -2150,19 +2215,18 @@ int split_weights(const float *W, int K, int Cin, int Cout, float *Ws, hipStream
 
 // Launch policy of wide 3^3 layers (64..159 input channels, a tile schedule).  All kernels give the same
 // bits; the bounds only move time.
-// With at least this many (group of four tiles, output block) units: the kernel whose blocks share the
-// weight tiles through LDS (faster from about 60k sites at 64 channels).
-constexpr int64_t SHARED_MIN_UNITS = 896;
+// With at least this many (group of four tiles, output block) units, and at most two output blocks: the kernel whose blocks
+// share the weight tiles through LDS.  64 -> 64, four layers with batch norms, shared / two blocks a split wavefront: 60k sites
+// 282 / 268 us, 90k 346 / 391, 150k 567 / 580.  With three and four output blocks the split kernel, which gathers once for all
+// or for two of them, is ahead everywhere: 96 -> 96 at 39k sites 437 / 315, at 333k 2335 / 2133, 112 -> 112 at 60k 714 / 686.
+constexpr int64_t SHARED_MIN_UNITS = 1100;
 static std::atomic<int64_t> g_shared_min_units{SHARED_MIN_UNITS};
-// Below that, with at least this many (tile, output block) units - half as many again for layers of more
-// than 64 input channels, whose units are longer - the kernel that gives every unit a wavefront of its own
-// (64 -> 64 at 39k sites = 2452 units: 50 us against 56 us; 2084 units: 48 against 50; 1840: 41 against 44;
-// 1716: 41.1 against 41.5; 1472: 41 against 39 - the split kernel's launch is whole rounds of 1024 blocks, four to
-// a compute unit, this kernel's is the SIMD with the most units).
-// Those figures are from the fp32 instruction; with bf16 parts the order is the same.  Four layers with their batch norms,
-// wavefront per unit / one block per unit / shared weights: 64 -> 64 at 39k sites 244 / 250 / 319 us, at 150k
-// 655 / 685 / 607, 96 -> 96 at 10k 264 / 185 / 413.
+// Below that, where the split kernel has one output block a wavefront: with at least this many (tile, output block) units - half
+// as many again for layers of more than 64 input channels, whose units are longer - the kernel that gives every unit a
+// wavefront of its own (64 -> 32 at 150k sites 75 us against 79 in the split kernel; with fp32 instructions the two met at
+// some 1700 units).
 constexpr int64_t OWN_MIN_UNITS = 1750;
+constexpr int64_t NARROW_SPLIT_WAVES = 8192, MANY_BLOCKS_MIN_WAVES = 2400;  // (see the launch shapes below)
 static std::atomic<int64_t> g_own_min_units{OWN_MIN_UNITS};
 // Narrow 3^3 layers (Cin, Cout <= 32) with at least this many 32-row tiles run on the persistent
 // kernel that keeps the whole filter in LDS; smaller ones on the one-wavefront-per-tile kernel.
@@ -2270,8 +2334,9 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const int NB0 = split ? 1 : conv_nb_per_group(Cout);
     const int nbtp = conv_nbt_padded(Cout);
     int S = 1;
+    const bool narrow = mode == MAP_NBR && K == 27 && !split;  // (two partial sums, whoever forms them)
     if (split) S = K == 27 ? (Cin >= 160 ? 8 : 4) : ((Cin >= 96 || two) ? 4 : 1);  // K == 8: conv and deconv
-    const int NB = (S == 1 && Cin >= 96) ? 1 : NB0;
+    int NB = (S == 1 && Cin >= 96) ? 1 : NB0;
     // (the split across blocks is for scales with few tiles; in a U-Net the width grows with the depth,
     // and a layer that narrows to at most 96 channels sits at a fine scale with many tiles)
     // (eight blocks from 224 -> 192 channels: the two coarsest scales of a seven-scale U-Net, a few tiles,
@@ -2283,11 +2348,27 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       S = 4;
     }
     if (G > 1) S = 4;
-    const bool wide_planned = mode == MAP_NBR && K == 27 && S == 4 && G == 1 && !lat && plan.map && plan.sched &&
+    // A tile of a narrow layer: a wavefront for each partial sum and output block up to NARROW_SPLIT_WAVES of them, one wavefront
+    // for all beyond.  Kernel times, split / not: 32 -> 32 at 6k sites 13 / 20 us, 48 -> 48 at 2k 18 / 41; four layers with
+    // batch norms 48 -> 48 at 60k (7504 wavefronts) 247 / 253, 32 -> 32 at 37k 165 / 173.  (Four partial sums for two-chunk
+    // layers: U-Net of 16 channels on 6k voxels 648 us and not 690, but 48 -> 48 at 150k 540 and not 424.)
+    if (narrow && !pw && tiles * nbt * 2 <= NARROW_SPLIT_WAVES) {
+      S = 2;
+      NB = 1;
+    }
+    // Wide layers: two or three output blocks a wavefront, which gathers and splits a row for all of them, while that
+    // leaves MANY_BLOCKS_MIN_WAVES wavefronts.  Kernel times, several / one: 64 -> 64 at 39k sites (4848 wavefronts left) 41 /
+    // 48 us (the wavefront-per-unit kernel), 192 -> 96 at 10k (2528) 49 / 64, 128 -> 64 at 39k (4848) 64 / 73, but
+    // 96 -> 96 at 10k (1264) 37 / 32 and 128 -> 128 at 2.6k (1296) 22 / 19.
+    if (mode == MAP_NBR && K == 27 && !latency && !pw) {
+      const int many = S == 4 ? (nbt % 2 == 0 ? 2 : nbt % 3 == 0 ? 3 : 1) : S == 8 && nbt == 3 ? 3 : 1;
+      if (many > 1 && tiles * (nbt / many) * S * G >= MANY_BLOCKS_MIN_WAVES) NB = many;
+    }
+    const bool wide_planned = mode == MAP_NBR && K == 27 && Cin >= 64 && S == 4 && G == 1 && !lat && plan.map && plan.sched &&
                               small_ids;
     // (a layer with one output block has half the weight bytes per gathered row to share: 64 -> 32 at 150k
     // sites takes 95 us there against 88 us with a wavefront per unit, so its bound is twice as high)
-    if (wide_planned && cdiv(tiles, 4) * nbt >= g_shared_min_units.load(std::memory_order_relaxed) * (nbt == 1 ? 2 : 1)) {
+    if (wide_planned && (nbt <= 2 || pw) && cdiv(tiles, 4) * nbt >= g_shared_min_units.load(std::memory_order_relaxed) * (nbt == 1 ? 2 : 1)) {
       // blocks of four tiles that share the weight tiles through LDS
       // with enough units left, two output blocks per gathered chunk (eight accumulators: two
       // wavefronts per SIMD instead of three, but a third fewer bytes per MFMA)
@@ -2321,7 +2402,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       return INSC_OK;
     }
     const int64_t own_min = g_own_min_units.load(std::memory_order_relaxed);
-    if (wide_planned && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
+    if (wide_planned && NB == 1 && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
       // one wavefront per (tile, output block): enough units that every SIMD gets one to three
       auto kernel = pw ? conv_own_kernel<4, 2, true> : conv_own_kernel<4, 2, false>;
       hipLaunchKernelGGL(kernel, dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
@@ -2332,13 +2413,13 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     }
     const unsigned gx = (unsigned)(S == 1 ? cdiv(tiles, CONV_WAVES) : tiles);
     const int GZ = two ? 2 * G : G;  // blocks per (tile, output block): G per source
-    dim3 grid(gx, (unsigned)(NB == 1 ? nbt : nbtp / NB), (unsigned)GZ), block((S == 1 ? CONV_WAVES : S) * 64);
+    dim3 grid(gx, (unsigned)cdiv(nbt, NB), (unsigned)GZ), block((S == 1 ? CONV_WAVES : S) * 64);
     float *part = nullptr;
     int32_t *pcount = nullptr;
     if (GZ > 1) {
       const size_t units = (size_t)gx * grid.y;
       void *ws;
-      int rc = workspace(WS_CONV, s, units * GZ * 1024 * sizeof(float), &ws);
+      int rc = workspace(WS_CONV, s, units * GZ * NB * 1024 * sizeof(float), &ws);
       if (rc) return rc;
       part = (float *)ws;
       if ((rc = zero_counters(s, units * (size_t)S, &pcount))) return rc;  // one counter per wavefront of a unit
@@ -2348,6 +2429,10 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const bool pairs = !latency && (int64_t)grid.x * grid.y * grid.z * (block.x / 64) >= (int64_t)plan.cus * 4;
 #define INSC_CONV_LAUNCH(NBV, KV, MV, SV)                                                                       \
   hipLaunchKernelGGL((pw ? conv_mfma_kernel<NBV, KV, MV, SV, true, false> : pairs ? conv_mfma_kernel<NBV, KV, MV, SV, false, true> : conv_mfma_kernel<NBV, KV, MV, SV, false, false>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
+                     map0, map1, rows, d_n_rows, n_rows, Cin, Cout, nbtp, tile_flags, in_bytes, wp_bytes, ep, part,  \
+                     pcount, plan)
+#define INSC_CONV_LAUNCH_MANY(NBV, SV)                                                                            \
+  hipLaunchKernelGGL((conv_mfma_kernel<NBV, 27, MAP_NBR, SV, false, true>), grid, block, 0, s, in, ld_in, out, ld_out, Wp, bias,  \
                      map0, map1, rows, d_n_rows, n_rows, Cin, Cout, nbtp, tile_flags, in_bytes, wp_bytes, ep, part,  \
                      pcount, plan)
 #define INSC_CONV_CASE(NBV)                                      \
@@ -2365,8 +2450,16 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     break;
     if (S > 1 && mode == MAP_NBR && K == 27) {
       switch (S) {
-        case 4: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 4); break;
-        case 8: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 8); break;
+        case 2: INSC_CONV_LAUNCH(1, 27, MAP_NBR, 2); break;
+        case 4:
+          if (NB == 1) INSC_CONV_LAUNCH(1, 27, MAP_NBR, 4);
+          else if (NB == 2) INSC_CONV_LAUNCH_MANY(2, 4);
+          else INSC_CONV_LAUNCH_MANY(3, 4);
+          break;
+        case 8:
+          if (NB == 3) INSC_CONV_LAUNCH_MANY(3, 8);
+          else INSC_CONV_LAUNCH(1, 27, MAP_NBR, 8);
+          break;
         default: shape_ok = false;
       }
     } else if (S > 1 && mode == MAP_NBR && K == 8) {
@@ -2393,6 +2486,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       return INSC_ERR_ARG;
     }
 #undef INSC_CONV_LAUNCH
+#undef INSC_CONV_LAUNCH_MANY
 #undef INSC_CONV_CASE
   } else {
     if (!W) {
