@@ -246,7 +246,10 @@ __global__ void grid_assign_kernel(Slot *table, const int32_t *__restrict__ coor
 // (an incremental frame): thread t owns a contiguous run of rows, so the ids come out in row
 // order exactly as from the scan-based passes.  site_of_point holds the rows' states on entry and
 // their sites on exit.
-constexpr int FINISH_SMALL_MAX = 16384;
+constexpr int FINISH_SMALL_MAX = 16384;  // (16 rows a thread)
+// A single grid's inserts take it up to 4096 rows: 3.6k rows 13 us, 14k 59 - a thread's rows one after the other, on one
+// compute unit - against 25 in the passes over the whole chip.
+constexpr int INSERT_ONE_MAX = 4096;
 __global__ __launch_bounds__(1024) void grid_finish_small_kernel(Slot *table, const int32_t *__restrict__ coords4,
                                                                  const int32_t *__restrict__ slot_of_point, int P,
                                                                  int32_t *d_n, int32_t *__restrict__ site_coords,
@@ -886,7 +889,7 @@ static int grid_insert_launch(insc_grid *g, const int32_t *d_coords4, int64_t P,
   const int64_t mask = g->n_slots - 1;
   const unsigned nb = grid_for(P, 256);
   int32_t *total = g->flags + g->scratch_rows;  // spare int after the flags
-  const bool small = P <= FINISH_SMALL_MAX;
+  const bool small = P <= INSERT_ONE_MAX;
   const int64_t n_parts = g->n_slots >> PART_SHIFT;
   if (!small && g->n_upper == 0 && g->part && n_parts >= 1 && n_parts <= PART_MAX) {  // empty: built in LDS
     int32_t *cnt = g->part, *cursor = cnt + PART_MAX * PART_PAD, *base = cursor + PART_MAX * PART_PAD;
@@ -962,7 +965,27 @@ constexpr int SORT_NEW_MAX = 8192;
 // LDS of the two appends: the keys of the new sites in two buffers that a merge round reads and writes in turn
 struct OrderLds {
   uint64_t key[2][SORT_NEW_MAX];
+  uint64_t bits[16][28];  // of each wavefront: the neighbour bits of its 64 sites (pattern_of_site)
 };
+// The word of site first + i (past n: all key bits set, so it ends up last), and that of the other lanes' sites - i and lane
+// agree mod 64 - sorted over the wavefront: a bitonic network.
+__device__ __forceinline__ uint64_t order_word_sorted(int first, int n, int i, const int32_t *__restrict__ coords,
+                                                      const int32_t *__restrict__ nbr, uint64_t *bits) {
+  const int lane = threadIdx.x & 63;
+  uint64_t k = ~8191ull | (uint64_t)i;
+  const uint32_t m = pattern_of_site(nbr, (int64_t)first + i - lane, min(64, n - (i - lane)), bits);
+  if (i < n) k = (order_key(reinterpret_cast<const int4 *>(coords)[first + i], m) << 13) | (uint64_t)i;
+#pragma unroll
+  for (int kk = 2; kk <= 64; kk <<= 1) {
+#pragma unroll
+    for (int j = kk >> 1; j > 0; j >>= 1) {
+      const uint64_t y = __shfl_xor(k, j, 64);
+      const bool keep_small = ((lane & j) == 0) == ((lane & kk) == 0);
+      k = keep_small ? (k < y ? k : y) : (k < y ? y : k);
+    }
+  }
+  return k;
+}
 // Sorted by (key, arrival) - one 64-bit word per site, sort key in the upper 51 bits, index among the new
 // sites in the lower 13, so no two words are equal - by one workgroup (all of it on one compute unit: what
 // it costs is the number of instructions, ~14 us for 3000 sites): every wavefront sorts runs of 64
@@ -975,7 +998,7 @@ __device__ __forceinline__ void order_append_sorted_body(const int first, const 
                                                          const int32_t *__restrict__ coords,
                                                          const int32_t *__restrict__ nbr, int32_t *__restrict__ order,
                                                          int32_t *__restrict__ pos, OrderLds &L) {
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   if (n <= 0) return;
   if (n > SORT_NEW_MAX) {
     for (int i = tid; i < n; i += 1024) {
@@ -986,25 +1009,7 @@ __device__ __forceinline__ void order_append_sorted_body(const int first, const 
   }
   const int N = (n + 63) & ~63;  // whole runs of 64; the words past n have all key bits set and end up last
   for (int i = tid; i < N; i += 1024) {
-    uint64_t k = ~8191ull | (uint64_t)i;
-    if (i < n) {
-      const int v = first + i;
-      const int4 c = reinterpret_cast<const int4 *>(coords)[v];
-      uint32_t m = 0;
-      for (int j = 0; j < 27; j++) m |= (nbr[(int64_t)v * 27 + j] >= 0 ? 1u : 0u) << j;
-      k = (order_key(c, m) << 13) | (uint64_t)i;
-    }
-    // the run of 64 that this word belongs to is held by one wavefront (i and lane agree mod 64): sorted here
-#pragma unroll
-    for (int kk = 2; kk <= 64; kk <<= 1) {
-#pragma unroll
-      for (int j = kk >> 1; j > 0; j >>= 1) {
-        const uint64_t y = __shfl_xor(k, j, 64);
-        const bool keep_small = ((lane & j) == 0) == ((lane & kk) == 0);
-        k = keep_small ? (k < y ? k : y) : (k < y ? y : k);
-      }
-    }
-    L.key[0][i] = k;
+    L.key[0][i] = order_word_sorted(first, n, i, coords, nbr, L.bits[tid >> 6]);
   }
   __syncthreads();
   int src = 0;
@@ -1134,21 +1139,127 @@ __device__ __forceinline__ void order_append_grouped_body(const int first, const
 // both orders of a scale by one workgroup: the processing order of the 3^3 layers, then - where the
 // scale has a coarser one above it - the order grouped by the position inside the parent cell
 struct OrderBothJob {
-  const int32_t *d_n, *coords, *nbr, *offset;  // offset null: no second order
+  const int32_t *d_n, *coords, *nbr, *offset;  // offset null: no second order; d_n null: `first` and `n` say which sites
   int32_t *order, *pos, *bo_order, *bo_pos;
   int all;  // order every site of the grid, not only those of the last insert
+  int first, n;
 };
+__device__ __forceinline__ void order_range(const OrderBothJob &j, int &first, int &n) {
+  first = !j.d_n ? j.first : j.all ? 0 : j.d_n[1];
+  n = !j.d_n ? j.n : j.d_n[0] - first;
+}
 struct OrderBothBatch {
   OrderBothJob job[16];
 };
 __global__ __launch_bounds__(1024) void order_append_both_batch_kernel(OrderBothBatch b) {
   __shared__ OrderLds L;
   const OrderBothJob &j = b.job[blockIdx.x];
-  const int first = j.all ? 0 : j.d_n[1], n = j.d_n[0] - first;
+  int first, n;
+  order_range(j, first, n);
   order_append_sorted_body(first, n, j.coords, j.nbr, j.order, j.pos, L);
   if (!j.offset) return;
   __syncthreads();  // the order written above is read below (by other threads than wrote it), and the LDS is reused
   order_append_grouped_body(first, n, j.offset, j.order, j.bo_order, j.bo_pos, L.key[0]);
+}
+// The same in three launches, for more than a run of 1024 words: one workgroup per run sorts it, one per run finds the
+// places of its words among all (the runs before it and the smaller words of the others, counted by binary searches in
+// LDS), one per scale groups them by offset.  By one workgroup 6000 sites took 70 us, 65 of them on the address unit of
+// its one compute unit (27 map entries of every site, a line each); read a site's entries side by side 44; in
+// three launches 19.
+constexpr int ORDER_RUN = 1024;
+__global__ __launch_bounds__(ORDER_RUN) void order_runs_kernel(OrderBothBatch b, uint64_t *__restrict__ words) {
+  __shared__ uint64_t key[2][ORDER_RUN];
+  __shared__ uint64_t bits[16][28];
+  const OrderBothJob &j = b.job[blockIdx.y];
+  int first, n;
+  order_range(j, first, n);
+  const int tid = threadIdx.x, i = blockIdx.x * ORDER_RUN + tid;
+  if (n > SORT_NEW_MAX) {  // (arrival order)
+    for (int q = i; q < n; q += gridDim.x * ORDER_RUN) {
+      j.order[first + q] = first + q;
+      if (j.pos) j.pos[first + q] = first + q;
+    }
+    return;
+  }
+  if ((int)blockIdx.x * ORDER_RUN >= n) return;  // (the whole block)
+  key[0][tid] = order_word_sorted(first, n, i, j.coords, j.nbr, bits[tid >> 6]);
+  __syncthreads();
+  int src = 0;
+#pragma unroll
+  for (int lg = 6; lg < 10; lg++) {
+    const int len = 1 << lg, run = tid >> lg;
+    const uint64_t *a = key[src], *sib = a + ((run ^ 1) << lg);
+    const uint64_t w = a[tid];
+    int lo = 0;
+    for (int step = len; step >= 1; step >>= 1)
+      if (lo + step <= len && sib[lo + step - 1] < w) lo += step;
+    key[src ^ 1][((run >> 1) << (lg + 1)) + (tid & (len - 1)) + lo] = w;
+    __syncthreads();
+    src ^= 1;
+  }
+  words[(int64_t)blockIdx.y * SORT_NEW_MAX + i] = key[src][tid];
+}
+__global__ __launch_bounds__(ORDER_RUN) void order_merge_kernel(OrderBothBatch b, const uint64_t *__restrict__ words) {
+  __shared__ uint64_t all[SORT_NEW_MAX];
+  const OrderBothJob &j = b.job[blockIdx.y];
+  int first, n;
+  order_range(j, first, n);
+  if (n > SORT_NEW_MAX || (int)blockIdx.x * ORDER_RUN >= n) return;
+  const int tid = threadIdx.x, runs = (n + ORDER_RUN - 1) / ORDER_RUN;
+  words += (int64_t)blockIdx.y * SORT_NEW_MAX;
+  for (int r = 0; r < runs; r++) all[r * ORDER_RUN + tid] = words[r * ORDER_RUN + tid];
+  __syncthreads();
+  const uint64_t w = all[blockIdx.x * ORDER_RUN + tid];
+  constexpr int RUNS = SORT_NEW_MAX / ORDER_RUN;
+  int lo[RUNS];
+#pragma unroll
+  for (int r = 0; r < RUNS; r++) lo[r] = 0;
+  for (int step = ORDER_RUN; step >= 1; step >>= 1) {
+#pragma unroll
+    for (int r = 0; r < RUNS; r++)
+      if (r < runs && lo[r] + step <= ORDER_RUN && all[r * ORDER_RUN + lo[r] + step - 1] < w) lo[r] += step;
+  }
+  int at = 0;  // (no two words are equal: in its own run a word counts those before it)
+#pragma unroll
+  for (int r = 0; r < RUNS; r++) at += r < runs ? lo[r] : 0;
+  if (at >= n) return;  // (a word past n)
+  const int v = first + (int)(w & 8191);
+  j.order[first + at] = v;
+  if (j.pos) j.pos[v] = first + at;
+}
+__global__ __launch_bounds__(1024) void order_group_kernel(OrderBothBatch b) {
+  __shared__ uint64_t sums[32];
+  const OrderBothJob &j = b.job[blockIdx.x];
+  if (!j.offset) return;
+  int first, n;
+  order_range(j, first, n);
+  order_append_grouped_body(first, n, j.offset, j.order, j.bo_order, j.bo_pos, sums);
+}
+static int order_launch(const OrderBothBatch &b, int n, int64_t n_upper, hipStream_t s) {
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (n_upper > ORDER_RUN) INSC_HIP(hipStreamIsCapturing(s, &capturing));
+  if (n_upper <= ORDER_RUN || capturing != hipStreamCaptureStatusNone) {  // (a captured call takes no memory)
+    hipLaunchKernelGGL(order_append_both_batch_kernel, dim3((unsigned)n), dim3(1024), 0, s, b);
+    INSC_LAUNCH_CHECK();
+    return INSC_OK;
+  }
+  void *ws;
+  const int rc = workspace(WS_SORT, s, sizeof(uint64_t) * SORT_NEW_MAX * (size_t)n, &ws);
+  if (rc) return rc;
+  const dim3 grid((unsigned)std::min<int64_t>(cdiv(n_upper, ORDER_RUN), SORT_NEW_MAX / ORDER_RUN), (unsigned)n);
+  hipLaunchKernelGGL(order_runs_kernel, grid, dim3(ORDER_RUN), 0, s, b, (uint64_t *)ws);
+  hipLaunchKernelGGL(order_merge_kernel, grid, dim3(ORDER_RUN), 0, s, b, (const uint64_t *)ws);
+  bool grouped = false;
+  for (int i = 0; i < n; i++) grouped = grouped || b.job[i].offset;
+  if (grouped) hipLaunchKernelGGL(order_group_kernel, dim3((unsigned)n), dim3(1024), 0, s, b);
+  INSC_LAUNCH_CHECK();
+  return INSC_OK;
+}
+// the sites first .. first + n - 1 (at most order_sorted_max() of them) in processing order
+int order_sites(const insc_grid *g, const int32_t *d_nbr, int64_t first, int64_t n, int32_t *d_order, hipStream_t s) {
+  OrderBothBatch b;
+  b.job[0] = OrderBothJob{nullptr, g->coords, d_nbr, nullptr, d_order, nullptr, nullptr, nullptr, 0, (int)first, (int)n};
+  return order_launch(b, 1, n, s);
 }
 
 int64_t order_sorted_max() { return SORT_NEW_MAX; }
@@ -1803,10 +1914,8 @@ int order_append_new_sites_both_batch(const insc_grid *const *grids, const int32
   }
   OrderBothBatch b;
   for (int i = 0; i < n; i++)
-    b.job[i] = OrderBothJob{grids[i]->d_n, grids[i]->coords, d_nbr[i], d_offset[i], d_order[i], d_pos[i], d_bo_order[i], d_bo_pos[i], all ? 1 : 0};
-  hipLaunchKernelGGL(order_append_both_batch_kernel, dim3((unsigned)n), dim3(1024), 0, s, b);
-  INSC_LAUNCH_CHECK();
-  return INSC_OK;
+    b.job[i] = OrderBothJob{grids[i]->d_n, grids[i]->coords, d_nbr[i], d_offset[i], d_order[i], d_pos[i], d_bo_order[i], d_bo_pos[i], all ? 1 : 0, 0, 0};
+  return order_launch(b, n, n_new_upper, s);
 }
 
 }  // namespace insc
