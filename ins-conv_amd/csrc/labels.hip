@@ -27,14 +27,36 @@ struct insc_labels {
 
 namespace insc {
 
+// First maximum of a row, as torch.max / torch.argmax.  The scores are asked for twenty at a time, in 16-byte loads where the
+// rows allow it: one by one - a lane per row, a line per lane - 200k rows of 20 classes took 33 us of a frame's update.
 __device__ __forceinline__ void row_max(const float *__restrict__ x, int C, int &arg, float &val) {
+  constexpr int N = 20;
+  const bool wide = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
   arg = 0;
   val = x[0];
-  for (int c = 1; c < C; c++)
-    if (x[c] > val) {  // first maximum, as torch.max / torch.argmax
-      val = x[c];
-      arg = c;
+  for (int c0 = 0; c0 < C; c0 += N) {
+    float v[N];
+    if (wide && c0 + N <= C) {
+#pragma unroll
+      for (int i = 0; i < N / 4; i++) {
+        const float4 q = reinterpret_cast<const float4 *>(x + c0)[i];
+        v[4 * i] = q.x;
+        v[4 * i + 1] = q.y;
+        v[4 * i + 2] = q.z;
+        v[4 * i + 3] = q.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; i++) v[i] = c0 + i < C ? x[c0 + i] : 0.0f;
     }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (c0 + i < C && v[i] > val) {
+        val = v[i];
+        arg = c0 + i;
+      }
+    }
+  }
 }
 
 __global__ void labels_push_kernel(const int32_t *__restrict__ sop, int64_t P, int32_t *__restrict__ head,
