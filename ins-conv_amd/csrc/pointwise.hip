@@ -320,6 +320,19 @@ int launch_input_finish(const float *d_sum, const int32_t *d_cnt, int mode, floa
   return INSC_OK;
 }
 
+// Coordinate rows of three or four columns, 32 or 64 bits wide (narrowed as a conversion does it), widened to (x, y, z, batch);
+// *bad = 1 where one lies outside 0 .. 65535 (batch 0 .. 32767).  Bound by the rows' bytes: 28 to 48 a point.
+template <class T>
+__global__ __launch_bounds__(256) void coords4_kernel(const T *__restrict__ in, int cols, int64_t ld, int64_t P,
+                                                      int32_t *__restrict__ out4, int32_t *__restrict__ bad) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  const T *row = in + p * ld;
+  const int4 c = make_int4((int)row[0], (int)row[1], (int)row[2], cols == 4 ? (int)row[3] : 0);
+  reinterpret_cast<int4 *>(out4)[p] = c;
+  if (bad && ((unsigned)c.x > 65535u || (unsigned)c.y > 65535u || (unsigned)c.z > 65535u || (unsigned)c.w > 32767u)) *bad = 1;
+}
+
 }  // namespace insc
 
 using namespace insc;
@@ -340,6 +353,23 @@ int insc_add(const float *d_a, int64_t ld_a, const float *d_b, int64_t ld_b, flo
   INSC_REQUIRE(n_rows >= 0 && C > 0 && ld_a >= C && ld_b >= C && ld_out >= C, INSC_ERR_ARG, "insc_add: bad sizes");
   INSC_REQUIRE(n_rows == 0 || (d_a && d_b && d_out), INSC_ERR_ARG, "insc_add: null pointer");
   return launch_add(d_a, ld_a, d_b, ld_b, d_out, ld_out, d_rows, d_n_rows, n_rows, C, nullptr, (hipStream_t)stream);
+}
+
+int insc_coords4(const void *d_coords, int bits, int cols, int64_t ld, int64_t P, int32_t *d_out4, int32_t *bad, void *stream) {
+  INSC_REQUIRE((bits == 32 || bits == 64) && (cols == 3 || cols == 4) && ld >= cols && P >= 0, INSC_ERR_ARG,
+               "insc_coords4: rows of 3 or 4 integers of 32 or 64 bits");
+  INSC_REQUIRE(P == 0 || (d_coords && d_out4 && ((uintptr_t)d_out4 & 15) == 0), INSC_ERR_ARG,
+               "insc_coords4: null pointer, or output rows that are not 16-byte aligned");
+  if (P == 0) return INSC_OK;
+  hipStream_t s = (hipStream_t)stream;
+  if (bits == 64)
+    hipLaunchKernelGGL(coords4_kernel<int64_t>, dim3(grid_for(P, 256)), dim3(256), 0, s, (const int64_t *)d_coords, cols, ld, P,
+                       d_out4, bad);
+  else
+    hipLaunchKernelGGL(coords4_kernel<int32_t>, dim3(grid_for(P, 256)), dim3(256), 0, s, (const int32_t *)d_coords, cols, ld, P,
+                       d_out4, bad);
+  INSC_LAUNCH_CHECK();
+  return INSC_OK;
 }
 
 int insc_copy_rows(const float *d_in, int64_t ld_in, float *d_out, int64_t ld_out, const int32_t *d_rows,

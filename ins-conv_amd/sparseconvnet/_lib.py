@@ -49,6 +49,7 @@ _SIGS = {
     "insc_deconv_down2": [vp, c_i64, c_i64, vp, c_i64, vp, vp, vp, vp, vp, vp, vp, c_i64, c_int, c_int, vp],
     "insc_bn_leaky": [vp, c_i64, vp, c_i64, vp, vp, vp, vp, c_f32, c_f32, vp, vp, c_i64, c_int, vp],
     "insc_add": [vp, c_i64, vp, c_i64, vp, c_i64, vp, vp, c_i64, c_int, vp],
+    "insc_coords4": [vp, c_int, c_int, c_i64, c_i64, vp, vp, vp],
     "insc_copy_rows": [vp, c_i64, vp, c_i64, vp, vp, c_i64, c_int, vp],
     "insc_input_accumulate": [vp, c_i64, c_int, vp, c_int, vp, vp, c_i64, vp],
     "insc_input_finish": [vp, vp, c_int, vp, c_i64, vp, vp, c_i64, c_int, vp],

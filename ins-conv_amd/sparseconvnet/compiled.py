@@ -179,9 +179,7 @@ class CompiledNet(object):
         """int32 on the device.  The reference's callers pass int64 coordinates, on the host
         (ioLayers.py:52-69 converts to a CPU LongTensor) or on the GPU (demo.py:20): narrowed on
         the side where they are, so that the host-to-device copy carries half the bytes."""
-        if coords.dtype != torch.int32:
-            coords = coords.to(torch.int32)
-        return coords.to(self.device).contiguous()
+        return SCN.to_device(coords, self.device).to(torch.int32).contiguous()
 
     def _changed(self):
         """Whether a parameter moved or changed since the weights were packed.  Looked at AFTER a
