@@ -190,6 +190,7 @@ def ptr(t):
 
 
 def stream_ptr():
-    import torch
+    from torch import _C
 
-    return torch.cuda.current_stream().cuda_stream
+    # (the current stream's handle without a Stream object around it: under 1 us a call instead of some 4)
+    return _C._cuda_getCurrentRawStream(_C._cuda_getDevice())
