@@ -139,17 +139,21 @@ __device__ __forceinline__ uint64_t order_key(int4 c, uint32_t m) {
 }
 // The neighbour pattern (bit k: neighbour k exists) of site v0 + lane, 0 beyond `count` sites; a wavefront's 64 rows of the map
 // are read side by side, 27 loads of 256 bytes, and the bits sorted out in LDS (28 words of its own).  With every lane at a row
-// of its own, 108 bytes apart, each load takes the address unit some 54 lines instead of three: 200k sites 5.5 us, 3.4 so.
+// of its own, 108 bytes apart, each load takes the address unit some 54 lines instead of three, which is what a kernel of one
+// or a few workgroups waits for (6000 sites in one workgroup: 65 us, 39 so).  Over the whole chip it does not pay (200k
+// sites 5.5 us, 7.1 so): the key kernels of rulebook.hip, which fill it, read their own rows.
 __device__ __forceinline__ uint32_t pattern_of_site(const int32_t *__restrict__ nbr, int64_t v0, int count, uint64_t *bits) {
   const int lane = threadIdx.x & 63;
+  if (count <= 0) return 0u;  // (the same for every lane)
   const int32_t *row = nbr + v0 * 27;
+  const int last = count * 27 - 1;
   int id[27];
 #pragma unroll
-  for (int i = 0; i < 27; i++) id[i] = i * 64 + lane < count * 27 ? row[i * 64 + lane] : -1;
+  for (int i = 0; i < 27; i++) id[i] = row[min(i * 64 + lane, last)];  // (no load under a branch: each would be waited for)
   uint64_t mine = 0;
 #pragma unroll
   for (int i = 0; i < 27; i++) {
-    const uint64_t have = __ballot(id[i] >= 0);
+    const uint64_t have = __ballot(id[i] >= 0 && i * 64 + lane <= last);
     mine = lane == i ? have : mine;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // (the words of the 64 sites before have been read)

@@ -1165,7 +1165,7 @@ __global__ __launch_bounds__(1024) void order_append_both_batch_kernel(OrderBoth
 // places of its words among all (the runs before it and the smaller words of the others, counted by binary searches in
 // LDS), one per scale groups them by offset.  By one workgroup 6000 sites took 70 us, 65 of them on the address unit of
 // its one compute unit (27 map entries of every site, a line each); read a site's entries side by side 44; in
-// three launches 19.
+// three launches 31 (10, 10 and 11).
 constexpr int ORDER_RUN = 1024;
 __global__ __launch_bounds__(ORDER_RUN) void order_runs_kernel(OrderBothBatch b, uint64_t *__restrict__ words) {
   __shared__ uint64_t key[2][ORDER_RUN];

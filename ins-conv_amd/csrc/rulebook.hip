@@ -40,13 +40,12 @@ __global__ void pairs_write_kernel(const int32_t *__restrict__ nbr, int64_t N, i
 // which costs some locality and nothing else.
 __global__ void order_key_kernel(const int32_t *__restrict__ coords, const int32_t *__restrict__ nbr, int64_t first,
                                  int64_t n, uint64_t *__restrict__ keys, int32_t *__restrict__ vals) {
-  __shared__ uint64_t bits[4][28];
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, t0 = t - (threadIdx.x & 63);
-  if (t0 >= n) return;  // (the whole wavefront)
-  const int64_t i = first + t;
-  const uint32_t m = pattern_of_site(nbr, first + t0, (int)min((int64_t)64, n - t0), bits[threadIdx.x >> 6]);
+  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  const int4 c = reinterpret_cast<const int4 *>(coords)[i];
+  const int64_t i = first + t;
+  int4 c = reinterpret_cast<const int4 *>(coords)[i];
+  uint32_t m = 0;
+  for (int k = 0; k < 27; k++) m |= (nbr[i * 27 + k] >= 0 ? 1u : 0u) << k;
   keys[t] = order_key(c, m);
   vals[t] = (int)i;
 }
@@ -72,12 +71,11 @@ struct OrderBuildBatchDev {
 };
 __global__ void order_key_batch_kernel(OrderBuildBatchDev b) {
   const OrderBuildJobDev &j = b.job[blockIdx.y];
-  __shared__ uint64_t bits[4][28];
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, t0 = t - (threadIdx.x & 63);
-  if (t0 >= j.n) return;  // (the whole wavefront)
-  const uint32_t m = pattern_of_site(j.nbr, t0, (int)min((int64_t)64, j.n - t0), bits[threadIdx.x >> 6]);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= j.n) return;
   const int4 c = reinterpret_cast<const int4 *>(j.coords)[t];
+  uint32_t m = 0;
+  for (int k = 0; k < 27; k++) m |= (j.nbr[t * 27 + k] >= 0 ? 1u : 0u) << k;
   j.keys[t] = order_key(c, m);
   j.vals[t] = (int)t;
 }
@@ -259,7 +257,7 @@ int insc_order_build(const insc_grid *g, const int32_t *d_nbr, int64_t first, in
   INSC_REQUIRE(n == 0 || (d_nbr && d_order), INSC_ERR_ARG, "insc_order_build: null pointer");
   if (n == 0) return INSC_OK;
   hipStream_t s = (hipStream_t)stream;
-  // (a scan's scales of 1k and 4k sites: 48 and 57 us of radix passes in eleven launches, 9 and 14 in one and two)
+  // (a scan's scales of 1k and 4k sites: 48 and 57 us of radix passes in eleven launches, 15 and 16 in one and two)
   if (n <= order_sorted_max()) return order_sites(g, d_nbr, first, n, d_order, s);
   void *ws;
   int rc = workspace(WS_API, s, (sizeof(uint64_t) + sizeof(int32_t)) * (size_t)n, &ws);
