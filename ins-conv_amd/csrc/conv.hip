@@ -575,6 +575,16 @@ __device__ __forceinline__ void add_plain_products(f16v &sums, const Ids &id_of,
   }
 }
 
+// The first six 64-byte lines of the kernel's arguments, asked for at once and waited for once.  They are in no cache when a
+// launch begins, and the compiler loads them where they are used: a trip to memory per line, one after the other.  (U-Net of
+// 16 channels on 6k voxels 577 -> 567 us, of 32 on 150k 2170 -> 2130.  The kernels whose blocks stay for many tiles gain
+// nothing.)
+__device__ __forceinline__ void request_six_lines_of_arguments() {
+  const __attribute__((address_space(4))) uint32_t *a =
+      (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" ::"s"(a[0]), "s"(a[16]), "s"(a[32]), "s"(a[48]), "s"(a[64]), "s"(a[80]));
+}
+
 // The rows of a tile: residual sum, the raw rows, the batch norm's rows - whole passes over the sixteen rows of a lane, so
 // that nothing branches per row.  Rows that do not exist (my_row < 0) go out of range.
 __device__ __forceinline__ void element_offsets(int my_row, uint32_t ld4, uint32_t (&off)[16]) {
@@ -655,9 +665,11 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep,
     float *__restrict__ part, int32_t *__restrict__ pcount, TilePlan plan) {
   constexpr int WAVES = S == 1 ? CONV_WAVES : S;
-  __shared__ int nbl[S == 1 ? WAVES : 1][TILE_M * K];
+  constexpr int NSTAGE = (TILE_M * K + 64 * S - 1) / (64 * S);
+  __shared__ int nbl[S == 1 ? WAVES : 1][NSTAGE * 64 * S];  // (whole passes: the last one's store needs no condition)
   __shared__ float red[S > 1 ? S : 1][S > 1 ? NB * 16 * 64 : 1];  // (slot S - 1: only when all wavefronts share the tail)
   __shared__ unsigned wmask[S];
+  request_six_lines_of_arguments();  // (they take 360 bytes)
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   // (the wavefront's number as a scalar: the item cursor below then runs on the scalar unit)
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
@@ -709,78 +721,115 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
 
   // blocks beyond the row count leave at once (launches are sized by an upper bound of it)
   if ((S == 1 ? (int64_t)bx * WAVES : (int64_t)bx) * TILE_M >= n) return;
-  // a tile is skipped when it lies beyond the row count or, with tile flags, is not marked
-  const bool live = t0 < n && (!tile_flags || tile_flags[t0 >> 5]);
-  int my_row = -1;
-  if (live && t0 + r < n) my_row = rows ? rows[t0 + r] : (int)(t0 + r);
-  // (residual-frame batch norm in the epilogue: the saved row of this lane's row, asked for here so
-  // that the main loop hides the load)
-  int my_pe = -1;
-  if (S > 1 && ep.pre_exist && my_row >= 0) my_pe = ep.pre_exist[my_row];
-
-  // (a row of a deconvolution has one input row, at one offset)
-  int my_offset = -1, my_parent = -1;
-  if (MODE == MAP_PARENT && my_row >= 0) {
-    my_offset = map1[my_row];
-    my_parent = map0[my_row];
+  // a tile is skipped when it lies beyond the row count or, with tile flags, is not marked: the whole block (S > 1) or one
+  // wavefront, and barriers are among the wavefronts of one tile only
+  if (t0 >= n || (tile_flags && !tile_flags[t0 >> 5])) return;
+  // Up to the first gather a small launch does little but wait for memory that no cache holds yet, so nothing here loads
+  // under a condition of its own (each such load would be waited for before the next) and what needs no map goes first:
+  // the bias and the per-channel scale / shift of the fused batch norms, zero beyond Cout.  Then the row ids, the tile's
+  // slice of the neighbour map and its offsets in one trip.  (3^3 layers of 16, 32 and 48 channels at 6k, 1.5k and 400
+  // sites 12.3 -> 10.7, 13.7 -> 12.2 and 19.1 -> 17.3 us, with the arguments asked for at once.)
+  float bias_of[NB], ew[NB], eb[NB], sw[NB], sb[NB];
+  {
+    const uint32_t width = (uint32_t)Cout * 4u;
+    const bool side = MODE == MAP_PARENT && ep.side_in;
+    const __amdgpu_buffer_rsrc_t rbias = make_rsrc(bias, bias && (S == 1 || ws == 0) ? width : 0u),
+                                 rew = make_rsrc(ep.w, ep.out2 ? width : 0u), reb = make_rsrc(ep.b, ep.out2 ? width : 0u),
+                                 rsw = make_rsrc(ep.side_w, side ? width : 0u), rsb = make_rsrc(ep.side_b, side ? width : 0u);
+    auto at = [&](__amdgpu_buffer_rsrc_t from, int b) {
+      return __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b32(from, ((cb0 + b) * 32 + r) * 4, 0, 0));
+    };
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      bias_of[b] = at(rbias, b);
+      ew[b] = at(rew, b);
+      eb[b] = at(reb, b);
+      sw[b] = sb[b] = 0.0f;
+      if (MODE == MAP_PARENT) {
+        sw[b] = at(rsw, b);
+        sb[b] = at(rsb, b);
+      }
+    }
   }
+  const bool in_range = t0 + r < n;
+  int listed = (int)min(t0 + r, n - 1), my_row;
+  if (rows) listed = rows[listed];
 
-  // stage the tile's slice of the neighbour map in LDS and find the offsets it uses; all the
-  // loads are issued before the first one is consumed.  With a tile plan (the map transposed into
-  // processing order, one 128-byte run per (offset, tile), and the offsets of every tile) the
-  // loads are coalesced, need no row id and the LDS copy is offset-major.
+  // Stage the tile's slice of the neighbour map in LDS and find the offsets it uses.  With a tile plan (the map transposed
+  // into processing order, one 128-byte run per (offset, tile), and the offsets of every tile) the loads are coalesced, need
+  // no row id and the LDS copy is offset-major.
   const bool planned = MODE == MAP_NBR && K == 27 && plan.map != nullptr;
   int *nl = nbl[S == 1 ? wave : 0];
   unsigned mymask = 0;
-  constexpr int NSTAGE = (TILE_M * K + 64 * S - 1) / (64 * S);
   int staged[NSTAGE];
   if (planned) {
+    // (the launch checked that 32-bit offsets reach all of the plan; entries beyond the 27th offset are out of range)
+    const uint32_t pld4 = (uint32_t)plan.ld * 4u;
+    const __amdgpu_buffer_rsrc_t rplan = make_rsrc(plan.map, 27u * pld4);
+    const uint32_t first = (uint32_t)t0 * 4u + (uint32_t)r * 4u + (uint32_t)h * pld4;
+    mymask = plan.tmask[t0 >> 5];
 #pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;  // e = k * 32 + row
-      staged[i] = (live && e < TILE_M * K) ? plan.map[(int64_t)(e >> 5) * plan.ld + t0 + (e & 31)] : -1;
-    }
-    if (live) mymask = plan.tmask[t0 >> 5];
+    for (int i = 0; i < NSTAGE; i++)  // entry e = k * 32 + row, e = (i * S + wave) * 64 + lane
+      staged[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rplan, (int)(first + (uint32_t)((S == 1 ? i : i * S + wave) * 2) * pld4), 0, 0);
+    asm volatile("" : "+v"(listed));  // (not waited for until the map is on its way)
+    my_row = in_range ? listed : -1;
 #pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
-      if (e < TILE_M * K) nl[e] = staged[i];
-    }
+    for (int i = 0; i < NSTAGE; i++) nl[(S == 1 ? i : i * S + wave) * 64 + lane] = staged[i];
   } else {
-#pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
-      const int rr = e / K, kk = e - rr * K;
-      const int rid = __shfl(my_row, rr & (TILE_M - 1), 64);
-      int v = -1;
-      const int offset_of = __shfl(my_offset, rr & (TILE_M - 1), 64), parent_of = __shfl(my_parent, rr & (TILE_M - 1), 64);
-      if (e < TILE_M * K && rid >= 0) {
-        if (MODE == MAP_NBR)
-          v = map0[(int64_t)rid * K + kk];
-        else if (MODE == MAP_IDENTITY)
-          v = rid;
-        else
-          v = offset_of == kk ? parent_of : -1;
-      }
-      staged[i] = v;
+    my_row = in_range ? listed : -1;
+    // (rows that do not exist read the map of one that does)
+    const int some_row = max(__builtin_amdgcn_readfirstlane(my_row), 0);
+    // (a row of a deconvolution has one input row, at one offset)
+    int my_offset = -1, my_parent = -1;
+    if (MODE == MAP_PARENT) {
+      my_offset = map1[my_row < 0 ? some_row : my_row];
+      my_parent = map0[my_row < 0 ? some_row : my_row];
     }
 #pragma unroll
     for (int i = 0; i < NSTAGE; i++) {
       const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
-      if (e < TILE_M * K) {
-        nl[e] = staged[i];
-        if (staged[i] >= 0) mymask |= 1u << (e % K);
+      const int rr = (e / K) & (TILE_M - 1), kk = e - (e / K) * K;
+      const int rid = __shfl(my_row, rr, 64);
+      if (MODE == MAP_NBR) {
+        const int v = map0[(int64_t)(rid < 0 ? some_row : rid) * K + kk];
+        staged[i] = rid < 0 || e >= TILE_M * K ? -1 : v;
+      } else if (MODE == MAP_IDENTITY) {
+        staged[i] = e < TILE_M * K ? rid : -1;
+      } else {
+        const int offset_of = __shfl(my_offset, rr, 64), parent_of = __shfl(my_parent, rr, 64);
+        staged[i] = rid >= 0 && offset_of == kk ? parent_of : -1;
       }
     }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) mymask |= (unsigned)__shfl_xor((int)mymask, d, 64);
+    for (int i = 0; i < NSTAGE; i++) {
+      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
+      nl[e] = staged[i];
+      mymask |= (staged[i] >= 0 ? 1u : 0u) << (e % K);
+    }
+    if constexpr (64 % K == 0) {
+      // (every entry of a lane is at the same offset)
+      uint64_t some = __ballot(mymask != 0);
+#pragma unroll
+      for (int d = 32; d >= K; d >>= 1) some |= some >> d;
+      mymask = (unsigned)some & ((1u << K) - 1u);
+    } else {
+#pragma unroll
+      for (int d = 32; d > 0; d >>= 1) mymask |= (unsigned)__shfl_xor((int)mymask, d, 64);
+    }
+    if (S > 1 && lane == 0) wmask[wave] = mymask;
   }
-  if (S > 1 && lane == 0) wmask[wave] = mymask;
-  __syncthreads();
-  if (!live) return;  // the whole block (S > 1) or wavefront (S == 1) is idle; no barrier follows
+  if (S > 1) {
+    __syncthreads();
+  } else {
+    // (a wavefront's own entries)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
   // Split launches: what the tail of this wavefront will read besides the sums - the other operand of a
   // folded element-wise sum, the saved rows of a residual frame's batch norm - is asked for here, for
-  // the rows the wavefront finishes, so that the main loop hides these loads.
+  // the rows the wavefront finishes, so that the main loop hides these loads.  (Rows and columns that do
+  // not exist get the values of ones that do, and are not written.)
   constexpr int NVP = S > 1 ? 16 / S : 1;
   float pre_res[NB][NVP], pre_pin[NVP], pre_pout[NVP];
   int pre_pe[NVP];
@@ -788,15 +837,36 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     const int c = cb0 * 32 + r;
 #pragma unroll
     for (int j = 0; j < NVP; j++) {
-      const int v = wave * NVP + j, src_lane = 8 * (v >> 2) + 4 * h + (v & 3);
-      const int row = __shfl(my_row, src_lane, 64);
-      pre_pe[j] = __shfl(my_pe, src_lane, 64);
+      pre_pe[j] = -1;
+      pre_pin[j] = pre_pout[j] = 0.0f;
 #pragma unroll
-      for (int b = 0; b < NB; b++)
-        pre_res[b][j] = (ep.res && row >= 0 && c + b * 32 < Cout) ? ep.res[(int64_t)row * ep.ldr + c + b * 32] : 0.0f;
-      const bool sv = pre_pe[j] >= 0 && c < Cout;
-      pre_pin[j] = sv ? ep.pre_in[(int64_t)pre_pe[j] * ep.ld_pin + c] : 0.0f;
-      pre_pout[j] = sv ? ep.pre_out[(int64_t)pre_pe[j] * ep.ld_pout + c] : 0.0f;
+      for (int b = 0; b < NB; b++) pre_res[b][j] = 0.0f;
+    }
+    if (ep.res) {
+#pragma unroll
+      for (int j = 0; j < NVP; j++) {
+        const int v = wave * NVP + j, row = __shfl(my_row, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+#pragma unroll
+        for (int b = 0; b < NB; b++) pre_res[b][j] = ep.res[(int64_t)max(row, 0) * ep.ldr + min(c + b * 32, Cout - 1)];
+      }
+    }
+    if (MODE == MAP_NBR && K == 27 && ep.pre_exist) {
+      const int pe = ep.pre_exist[max(my_row, 0)], my_pe = my_row < 0 ? -1 : pe;
+#pragma unroll
+      for (int j = 0; j < NVP; j++) {
+        const int v = wave * NVP + j;
+        pre_pe[j] = __shfl(my_pe, 8 * (v >> 2) + 4 * h + (v & 3), 64);
+      }
+      const uint64_t saved = __ballot(my_pe >= 0);
+      if (saved) {  // (the saved matrices may have no rows at all)
+        const int some_saved = __builtin_amdgcn_readlane(my_pe, __builtin_ctzll(saved)), cc = min(c, Cout - 1);
+#pragma unroll
+        for (int j = 0; j < NVP; j++) {
+          const int64_t row = pre_pe[j] < 0 ? some_saved : pre_pe[j];
+          pre_pin[j] = ep.pre_in[row * ep.ld_pin + cc];
+          pre_pout[j] = ep.pre_out[row * ep.ld_pout + cc];
+        }
+      }
     }
   }
   // Offsets some row of the tile uses.  With S wavefronts per tile, the (offset k, chunk ch)
@@ -809,19 +879,24 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     rest = (unsigned)__builtin_amdgcn_readfirstlane((int)mymask);
     nitems = __builtin_popcount(rest) * nch;
   } else {
-    unsigned act = 0;
+    unsigned act = mymask;
+    if (!planned) {
 #pragma unroll
-    for (int w = 0; w < S; w++) act |= wmask[w];
+      for (int w = 0; w < S; w++) act |= wmask[w];
+    }
     act = (unsigned)__builtin_amdgcn_readfirstlane((int)act);
-    // (lane k looks at offset k: one ballot and a sum over the lanes instead of a scalar loop over the offsets)
+    // (lane k looks at offset k: ballots instead of a scalar loop over the offsets; an offset holds nch / ST items of this
+    // wavefront, one more where c0 is below the remainder)
     // (two wavefronts: a narrow layer's two partial sums)
     const int c0 = S == 2 ? ((ws ^ lane) & 1) * nch : (ws - lane * nch) & (ST - 1);
     const bool has = lane < K && ((act >> (lane & 31)) & 1u) && c0 < nch;
     rest = (unsigned)__ballot(has);
-    int cnt = !has ? 0 : S == 2 ? nch : (nch - c0 + ST - 1) >> __builtin_ctz(ST);
-#pragma unroll
-    for (int d = 16; d > 0; d >>= 1) cnt += __shfl_xor(cnt, d, 64);
-    nitems = __builtin_amdgcn_readfirstlane(cnt);
+    if (S == 2) {
+      nitems = __builtin_popcount(rest) * nch;
+    } else {
+      const unsigned more = (unsigned)__ballot(has && c0 < (nch & (ST - 1)));
+      nitems = __builtin_popcount(act) * (nch >> __builtin_ctz(ST)) + __builtin_popcount(more);
+    }
   }
 
   // (one wavefront, several partial sums: the running one and the sum of the finished ones)
@@ -830,24 +905,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
   f16v total[SEQ ? NB : 1];
   int cur = 0;  // the partial sum in sums
 #pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const int c = (cb0 + b) * 32 + r;
-    sum_start(sums[b], (bias && c < Cout && (S == 1 || ws == 0)) ? bias[c] : 0.0f);
-  }
-
-  // per-channel scale / shift of the fused batch norm for this lane's columns (loaded here so
-  // that the latency is hidden behind the main loop)
-  float ew[NB], eb[NB], sw[NB], sb[NB];
-#pragma unroll
-  for (int b = 0; b < NB; b++) {
-    const int c = (cb0 + b) * 32 + r;
-    const bool on = ep.out2 && c < Cout;
-    ew[b] = on ? ep.w[c] : 0.0f;
-    eb[b] = on ? ep.b[c] : 0.0f;
-    const bool son = MODE == MAP_PARENT && ep.side_in && c < Cout;
-    sw[b] = son ? ep.side_w[c] : 0.0f;
-    sb[b] = son ? ep.side_b[c] : 0.0f;
-  }
+  for (int b = 0; b < NB; b++) sum_start(sums[b], bias_of[b]);
 
   if (rest) {
     // Work items of this tile: (active offset k, 32-channel chunk ch), offsets ascending, chunks
@@ -975,6 +1033,9 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
       for (int v = 0; v < 16; v++) acc[b][v] = total[b][v] + acc[b][v];
     }
   }
+  // (rows whose byte offsets fit 32 bits, through 24-bit multiplies, in every matrix that is written or added)
+  const int64_t widest = 4 * max(max(ld_out, ep.ld2), max(ep.ldr, ep.ld_side));
+  const bool fits = widest < (1 << 24) && __all(my_row < (1 << 24) && (int64_t)my_row * widest < (int64_t)ROWS_REACH);
   if (S == 1) {
     // (one block at a time: copies of all blocks' repeated sums would cost NB = 3 its second wavefront per SIMD, 32 -> 96 at
     // 200k sites 99 -> 124 us)
@@ -1133,6 +1194,26 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
       }
       continue;
     }
+    if (!(MODE == MAP_PARENT && ep.side_in) && fits) {
+      const uint32_t c4 = (uint32_t)c * 4u;
+      if (out) {
+        const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, BUF_OOB);
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(a[b][j]), rout,
+                                                (int)(rid[j] < 0 ? BUF_OOB : __umul24((unsigned)rid[j], (uint32_t)ld_out * 4u) + c4), 0, 0);
+      }
+      if (ep.out2) {
+        const __amdgpu_buffer_rsrc_t rout2 = make_rsrc(ep.out2, BUF_OOB);
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+          const float y = fmaf(a[b][j], ew[b], eb[b]);  // fused batch norm + leaky ReLU
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y * ((y > 0.0f) ? 1.0f : ep.leak)), rout2,
+                                                (int)(rid[j] < 0 ? BUF_OOB : __umul24((unsigned)rid[j], (uint32_t)ep.ld2 * 4u) + c4), 0, 0);
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int j = 0; j < NV; j++) {
       if (rid[j] < 0) continue;
@@ -1150,13 +1231,11 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     return;
   }
 
-  // Rows that 32-bit offsets reach go out in whole passes without a branch per row: with one, the 16 stores of every matrix
+  // Such rows go out in whole passes without a branch per row: with one, the 16 stores of every matrix
   // and block, and the loads of a joined matrix's other half, went one by one.  A deconvolution's map (two words a row) is
   // loaded once and handed round for the same reason, not 8 times under a condition.  Deconvolutions of 6k, 37k and 150k
   // sites to one block of columns 15.9 -> 7.5, 17.6 -> 8.9 and 54 -> 29 us, of 1k sites to two 20.9 -> 11.9.
   {
-    const int64_t widest = 4 * max(max(ld_out, ep.ld2), max(ep.ldr, ep.ld_side));
-    const bool fits = widest < (1 << 24) && __all(my_row < (1 << 24) && (int64_t)my_row * widest < (int64_t)ROWS_REACH);
     if (__builtin_expect(fits, 1)) {
       const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u),
                                    rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
