@@ -19,6 +19,12 @@ def test_sort_edges(S, n):
     primitives.test_sort_stable(S, n, 16)
 
 
+# frames of 256, second ones of 320, 1024, 1025 and 16383 points: rounds of 1024 rows, up to the last workgroup that ranks alone
+@pytest.mark.parametrize("P", [256, 820, 821, 13107])
+def test_frame_edges(S, P):
+    primitives.test_insert_at_all_scales_equals_the_scale_by_scale_chain(S, P)
+
+
 # one tile and less, a last group of one to four, a block of positions, more tiles than one round of the schedule (8 x 1024)
 @pytest.mark.parametrize("n,listed", [(1, False), (31, True), (33, False), (129, True), (256, False), (257, True), (2049 * 32, True),
                                       (8193 * 32 + 5, False)])
