@@ -785,36 +785,59 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
       my_offset = map1[my_row < 0 ? some_row : my_row];
       my_parent = map0[my_row < 0 ? some_row : my_row];
     }
+    if constexpr (MODE == MAP_NBR && K == 27) {
+      // A lane stays with one offset, half a wavefront with a row: the row ids come from their lanes through the scalar
+      // unit, and the offsets in use are what the ballots of all rows have in common, without a reduction over the lanes.
+      constexpr int PAIRS_OF_ROWS = TILE_M / (2 * S);
+      const int kk = min(r, K - 1);
+      int v[PAIRS_OF_ROWS];
 #pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
-      const int rr = (e / K) & (TILE_M - 1), kk = e - (e / K) * K;
-      const int rid = __shfl(my_row, rr, 64);
-      if (MODE == MAP_NBR) {
-        const int v = map0[(int64_t)(rid < 0 ? some_row : rid) * K + kk];
-        staged[i] = rid < 0 || e >= TILE_M * K ? -1 : v;
-      } else if (MODE == MAP_IDENTITY) {
-        staged[i] = e < TILE_M * K ? rid : -1;
-      } else {
-        const int offset_of = __shfl(my_offset, rr, 64), parent_of = __shfl(my_parent, rr, 64);
-        staged[i] = rid >= 0 && offset_of == kk ? parent_of : -1;
+      for (int i = 0; i < PAIRS_OF_ROWS; i++) {
+        const int rr = (S == 1 ? i : i * S + wave) * 2;
+        const int ra = __builtin_amdgcn_readlane(my_row, rr), rb = __builtin_amdgcn_readlane(my_row, rr + 1), rid = h ? rb : ra;
+        v[i] = map0[(int64_t)(rid < 0 ? some_row : rid) * K + kk];
       }
-    }
+      uint64_t used = 0;
 #pragma unroll
-    for (int i = 0; i < NSTAGE; i++) {
-      const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
-      nl[e] = staged[i];
-      mymask |= (staged[i] >= 0 ? 1u : 0u) << (e % K);
-    }
-    if constexpr (64 % K == 0) {
+      for (int i = 0; i < PAIRS_OF_ROWS; i++) {
+        const int rr = (S == 1 ? i : i * S + wave) * 2;
+        const int ra = __builtin_amdgcn_readlane(my_row, rr), rb = __builtin_amdgcn_readlane(my_row, rr + 1);
+        if ((h ? rb : ra) < 0) v[i] = -1;
+        used |= __ballot(v[i] >= 0);
+      }
+      mymask = (unsigned)(used | used >> 32) & 0x7FFFFFFu;
+      if (r < K) {
+#pragma unroll
+        for (int i = 0; i < PAIRS_OF_ROWS; i++) nl[((S == 1 ? i : i * S + wave) * 2 + h) * K + r] = v[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NSTAGE; i++) {
+        const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
+        const int rr = (e / K) & (TILE_M - 1), kk = e - (e / K) * K;
+        const int rid = __shfl(my_row, rr, 64);
+        if (MODE == MAP_NBR) {
+          const int v = map0[(int64_t)(rid < 0 ? some_row : rid) * K + kk];
+          staged[i] = rid < 0 || e >= TILE_M * K ? -1 : v;
+        } else if (MODE == MAP_IDENTITY) {
+          staged[i] = e < TILE_M * K ? rid : -1;
+        } else {
+          const int offset_of = __shfl(my_offset, rr, 64), parent_of = __shfl(my_parent, rr, 64);
+          staged[i] = rid >= 0 && offset_of == kk ? parent_of : -1;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NSTAGE; i++) {
+        const int e = (S == 1 ? i : i * S + wave) * 64 + lane;
+        nl[e] = staged[i];
+        mymask |= (staged[i] >= 0 ? 1u : 0u) << (e % K);
+      }
       // (every entry of a lane is at the same offset)
+      static_assert((MODE == MAP_NBR && K == 27) || 64 % K == 0, "");
       uint64_t some = __ballot(mymask != 0);
 #pragma unroll
       for (int d = 32; d >= K; d >>= 1) some |= some >> d;
       mymask = (unsigned)some & ((1u << K) - 1u);
-    } else {
-#pragma unroll
-      for (int d = 32; d > 0; d >>= 1) mymask |= (unsigned)__shfl_xor((int)mymask, d, 64);
     }
     if (S > 1 && lane == 0) wmask[wave] = mymask;
   }
