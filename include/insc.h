@@ -229,8 +229,8 @@ int insc_conv_ssc_plan(const float *d_in, int64_t ld_in, int64_t n_in_rows, floa
                        void *stream);
 /* Launch policy of a 3^3 layer of 64..159 input channels with a tile schedule: by default one block per
  * (tile, 32-column output block) pair; with at least `units` (four consecutive tiles, output block) pairs
- * (default 896) the kernel whose blocks share the weight tiles through LDS.  Same bits in all cases: tuning and
- * test knobs with no counterpart in the reference.  (The persistent-block kernel that the first one chose was slower
+ * (default 1100, and at most two output blocks) the kernel whose blocks share the weight tiles through LDS.  Same bits in
+ * all cases: tuning and test knobs with no counterpart in the reference.  (The persistent-block kernel that the first one chose was slower
  * at every size and is gone; the call is accepted and changes nothing.) */
 int insc_conv_set_persistent_min_units(int64_t units);
 int insc_conv_set_shared_weights_min_units(int64_t units);
