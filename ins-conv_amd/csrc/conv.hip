@@ -76,10 +76,14 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(const float *__restri
 // back from LDS by the threads of the row (one 16-byte broadcast read per offset): with every thread
 // fetching its row's 27 ids and 81 values itself the kernel was bound by the number of load instructions
 // (92 us for 150k rows and 32 output channels).
+// A batch's values are two trips to memory away (three with a row list): they are asked for while the batch before is computed,
+// its ids one batch earlier still, none under a condition.  Whether a neighbour exists rides in the fourth word where the
+// input leaves it free.  (Fetched batch by batch, a word of its own in LDS: 150k rows of 3 -> 32 channels 58.8 us, 42.5 so.)
+// Four wavefronts a SIMD with one pair a thread; with two pairs 128 registers would spill.
 // ---------------------------------------------------------------------------------------
 constexpr int STEM_ROWS = 16;  // rows per batch at most (those of 256 / Cout rows that a block handles at a time)
-template <int CIN>
-__global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict__ in, int64_t ld_in,
+template <int CIN, int NE>
+__global__ __launch_bounds__(256, CIN < 4 && NE == 1 ? 4 : 2) void conv_stem_kernel(const float *__restrict__ in, int64_t ld_in,
                                                         float *__restrict__ out, int64_t ld_out,
                                                         const float *__restrict__ W, const float *__restrict__ bias,
                                                         const int32_t *__restrict__ map0,
@@ -89,12 +93,43 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
                                                         BnEpilogue ep) {
   constexpr int K = 27;
   __shared__ float4 xs[2][STEM_ROWS][K];  // input values of (row, offset); two batches in turn
-  __shared__ int vs[2][STEM_ROWS][K];     // 1: the row has a neighbour at the offset
+  __shared__ int vs[CIN == 4 ? 2 : 1][CIN == 4 ? STEM_ROWS : 1][K];  // 1: the row has a neighbour there (CIN < 4: xs[..].w)
   __shared__ int rid[2][STEM_ROWS];       // row of the batch, -1: none
   const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
   const int cpb = min(256 / Cout, STEM_ROWS);  // rows per batch (Cout <= 256)
   const int lr = threadIdx.x / Cout, co = threadIdx.x % Cout;
   const bool worker = lr < cpb;
+  const int64_t step = (int64_t)gridDim.x * cpb;
+  if ((int64_t)blockIdx.x * cpb >= n) return;  // (the whole block)
+
+  // fetch: NE (row, offset) pairs per thread, two where a batch has more than 256 of them
+  int row_of[NE], src_of[NE];
+  float x_of[NE][CIN];
+  bool have[NE];
+  auto load_ids = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      const int e = (int)threadIdx.x + i * 256, er = e / K, k = e - er * K;
+      const int64_t t = t0 + er, tc = min(t, n - 1);
+      const int r = rows ? rows[tc] : (int)tc;
+      const bool on = t < n && r >= 0 && (!row_mask || row_mask[max(r, 0)]);
+      const int src = map0[(int64_t)(on ? r : 0) * K + k];
+      row_of[i] = on ? r : -1;
+      src_of[i] = on ? src : -1;
+    }
+  };
+  auto gather = [&]() {
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      have[i] = src_of[i] >= 0;
+      const float *p = have[i] ? in + (int64_t)src_of[i] * ld_in : W;  // (no condition: any CIN words that exist)
+#pragma unroll
+      for (int ci = 0; ci < CIN; ci++) x_of[i][ci] = p[ci];
+    }
+  };
+
+  int64_t t0 = (int64_t)blockIdx.x * cpb;
+  load_ids(t0);
   float w[K][CIN];
 #pragma unroll
   for (int k = 0; k < K; k++)
@@ -102,26 +137,31 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
     for (int ci = 0; ci < CIN; ci++) w[k][ci] = worker ? W[((int64_t)k * CIN + ci) * Cout + co] : 0.0f;
   const float bv = (bias && worker) ? bias[co] : 0.0f;
   const float ew = (ep.out2 && worker) ? ep.w[co] : 0.0f, eb = (ep.out2 && worker) ? ep.b[co] : 0.0f;
-  int buf = 0;
-  for (int64_t t0 = (int64_t)blockIdx.x * cpb; t0 < n; t0 += (int64_t)gridDim.x * cpb, buf ^= 1) {
-    // fetch: one (row, offset) per thread
-    for (int e = threadIdx.x; e < cpb * K; e += 256) {
-      const int er = e / K, k = e - er * K;
-      const int64_t t = t0 + er;
-      int row = t < n ? (rows ? rows[t] : (int)t) : -1;
-      if (row >= 0 && row_mask && !row_mask[row]) row = -1;
-      const int src = row >= 0 ? map0[(int64_t)row * K + k] : -1;
-      float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (src >= 0) {
-        const float *p = in + (int64_t)src * ld_in;
+  gather();
+  int row_here[NE];
 #pragma unroll
-        for (int ci = 0; ci < CIN; ci++) x[ci] = p[ci];
-      }
+  for (int i = 0; i < NE; i++) row_here[i] = row_of[i];
+  load_ids(t0 + step);  // (batches past the end read the last row's ids and hold no row)
+  for (int buf = 0; t0 < n; t0 += step, buf ^= 1) {
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      const int e = (int)threadIdx.x + i * 256, er = e / K, k = e - er * K;
+      if (e >= cpb * K) break;
+      float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int ci = 0; ci < CIN; ci++) x[ci] = have[i] ? x_of[i][ci] : 0.0f;
+      if constexpr (CIN < 4) x[3] = have[i] ? 1.0f : 0.0f;
       xs[buf][er][k] = make_float4(x[0], x[1], x[2], x[3]);
-      vs[buf][er][k] = src >= 0 ? 1 : 0;
-      if (k == 0) rid[buf][er] = row;
+      if constexpr (CIN == 4) vs[buf][er][k] = have[i] ? 1 : 0;
+      if (k == 0) rid[buf][er] = row_here[i];
     }
     __syncthreads();  // (one barrier per batch: the next batch fills the other buffer)
+    // the next batch's values and the ids of the one after are in flight while this one is computed
+    gather();
+#pragma unroll
+    for (int i = 0; i < NE; i++) row_here[i] = row_of[i];
+    load_ids(t0 + 2 * step);
+    __builtin_amdgcn_sched_barrier(0);
     const int row = worker ? rid[buf][lr] : -1;
     if (row < 0) continue;
     float acc = bv;
@@ -132,7 +172,10 @@ __global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict_
       float a = acc;
 #pragma unroll
       for (int ci = 0; ci < CIN; ci++) a = fmaf(x[ci], w[k][ci], a);
-      acc = vs[buf][lr][k] ? a : acc;
+      bool there;
+      if constexpr (CIN == 4) there = vs[buf][lr][k] != 0;
+      else there = xv.w != 0.0f;
+      acc = there ? a : acc;
     }
     if (ep.res) acc += ep.res[(int64_t)row * ep.ldr + co];
     if (out) out[(int64_t)row * ld_out + co] = acc;
@@ -2694,7 +2737,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       // enough blocks to fill the machine, few enough that the weights are fetched rarely
       const dim3 sg(grid_for(n_rows, std::min(cpb, STEM_ROWS), (unsigned)device_cus() * 8));
 #define INSC_STEM(CI)                                                                                          \
-  hipLaunchKernelGGL(conv_stem_kernel<CI>, sg, dim3(256), 0, s, in, ld_in, out, ld_out, W, bias, map0, rows, \
+  hipLaunchKernelGGL((cpb > 9 ? conv_stem_kernel<CI, 2> : conv_stem_kernel<CI, 1>), sg, dim3(256), 0, s, in, ld_in, out, ld_out, W, bias, map0, rows, \
                      d_n_rows, n_rows, Cout, row_mask, ep)
       if (Cin == 1)
         INSC_STEM(1);
