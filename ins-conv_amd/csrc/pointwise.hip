@@ -320,7 +320,12 @@ int launch_input_finish(const float *d_sum, const int32_t *d_cnt, int mode, floa
   return INSC_OK;
 }
 
-// Coordinate rows of three or four columns, 32 or 64 bits wide (narrowed as a conversion does it), widened to (x, y, z, batch);
+// A coordinate that 32 bits do not hold becomes one at their end, which is as far outside every grid: cut to its low bits it
+// would pass for another voxel's.  (Not the very lowest, which marks rows that an insert skips.)
+__device__ __forceinline__ int narrowed(int64_t x) {
+  return (int)(x < INT32_MIN ? (int64_t)INT32_MIN + 1 : x > INT32_MAX ? (int64_t)INT32_MAX : x);
+}
+// Coordinate rows of three or four columns, 32 or 64 bits wide, as (x, y, z, batch) in 32 bits;
 // *bad = 1 where one lies outside 0 .. 65535 (batch 0 .. 32767).  Bound by the rows' bytes: 28 to 48 a point.
 template <class T>
 __global__ __launch_bounds__(256) void coords4_kernel(const T *__restrict__ in, int cols, int64_t ld, int64_t P,
@@ -328,7 +333,7 @@ __global__ __launch_bounds__(256) void coords4_kernel(const T *__restrict__ in, 
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= P) return;
   const T *row = in + p * ld;
-  const int4 c = make_int4((int)row[0], (int)row[1], (int)row[2], cols == 4 ? (int)row[3] : 0);
+  const int4 c = make_int4(narrowed(row[0]), narrowed(row[1]), narrowed(row[2]), cols == 4 ? narrowed(row[3]) : 0);
   reinterpret_cast<int4 *>(out4)[p] = c;
   if (bad && ((unsigned)c.x > 65535u || (unsigned)c.y > 65535u || (unsigned)c.z > 65535u || (unsigned)c.w > 32767u)) *bad = 1;
 }

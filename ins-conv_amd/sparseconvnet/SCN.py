@@ -336,12 +336,21 @@ class Metadata_3(object):
 # =========================================================================================
 def to_device(coords, device):
     """Integer coordinates on the device: those of the host narrowed to 32 bits on the way into page-locked memory, from
-    where the copy runs at the link's rate (220k points: 160 us as they are, 75 so)."""
+    where the copy runs at the link's rate (220k points: 160 us as they are, 75 so).  Values that 32 bits do not hold stay
+    out of range, as in insc_coords4; the host looks for them while the copy runs."""
     if coords.is_cuda or not coords.numel():
         return coords.to(device)
-    staged = torch.empty(coords.shape, dtype=torch.int32, pin_memory=True)
-    staged.copy_(coords)
-    return staged.to(device, non_blocking=True)
+
+    def stage(c):
+        staged = torch.empty(c.shape, dtype=torch.int32, pin_memory=True)
+        return staged.copy_(c).to(device, non_blocking=True)
+
+    out = stage(coords)
+    if coords.dtype == torch.int64:
+        lo, hi = torch.aminmax(coords)
+        if int(lo) < -1 << 31 or int(hi) >= 1 << 31:
+            out = stage(torch.where(coords < -1 << 31, (-1 << 31) + 1, coords.clamp(max=(1 << 31) - 1)))
+    return out
 
 
 def _coords4(coords, device, bad=None):

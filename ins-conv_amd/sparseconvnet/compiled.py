@@ -178,8 +178,12 @@ class CompiledNet(object):
     def _coords(self, coords):
         """int32 on the device.  The reference's callers pass int64 coordinates, on the host
         (ioLayers.py:52-69 converts to a CPU LongTensor) or on the GPU (demo.py:20): narrowed on
-        the side where they are, so that the host-to-device copy carries half the bytes."""
-        return SCN.to_device(coords, self.device).to(torch.int32).contiguous()
+        the side where they are, so that the host-to-device copy carries half the bytes.  Values
+        that 32 bits do not hold stay out of range."""
+        c = SCN.to_device(coords, self.device)
+        if c.dtype == torch.int64 and c.dim() == 2 and c.size(1) in (3, 4):
+            c = SCN._coords4(c, self.device)
+        return c.to(torch.int32).contiguous()
 
     def _changed(self):
         """Whether a parameter moved or changed since the weights were packed.  Looked at AFTER a

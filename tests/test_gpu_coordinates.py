@@ -26,14 +26,51 @@ def test_coordinate_rows(dtype, cuda):
         assert got.is_contiguous() and torch.equal(got.cpu(), want) and int(bad[0]) == 0
 
 
+# values whose low 32 bits are a coordinate among them
+@pytest.mark.parametrize("cuda", [False, True])
 @pytest.mark.parametrize("at,value,ok", [(0, -1, False), (1, 65535, True), (2, 65536, False), (3, 32767, True), (3, 32768, False),
-                                         (3, -1, False), (0, 1 << 32, True), (0, (1 << 32) - 1, False)])
-def test_coordinates_out_of_range(at, value, ok):
+                                         (3, -1, False), (0, 1 << 32, False), (0, (1 << 32) - 1, False), (1, -(1 << 40), False),
+                                         (2, (1 << 32) + 9, False), (3, 7 - (1 << 33), False), (0, -(1 << 31), False)])
+def test_coordinates_out_of_range(at, value, ok, cuda):
     from sparseconvnet import SCN as S
 
     rows = torch.zeros((700, 4), dtype=torch.int64)
-    rows[699, at] = value  # (narrowed to 32 bits first, as ever)
+    rows[699, at] = value
     bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-    S._coords4(rows, torch.device("cuda:0"), bad)
+    got = S._coords4(rows.cuda() if cuda else rows, torch.device("cuda:0"), bad)
     torch.cuda.synchronize()
     assert int(bad[0]) == (0 if ok else 1)
+    assert bool((got[:699] == 0).all()) and (not ok or int(got[699, at]) == value)
+
+
+@pytest.mark.parametrize("cuda", [False, True])
+@pytest.mark.parametrize("value", [1 << 32, 5 - (1 << 33)])
+def test_a_coordinate_beyond_32_bits_is_no_other_voxel(cuda, value):
+    import sparseconvnet as scn
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import InscError
+    from workloads.netdefs import NaiveUNet
+
+    pts = torch.tensor([[0, 0, 0], [5, 0, 0], [7, 8, 9]])
+    far = pts.clone()
+    far[2, 0] = value
+    pts, far = (pts.cuda(), far.cuda()) if cuda else (pts, far)
+    t = S.Result_3()
+    t.set(pts, torch.eye(3)[[2, 2, 2]])
+    t.set(far[2:], torch.eye(3)[:1])
+    with pytest.raises(InscError) as e:  # (by the next call that waits)
+        len(t)
+    assert e.value.code == -5
+    assert t.multiQuery(far[2:]).item() == t.multiQuery(far[2:] * 0 + 999).item()  # (no such voxel)
+    assert t.multiQuery(pts).tolist() == [2, 2, 2]
+    feats = torch.ones((3, 3), device="cuda")
+    layer = scn.InputLayer(3, 4096, mode=4)
+    with pytest.raises(InscError) as e:
+        layer([far, feats, 1])
+    assert e.value.code == -5
+    net = scn.compile(NaiveUNet(m=16, levels=2, seed=1).cuda().sparseModel, capacity_sites=4096)
+    with torch.no_grad():
+        net([pts, feats, 1], increment=False)
+        with pytest.raises(InscError) as e:
+            net([far, feats, 1], increment=True)
+    assert e.value.code == -5
