@@ -330,12 +330,13 @@ __device__ __forceinline__ int narrowed(int64_t x) {
 template <class T>
 __global__ __launch_bounds__(256) void coords4_kernel(const T *__restrict__ in, int cols, int64_t ld, int64_t P,
                                                       int32_t *__restrict__ out4, int32_t *__restrict__ bad) {
-  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P) return;
-  const T *row = in + p * ld;
-  const int4 c = make_int4(narrowed(row[0]), narrowed(row[1]), narrowed(row[2]), cols == 4 ? narrowed(row[3]) : 0);
-  reinterpret_cast<int4 *>(out4)[p] = c;
-  if (bad && ((unsigned)c.x > 65535u || (unsigned)c.y > 65535u || (unsigned)c.z > 65535u || (unsigned)c.w > 32767u)) *bad = 1;
+  // (a launch has at most 2^20 blocks)
+  for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (int64_t)gridDim.x * blockDim.x) {
+    const T *row = in + p * ld;
+    const int4 c = make_int4(narrowed(row[0]), narrowed(row[1]), narrowed(row[2]), cols == 4 ? narrowed(row[3]) : 0);
+    reinterpret_cast<int4 *>(out4)[p] = c;
+    if (bad && ((unsigned)c.x > 65535u || (unsigned)c.y > 65535u || (unsigned)c.z > 65535u || (unsigned)c.w > 32767u)) *bad = 1;
+  }
 }
 
 }  // namespace insc

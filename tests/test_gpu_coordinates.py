@@ -74,3 +74,21 @@ def test_a_coordinate_beyond_32_bits_is_no_other_voxel(cuda, value):
         with pytest.raises(InscError) as e:
             net([far, feats, 1], increment=True)
     assert e.value.code == -5
+
+
+def test_more_rows_than_threads_in_a_launch():
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
+
+    ensure_init(0)
+    P = (1 << 28) + 257
+    rows = torch.zeros((P, 3), dtype=torch.int32, device="cuda")
+    rows[-1] = torch.tensor([4, 5, 6])
+    rows[1 << 28, 1] = -3
+    out = torch.full((P, 4), -9, dtype=torch.int32, device="cuda")
+    bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    lib.insc_coords4(ptr(rows), 32, 3, S.I64(3), S.I64(P), ptr(out), ptr(bad), stream_ptr())
+    torch.cuda.synchronize()
+    assert int(bad[0]) == 1
+    assert out[-1].tolist() == [4, 5, 6, 0] and out[1 << 28].tolist() == [0, -3, 0, 0]
+    assert all(torch.equal(a[:, :3], b) and not bool(a[:, 3].any()) for a, b in zip(out.split(1 << 26), rows.split(1 << 26)))
