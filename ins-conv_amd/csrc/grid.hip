@@ -811,11 +811,19 @@ static int grid_alloc_table(insc_grid *g, int64_t capacity_sites) {
   return INSC_OK;
 }
 
+// whether s is being captured (the null stream never is)
+static int stream_captured(hipStream_t s, bool *captured) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (s != nullptr) INSC_HIP(hipStreamIsCapturing(s, &cap));
+  *captured = cap != hipStreamCaptureStatusNone;
+  return INSC_OK;
+}
+
 int grid_wait_made(const insc_grid *g, hipStream_t s) {
   if (s == nullptr || !g->made_pending.load(std::memory_order_acquire)) return INSC_OK;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  INSC_HIP(hipStreamIsCapturing(s, &cap));
-  if (cap != hipStreamCaptureStatusNone) return INSC_OK;  // (a capture cannot wait for what was queued before it)
+  bool captured;
+  const int rc = stream_captured(s, &captured);
+  if (rc || captured) return rc;  // (a capture cannot wait for what was queued before it)
   INSC_HIP(hipStreamWaitEvent(s, g->made, 0));
   return INSC_OK;
 }
@@ -891,7 +899,14 @@ static int grid_insert_launch(insc_grid *g, const int32_t *d_coords4, int64_t P,
   int32_t *total = g->flags + g->scratch_rows;  // spare int after the flags
   const bool small = P <= INSERT_ONE_MAX;
   const int64_t n_parts = g->n_slots >> PART_SHIFT;
-  if (!small && g->n_upper == 0 && g->part && n_parts >= 1 && n_parts <= PART_MAX) {  // empty: built in LDS
+  bool in_lds = !small && g->n_upper == 0 && g->part && n_parts >= 1 && n_parts <= PART_MAX;  // (empty: built in LDS)
+  if (in_lds) {
+    // (a graph is launched again over the sites of the launch before: nothing says that the grid is empty then)
+    bool captured;
+    if ((rc = stream_captured(s, &captured))) return rc;
+    in_lds = !captured;
+  }
+  if (in_lds) {
     int32_t *cnt = g->part, *cursor = cnt + PART_MAX * PART_PAD, *base = cursor + PART_MAX * PART_PAD;
     int32_t *part_rows = g->slot_of_point, *state = part_rows + g->scratch_rows, *where = state + g->scratch_rows;
     uint64_t *part_keys = reinterpret_cast<uint64_t *>(where + g->scratch_rows);
@@ -1236,9 +1251,12 @@ __global__ __launch_bounds__(1024) void order_group_kernel(OrderBothBatch b) {
   order_append_grouped_body(first, n, j.offset, j.order, j.bo_order, j.bo_pos, sums);
 }
 static int order_launch(const OrderBothBatch &b, int n, int64_t n_upper, hipStream_t s) {
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (n_upper > ORDER_RUN) INSC_HIP(hipStreamIsCapturing(s, &capturing));
-  if (n_upper <= ORDER_RUN || capturing != hipStreamCaptureStatusNone) {  // (a captured call takes no memory)
+  bool captured = false;
+  if (n_upper > ORDER_RUN) {
+    const int rc = stream_captured(s, &captured);
+    if (rc) return rc;
+  }
+  if (n_upper <= ORDER_RUN || captured) {  // (a captured call takes no memory)
     hipLaunchKernelGGL(order_append_both_batch_kernel, dim3((unsigned)n), dim3(1024), 0, s, b);
     INSC_LAUNCH_CHECK();
     return INSC_OK;

@@ -72,3 +72,37 @@ def test_inserts_around_what_one_workgroup_ranks(orc, P):
     sop, osc, _ = orc.grid_build(pts)
     assert (sc.coords_view().cpu().numpy() == osc).all()
     assert (both.cpu().numpy() == sop[P:]).all()
+
+
+@pytest.mark.parametrize("P", [4000, 5000, 16384, 30000])
+@pytest.mark.parametrize("cleared", [False, True])
+def test_captured_inserts_meet_the_sites_of_the_launch_before(orc, P, cleared):
+    """An insert captured while the grid was empty: launched again, it finds its own sites (unless the graph clears them)."""
+    from sparseconvnet import SCN as S
+    from sparseconvnet._lib import lib, ptr, stream_ptr
+
+    rng = np.random.default_rng(P)
+    side = int(P ** (1 / 3)) + 1
+    pts = np.concatenate([rng.integers(0, side, (P, 3)), np.zeros((P, 1), np.int64)], 1).astype(np.int32)
+    m, sc = metadata(pts[::-1], 2 * P)  # (scratch memory for P rows)
+    want, osc, _ = orc.grid_build(pts)
+    c = torch.from_numpy(pts).cuda()
+    sop = torch.empty(P, dtype=torch.int32, device="cuda")
+    n = I64(0)
+    clear = lambda: lib.insc_grid_clear(sc.grid, stream_ptr())
+    clear()
+    lib.insc_grid_size(sc.grid, ctypes.byref(n), stream_ptr())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if cleared:
+            clear()
+        lib.insc_grid_insert(sc.grid, ptr(c), I64(P), ptr(sop), None, stream_ptr())
+    for _ in range(3):
+        sop.fill_(-5)
+        graph.replay()
+        torch.cuda.synchronize()
+        count = S._from_ptr(lib.insc_grid_count_ptr(sc.grid), (1,), torch.int32, torch.device("cuda:0"))
+        coords = S._from_ptr(lib.insc_grid_coords(sc.grid), (len(osc), 4), torch.int32, torch.device("cuda:0"))
+        assert int(count[0]) == len(osc)
+        assert (sop.cpu().numpy() == want).all() and (coords.cpu().numpy() == osc).all()
