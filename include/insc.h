@@ -261,10 +261,10 @@ int insc_bn_leaky(const float *d_in, int64_t ld_in, float *d_out, int64_t ld_out
 /* out = a + b on the listed rows (AddTable, sparseconvnet/tables.py:28-40). */
 int insc_add(const float *d_a, int64_t ld_a, const float *d_b, int64_t ld_b, float *d_out, int64_t ld_out,
              const int32_t *d_rows, const int32_t *d_n_rows, int64_t n_rows, int C, void *stream);
-/* Coordinate rows as callers hold them - [P, cols] integers of 32 or 64 bits, cols 3 (batch 0) or 4, row stride ld - as the
- * (x, y, z, batch) quadruples that the grid calls take (d_out4, 16-byte aligned); 64-bit values that 32 bits do not
- * hold become others that are out of range.  bad (nullable, device-writable): set to 1 if a coordinate lies outside 0..65535 or a
- * batch index outside 0..32767, whatever its width, else left alone. */
+/* Coordinate rows as callers hold them - [P, cols] integers of 32 or 64 bits, or floats that hold integers (bits -32), cols 3
+ * (batch 0) or 4, row stride ld - as the (x, y, z, batch) quadruples that the grid calls take (d_out4, 16-byte aligned); values
+ * that 32 bits do not hold become others that are out of range.  bad (nullable, device-writable): set to 1 if a coordinate lies
+ * outside 0..65535 or a batch index outside 0..32767, whatever its width, else left alone. */
 int insc_coords4(const void *d_coords, int bits, int cols, int64_t ld, int64_t P, int32_t *d_out4, int32_t *bad, void *stream);
 /* out[r, :] = in[r, :] on the listed rows (column-slice copy used for JoinTable,
  * sparseconvnet/tables.py:13-25). */

@@ -325,7 +325,11 @@ int launch_input_finish(const float *d_sum, const int32_t *d_cnt, int mode, floa
 __device__ __forceinline__ int narrowed(int64_t x) {
   return (int)(x < INT32_MIN ? (int64_t)INT32_MIN + 1 : x > INT32_MAX ? (int64_t)INT32_MAX : x);
 }
-// Coordinate rows of three or four columns, 32 or 64 bits wide, as (x, y, z, batch) in 32 bits;
+__device__ __forceinline__ int narrowed(int x) { return x; }
+__device__ __forceinline__ int narrowed(float x) {  // (floats hold every coordinate that is in range)
+  return x <= -2147483648.0f ? INT32_MIN + 1 : x >= 2147483648.0f ? INT32_MAX : (int)x;
+}
+// Coordinate rows of three or four columns, integers of 32 or 64 bits or floats, as (x, y, z, batch) in 32 bits;
 // *bad = 1 where one lies outside 0 .. 65535 (batch 0 .. 32767).  Bound by the rows' bytes: 28 to 48 a point.
 template <class T>
 __global__ __launch_bounds__(256) void coords4_kernel(const T *__restrict__ in, int cols, int64_t ld, int64_t P,
@@ -362,8 +366,8 @@ int insc_add(const float *d_a, int64_t ld_a, const float *d_b, int64_t ld_b, flo
 }
 
 int insc_coords4(const void *d_coords, int bits, int cols, int64_t ld, int64_t P, int32_t *d_out4, int32_t *bad, void *stream) {
-  INSC_REQUIRE((bits == 32 || bits == 64) && (cols == 3 || cols == 4) && ld >= cols && P >= 0, INSC_ERR_ARG,
-               "insc_coords4: rows of 3 or 4 integers of 32 or 64 bits");
+  INSC_REQUIRE((bits == 32 || bits == 64 || bits == -32) && (cols == 3 || cols == 4) && ld >= cols && P >= 0, INSC_ERR_ARG,
+               "insc_coords4: rows of 3 or 4 integers of 32 or 64 bits or floats");
   INSC_REQUIRE(P == 0 || (d_coords && d_out4 && ((uintptr_t)d_out4 & 15) == 0), INSC_ERR_ARG,
                "insc_coords4: null pointer, or output rows that are not 16-byte aligned");
   if (P == 0) return INSC_OK;
@@ -371,6 +375,9 @@ int insc_coords4(const void *d_coords, int bits, int cols, int64_t ld, int64_t P
   if (bits == 64)
     hipLaunchKernelGGL(coords4_kernel<int64_t>, dim3(grid_for(P, 256)), dim3(256), 0, s, (const int64_t *)d_coords, cols, ld, P,
                        d_out4, bad);
+  else if (bits == -32)
+    hipLaunchKernelGGL(coords4_kernel<float>, dim3(grid_for(P, 256)), dim3(256), 0, s, (const float *)d_coords, cols, ld, P, d_out4,
+                       bad);
   else
     hipLaunchKernelGGL(coords4_kernel<int32_t>, dim3(grid_for(P, 256)), dim3(256), 0, s, (const int32_t *)d_coords, cols, ld, P,
                        d_out4, bad);

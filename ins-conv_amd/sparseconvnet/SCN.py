@@ -335,22 +335,17 @@ class Metadata_3(object):
 # helpers shared by the op functions
 # =========================================================================================
 def to_device(coords, device):
-    """Integer coordinates on the device: those of the host narrowed to 32 bits on the way into page-locked memory, from
-    where the copy runs at the link's rate (220k points: 160 us as they are, 75 so).  Values that 32 bits do not hold stay
-    out of range, as in insc_coords4; the host looks for them while the copy runs."""
+    """Coordinates on the device, those of the host in 32 bits and by way of page-locked memory, from where the copy runs at
+    the link's rate (220k points: 160 us as they are, 75 so).  64-bit integers travel as floats, which hold every coordinate
+    that is in range and leave the others out of it; their low 32 bits need not.  (A conversion to integers and a second pass
+    of the host that looks for them: the slowest passes of a scanning session took 25-30 ms, 16-19 so, 14 in the median.)"""
     if coords.is_cuda or not coords.numel():
         return coords.to(device)
+    staged = torch.empty(coords.shape, dtype=torch.float32 if coords.dtype == torch.int64 else torch.int32, pin_memory=True)
+    return staged.copy_(coords).to(device, non_blocking=True)
 
-    def stage(c):
-        staged = torch.empty(c.shape, dtype=torch.int32, pin_memory=True)
-        return staged.copy_(c).to(device, non_blocking=True)
 
-    out = stage(coords)
-    if coords.dtype == torch.int64:
-        lo, hi = torch.aminmax(coords)
-        if int(lo) < -1 << 31 or int(hi) >= 1 << 31:
-            out = stage(torch.where(coords < -1 << 31, (-1 << 31) + 1, coords.clamp(max=(1 << 31) - 1)))
-    return out
+_COORD_BITS = {torch.int32: 32, torch.int64: 64, torch.float32: -32}
 
 
 def _coords4(coords, device, bad=None):
@@ -359,12 +354,12 @@ def _coords4(coords, device, bad=None):
     if coords.dim() != 2 or coords.size(1) not in (3, 4):
         raise ValueError("coords must be [P,3] or [P,4]")
     c = to_device(coords, device)
-    if c.dtype not in (torch.int32, torch.int64):
+    if c.dtype not in _COORD_BITS:
         c = c.to(torch.int32)
     if c.stride(1) != 1 or c.stride(0) < c.size(1):
         c = c.contiguous()
     out = torch.empty((c.size(0), 4), dtype=torch.int32, device=c.device)
-    lib.insc_coords4(ptr(c), 64 if c.dtype == torch.int64 else 32, c.size(1), max(c.stride(0), c.size(1)), c.size(0), ptr(out),
+    lib.insc_coords4(ptr(c), _COORD_BITS[c.dtype], c.size(1), max(c.stride(0), c.size(1)), c.size(0), ptr(out),
                      ptr(bad), stream_ptr())
     return out
 

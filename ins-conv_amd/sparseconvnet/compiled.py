@@ -181,7 +181,7 @@ class CompiledNet(object):
         the side where they are, so that the host-to-device copy carries half the bytes.  Values
         that 32 bits do not hold stay out of range."""
         c = SCN.to_device(coords, self.device)
-        if c.dtype == torch.int64 and c.dim() == 2 and c.size(1) in (3, 4):
+        if c.dtype != torch.int32 and c.dim() == 2 and c.size(1) in (3, 4):
             c = SCN._coords4(c, self.device)
         return c.to(torch.int32).contiguous()
 

@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("cuda", [False, True])
-@pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.int16, torch.float64])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.int16, torch.float64, torch.float32])
 def test_coordinate_rows(dtype, cuda):
     from sparseconvnet import SCN as S
     from sparseconvnet._lib import ensure_init
