@@ -75,15 +75,88 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(const float *__restri
 // and input values of a batch of rows are fetched once per block, one (row, offset) per thread, and read
 // back from LDS by the threads of the row (one 16-byte broadcast read per offset): with every thread
 // fetching its row's 27 ids and 81 values itself the kernel was bound by the number of load instructions
-// (92 us for 150k rows and 32 output channels).
-// A batch's values are two trips to memory away (three with a row list): they are asked for while the batch before is computed,
-// its ids one batch earlier still, none under a condition.  Whether a neighbour exists rides in the fourth word where the
-// input leaves it free.  (Fetched batch by batch, a word of its own in LDS: 150k rows of 3 -> 32 channels 58.8 us, 42.5 so.)
-// Four wavefronts a SIMD with one pair a thread; with two pairs 128 registers would spill.
+// (92 us for 150k rows and 32 output channels).  With three channels the fourth word of the values says whether the
+// neighbour exists (a word of its own in LDS: 150k rows of 3 -> 16 channels 38 us, 34 so; with one channel nothing is gained).
 // ---------------------------------------------------------------------------------------
 constexpr int STEM_ROWS = 16;  // rows per batch at most (those of 256 / Cout rows that a block handles at a time)
+template <int CIN>
+__global__ __launch_bounds__(256) void conv_stem_kernel(const float *__restrict__ in, int64_t ld_in,
+                                                        float *__restrict__ out, int64_t ld_out,
+                                                        const float *__restrict__ W, const float *__restrict__ bias,
+                                                        const int32_t *__restrict__ map0,
+                                                        const int32_t *__restrict__ rows,
+                                                        const int32_t *__restrict__ d_n_rows, int64_t n_rows,
+                                                        int Cout, const uint8_t *__restrict__ row_mask,
+                                                        BnEpilogue ep) {
+  constexpr int K = 27;
+  __shared__ float4 xs[2][STEM_ROWS][K];  // input values of (row, offset); two batches in turn
+  constexpr bool FLAG = CIN == 3;         // whether a neighbour exists rides in the free fourth word
+  __shared__ int vs[FLAG ? 1 : 2][FLAG ? 1 : STEM_ROWS][K];  // 1: the row has a neighbour at the offset
+  __shared__ int rid[2][STEM_ROWS];       // row of the batch, -1: none
+  const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
+  const int cpb = min(256 / Cout, STEM_ROWS);  // rows per batch (Cout <= 256)
+  const int lr = threadIdx.x / Cout, co = threadIdx.x % Cout;
+  const bool worker = lr < cpb;
+  float w[K][CIN];
+#pragma unroll
+  for (int k = 0; k < K; k++)
+#pragma unroll
+    for (int ci = 0; ci < CIN; ci++) w[k][ci] = worker ? W[((int64_t)k * CIN + ci) * Cout + co] : 0.0f;
+  const float bv = (bias && worker) ? bias[co] : 0.0f;
+  const float ew = (ep.out2 && worker) ? ep.w[co] : 0.0f, eb = (ep.out2 && worker) ? ep.b[co] : 0.0f;
+  int buf = 0;
+  for (int64_t t0 = (int64_t)blockIdx.x * cpb; t0 < n; t0 += (int64_t)gridDim.x * cpb, buf ^= 1) {
+    // fetch: one (row, offset) per thread
+    for (int e = threadIdx.x; e < cpb * K; e += 256) {
+      const int er = e / K, k = e - er * K;
+      const int64_t t = t0 + er;
+      int row = t < n ? (rows ? rows[t] : (int)t) : -1;
+      if (row >= 0 && row_mask && !row_mask[row]) row = -1;
+      const int src = row >= 0 ? map0[(int64_t)row * K + k] : -1;
+      float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (src >= 0) {
+        const float *p = in + (int64_t)src * ld_in;
+#pragma unroll
+        for (int ci = 0; ci < CIN; ci++) x[ci] = p[ci];
+      }
+      if constexpr (FLAG) x[3] = src >= 0 ? 1.0f : 0.0f;
+      else vs[buf][er][k] = src >= 0 ? 1 : 0;
+      xs[buf][er][k] = make_float4(x[0], x[1], x[2], x[3]);
+      if (k == 0) rid[buf][er] = row;
+    }
+    __syncthreads();  // (one barrier per batch: the next batch fills the other buffer)
+    const int row = worker ? rid[buf][lr] : -1;
+    if (row < 0) continue;
+    float acc = bv;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const float4 xv = xs[buf][lr][k];
+      const float x[4] = {xv.x, xv.y, xv.z, xv.w};
+      float a = acc;
+#pragma unroll
+      for (int ci = 0; ci < CIN; ci++) a = fmaf(x[ci], w[k][ci], a);
+      bool there;
+      if constexpr (FLAG) there = xv.w != 0.0f;
+      else there = vs[buf][lr][k] != 0;
+      acc = there ? a : acc;
+    }
+    if (ep.res) acc += ep.res[(int64_t)row * ep.ldr + co];
+    if (out) out[(int64_t)row * ld_out + co] = acc;
+    if (ep.out2) {
+      const float y = fmaf(acc, ew, eb);
+      ep.out2[(int64_t)row * ep.ld2 + co] = y * ((y > 0.0f) ? 1.0f : ep.leak);
+    }
+  }
+}
+
+// The same, a batch ahead.  A batch's values are two trips to memory away (three with a row list): they are asked for while the
+// batch before is computed, its ids one batch earlier still, none under a condition.  Whether a neighbour exists rides in the
+// fourth word where the input leaves it free.  (150k rows of 3 -> 32 channels 58.8 us batch by batch, 42.5 so.)  What it costs
+// is a prologue, two batches of loads past the end and, with NE = 2, loads for pairs that a batch does not have; the
+// rule at the launch says where that pays.  Four wavefronts a SIMD with one pair a thread; with two pairs 128 registers would
+// spill.  (One kernel for both forms, its parts in shared lambdas, took 1 us more a launch.)
 template <int CIN, int NE>
-__global__ __launch_bounds__(256, CIN < 4 && NE == 1 ? 4 : 2) void conv_stem_kernel(const float *__restrict__ in, int64_t ld_in,
+__global__ __launch_bounds__(256, CIN < 4 && NE == 1 ? 4 : 2) void conv_stem_ahead_kernel(const float *__restrict__ in, int64_t ld_in,
                                                         float *__restrict__ out, int64_t ld_out,
                                                         const float *__restrict__ W, const float *__restrict__ bias,
                                                         const int32_t *__restrict__ map0,
@@ -2736,17 +2809,31 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     if (mode == MAP_NBR && K == 27 && Cin <= 4) {
       // enough blocks to fill the machine, few enough that the weights are fetched rarely
       const dim3 sg(grid_for(n_rows, std::min(cpb, STEM_ROWS), (unsigned)device_cus() * 8));
-#define INSC_STEM(CI)                                                                                          \
-  hipLaunchKernelGGL((cpb > 9 ? conv_stem_kernel<CI, 2> : conv_stem_kernel<CI, 1>), sg, dim3(256), 0, s, in, ld_in, out, ld_out, W, bias, map0, rows, \
-                     d_n_rows, n_rows, Cout, row_mask, ep)
-      if (Cin == 1)
-        INSC_STEM(1);
-      else if (Cin == 2)
-        INSC_STEM(2);
-      else if (Cin == 3)
-        INSC_STEM(3);
-      else
-        INSC_STEM(4);
+#define INSC_STEM(...)                                                                                         \
+  hipLaunchKernelGGL((__VA_ARGS__), sg, dim3(256), 0, s, in, ld_in, out, ld_out, W, bias, map0, rows, d_n_rows, n_rows, Cout, row_mask, ep)
+      // A batch ahead or batch by batch (same bits).  Up to 256 (row, offset) pairs a batch, one a thread: with three channels
+      // always ahead (3 -> 32, us batch by batch / ahead: 6k rows 6.7 / 6.3, 37k 17.9 / 15.6, 400k 131 / 87); with two or four from
+      // some five batches a block (2 -> 64: 37k rows, four batches, 20.1 / 21.6, 100k, twelve, 52.5 / 47.5; 4 -> 64: 37k 32.0 /
+      // 32.6, 100k 82 / 70); with one, whose batches are short, from twelve (1 -> 32: 100k 20.4 / 20.2, 400k 63.8 / 58.7).
+      // Two pairs a thread: ahead with two channels (2 -> 16: 37k 11.0 / 12.4, 100k 23.1 / 22.7, 400k 80 / 65), else batch by
+      // batch (1 -> 16: 37k 7.7 / 10.3, 400k 45 / 57; 3 -> 16: 37k 12.5 / 16.7, 400k 82 / 87; 4 -> 16: 37k 18.7 / 24.1, 400k 125 / 119).
+      const int batch = std::min(cpb, STEM_ROWS);
+      const int64_t batches = expect_rows / ((int64_t)batch * sg.x);  // of a block
+      const bool two = batch * 27 > 256;
+      if (Cin == 1) {
+        if (!two && batches >= 12) INSC_STEM(conv_stem_ahead_kernel<1, 1>);
+        else INSC_STEM(conv_stem_kernel<1>);
+      } else if (Cin == 2) {
+        if (batches < 5) INSC_STEM(conv_stem_kernel<2>);
+        else if (two) INSC_STEM(conv_stem_ahead_kernel<2, 2>);
+        else INSC_STEM(conv_stem_ahead_kernel<2, 1>);
+      } else if (Cin == 3) {
+        if (!two) INSC_STEM(conv_stem_ahead_kernel<3, 1>);
+        else INSC_STEM(conv_stem_kernel<3>);
+      } else {
+        if (!two && batches >= 5) INSC_STEM(conv_stem_ahead_kernel<4, 1>);
+        else INSC_STEM(conv_stem_kernel<4>);
+      }
 #undef INSC_STEM
       INSC_LAUNCH_CHECK();
       return INSC_OK;

@@ -1,6 +1,6 @@
-"""3^3 layers of one to four input channels: batches of rows are fetched ahead of the one that is computed.  Row counts around
-a batch, widths that take one and two (row, offset) pairs a thread, row lists and an absent neighbour next to weights that are
-not finite, against 64-bit sums."""
+"""3^3 layers of one to four input channels: batches of rows are fetched one by one or ahead of the one that is computed.  Row
+counts around a batch, widths that take one and two (row, offset) pairs a thread, row lists and an absent neighbour next to
+weights that are not finite, against 64-bit sums; and both forms against each other, where a block has many batches."""
 import numpy as np
 import pytest
 import torch
@@ -54,3 +54,35 @@ def test_stem(scene, cin, cout, n_rows):
     assert (got[~fin] == ref[~fin]).all()
     # (one rounding per product-and-add: at most 27 * cin + 1 of half a unit each of a sum no larger than `size`)
     assert (np.abs(got - ref)[fin] <= (27 * cin + 1) * 2.0 ** -24 * size[fin]).all()
+
+
+# each form that runs ahead of its batch: 256 / cout rows a batch (16 at most), 2048 blocks, five or twelve batches each and a bit
+@pytest.mark.parametrize("cin,cout,n", [(1, 256, 24581), (2, 16, 163845), (2, 20, 122885), (2, 128, 20487), (3, 90, 4100),
+                                        (4, 64, 40970)])
+def test_a_batch_ahead_gives_the_same_bits(cin, cout, n):
+    from sparseconvnet.SCN import I64, lib, ptr, stream_ptr
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    nbr = torch.randint(-2 * n, n, (n, 27), generator=g, device="cuda", dtype=torch.int32).clamp_(min=-1)
+    x = torch.randn((n, cin), generator=g, device="cuda")
+    W = torch.randn((27, cin, cout), generator=g, device="cuda")
+    b = torch.randn(cout, generator=g, device="cuda")
+    order = torch.randperm(n, generator=g, device="cuda").to(torch.int32)
+
+    def run(rows):
+        out = torch.full((n, cout), 7.0, device="cuda")
+        for r in rows:
+            lib.insc_conv_nbr(ptr(x), I64(cin), I64(n), ptr(out), I64(cout), ptr(W), None, ptr(b), ptr(nbr), 27, ptr(r), None,
+                              I64(len(r)), cin, cout, None, stream_ptr())
+        return out
+
+    many, few = run([order]), run(order.split(1000))
+    ref, size = b.double().repeat(n, 1), b.double().abs().repeat(n, 1)
+    for k in range(27):
+        at = (nbr[:, k] >= 0).nonzero()[:, 0]
+        xk = x[nbr[at, k].long()].double()
+        ref[at] += xk @ W[k].double()
+        size[at] += xk.abs() @ W[k].double().abs()
+    for got in (many, few):
+        assert bool(((got.double() - ref).abs() <= (27 * cin + 1) * 2.0 ** -24 * size).all())
+    assert torch.equal(many, few)
