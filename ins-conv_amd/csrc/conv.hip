@@ -1038,10 +1038,14 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     }
   }
 
-  // (one wavefront, several partial sums: the running one and the sum of the finished ones)
-  constexpr bool SEQ = S == 1 && K == 27 && MODE == MAP_NBR;
+  // (one wavefront, two partial sums: the running one and the finished one.  With three output blocks a wavefront the finished
+  // one waits in LDS: in registers it goes over the 256 that leave a second wavefront per SIMD, and the 34 that spilled cost
+  // more than the loads here or, without a cap, that wavefront: 48 -> 96 at 150k sites 232, 185 and 155 us, 16 -> 96 112, 91 and 75.
+  // Two and four blocks take the same time either way.)
+  constexpr bool SEQ = S == 1 && K == 27 && MODE == MAP_NBR, HELD = SEQ && NB == 3;
+  __shared__ float held[HELD ? WAVES : 1][HELD ? NB * 16 * 64 : 1];
   Sum sums[NB];
-  f16v total[SEQ ? NB : 1];
+  f16v total[SEQ && !HELD ? NB : 1];
   int cur = 0;  // the partial sum in sums
 #pragma unroll
   for (int b = 0; b < NB; b++) sum_start(sums[b], bias_of[b]);
@@ -1128,7 +1132,10 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
         for (int b = 0; b < NB; b++) {
           const f16v part = sum_of(sums[b]);
 #pragma unroll
-          for (int v = 0; v < 16; v++) total[b][v] = cur == 0 ? part[v] : total[b][v] + part[v];
+          for (int v = 0; v < 16; v++) {
+            if constexpr (HELD) held[wave][(b * 16 + v) * 64 + lane] = part[v];
+            else total[b][v] = part[v];
+          }
           sum_start(sums[b], 0.0f);
         }
         cur = c0.p;
@@ -1169,7 +1176,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
     acc[b] = sum_of(sums[b]);
     if (SEQ && cur != 0) {
 #pragma unroll
-      for (int v = 0; v < 16; v++) acc[b][v] = total[b][v] + acc[b][v];
+      for (int v = 0; v < 16; v++) acc[b][v] = (HELD ? held[wave][(b * 16 + v) * 64 + lane] : total[HELD ? 0 : b][v]) + acc[b][v];
     }
   }
   // (rows whose byte offsets fit 32 bits, through 24-bit multiplies, in every matrix that is written or added)
