@@ -242,14 +242,16 @@ __global__ void grid_assign_kernel(Slot *table, const int32_t *__restrict__ coor
   }
 }
 
-// Passes 2-3 and the counter update in one workgroup, for inserts of up to FINISH_SMALL_MAX rows
-// (an incremental frame): thread t owns a contiguous run of rows, so the ids come out in row
+// Passes 2-3 and the counter update in one workgroup: thread t owns a contiguous run of rows, so the ids come out in row
 // order exactly as from the scan-based passes.  site_of_point holds the rows' states on entry and
-// their sites on exit.
+// their sites on exit.  insc_grid_insert_noalloc, which has no memory for the passes, takes it always, up to FINISH_SMALL_MAX
+// rows; frames at all scales at once (frame_finish_kernel) are ranked by a workgroup a scale up to the same number.
 constexpr int FINISH_SMALL_MAX = 16384;  // (16 rows a thread)
-// A single grid's inserts take it up to 4096 rows: 3.6k rows 13 us, 14k 59 - a thread's rows one after the other, on one
-// compute unit - against 25 in the passes over the whole chip.
-constexpr int INSERT_ONE_MAX = 4096;
+// Other inserts take it up to 7168 rows (seven a thread).  It goes through a thread's rows one after the other on one compute
+// unit, the passes over the whole chip are two or three launches more: 6k rows 18 us against 16, 8k 33 against 19, 16k 64 against 27
+// (kernels), but calls that the host sets the pace of, as two updates and a query of a label table, 4.2k points 125 us against
+// 144, 7k 128 against 147, and 7.4k, by the passes either way, 147.
+constexpr int INSERT_ONE_MAX = 7168;
 __global__ __launch_bounds__(1024) void grid_finish_small_kernel(Slot *table, const int32_t *__restrict__ coords4,
                                                                  const int32_t *__restrict__ slot_of_point, int P,
                                                                  int32_t *d_n, int32_t *__restrict__ site_coords,

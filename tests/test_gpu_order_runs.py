@@ -61,7 +61,7 @@ def test_order_of_short_scales(n, captured):
     assert (got[n_old:] == n_old + np.argsort(key, kind="stable")).all()
 
 
-@pytest.mark.parametrize("P", [4095, 4096, 4097, 16384, 16385])
+@pytest.mark.parametrize("P", [4095, 4096, 4097, 7168, 7169, 16384, 16385])
 def test_inserts_around_what_one_workgroup_ranks(orc, P):
     rng = np.random.default_rng(P)
     pts = np.concatenate([rng.integers(0, 22, (2 * P, 3)), np.zeros((2 * P, 1), np.int64)], 1).astype(np.int32)  # many repeats
