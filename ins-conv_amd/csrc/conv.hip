@@ -549,7 +549,6 @@ __device__ __forceinline__ void mac_chunk(Sum &acc, const Parts (&a)[2], const W
 // and the hardware returns zeros, and the weight tile is addressed by a scalar offset.
 // offsets at or beyond this bound make a buffer load return zeros
 constexpr uint32_t BUF_OOB = 0xFFFFF000u;  // room for the per-load immediate on top
-constexpr uint32_t ROWS_REACH = 0xFFFE0000u;  // row offsets below this leave room for a row's columns
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
@@ -1181,7 +1180,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
   }
   // (rows whose byte offsets fit 32 bits, through 24-bit multiplies, in every matrix that is written or added)
   const int64_t widest = 4 * max(max(ld_out, ep.ld2), max(ep.ldr, ep.ld_side));
-  const bool fits = widest < (1 << 24) && __all(my_row < (1 << 24) && (int64_t)my_row * widest < (int64_t)ROWS_REACH);
+  const bool fits = widest < (1 << 24) && __all(my_row < (1 << 24) && (int64_t)my_row * widest + 4 * (int64_t)Cout <= (int64_t)BUF_OOB);
   if (S == 1) {
     // (one block at a time: copies of all blocks' repeated sums would cost NB = 3 its second wavefront per SIMD, 32 -> 96 at
     // 200k sites 99 -> 124 us)

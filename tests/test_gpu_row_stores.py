@@ -58,3 +58,32 @@ def test_rows_of_any_stride(Cin, Cout, n, up):
     bound = (4 * Cin + 5) * 2.0 ** -23 * size + 1e-30
     assert bool(((got[:, :Cout].double() - want).abs() <= bound)[done].all())
     assert bool((got[:, Cout] == 7.0).all()) and bool((got[~done] == 7.0).all())
+
+
+# a row that begins below the reach of 32-bit offsets and ends beyond it, in one and in four wavefronts a tile
+@pytest.mark.parametrize("Cin", [16, 96])
+def test_a_row_that_crosses_the_reach_of_32_bit_offsets(Cin):
+    from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
+
+    ensure_init(0)
+    Cout, ld, n = 40000, 40004, 26842
+    edge = 26840
+    assert edge * ld * 4 < 0xFFFE0000 and edge * ld * 4 + Cout * 4 > 0xFFFFF000
+    g = torch.Generator(device="cuda").manual_seed(Cin)
+    x = torch.randn((64, Cin), generator=g, device="cuda")
+    W = torch.randn((8, Cin, Cout), generator=g, device="cuda") * (1.0 / Cin) ** 0.5
+    nbr = torch.randint(0, 64, (n, 8), generator=g, device="cuda", dtype=torch.int32)
+    out = torch.full((n, ld), 7.0, device="cuda")
+
+    def run(rows):
+        r = torch.tensor(rows, dtype=torch.int32, device="cuda")
+        lib.insc_conv_nbr(ptr(x), I64(Cin), I64(64), ptr(out), I64(ld), ptr(W), None, None, ptr(nbr), 8, ptr(r), None,
+                          I64(len(rows)), Cin, Cout, None, stream_ptr())
+
+    run([edge, 3])
+    for r in (edge, 3):
+        want, size = (sum(f(x[nbr[r, k].long()].double()) @ f(W[k].double()) for k in range(8)) for f in (lambda t: t, torch.abs))
+        assert bool(((out[r, :Cout].double() - want).abs() <= (4 * Cin + 5) * 2.0 ** -23 * size + 1e-30).all())
+    assert bool((out[:, Cout:] == 7.0).all())
+    out[[edge, 3]] = 7.0
+    assert bool((out == 7.0).all())
