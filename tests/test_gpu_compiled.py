@@ -66,6 +66,32 @@ def test_compiled_full_and_incremental(levels, m, launch_policy):
         assert torch.equal(out, ref)
 
 
+# 3^3 layers in the forms of larger scenes, with the executor's epilogues (residual sum, batch norm into a second matrix) and,
+# in the incremental frame, its dirty-tile flags: a wavefront for both partial sums, two blocks of columns (48 -> 48 at 69k sites:
+# over 8192 wavefronts of one sum and block); three blocks a wavefront (96 -> 96 and 192 -> 96 at 21k: at least 2400 wavefronts
+# remain); two blocks a wavefront with sums that meet across four and across two blocks of wavefronts (192 -> 192 at the scale
+# above, 128 -> 128 at 21k).
+@pytest.mark.parametrize("m,n,new", [(48, 69000, 900), (96, 21000, 700), (128, 21000, 700)])
+def test_epilogues_of_the_forms_of_larger_scenes(m, n, new):
+    import sparseconvnet as scn
+    from workloads import scenes
+    from workloads.netdefs import NaiveUNet
+
+    vox = scenes.boxes_scene(seed=m, n=n + new, grid=256, lo_rng=(8, 200), size_rng=(12, 40))
+    rng = np.random.default_rng(m)
+    rgb = rng.uniform(0, 1, (n + new, 3)).astype(np.float32)
+    model = NaiveUNet(m=m, levels=2, seed=m).cuda()
+    ref_model = copy.deepcopy(model)
+    net = scn.compile(model.sparseModel, capacity_sites=n + new)
+    with torch.no_grad():
+        for f, upto in enumerate((n, n + new)):
+            seen = 0 if f == 0 else n
+            out = net(_inp(vox[seen:upto], rgb[seen:upto]), increment=f > 0, all_points=True)
+            ref = ref_model.sparseModel(_inp(vox[:upto], rgb[:upto]), False)
+            assert out.shape == ref.shape and torch.equal(out, ref)
+        assert net.sites_per_level()[0] == n + new and net.sites_per_level()[1] > 4096
+
+
 def test_compiled_rejects_incremental_without_state():
     import sparseconvnet as scn
     from workloads.netdefs import NaiveUNet
