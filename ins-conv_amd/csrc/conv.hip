@@ -575,7 +575,8 @@ __device__ __forceinline__ Frag gather_chunk(__amdgpu_buffer_rsrc_t rin, bool on
 // 500k sites of 32 channels at 8.5 and 11.1.  (A line a quad reaches 17.0 and 12.3, but its exchange over four lanes takes 32
 // instructions and not 16: 32 -> 32 at 500k sites 104, 99 and 102 us a layer with one, two and four lanes a row.)
 // Kernels whose launches are shorter than a few wavefronts per SIMD wait for their own instructions, not for the address
-// unit, and gather row by row (U-Net on 6k voxels 977 us, two lanes a row 1020).
+// unit, and gather row by row (U-Net on 6k voxels 977 us, two lanes a row 1020).  So do the kernels that split packed fp32 weights
+// as they go, which wait for their vector instructions: 112 -> 112 at 60k sites 230 us two lanes a row, 209 row by row.
 template <int CTRL>
 __device__ __forceinline__ uint32_t lane_perm(uint32_t x) {  // (an operand modifier of the instruction that uses it)
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
@@ -617,6 +618,15 @@ __device__ __forceinline__ Frag own_rows(Frag f) {
   exchange(f.q[0], f.q[1]);
   exchange(f.q[2], f.q[3]);
   return f;
+}
+// either of the two; PAIRS: two lanes a row
+template <bool PAIRS>
+__device__ __forceinline__ Frag gather_rows(__amdgpu_buffer_rsrc_t rin, bool on, uint32_t base, int lane, uint32_t piece, bool full) {
+  return PAIRS ? gather_pairs(rin, on, base, piece, full) : gather_chunk(rin, on, base, lane >> 5, full);
+}
+template <bool PAIRS>
+__device__ __forceinline__ Frag rows_of(const Frag &f) {
+  return PAIRS ? own_rows(f) : f;
 }
 // weight tile `tile` of the filter (on false: zeros)
 template <bool PW>
@@ -772,7 +782,7 @@ __device__ __forceinline__ int pick_offset(unsigned rest, bool centre_first) {
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
 template <int NB, int K, int MODE, int S, bool PW, bool PAIRS>
-__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2 && K == 27) ? 2 : 1) void conv_mfma_kernel(
+__global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, S == 8 && PW ? 4 /* two blocks a compute unit */ : NB == 3 || (NB == 2 && K == 27) ? 2 : 1) void conv_mfma_kernel(
     const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
     const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ map0,
     const int32_t *__restrict__ map1, const int32_t *__restrict__ rows,
@@ -1101,7 +1111,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
       const int src = nl[planned ? kk * TILE_M + r : r * K + kk];
       const bool on = c.k >= 0 && src >= 0, full = Cin - c.ch * 32 >= 32;
       const uint32_t base = (uint32_t)src * ld4 + (uint32_t)(c.ch * 128);
-      return PAIRS ? gather_pairs(rin, on, base, piece, full) : gather_chunk(rin, on, base, h, full);
+      return gather_rows<PAIRS>(rin, on, base, lane, piece, full);
     };
     auto wload = [&](const Cursor &c, int b) -> WFrag<PW> {
       return load_wtile<PW>(rw, ((c.k < 0 ? 0 : c.k) * nch + c.ch) * nbtp + cb0 + b, c.k >= 0, lane16);
@@ -1147,7 +1157,7 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, NB == 3 || (NB == 2
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         if (b == 0) {
-          const Frag a = PAIRS ? own_rows(g[u]) : g[u];
+          const Frag a = rows_of<PAIRS>(g[u]);
           as[0] = split8(a.q[0], a.q[1]);
           as[1] = split8(a.q[2], a.q[3]);
         }
@@ -1655,7 +1665,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
   };
   auto gather = [&](int q, int src, uint32_t base) -> Frag {
     const bool on = q >= 0 && src >= 0 && base != BUF_OOB;  // (a load sent out of range returns 0, which would pass for a site)
-    return gather_pairs(rin, on, (uint32_t)src * ld4, piece, KS == 2);
+    return gather_rows<!PW>(rin, on, (uint32_t)src * ld4, lane, piece, KS == 2);
   };
 
   // Software pipeline over tiles: while tile t is computed, the neighbour ids of the first items of the next
@@ -1739,7 +1749,7 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
       auto compute = [&](auto U) {
         constexpr int u = decltype(U)::value;
         Parts as[2];
-        const Frag a = own_rows(g[u]);
+        const Frag a = rows_of<!PW>(g[u]);
         as[0] = split8(a.q[0], a.q[1]);
         if constexpr (KS == 2) as[1] = split8(a.q[2], a.q[3]);
         mac_chunk(sum, as, bw, KS == 2);
@@ -1984,7 +1994,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
         const int kk = c.k < 0 ? 0 : c.k;
         const int src = nlw[kk * TILE_M + r];
         const bool on = c.k >= 0 && ((mine >> kk) & 1u) && src >= 0;
-        return gather_pairs(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), piece, Cin - c.ch * 32 >= 32);
+        return gather_rows<!PW>(rin, on, (uint32_t)src * ld4 + (uint32_t)(c.ch * 128), lane, piece, Cin - c.ch * 32 >= 32);
       };
       auto compute = [&](const Step &c, const Frag &a, const u32x4 (*wl)[PC * 64]) {
         if (c.k < 0 || !((mine >> c.k) & 1u)) return;  // (the same for every lane of the wavefront)
@@ -1999,7 +2009,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
           }
           cur = c.p;
         }
-        const Frag w = own_rows(a);
+        const Frag w = rows_of<!PW>(a);
         const Parts as[2] = {split8(w.q[0], w.q[1]), split8(w.q[2], w.q[3])};
 #pragma unroll
         for (int o = 0; o < NB; o++) {
@@ -2205,8 +2215,8 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
     auto gather = [&](const Cursor &cu) -> Frag {
       const int kk = cu.k < 0 ? 0 : cu.k;
       const int src = nl[kk * TILE_M + r];
-      return gather_pairs(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), piece,
-                          Cin - cu.ch * 32 >= 32);
+      return gather_rows<!PW>(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), lane, piece,
+                              Cin - cu.ch * 32 >= 32);
     };
     auto wload = [&](const Cursor &cu) -> WFrag<PW> {
       return load_wtile<PW>(rw, ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob, cu.k >= 0, lane16);
@@ -2244,7 +2254,7 @@ __global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(
             sum_start(acc, 0.0f);
             cur = c0.p;
           }
-          const Frag a = own_rows(g[uu]);
+          const Frag a = rows_of<!PW>(g[uu]);
           const Parts as[2] = {split8(a.q[0], a.q[1]), split8(a.q[2], a.q[3])};
           mac_chunk(acc, as, bw[uu], full);
         }
