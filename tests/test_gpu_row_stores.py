@@ -11,9 +11,10 @@ I64 = ctypes.c_int64
 WIDE = (1 << 22) + 8  # floats per row: 16 MiB, more than 24-bit row strides
 
 
-# a tile less a row, one and a row; ragged columns; one to four output blocks a wavefront, a tile over several
+# a tile less a row, one and a row; ragged columns; one to four output blocks a wavefront, a tile over several; columns beyond
+# the 1024 between the offset of a row that does not exist and 4 GB
 @pytest.mark.parametrize("up", [False, True])
-@pytest.mark.parametrize("Cin,Cout,n", [(32, 16, 31), (16, 33, 33), (48, 64, 1), (64, 90, 32), (32, 128, 70), (96, 40, 45), (96, 100, 5000)])
+@pytest.mark.parametrize("Cin,Cout,n", [(32, 16, 31), (16, 33, 33), (48, 64, 1), (64, 90, 32), (32, 128, 70), (96, 40, 45), (96, 100, 5000), (32, 1060, 45), (96, 1060, 45)])
 def test_rows_of_any_stride(Cin, Cout, n, up):
     from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
 
