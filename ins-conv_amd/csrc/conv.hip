@@ -2690,9 +2690,13 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     }
     const bool wide_planned = mode == MAP_NBR && K == 27 && Cin >= 64 && S == 4 && G == 1 && !lat && plan.map && plan.sched &&
                               small_ids;
-    // (a layer with one output block has half the weight bytes per gathered row to share: 64 -> 32 at 150k
-    // sites takes 95 us there against 88 us with a wavefront per unit, so its bound is twice as high)
-    if (wide_planned && (nbt <= 2 || pw) && cdiv(tiles, 4) * nbt >= g_shared_min_units.load(std::memory_order_relaxed) * (nbt == 1 ? 2 : 1)) {
+    // (Twice as high a bound for a layer with one output block, which has half the weight bytes per gathered row to share
+    // (64 -> 32 at 60k sites, shared / split 60 / 39 us, at 100k 70 / 62, at 200k 137 / 137), and for the five or seven blocks that are
+    // taken one a wavefront; not with packed weights.
+    // Kernel times, shared / split: 64 -> 160 at 40k sites (1565 units) 101 / 99 us, 96 -> 160 144 / 138, at 60k (2345) 143 / 145 and
+    // 203 / 209, at 100k 240 / 264 and 350 / 383.)
+    const int64_t shared_min = g_shared_min_units.load(std::memory_order_relaxed) * (nbt == 1 || (nbt > 2 && !pw) ? 2 : 1);
+    if (wide_planned && (NB == 1 || nbt == 2) && cdiv(tiles, 4) * nbt >= shared_min) {
       // blocks of four tiles that share the weight tiles through LDS
       // with enough units left, two output blocks per gathered chunk (eight accumulators: two
       // wavefronts per SIMD instead of three, but a third fewer bytes per MFMA)
