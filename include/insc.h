@@ -227,20 +227,17 @@ int insc_conv_ssc_plan(const float *d_in, int64_t ld_in, int64_t n_in_rows, floa
                        const int32_t *d_plan, int64_t plan_ld, const uint32_t *d_tmask, const int32_t *d_sched,
                        const int32_t *d_order, const int32_t *d_n_rows, int64_t n_rows, int Cin, int Cout,
                        void *stream);
-/* Launch policy of a 3^3 layer of 64..159 input channels with a tile schedule: by default one block per
- * (tile, 32-column output block) pair; with at least `units` (four consecutive tiles, output block) pairs
- * (default 1100, and at most two output blocks) the kernel whose blocks share the weight tiles through LDS.  Same bits in
- * all cases: tuning and test knobs with no counterpart in the reference.  (The persistent-block kernel that the first one chose was slower
- * at every size and is gone; the call is accepted and changes nothing.) */
-int insc_conv_set_persistent_min_units(int64_t units);
+/* Launch policy of a 3^3 layer of 64..159 input channels with a tile schedule: with at least `units` (four consecutive tiles,
+ * 32-column output block) pairs (default 1100 where there are two output blocks, twice that with one or an odd number from five
+ * up) the kernel whose blocks share the weight tiles through LDS; else a workgroup takes a tile and one to three of
+ * its output blocks.  Same bits in all cases: a tuning and test knob with no counterpart in the reference. */
 int insc_conv_set_shared_weights_min_units(int64_t units);
-/* ... and between the two, from `units` (tile, output block) pairs up (default 1750; half as many again
- * for more than 64 input channels), on the kernel that gives every pair a wavefront of its own.  Same
- * bits again. */
+/* Two more bounds, for kernels that were slower at every size and are gone: the calls are accepted and change nothing. */
+int insc_conv_set_persistent_min_units(int64_t units);
 int insc_conv_set_wavefront_per_unit_min_units(int64_t units);
 /* A 3^3 layer with at most 32 input and 32 output channels runs, from `tiles` 32-row tiles up
  * (default 2048, i.e. 65k sites; four times as many without a tile plan), on persistent blocks that keep the whole filter in LDS; below,
- * one wavefront per tile.  Same bits in both cases: a tuning and test knob like the two above. */
+ * one wavefront per tile.  Same bits in both cases: a tuning and test knob like the first above. */
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles);
 /* All of these back to their defaults. */
 int insc_conv_reset_launch_policy(void);

@@ -2109,184 +2109,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB > 1 ? 2 
   }
 }
 
-// ---------------------------------------------------------------------------------------
-// Wide 3^3 layers of middling size (a few hundred to a few thousand tiles): one wavefront per unit
-// (tile, output block), nothing shared between wavefronts - no barrier, no partial sums through LDS,
-// no wait for the slowest of four.  To give the bits of conv_mfma_kernel<1, 27, MAP_NBR, ST> the
-// wavefront forms that kernel's ST partial sums one after the other (as the kernel above).  Units
-// follow the cost-ordered tile schedule, output blocks of a tile side by side on neighbouring SIMDs of
-// one compute unit, so they meet the tile's map slice and gathered rows in L1.
-// What bounds it: 10 KB through L1 per item (4 KB of rows, 6 KB of weights): 64 -> 64 at 39k sites 52 us in fp32, 48 now.
-// ---------------------------------------------------------------------------------------
-// D = items in flight per wavefront (2 with three wavefronts per SIMD; deeper rings at two wavefronts per
-// SIMD measured the same, and so did fewer wavefronts that draw their units from a counter: what the
-// launch lasts is the SIMD with the largest sum of items, hence the fixed assignment below).
-// (two wavefronts per SIMD: at three the sums, parts and weights do not fit the registers - 64 -> 64 at 39k sites
-// 55 us with 30 of them spilled against 47)
-constexpr int OWN_WAVES = 8;  // one block per compute unit
-template <int ST, int D, bool PW>
-__global__ __launch_bounds__(OWN_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_own_kernel(
-    const float *__restrict__ in, int64_t ld_in, float *__restrict__ out, int64_t ld_out,
-    const float *__restrict__ Wp, const float *__restrict__ bias, const int32_t *__restrict__ rows,
-    const int32_t *__restrict__ d_n_rows, int64_t n_rows, int Cin, int Cout, int nbt, int nbtp,
-    const uint8_t *__restrict__ tile_flags, uint32_t in_bytes, uint32_t wp_bytes, BnEpilogue ep, TilePlan plan) {
-  constexpr int K = 27;
-  constexpr int NSTAGE = (TILE_M * K + 63) / 64;
-  __shared__ int nlb[OWN_WAVES][TILE_M * K];
-  const int64_t n = d_n_rows ? min((int64_t)*d_n_rows, n_rows) : n_rows;
-  const int64_t ntiles = (n + TILE_M - 1) / TILE_M, units = ntiles * nbt;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const int r = lane & 31;
-  const int nch = conv_nch(Cin);
-  int *nl = nlb[wave];
-  // (wavefronts are on their own: no workgroup barrier anywhere below)
-  // offsets that hold items of partial sum p
-  unsigned hm[ST];
-#pragma unroll
-  for (int p = 0; p < ST; p++) hm[p] = (unsigned)__ballot(lane < K && ((p - lane * nch) & (ST - 1)) < nch);
-  // One block per compute unit; wavefront w sits on SIMD w % 4, so bin = (block, w % 4) names a SIMD and
-  // turn = w / 4 one of its two wavefronts.  Units come by falling cost: the first turn hands them to the
-  // bins in order, every later turn in reverse order, so the SIMDs that drew the expensive units of the
-  // first turn get the cheap ones afterwards (largest sum of a SIMD at 39k sites and 64 channels: 72 items against
-  // 90 when every SIMD takes three units in a row; 66 is the best any assignment reaches).
-  const int64_t nbins = (int64_t)gridDim.x * 4;
-  const int64_t bin = (int64_t)blockIdx.x * 4 + (wave & 3);
-  for (int64_t rnd = wave >> 2; rnd * nbins < units; rnd += OWN_WAVES / 4) {
-  const int64_t u = rnd * nbins + (rnd == 0 ? bin : nbins - 1 - bin);
-  if (u >= units) continue;
-  const int tile = __builtin_amdgcn_readfirstlane(plan.sched[u / nbt]);
-  const int ob = (int)(u % nbt);
-  if (tile_flags && !tile_flags[tile]) continue;
-  // (the slice of the last unit has been read to the end before this one overwrites it)
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  // the tile's slice of the map: 27 coalesced runs of the plan
-  int st[NSTAGE];
-#pragma unroll
-  for (int i = 0; i < NSTAGE; i++) {
-    const int e = i * 64 + lane;  // e = k * 32 + row
-    st[i] = e < TILE_M * K ? plan.map[(int64_t)(e >> 5) * plan.ld + (int64_t)tile * TILE_M + (e & 31)] : -1;
-  }
-  const int64_t pr = (int64_t)tile * TILE_M + r;
-  const int my_row = pr < n ? (rows ? rows[pr] : (int)pr) : -1;
-  const unsigned tmask = (unsigned)__builtin_amdgcn_readfirstlane((int)plan.tmask[tile]);
-  const int c = ob * 32 + r;
-  const float bv = (bias && c < Cout) ? bias[c] : 0.0f;
-  const float ew = (ep.out2 && c < Cout) ? ep.w[c] : 0.0f;
-  const float eb = (ep.out2 && c < Cout) ? ep.b[c] : 0.0f;
-#pragma unroll
-  for (int i = 0; i < NSTAGE; i++) {
-    const int e = i * 64 + lane;
-    if (e < TILE_M * K) nl[e] = st[i];
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-  // the running partial sum and the sum of the finished ones; bias in partial sum 0
-  Sum acc;
-  sum_start(acc, bv);
-  f16v total;
-  int cur = 0;  // the partial sum in acc
-  if (tmask) {
-    struct Cursor {
-      int k, ch, p;
-      unsigned rest;
-    };
-    auto step = [&](const Cursor &cu) -> Cursor {  // past the end: k = -1
-      Cursor nx = cu;
-      nx.ch = cu.ch + ST;
-      if (nx.ch >= nch || cu.k < 0) {
-#pragma unroll
-        for (int p = 1; p < ST; p++) {
-          if (nx.rest == 0 && nx.p < p) {
-            nx.p = p;
-            nx.rest = tmask & hm[p];
-          }
-        }
-        nx.k = nx.rest ? __builtin_ctz(nx.rest) : -1;
-        nx.ch = (nx.p - nx.k * nch) & (ST - 1);
-        nx.rest &= nx.rest - 1;
-      }
-      return nx;
-    };
-    const __amdgpu_buffer_rsrc_t rin = make_rsrc(in, in_bytes), rw = make_rsrc(Wp, wp_bytes);
-    const uint32_t ld4 = (uint32_t)ld_in * 4u, lane16 = (uint32_t)lane * 16u, piece = pair_piece(lane);
-    auto gather = [&](const Cursor &cu) -> Frag {
-      const int kk = cu.k < 0 ? 0 : cu.k;
-      const int src = nl[kk * TILE_M + r];
-      return gather_rows<!PW>(rin, cu.k >= 0 && src >= 0, (uint32_t)src * ld4 + (uint32_t)(cu.ch * 128), lane, piece,
-                              Cin - cu.ch * 32 >= 32);
-    };
-    auto wload = [&](const Cursor &cu) -> WFrag<PW> {
-      return load_wtile<PW>(rw, ((cu.k < 0 ? 0 : cu.k) * nch + cu.ch) * nbtp + ob, cu.k >= 0, lane16);
-    };
-    const int nitems = __builtin_popcount(tmask) * nch;
-    Cursor first;
-    first.k = -1;
-    first.ch = nch;
-    first.p = 0;
-    first.rest = tmask & hm[0];
-    first = step(first);
-    Frag g[D];
-    WFrag<PW> bw[D];
-    Cursor ci = first, c0 = first;
-#pragma unroll
-    for (int d = 0; d < D - 1; d++) {
-      g[d] = gather(ci);
-      bw[d] = wload(ci);
-      ci = step(ci);
-    }
-    for (int t0i = 0; t0i < nitems; t0i += D) {
-#pragma unroll
-      for (int uu = 0; uu < D; uu++) {
-        g[(uu + D - 1) % D] = gather(ci);
-        bw[(uu + D - 1) % D] = wload(ci);
-        ci = step(ci);
-        const bool full = Cin - c0.ch * 32 >= 32;
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        if (t0i + uu < nitems) {
-          if (c0.p != cur) {
-            const f16v part = sum_of(acc);
-#pragma unroll
-            for (int v = 0; v < 16; v++) total[v] = cur == 0 ? part[v] : total[v] + part[v];
-            sum_start(acc, 0.0f);
-            cur = c0.p;
-          }
-          const Frag a = rows_of<!PW>(g[uu]);
-          const Parts as[2] = {split8(a.q[0], a.q[1]), split8(a.q[2], a.q[3])};
-          mac_chunk(acc, as, bw[uu], full);
-        }
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        c0 = step(c0);
-      }
-    }
-  }
-  // rows and epilogue (D layout of the 32x32 MFMA: lane holds column (lane & 31), rows 8*(v/4) + 4*(lane>>5) + (v&3))
-  const __amdgpu_buffer_rsrc_t rout = make_rsrc(out, out ? BUF_OOB : 0u), rout2 = make_rsrc(ep.out2, ep.out2 ? BUF_OOB : 0u);
-  const __amdgpu_buffer_rsrc_t rres = make_rsrc(ep.res, ep.res ? BUF_OOB : 0u);
-  const uint32_t ldo4 = (uint32_t)ld_out * 4u, ldo24 = (uint32_t)ep.ld2 * 4u, ldr4 = (uint32_t)ep.ldr * 4u;
-  f16v sum = sum_of(acc);
-  if (cur != 0) {
-#pragma unroll
-    for (int v = 0; v < 16; v++) sum[v] = total[v] + sum[v];
-  }
-  unscale<16>(sum);
-  repair_sums<16>(sum, 0, [&]() -> f16v {
-    f16v x;
-#pragma unroll
-    for (int v = 0; v < 16; v++) x[v] = bv;
-    add_plain_products<PW>(x, [&](int k) { return plan.map[(int64_t)k * plan.ld + (int64_t)tile * TILE_M + (lane_again() & 31)]; }, K,
-                       make_rsrc(in, in_bytes), (uint32_t)ld_in * 4u, make_rsrc(Wp, wp_bytes), Cin, nch, nbtp, ob);
-    return x;
-  });
-  store_tile(sum, my_row, ob * 32, c < Cout, rout, ldo4, rout2, ldo24, rres, ldr4, ew, eb, ep.leak, out != nullptr, ep.out2 != nullptr,
-             ep.res != nullptr);
-  }  // units of this wavefront
-}
-
 __global__ void count_rules_kernel(const int32_t *__restrict__ map0, int K, const int32_t *__restrict__ rows,
                                    const int32_t *__restrict__ d_n_rows, int64_t n_rows,
                                    unsigned long long *__restrict__ total) {
@@ -2545,13 +2367,9 @@ int split_weights(const float *W, int K, int Cin, int Cout, float *Ws, hipStream
 // or for two of them, is ahead everywhere: 96 -> 96 at 39k sites 437 / 315, at 333k 2335 / 2133, 112 -> 112 at 60k 714 / 686.
 constexpr int64_t SHARED_MIN_UNITS = 1100;
 static std::atomic<int64_t> g_shared_min_units{SHARED_MIN_UNITS};
-// Below that, where the split kernel has one output block a wavefront: with at least this many (tile, output block) units - half
-// as many again for layers of more than 64 input channels, whose units are longer - the kernel that gives every unit a
-// wavefront of its own (64 -> 32 at 150k sites 75 us against 79 in the split kernel; with fp32 instructions the two met at
-// some 1700 units).
-constexpr int64_t OWN_MIN_UNITS = 1750;
+// (Between the two lay a kernel with a wavefront for every (tile, output block): 64 -> 32 at 60k sites 52 us against 40 in the split
+// kernel, which gathers two lanes a row as well, at 100k 74 / 63, at 200k 131 / 130; 64 -> 160 at 25k 70 / 65.)
 constexpr int64_t NARROW_SPLIT_WAVES = 8192, MANY_BLOCKS_MIN_WAVES = 2400;  // (see the launch shapes below)
-static std::atomic<int64_t> g_own_min_units{OWN_MIN_UNITS};
 // Narrow 3^3 layers (Cin, Cout <= 32) with at least this many 32-row tiles run on the persistent
 // kernel that keeps the whole filter in LDS; smaller ones on the one-wavefront-per-tile kernel.
 // Same bits either way.
@@ -2682,7 +2500,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     }
     // Wide layers: two or three output blocks a wavefront, which gathers and splits a row for all of them, while that
     // leaves MANY_BLOCKS_MIN_WAVES wavefronts.  Kernel times, several / one: 64 -> 64 at 39k sites (4848 wavefronts left) 41 /
-    // 48 us (the wavefront-per-unit kernel), 192 -> 96 at 10k (2528) 49 / 64, 128 -> 64 at 39k (4848) 64 / 73, but
+    // 48 us, 192 -> 96 at 10k (2528) 49 / 64, 128 -> 64 at 39k (4848) 64 / 73, but
     // 96 -> 96 at 10k (1264) 37 / 32 and 128 -> 128 at 2.6k (1296) 22 / 19.
     if (mode == MAP_NBR && K == 27 && !latency && !pw) {
       const int many = S == 4 ? (nbt % 2 == 0 ? 2 : nbt % 3 == 0 ? 3 : 1) : S == 8 && nbt == 3 ? 3 : 1;
@@ -2726,16 +2544,6 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       const unsigned nblk = (unsigned)std::min<int64_t>((int64_t)device_cus() * per_cu2, wunits);
       hipLaunchKernelGGL(kernel, dim3(nblk), dim3(256), 0, s, in, ld_in, out, ld_out, Wp, bias, rows,
                          d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep, plan);
-      INSC_LAUNCH_CHECK();
-      return INSC_OK;
-    }
-    const int64_t own_min = g_own_min_units.load(std::memory_order_relaxed);
-    if (wide_planned && NB == 1 && tiles * nbt >= (Cin > 64 ? own_min + own_min / 2 : own_min)) {
-      // one wavefront per (tile, output block): enough units that every SIMD gets one to three
-      auto kernel = pw ? conv_own_kernel<4, 2, true> : conv_own_kernel<4, 2, false>;
-      hipLaunchKernelGGL(kernel, dim3((unsigned)device_cus()), dim3(OWN_WAVES * 64), 0, s, in, ld_in, out,
-                         ld_out, Wp, bias, rows, d_n_rows, n_rows, Cin, Cout, nbt, nbtp, tile_flags, in_bytes, wp_bytes, ep,
-                         plan);
       INSC_LAUNCH_CHECK();
       return INSC_OK;
     }
@@ -2871,7 +2679,7 @@ using namespace insc;
 
 extern "C" {
 
-// (kept for callers: the kernel that this bound chose was the slower one at every size and is gone)
+// (this and the next but one are kept for callers: the kernels that these bounds chose were the slower ones at every size and are gone)
 int insc_conv_set_persistent_min_units(int64_t units) {
   INSC_REQUIRE(units >= 1, INSC_ERR_ARG, "insc_conv_set_persistent_min_units: units must be >= 1");
   return INSC_OK;
@@ -2885,7 +2693,6 @@ int insc_conv_set_shared_weights_min_units(int64_t units) {
 
 int insc_conv_set_wavefront_per_unit_min_units(int64_t units) {
   INSC_REQUIRE(units >= 1, INSC_ERR_ARG, "insc_conv_set_wavefront_per_unit_min_units: units must be >= 1");
-  g_own_min_units.store(units, std::memory_order_relaxed);
   return INSC_OK;
 }
 
@@ -2897,7 +2704,6 @@ int insc_conv_set_filter_lds_min_tiles(int64_t tiles) {
 
 int insc_conv_reset_launch_policy(void) {
   g_shared_min_units.store(SHARED_MIN_UNITS, std::memory_order_relaxed);
-  g_own_min_units.store(OWN_MIN_UNITS, std::memory_order_relaxed);
   g_wl_min_tiles.store(WL_MIN_TILES, std::memory_order_relaxed);
   return INSC_OK;
 }
