@@ -2479,6 +2479,9 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     const bool narrow = mode == MAP_NBR && K == 27 && !split;  // (two partial sums, whoever forms them)
     if (split) S = K == 27 ? (Cin >= 160 ? 8 : 4) : ((Cin >= 96 || two) ? 4 : 1);  // K == 8: conv and deconv
     int NB = (S == 1 && Cin >= 96) ? 1 : NB0;
+    // (four blocks and two partial sums leave one wavefront a SIMD, two blocks two: 48 -> 128 without a plan at 100k sites 295 / 253 us,
+    // 16 -> 112 140 / 112, with one at 60k 89 / 88 and 48 / 42)
+    if (narrow && NB == 4) NB = 2;
     // (the split across blocks is for scales with few tiles; in a U-Net the width grows with the depth,
     // and a layer that narrows to at most 96 channels sits at a fine scale with many tiles)
     // (eight blocks from 224 -> 192 channels: the two coarsest scales of a seven-scale U-Net, a few tiles,
@@ -2494,7 +2497,9 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
     // for all beyond.  Kernel times, split / not: 32 -> 32 at 6k sites 13 / 20 us, 48 -> 48 at 2k 18 / 41; four layers with
     // batch norms 48 -> 48 at 60k (7504 wavefronts) 247 / 253, 32 -> 32 at 37k 165 / 173.  (Four partial sums for two-chunk
     // layers: U-Net of 16 channels on 6k voxels 648 us and not 690, but 48 -> 48 at 150k 540 and not 424.)
-    if (narrow && !pw && tiles * nbt * 2 <= NARROW_SPLIT_WAVES) {
+    // Without a plan every wavefront stages the map by itself, and more of them than fit the chip at once are slower:
+    // 32 -> 64 at 25k sites (3128) 33 / 29, 32 -> 32 at 60k (3752) 39 / 35, 48 -> 48 91 / 75, but 32 -> 32 at 40k (2500) 27 / 33.
+    if (narrow && !pw && tiles * nbt * 2 <= (plan.map ? NARROW_SPLIT_WAVES : (int64_t)plan.cus * 12)) {
       S = 2;
       NB = 1;
     }
@@ -2574,7 +2579,7 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
 #define INSC_CONV_CASE(NBV)                                      \
   case NBV:                                                      \
     if (mode == MAP_NBR && K == 27)                              \
-      INSC_CONV_LAUNCH(NBV, 27, MAP_NBR, 1);                     \
+      INSC_CONV_LAUNCH((NBV > 3 ? 2 : NBV), 27, MAP_NBR, 1);     \
     else if (mode == MAP_NBR && K == 8)                          \
       INSC_CONV_LAUNCH(NBV, 8, MAP_NBR, 1);                      \
     else if (mode == MAP_PARENT && K == 8)                       \

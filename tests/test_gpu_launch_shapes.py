@@ -49,9 +49,9 @@ def run(m, sc, x, W, Cout, bias, raw=True, plan=True, rows=None):
     return out
 
 
-# one chunk and two, a half chunk, one to three output blocks, a ragged one; the last three: too many tiles for a wavefront per sum
+# one chunk and two, a half chunk, one to three output blocks, a ragged one; the last five: too many tiles for a wavefront per sum
 @pytest.mark.parametrize("Cin,Cout,n", [(16, 16, 700), (32, 32, 5000), (32, 20, 33), (48, 48, 3000), (48, 100, 1900), (16, 72, 31),
-                                        (48, 48, 70000), (16, 96, 45000), (48, 90, 45000)])
+                                        (48, 48, 70000), (16, 96, 45000), (48, 90, 45000), (48, 100, 34000), (32, 130, 28000)])
 def test_narrow_layers(orc, Cin, Cout, n):
     from sparseconvnet._lib import lib
 
