@@ -236,7 +236,8 @@ int insc_conv_set_shared_weights_min_units(int64_t units);
 int insc_conv_set_persistent_min_units(int64_t units);
 int insc_conv_set_wavefront_per_unit_min_units(int64_t units);
 /* A 3^3 layer with at most 32 input and 32 output channels runs, from `tiles` 32-row tiles up
- * (default 2048, i.e. 65k sites; four times as many without a tile plan), on persistent blocks that keep the whole filter in LDS; below,
+ * (default 2048, i.e. 65k sites; three and a half times as many, 229k sites, with more than 16 input channels, weights that are not
+ * packed and a tile plan; four times as many without a plan), on persistent blocks that keep the whole filter in LDS; below,
  * one wavefront per tile.  Same bits in both cases: a tuning and test knob like the first above. */
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles);
 /* All of these back to their defaults. */

@@ -2445,10 +2445,14 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
                            out_rows * ep.ld2 * 4 < (int64_t)BUF_OOB && ep.ldr * 4 < (1 << 24) &&
                            out_rows * ep.ldr * 4 < (int64_t)BUF_OOB;
     // (below some two thousand tiles the persistent kernel's start-up - every block copies the whole filter into LDS -
-    // costs more than it saves: full U-Net forwards of 32 channels, here / per tile, 45k sites 1509 / 1462 us, 100k 1654 / 1669.
-    // Without a plan every tile looks its offsets up first: four times as many.  Both kernels give the same bits.)
+    // costs more than it saves; without a plan every tile looks its offsets up first: four times as many.  Of 32 input
+    // channels, split ahead, the filter takes all of LDS, one block a compute unit, and the bound is three and a half times as high: filter
+    // in LDS / per tile 66k sites 41 / 27 us, 100k 47 / 38, 200k 71 / 69, 300k 108 / 112; 16 -> 32 at 66k 24 / 22, at 100k 28 / 31, 32 -> 32 with
+    // packed weights 35 / 33 and 40 / 40, at 130k 46 / 53.  Both kernels give the same bits.)
+    const int64_t wl_set = g_wl_min_tiles.load(std::memory_order_relaxed);
+    const int64_t wl_min = Cin > 16 && !pw && plan.map ? 1 + (wl_set - 1) * 7 / 2 : wl_set;
     if (mode == MAP_NBR && K == 27 && Cin <= 32 && Cout <= 32 && map_bytes64 < (int64_t)BUF_OOB && small_ids &&
-        cdiv(expect_rows, TILE_M) / (plan.map ? 1 : 4) >= g_wl_min_tiles.load(std::memory_order_relaxed) && !latency) {
+        cdiv(expect_rows, TILE_M) / (plan.map ? 1 : 4) >= wl_min && !latency) {
       const uint32_t map_bytes = (uint32_t)map_bytes64;
       // persistent blocks, a multiple of the XCD count, at most one per compute unit
       const int64_t want = cdiv(tiles, WL_WAVES);

@@ -206,10 +206,10 @@ def test_the_kernels_of_wide_layers_on_tiny_and_ragged_scenes(S, n):
 
 
 @pytest.mark.parametrize("Cin,Cout,n", [(16, 16, 66000), (32, 32, 100000), (32, 20, 131000), (64, 64, 30000), (64, 64, 62000),
-                                        (96, 64, 45000), (64, 150, 57000)])
+                                        (96, 64, 45000), (64, 150, 57000), (32, 32, 235000)])
 def test_the_default_launch_policy_gives_the_bits_of_the_per_tile_kernel(S, Cin, Cout, n):
-    """Sizes at which the policy that ships leaves the kernel of small scenes: the filter in LDS from 65k sites, a wavefront
-    per unit from 28k at 64 channels, shared weights from 57k (two output blocks, and five)."""
+    """Sizes at which the policy that ships leaves the kernel of small scenes: the filter in LDS from 65k sites at 16
+    channels and 229k at 32, shared weights from 57k (two output blocks, and five)."""
     from sparseconvnet._lib import lib
 
     lib.insc_conv_reset_launch_policy()
