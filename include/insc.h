@@ -143,7 +143,9 @@ int insc_rulebook_down2(const insc_grid *fine, insc_grid *coarse, int64_t first,
  * next to each other, so that row tiles of the convolution kernel skip whole filter offsets.
  * Results of the convolution do not depend on it.  No counterpart in the reference (its chunk
  * builder, SubmanifoldRules_cuda.cpp:572-1112, serves the same purpose for its
- * shared-memory kernel). */
+ * shared-memory kernel).  Up to 8192 sites are sorted by merging, in one to three launches, more by radix passes; both take
+ * scratch memory of the stream (up to 1024 sites none), which is allocated when it has to grow.  In a stream that is being captured
+ * up to 8192 sites go to one workgroup, which takes none. */
 int insc_order_build(const insc_grid *g, const int32_t *d_nbr, int64_t first, int64_t n, int32_t *d_order,
                      void *stream);
 
@@ -165,8 +167,9 @@ int insc_order_build_scales(const insc_grid *const *grids, const int32_t *const 
                             int32_t *const *d_bo_order, int32_t *const *d_bo_pos, void *stream);
 
 /* The sites added by the grid's most recent insert - [count before it, count) - appended to the grid's
- * processing order in ONE launch (one workgroup, a radix sort in shared memory): d_order[first..count) =
- * those sites sorted among themselves by the key of insc_order_build (what that call gives for the same
+ * processing order (a merge sort in shared memory, one workgroup and launch for up to 1024 new sites; beyond, a workgroup per 1024,
+ * two launches or three that meet in scratch memory of the stream, allocated when it has to grow - in a stream that is being captured
+ * one workgroup and no scratch): d_order[first..count) = those sites sorted among themselves by the key of insc_order_build (what that call gives for the same
  * range), equal keys in id order;
  * d_pos (nullable) the inverse over the same range.  With d_offset (position inside the parent cell,
  * from insc_rulebook_down2) also d_bo_order / d_bo_pos: the same sites grouped by that position, each

@@ -776,8 +776,9 @@ __device__ __forceinline__ int pick_offset(unsigned rest, bool centre_first) {
 //         out round robin and the partial sums are added in wavefront order at the end.  This is for
 //         the coarse scales of a U-Net, where a layer has a handful of tiles but hundreds of
 //         channels and a single wavefront would run tens of thousands of dependent MFMAs.  Which
-//         terms a wavefront sums depends on k only, so a row's result is a function of S alone
-//         (S is a fixed property of the layer shape), never of the tile it happens to sit in.
+//         terms a wavefront sums depends on k and ch only, never on the tile a row happens to sit in.
+//         How a row's sum is grouped depends on the layer shape alone: S * G partial sums of a wide
+//         layer, two of a narrow one, whether one wavefront forms both (S == 1) or each has its own (S == 2).
 //         With gridDim.z = G > 1 the deal goes over S * G wavefronts in G blocks (different
 //         compute units): a coarse scale has so few tiles that the matrix cores of the few
 //         units holding them would bound the layer.
@@ -1498,8 +1499,8 @@ __global__ __launch_bounds__((S == 1 ? CONV_WAVES : S) * 64, S == 8 && PW ? 4 /*
 // room for a copy, and none is needed: lane r only ever wants the ids of row r).
 // The sums are formed exactly as in conv_mfma_kernel<1, 27, MAP_NBR, 1> (centre, then offsets ascending, same
 // MFMA sequence; the odd offsets' partial sum, with the centre, before the even ones'), so both kernels give the same bits.
-// What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in 103 us a layer (6.2 TB/s; a pure
-// gather reaches 8.7), against 35 us of matrix-core time; 115 us with fp32 instructions, whose 65 us it also waited for.
+// What bounds it: the gather - 500k sites, 32 -> 32: 640 MB of rows through L1 in 94 us a layer (6.8 TB/s; a gather alone, two
+// lanes a row, reaches 11.1), against 35 us of matrix-core time; 103 us with one lane a row, 115 with fp32 instructions.
 // (A contiguous eighth of the tiles per XCD instead of interleaved ones: 531 against 511 us for four layers.)
 // ---------------------------------------------------------------------------------------
 // (32 -> 32 in four layers with their batch norms, 500k / 150k sites: eight wavefronts 542 / 228 us, twelve 538 / 201;
@@ -1833,8 +1834,8 @@ __global__ __launch_bounds__(WL_WAVES * 64) void conv_wlds_kernel(
 // slots are compile-time choices (the step loop is unrolled by three): the compiler then knows that a read of one
 // weight buffer cannot touch a load into another that is still in flight (for a single array it would wait for every
 // outstanding load before each LDS read).
-// What bounds it (64 -> 64 at 500k sites, a launch 414 us in fp32, 342 now; four layers with batch norms 1920 and
-// 1540-1600): 2.2 GB from L2 into L1 per launch at 6.5 TB/s; matrix cores busy 41 %.  Not taken: eight tiles per block,
+// What bounds it (64 -> 64 at 500k sites, a launch 414 us in fp32, 325 now; four layers with batch norms 1920 and
+// 1530): 2.2 GB from L2 into L1 per launch at 6.5 TB/s; matrix cores busy 41 %.  Not taken: eight tiles per block,
 // which halves the weight bytes, 1542 us instead of 1436 (the wavefronts wait for one another); units in site order per
 // XCD, which would hit L2, 1741 instead of 1460 (unbalanced).
 // ---------------------------------------------------------------------------------------
@@ -2465,15 +2466,16 @@ int launch_conv(const float *in, int64_t ld_in, int64_t in_rows, float *out, int
       return INSC_OK;
     }
     const int nbt = (Cout + 31) / 32;
-    // Launch shape, a function of the layer shape only (so results never depend on the scene):
-    //  Cin < 64: each wavefront computes all output blocks of its tile (the gathered rows are
-    //    reused across them);
-    //  wider layers sit at the coarse scales of a U-Net, which have few tiles: one output block
-    //    per wavefront, and for 3^3 / 2^3 maps the items of a tile are dealt to S wavefronts
-    //    (four for 3^3) in each of G blocks.
+    // Launch shape.  How a row's sum is grouped is a function of the layer shape only (so results never depend on the scene);
+    // how many wavefronts and output blocks go with that depends on the size as well.
+    //  Cin < 64: two partial sums (3^3), formed by one wavefront for up to three output blocks of its tile or, in
+    //    small launches, by a wavefront each and per block;
+    //  wider layers sit at the coarse scales of a U-Net, which have few tiles: for 3^3 / 2^3 maps the items of a tile are
+    //    dealt to S wavefronts (four for 3^3) in each of G blocks, with one output block per wavefront or,
+    //    where that leaves enough wavefronts, two or three.
     // latency != 0 (residual frames: a few thousand rows at most, so a launch lasts as long as
     // its most expensive tile): the items of every 3^3 tile are dealt to four wavefronts whatever
-    // the width, and to more blocks for the wide layers.  Also a function of the layer shape only.
+    // the width, and to more blocks for the wide layers.
     const bool lat = latency && mode == MAP_NBR && K == 27 && Cin >= 32;
     const bool two = ep.src2_in != nullptr;  // (checked above: a shape that the split kernel serves)
     const bool split = lat || two || (Cin >= 64 && K > 1 && (mode == MAP_NBR || (mode == MAP_PARENT && Cin >= 96)));

@@ -29,6 +29,7 @@ namespace insc {
 
 // First maximum of a row, as torch.max / torch.argmax.  The scores are asked for twenty at a time, in 16-byte loads where the
 // rows allow it: one by one - a lane per row, a line per lane - 200k rows of 20 classes took 33 us of a frame's update.
+// Two updates with 200k rows, one by one / so: 2 classes 99 / 82 us, 13 109 / 88, 19 119 / 92, 20 120 / 84, 21 123 / 94, 40 173 / 92.
 __device__ __forceinline__ void row_max(const float *__restrict__ x, int C, int &arg, float &val) {
   constexpr int N = 20;
   const bool wide = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
