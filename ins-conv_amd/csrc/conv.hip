@@ -2690,6 +2690,9 @@ using namespace insc;
 
 extern "C" {
 
+// (bounds are held to what the rules can multiply: "never" may be asked for as the largest integer)
+constexpr int64_t BOUND_MAX = int64_t(1) << 48;
+
 // (this and the next but one are kept for callers: the kernels that these bounds chose were the slower ones at every size and are gone)
 int insc_conv_set_persistent_min_units(int64_t units) {
   INSC_REQUIRE(units >= 1, INSC_ERR_ARG, "insc_conv_set_persistent_min_units: units must be >= 1");
@@ -2698,7 +2701,7 @@ int insc_conv_set_persistent_min_units(int64_t units) {
 
 int insc_conv_set_shared_weights_min_units(int64_t units) {
   INSC_REQUIRE(units >= 1, INSC_ERR_ARG, "insc_conv_set_shared_weights_min_units: units must be >= 1");
-  g_shared_min_units.store(units, std::memory_order_relaxed);
+  g_shared_min_units.store(std::min(units, BOUND_MAX), std::memory_order_relaxed);
   return INSC_OK;
 }
 
@@ -2709,7 +2712,7 @@ int insc_conv_set_wavefront_per_unit_min_units(int64_t units) {
 
 int insc_conv_set_filter_lds_min_tiles(int64_t tiles) {
   INSC_REQUIRE(tiles >= 1, INSC_ERR_ARG, "insc_conv_set_filter_lds_min_tiles: tiles must be >= 1");
-  g_wl_min_tiles.store(tiles, std::memory_order_relaxed);
+  g_wl_min_tiles.store(std::min(tiles, BOUND_MAX), std::memory_order_relaxed);
   return INSC_OK;
 }
 
