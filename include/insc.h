@@ -384,7 +384,7 @@ int insc_net_op_count(const insc_net *net);
  * Like that call it forgets the cached state of earlier frames.  No counterpart in the reference, whose modules pass their tensors on every call. */
 int insc_net_rebind_op(insc_net *net, int op, const float *d_W, const float *d_bias, const float *d_mean,
                        const float *d_var, const float *d_gamma, const float *d_beta);
-/* One frame: d_coords int32 [P,coord_cols] (x,y,z[,batch]), d_feats float32 [P,in_channels].
+/* One frame: d_coords int32 [P,coord_cols] (x,y,z[,batch]; coord_cols -3 or -4: rows of 3 or 4 floats that hold integers), d_feats float32 [P,in_channels].
  * increment == 0 forgets all state and runs a full forward; increment != 0 appends the points
  * and recomputes only the rows they affect.  d_out (nullable) receives one row of the output
  * tensor per point of this frame (out_all == 0) or per point since the last full frame.
@@ -406,7 +406,7 @@ int insc_net_dirty_counts(insc_net *net, int max_sets, int *h_n_sets, int *h_lev
 /* One residual frame: the reference's own incremental forward (demo.py:26-38 with
  * increment=True; Incre_* operators, pybind.cpp:218-258) as one call.  The frame's points form a
  * site set of their own, features are differences to the state saved by the last
- * insc_net_forward, and that state is not modified.  d_out (nullable): [P,C], saved value +
+ * insc_net_forward, and that state is not modified.  d_coords, coord_cols: as there.  d_out (nullable): [P,C], saved value +
  * residual for every point of the frame (cuda_Incre_OutputLayer_updateOutput,
  * CUDA/IOLayers.cpp:339-368).  h_n_sites (nullable): sites of the frame at the input scale.
  * Returns once the frame's site counts are known; the layers may still be running on the stream. */

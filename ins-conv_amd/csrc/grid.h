@@ -52,6 +52,15 @@ int grid_wait_made(const insc_grid *g, hipStream_t s);
 // Point coordinate that the insert skips silently (site -1, no error): used to pad a fixed-size
 // launch whose real length is only known on the device.
 constexpr int32_t COORD_SKIP = INT32_MIN;
+// A coordinate that 32 bits do not hold becomes one at their end, which is as far outside every grid: cut to its low bits it
+// would pass for another voxel's.  (Not the very lowest, which is COORD_SKIP.)
+__device__ __forceinline__ int narrowed(int64_t x) {
+  return (int)(x < INT32_MIN ? (int64_t)INT32_MIN + 1 : x > INT32_MAX ? (int64_t)INT32_MAX : x);
+}
+__device__ __forceinline__ int narrowed(int x) { return x; }
+__device__ __forceinline__ int narrowed(float x) {  // (floats hold every coordinate that is in range)
+  return x <= -2147483648.0f ? INT32_MIN + 1 : x >= 2147483648.0f ? INT32_MAX : (int)x;
+}
 
 // Device-side variants used inside a frame: nothing here synchronises with the host.
 // All of them act on the sites added by the grid's most recent insert, [*d_n_prev, *d_n).
@@ -94,7 +103,7 @@ int incre_links_batch(const insc_grid *const *grids, const insc_grid *const *pre
 // (halved) into lv[1].grid and so on, with the parent /
 // offset / child link of every scale to the next coarser one filled in for the new sites.  Every
 // grid then reports the sites of this insert as its newest ([d_n[1], d_n[0])).  d_coords: int32
-// [P, cols] (cols 3 or 4).  If any coordinate is out of range nothing is inserted anywhere, *d_bad
+// [P, cols] (cols 3 or 4; -3 or -4: floats that hold integers).  If any coordinate is out of range nothing is inserted anywhere, *d_bad
 // = frame, and every row of d_sop is -1.  h_counts (nullable, host memory the device can write):
 // receives per scale the site count and error flags, then at [2 * n_levels] `frame` for a dropped frame else 0.
 struct FrameInsertLevel {

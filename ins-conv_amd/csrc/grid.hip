@@ -1383,8 +1383,10 @@ constexpr uint32_t REC_NONE = 0xFFFFFFFFu;  // no slot: bad coordinate, or the t
 __device__ __forceinline__ bool rec_is_slot(uint32_t r) { return r != REC_NONE && !(r & REC_SITE); }
 __device__ __forceinline__ int64_t rec_slot(uint32_t r) { return (int64_t)(r & ~REC_DUP); }
 __device__ __forceinline__ int4 frame_point(const int32_t *__restrict__ coords_in, int cols, int p, int l) {
-  const int32_t *c = coords_in + (int64_t)p * cols;
-  return make_int4(c[0] >> l, c[1] >> l, c[2] >> l, cols > 3 ? c[3] : 0);
+  const int n = abs(cols);
+  const int32_t *c = coords_in + (int64_t)p * n;
+  auto at = [&](int i) -> int { return cols < 0 ? narrowed(__int_as_float(c[i])) : c[i]; };
+  return make_int4(at(0) >> l, at(1) >> l, at(2) >> l, n > 3 ? at(3) : 0);
 }
 // rec[l * P + p]: what row p found at scale l - REC_SITE | id, the slot it claimed first, REC_DUP | the slot
 // another row claimed first, or REC_NONE (protocol: see grid_claim_kernel).  With flag / rep (frames
@@ -1399,8 +1401,8 @@ __global__ __launch_bounds__(256) void frame_claim_kernel(FrameInsertArgs a, con
   const int p = p_begin + blockIdx.x * 256 + threadIdx.x;  // (this launch serves rows p_begin .. p_end - 1)
   if (p >= p_end) return;
   const int64_t idx = (int64_t)l * P + p;
-  const int32_t *c0 = coords_in + (int64_t)p * cols;
-  if (!coord_ok(c0[0], c0[1], c0[2], cols > 3 ? c0[3] : 0)) {
+  int4 c = frame_point(coords_in, cols, p, 0);
+  if (!coord_ok(c.x, c.y, c.z, c.w)) {
     if (l == 0) bad[0] = frame;
     rec[idx] = REC_NONE;
     if (flag) {
@@ -1409,7 +1411,7 @@ __global__ __launch_bounds__(256) void frame_claim_kernel(FrameInsertArgs a, con
     }
     return;
   }
-  const int4 c = frame_point(coords_in, cols, p, l);
+  c = make_int4(c.x >> l, c.y >> l, c.z >> l, c.w);
   const uint64_t key = pack_key(c.x, c.y, c.z, c.w);
   auto claim = [&]() -> uint32_t {
     Walk w = walk_begin(key, L.mask);

@@ -8,6 +8,7 @@
 // batchNormalization.py:60-61, ioLayers.py:69,106-107) and a Metadata object per frame
 // (Metadata/Metadata.h:218-386); here it is one object with an explicit program.
 #include <algorithm>
+#include <cstdlib>
 #include <map>
 #include <set>
 #include <vector>
@@ -1116,7 +1117,7 @@ int insc_net_rebind_op(insc_net *net, int op, const float *d_W, const float *d_b
   return INSC_OK;
 }
 
-/* One frame.  d_coords: int32 [P, coord_cols] (x,y,z[,batch]); d_feats: float32 [P,in_channels].
+/* One frame.  d_coords: int32 [P, coord_cols] (x,y,z[,batch]), or floats (coord_cols -3, -4); d_feats: float32 [P,in_channels].
  * increment == 0: forget all state and run a full forward over these points.
  * increment != 0: append the points to the scene of the previous frames and recompute only
  *                 the rows they affect; the result equals a full forward over all points.
@@ -1130,7 +1131,7 @@ int insc_net_rebind_op(insc_net *net, int op, const float *d_W, const float *d_b
 int insc_net_forward(insc_net *net, const int32_t *d_coords, int coord_cols, const float *d_feats, int64_t P,
                      int increment, float *d_out, int out_all, int64_t *h_n_sites, void *stream) {
   INSC_REQUIRE(net && net->finalized, INSC_ERR_STATE, "insc_net_forward: net is not finalized");
-  INSC_REQUIRE(P >= 0 && (P == 0 || (d_coords && d_feats)) && (coord_cols == 3 || coord_cols == 4), INSC_ERR_ARG,
+  INSC_REQUIRE(P >= 0 && (P == 0 || (d_coords && d_feats)) && (std::abs(coord_cols) == 3 || std::abs(coord_cols) == 4), INSC_ERR_ARG,
                "insc_net_forward: bad arguments");
   INSC_REQUIRE(!increment || net->have_state, INSC_ERR_STATE,
                "insc_net_forward: incremental frame without a full frame before it (none yet, or the weights "
@@ -1627,7 +1628,7 @@ int insc_net_forward_residual(insc_net *net, const int32_t *d_coords, int coord_
   INSC_REQUIRE(net->keep_raw, INSC_ERR_STATE,
                "insc_net_forward_residual: call insc_net_enable_residual before insc_net_finalize");
   INSC_REQUIRE(net->have_state, INSC_ERR_STATE, "insc_net_forward_residual: residual frame before any full frame");
-  INSC_REQUIRE(P >= 0 && (P == 0 || (d_coords && d_feats)) && (coord_cols == 3 || coord_cols == 4), INSC_ERR_ARG,
+  INSC_REQUIRE(P >= 0 && (P == 0 || (d_coords && d_feats)) && (std::abs(coord_cols) == 3 || std::abs(coord_cols) == 4), INSC_ERR_ARG,
                "insc_net_forward_residual: bad arguments");
   if (h_n_sites) *h_n_sites = 0;
   if (P == 0) return INSC_OK;

@@ -320,15 +320,6 @@ int launch_input_finish(const float *d_sum, const int32_t *d_cnt, int mode, floa
   return INSC_OK;
 }
 
-// A coordinate that 32 bits do not hold becomes one at their end, which is as far outside every grid: cut to its low bits it
-// would pass for another voxel's.  (Not the very lowest, which marks rows that an insert skips.)
-__device__ __forceinline__ int narrowed(int64_t x) {
-  return (int)(x < INT32_MIN ? (int64_t)INT32_MIN + 1 : x > INT32_MAX ? (int64_t)INT32_MAX : x);
-}
-__device__ __forceinline__ int narrowed(int x) { return x; }
-__device__ __forceinline__ int narrowed(float x) {  // (floats hold every coordinate that is in range)
-  return x <= -2147483648.0f ? INT32_MIN + 1 : x >= 2147483648.0f ? INT32_MAX : (int)x;
-}
 // Coordinate rows of three or four columns, integers of 32 or 64 bits or floats, as (x, y, z, batch) in 32 bits;
 // *bad = 1 where one lies outside 0 .. 65535 (batch 0 .. 32767).  Bound by the rows' bytes: 28 to 48 a point.
 template <class T>

@@ -176,14 +176,16 @@ class CompiledNet(object):
         self._rebind()
 
     def _coords(self, coords):
-        """int32 on the device.  The reference's callers pass int64 coordinates, on the host
-        (ioLayers.py:52-69 converts to a CPU LongTensor) or on the GPU (demo.py:20): narrowed on
-        the side where they are, so that the host-to-device copy carries half the bytes.  Values
-        that 32 bits do not hold stay out of range."""
+        """On the device, and coord_cols of insc_net_forward.  The reference's callers pass int64 coordinates, on the host
+        (ioLayers.py:52-69 converts to a CPU LongTensor) or on the GPU (demo.py:20): those of
+        the host travel as floats, half the bytes, and the frame's kernels read them so; others
+        are made int32.  Values that 32 bits do not hold stay out of range."""
         c = SCN.to_device(coords, self.device)
+        if c.dtype == torch.float32:
+            return c.contiguous(), -int(c.size(1))
         if c.dtype != torch.int32 and c.dim() == 2 and c.size(1) in (3, 4):
             c = SCN._coords4(c, self.device)
-        return c.to(torch.int32).contiguous()
+        return c.to(torch.int32).contiguous(), int(c.size(1))
 
     def _changed(self):
         """Whether a parameter moved or changed since the weights were packed.  Looked at AFTER a
@@ -205,14 +207,14 @@ class CompiledNet(object):
         increment = bool(increment)
         if all_points is None:
             all_points = (not increment) or self.output_layer.all_points
-        c = self._coords(coords)
+        c, cols = self._coords(coords)
         f = feats.detach().to(device=self.device, dtype=torch.float32).contiguous()
         P = c.size(0)
         rows = (self._n_points if increment else 0) + P if all_points else P
         out = torch.empty((rows, self.out_channels), dtype=torch.float32, device=self.device)
         n = I64(0)
         for attempt in (0, 1):
-            lib.insc_net_forward(self.h, ptr(c), int(c.size(1)), ptr(f), I64(P), int(increment), ptr(out),
+            lib.insc_net_forward(self.h, ptr(c), cols, ptr(f), I64(P), int(increment), ptr(out),
                                  int(bool(all_points)), ctypes.byref(n), stream_ptr())
             if attempt or not self._changed():
                 break
@@ -231,12 +233,12 @@ class CompiledNet(object):
         the frame's points only; the saved state is not touched."""
         if not self.residual:
             raise RuntimeError("compile the model with residual=True to run residual frames")
-        c = self._coords(coords)
+        c, cols = self._coords(coords)
         f = feats.detach().to(device=self.device, dtype=torch.float32).contiguous()
         P = c.size(0)
         out = torch.empty((P, self.out_channels), dtype=torch.float32, device=self.device)
         n = I64(0)
-        lib.insc_net_forward_residual(self.h, ptr(c), int(c.size(1)), ptr(f), I64(P), ptr(out), ctypes.byref(n),
+        lib.insc_net_forward_residual(self.h, ptr(c), cols, ptr(f), I64(P), ptr(out), ctypes.byref(n),
                                       stream_ptr())
         self.n_sites_frame = int(n.value)
         return out

@@ -76,6 +76,29 @@ def test_a_coordinate_beyond_32_bits_is_no_other_voxel(cuda, value):
     assert e.value.code == -5
 
 
+# frames ranked by one workgroup a scale and, beyond 16384 points, by the passes over the chip
+@pytest.mark.parametrize("n,cols", [(300, 3), (2000, 4), (17000, 3), (17000, 4)])
+def test_a_frame_reads_coordinates_of_any_type(n, cols):
+    import sparseconvnet as scn
+    from workloads.netdefs import NaiveUNet
+
+    g = torch.Generator().manual_seed(n + cols)
+    rows = torch.cat([torch.randint(0, 2 * int(n ** (1 / 3)), (n, 3), generator=g) + torch.tensor([0, 65000, 300]),
+                      torch.randint(0, 3, (n, 1), generator=g)], 1)[:, :cols]
+    feats = torch.rand((n, 3), generator=g).cuda()
+    net = scn.compile(NaiveUNet(m=16, levels=3, seed=1).cuda().sparseModel, capacity_sites=2 * n, residual=True)
+    forms = [lambda t: t.cuda().to(torch.int32), lambda t: t, lambda t: t.cuda(), lambda t: t.cuda().float(), lambda t: t.float(),
+             lambda t: t.repeat(1, 2)[:, :cols], lambda t: t.to(torch.int32)]
+    k = n // 3
+    outs = []
+    with torch.no_grad():
+        for form in forms:
+            outs.append([net([form(rows[:n - k]), feats[:n - k], 3], increment=False).clone(),
+                         net([form(rows[n - 2 * k:]), feats[n - 2 * k:], 3], increment="residual").clone(),
+                         net([form(rows[n - k:]), feats[n - k:], 3], increment=True, all_points=True).clone()])
+    assert all(torch.equal(a, b) for o in outs[1:] for a, b in zip(outs[0], o))
+
+
 def test_more_rows_than_threads_in_a_launch():
     from sparseconvnet import SCN as S
     from sparseconvnet._lib import ensure_init, lib, ptr, stream_ptr
